@@ -374,6 +374,32 @@ inline void pack_event_bitmap(hipStream_t stream, const VT *ev, uint32_t n, uint
   hipLaunchKernelGGL(pack_event_bitmap_kernel<VT>, dim3(grid < 2048 ? grid : 2048), dim3(256), 0, stream, ev, n, bits);
 }
 
+// Copies n elements of x to LDS with all threads of the workgroup: 16-byte loads, eight of a lane in flight (a loop of
+// one 4-byte load per thread and turn is a chain of round trips: 35 of them, 25 us, for 138 KB and 1,024 threads).
+// `to` is 16-byte aligned; x may begin at any element.  The caller waits at a barrier.
+template <typename T>
+__device__ __forceinline__ void copy_to_lds(T *to, const T *__restrict__ x, uint32_t n) {
+  constexpr uint32_t kPer = 16 / sizeof(T), kUnroll = 8;
+  typedef T piece __attribute__((ext_vector_type(kPer), aligned(sizeof(T))));
+  typedef T lds_piece __attribute__((ext_vector_type(kPer)));
+  const uint32_t pieces = n / kPer;
+  for (uint32_t i0 = threadIdx.x; i0 < pieces; i0 += kUnroll * blockDim.x) {
+    piece v[kUnroll];
+#pragma unroll
+    for (uint32_t k = 0; k < kUnroll; ++k) {
+      const uint32_t i = i0 + k * blockDim.x;
+      v[k] = reinterpret_cast<const piece *>(x)[i < pieces ? i : pieces - 1u];
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < kUnroll; ++k) {
+      const uint32_t i = i0 + k * blockDim.x;
+      if (i < pieces) reinterpret_cast<lds_piece *>(to)[i] = v[k];
+    }
+  }
+  const uint32_t rest = pieces * kPer + threadIdx.x;
+  if (rest < n) to[rest] = x[rest];
+}
+
 __device__ __forceinline__ void atomic_add(float *p, float v) { unsafeAtomicAdd(p, v); }
 __device__ __forceinline__ void atomic_add(double *p, double v) { unsafeAtomicAdd(p, v); }
 

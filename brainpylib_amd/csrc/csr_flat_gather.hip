@@ -26,60 +26,78 @@
 // range in tail[wave] with the row's number.  A second, small kernel adds tail[w] and the heads of the waves
 // that follow, up to the wave the row ends in, and stores the row.  Both arrays hold one entry per wave of the
 // launch (the nonzero count is known on the device only; the number of waves is the launcher's).
+//
+// OUT: what the walk leaves behind.  kFlatSums: y = A x.  kFlatProducts: products[j] = v[row of j] * x[column of j]
+// for every nonzero j (the gradient of the weights), stored with the quads' own 16-byte width; the rows of the
+// nonzeros are at hand in the window anyway, v's 64 elements of the window lie beside it.  Both at once read the
+// indices and gather x once.  Measured: 1e7 nonzeros, both, x of 30,011 floats in LDS: 32 us, 3.7 TB/s of the 120 MB it
+// must move; 3e7 nonzeros, products alone, x of 120,011 floats: 126 us, bound by the lines that the gathers move out
+// of the L2s (2.7 GB, 54 us without those gathers).  An expanded list of the rows, two gathers and a product as
+// passes of their own took 215 and 850 us.
+// STAGED: one workgroup of 1,024 threads per CU keeps the first elements of x (138 KB) in LDS and gathers only the
+// rest from L2 (flat_stages()).
+#include <type_traits>
+
 #include "common.h"
 #include "csr_flat_gather.h"
 
 namespace bpl {
 namespace {
 
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef double f64x2 __attribute__((ext_vector_type(2)));
+// (aligned to their elements: the arrays may begin anywhere, and a 16-byte load of an address that is not a multiple
+// of 16 costs what it touches)
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef float f32x4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef double f64x2 __attribute__((ext_vector_type(2), aligned(8)));
 
-constexpr int kFlatThreads = 512;
-constexpr int kFlatWaves = kFlatThreads / kWave;
-constexpr unsigned kFlatPerCu = 2;
+enum : int { kFlatSums = 1, kFlatProducts = 2 };
+// 16 waves per CU either way: two workgroups, or one that has the LDS to itself (STAGED)
+constexpr int flat_threads(bool staged) { return staged ? 1024 : 512; }
+constexpr unsigned flat_per_cu(bool staged) { return staged ? 1u : 2u; }
+constexpr uint32_t kFlatStagedBytes = 138u * 1024u;  // (beside it: 16.6 KB of windows and accumulators, 20.7 KB for double)
 constexpr uint32_t kFlatRows = 64;  // rows of an indptr window (one per lane)
 constexpr uint32_t kNoRow = 0xffffffffu;
 
-template <typename F>
+// quads per lane and step, as many as 128 registers hold (with sums and products of floats at once two as well: the
+// elements of x and the weights both live until the rows are known)
+template <typename F, int OUT>
 struct FlatQuads {
-  static constexpr int value = sizeof(F) == 4 ? 4 : 2;  // quads per lane and step (registers)
+  static constexpr int value = sizeof(F) == 4 && OUT != (kFlatSums | kFlatProducts) ? 4 : 2;
 };
 
-// quads a wave owns: the same on the device (both kernels) from the nonzero count and the number of waves
-__device__ __forceinline__ uint32_t flat_quads_per_wave(uint32_t nnz, uint32_t waves, uint32_t step_quads) {
+// Quads a wave owns: the same on the device (both kernels) from the nonzero count and the number of waves, a multiple
+// of `unit`.  Whole wavefronts of quads: with 1e7 nonzeros and 4,096 waves a wave has two and a half steps, and three
+// for each would leave a fifth of the waves without any.  (The plain sums of x in L2 keep whole steps: that walk is at
+// 126 registers, and spills two if its steps may end anywhere.)
+__device__ __forceinline__ uint32_t flat_quads_per_wave(uint32_t nnz, uint32_t waves, uint32_t unit) {
   const uint32_t quads = nnz / 4u + (nnz % 4u ? 1u : 0u);
   const uint32_t per = quads / waves + (quads % waves ? 1u : 0u);
-  return (per + step_quads - 1u) / step_quads * step_quads;
+  return (per + unit - 1u) / unit * unit;
+}
+template <typename F, int OUT, bool STAGED>
+constexpr uint32_t flat_unit() {
+  return (OUT == kFlatSums && !STAGED) ? FlatQuads<F, OUT>::value * kWave : kWave;
 }
 
-// Four consecutive indices / weights, quad q of the array (n elements).  Only the array's last quad can
-// reach beyond its end: that one is read element by element.
-__device__ __forceinline__ u32x4 flat_index_quad(const uint32_t *__restrict__ p, uint32_t q, uint32_t n) {
-  if (4u * q + 4u <= n) return __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(p) + q);
-  u32x4 r = {0u, 0u, 0u, 0u};
-  if (4u * q + 0u < n) r.x = p[4u * q + 0u];
-  if (4u * q + 1u < n) r.y = p[4u * q + 1u];
-  if (4u * q + 2u < n) r.z = p[4u * q + 2u];
-  return r;
+// Four consecutive indices / weights, whole quad q of the array.
+__device__ __forceinline__ u32x4 flat_index_quad(const uint32_t *__restrict__ p, uint32_t q) {
+  return __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(p) + q);
 }
-__device__ __forceinline__ void flat_data_quad(const float *__restrict__ p, uint32_t q, uint32_t n, float (&v)[4]) {
-  if (4u * q + 4u <= n) {
-    const f32x4 t = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(p) + q);
-    v[0] = t.x, v[1] = t.y, v[2] = t.z, v[3] = t.w;
-  } else {
-    for (uint32_t t = 0; t < 4; ++t) v[t] = (4u * q + t < n) ? p[4u * q + t] : 0.f;
-  }
+__device__ __forceinline__ void flat_data_quad(const float *__restrict__ p, uint32_t q, float (&v)[4]) {
+  const f32x4 t = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(p) + q);
+  v[0] = t.x, v[1] = t.y, v[2] = t.z, v[3] = t.w;
 }
-__device__ __forceinline__ void flat_data_quad(const double *__restrict__ p, uint32_t q, uint32_t n, double (&v)[4]) {
-  if (4u * q + 4u <= n) {
-    const f64x2 a = __builtin_nontemporal_load(reinterpret_cast<const f64x2 *>(p) + 2u * q);
-    const f64x2 b = __builtin_nontemporal_load(reinterpret_cast<const f64x2 *>(p) + 2u * q + 1u);
-    v[0] = a.x, v[1] = a.y, v[2] = b.x, v[3] = b.y;
-  } else {
-    for (uint32_t t = 0; t < 4; ++t) v[t] = (4u * q + t < n) ? p[4u * q + t] : 0.;
-  }
+__device__ __forceinline__ void flat_data_quad(const double *__restrict__ p, uint32_t q, double (&v)[4]) {
+  const f64x2 a = __builtin_nontemporal_load(reinterpret_cast<const f64x2 *>(p) + 2u * q);
+  const f64x2 b = __builtin_nontemporal_load(reinterpret_cast<const f64x2 *>(p) + 2u * q + 1u);
+  v[0] = a.x, v[1] = a.y, v[2] = b.x, v[3] = b.y;
+}
+__device__ __forceinline__ void flat_store_quad(float *__restrict__ p, const float (&v)[4]) {
+  __builtin_nontemporal_store(f32x4{v[0], v[1], v[2], v[3]}, reinterpret_cast<f32x4 *>(p));
+}
+__device__ __forceinline__ void flat_store_quad(double *__restrict__ p, const double (&v)[4]) {
+  __builtin_nontemporal_store(f64x2{v[0], v[1]}, reinterpret_cast<f64x2 *>(p));
+  __builtin_nontemporal_store(f64x2{v[2], v[3]}, reinterpret_cast<f64x2 *>(p) + 1);
 }
 
 // The last row r in [0, n_row) with indptr[r] <= pos, for pos < indptr[n_row]: the wave searches together,
@@ -99,35 +117,53 @@ __device__ __forceinline__ uint32_t flat_row_of(const uint32_t *__restrict__ ind
   return lo;
 }
 
-template <typename F, bool HETER>
-__global__ __launch_bounds__(kFlatThreads, 4) void csr_flat_gather_kernel(
+template <typename F, bool HETER, int OUT, bool STAGED>
+__global__ __launch_bounds__(flat_threads(STAGED), 4) void csr_flat_gather_kernel(
     const F *__restrict__ data, const uint32_t *__restrict__ indices, const uint32_t *__restrict__ indptr,
-    const F *__restrict__ x, F *__restrict__ y, uint32_t n_row, uint32_t min_mean, uint32_t max_mean,
-    double *__restrict__ head, double *__restrict__ tail, uint32_t *__restrict__ tail_row) {
-  constexpr int U = FlatQuads<F>::value;
+    const F *__restrict__ x, F *__restrict__ y, uint32_t n_row, uint32_t n_col, uint32_t min_mean,
+    double *__restrict__ head, double *__restrict__ tail, uint32_t *__restrict__ tail_row, const F *__restrict__ v,
+    F *__restrict__ products) {
+  constexpr int U = FlatQuads<F, OUT>::value;
   constexpr uint32_t kStepQuads = U * kWave;
+  constexpr int kFlatWaves = flat_threads(STAGED) / kWave;
+  constexpr bool kSums = (OUT & kFlatSums) != 0, kProducts = (OUT & kFlatProducts) != 0;
+  constexpr bool kWeights = kSums && HETER;  // (the products of v and x alone do not need them)
+  extern __shared__ __attribute__((aligned(16))) unsigned char s_staged[];
   __shared__ uint32_t s_ptr_all[kFlatWaves][kFlatRows + 2];  // (entry 65: a sentinel)
-  __shared__ double s_sum_all[kFlatWaves][kFlatRows];
+  __shared__ double s_sum_all[kSums ? kFlatWaves : 1][kFlatRows];
+  __shared__ F s_v_all[kProducts ? kFlatWaves : 1][kFlatRows + 1];  // v of the window's rows (entry 64: never used)
   const uint32_t nnz = indptr[n_row];
   const uint32_t mean = nnz / n_row;
-  if (mean < min_mean || mean >= max_mean || nnz > kFlatMaxNnz) return;  // (the launcher's other kernel takes those matrices)
+  if (mean < min_mean || nnz > kFlatMaxNnz) return;  // (the launcher's other kernel takes those matrices)
+  if (kSums && nnz == 0) {
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n_row; i += gridDim.x * blockDim.x) y[i] = F(0);
+  }
   const uint32_t lane = static_cast<uint32_t>(lane_id()), wv = threadIdx.x / kWave;
   uint32_t *s_ptr = s_ptr_all[wv];
-  double *s_sum = s_sum_all[wv];
+  double *s_sum = s_sum_all[kSums ? wv : 0];
+  F *s_v = s_v_all[kProducts ? wv : 0];
+  F *s_x = reinterpret_cast<F *>(s_staged);
+  uint32_t staged = 0;
+  if constexpr (STAGED) {
+    constexpr uint32_t kFits = kFlatStagedBytes / sizeof(F);
+    staged = n_col < kFits ? n_col : kFits;
+    copy_to_lds(s_x, x, staged);
+    __syncthreads();
+  }
   const uint32_t waves = gridDim.x * kFlatWaves, w = blockIdx.x * kFlatWaves + wv;
-  const uint32_t per = flat_quads_per_wave(nnz, waves, kStepQuads);
-  if (lane == 0) head[w] = 0.0, tail[w] = 0.0, tail_row[w] = kNoRow;
+  const uint32_t per = flat_quads_per_wave(nnz, waves, flat_unit<F, OUT, STAGED>());
+  if (kSums && lane == 0) head[w] = 0.0, tail[w] = 0.0, tail_row[w] = kNoRow;
   const uint64_t first_quad = static_cast<uint64_t>(w) * per;
   if (4u * first_quad >= nnz) return;
   const uint32_t begin = static_cast<uint32_t>(4u * first_quad);  // the wave owns the nonzeros [begin, end)
   const uint32_t end = (4u * (first_quad + per) < nnz) ? static_cast<uint32_t>(4u * (first_quad + per)) : nnz;
-  const F w_homo = HETER ? F(0) : data[0];
+  const F w_homo = (HETER || !kSums) ? F(0) : data[0];
 
   // Invariant at the start of a step [s0, s1): r is the row that holds nonzero s0 or begins there (rows that
   // end at s0 or before are stored or left to the wave before); s_sum[0] holds what row r has gathered in
   // this wave so far, s_sum[1..63] are zero.  Wave 0 begins at row 0, so that leading empty rows are stored.
   uint32_t r = (w == 0) ? 0u : flat_row_of(indptr, n_row, begin, lane);
-  s_sum[lane] = 0.0;
+  if (kSums) s_sum[lane] = 0.0;
   if (lane == 0) s_ptr[kFlatRows + 1] = 0xffffffffu;
 
   // Two steps are under way at a time: the index and weight streams of step i + 1 are requested before the
@@ -135,59 +171,112 @@ __global__ __launch_bounds__(kFlatThreads, 4) void csr_flat_gather_kernel(
   // requested first of all: waiting for a load means waiting for every load issued before it.  (Keeping the
   // next step's gathers in flight as well needs more registers than two workgroups per CU leave: the
   // compiler spills, and a reloaded register is a load that waits for every gather before it: 750 us.)
+  // The loads carry no condition (a branch per load keeps the compiler from leaving them in flight): a lane beyond
+  // the array's last whole quad reads that one again and its elements are masked by their position, and the one to
+  // three nonzeros behind it are read where they are used.
   constexpr uint32_t kStep = 4u * kStepQuads;
+  const uint32_t whole = nnz / 4u;
   auto load_streams = [&](uint32_t s0, u32x4 (&ci)[U], F (&cd)[U][4]) {  // lane l: quads s0 / 4 + l, + 64, ...
+    if (s0 >= end || whole == 0) return;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const uint32_t q = s0 / 4u + static_cast<uint32_t>(u) * kWave + lane;
-      ci[u] = u32x4{0u, 0u, 0u, 0u};
-      if (s0 < end && 4u * q < end) ci[u] = flat_index_quad(indices, q, nnz);
+      ci[u] = flat_index_quad(indices, q < whole ? q : whole - 1u);
     }
-    if (HETER) {
+    if constexpr (kWeights) {
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const uint32_t q = s0 / 4u + static_cast<uint32_t>(u) * kWave + lane;
-#pragma unroll
-        for (int t = 0; t < 4; ++t) cd[u][t] = F(0);
-        if (s0 < end && 4u * q < end) flat_data_quad(data, q, nnz, cd[u]);
+        flat_data_quad(data, q < whole ? q : whole - 1u, cd[u]);
       }
     }
   };
-  u32x4 ci[U];
-  F cd[U][4];
+  u32x4 ci[U] = {};
+  F cd[U][4] = {};
   load_streams(begin, ci, cd);
   for (uint32_t s0 = begin; s0 < end; s0 += kStep) {
     const uint32_t s1 = (end - s0 > kStep) ? s0 + kStep : end;
     uint32_t ptr_lane, ptr_last;
+    F v_lane = F(0);
     auto load_window = [&]() {
       const uint64_t k = static_cast<uint64_t>(r) + lane;
+      if constexpr (kProducts) v_lane = k < n_row ? v[k] : F(0);
       ptr_lane = k <= n_row ? indptr[k] : 0xffffffffu;
-      ptr_last = static_cast<uint64_t>(r) + kFlatRows <= n_row ? indptr[r + kFlatRows] : 0xffffffffu;  // (one address: a broadcast)
+      ptr_last = static_cast<uint64_t>(r) + kFlatRows <= n_row ? indptr[r + kFlatRows] : 0xffffffffu;
     };
     load_window();
+    if (s1 == nnz && (nnz & 3u) != 0u) {  // (the wave that ends the array: its last one to three nonzeros)
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (s0 / 4u + static_cast<uint32_t>(u) * kWave + lane != whole) continue;
+        const uint32_t p0 = 4u * whole;
+        ci[u] = u32x4{indices[p0], p0 + 1u < nnz ? indices[p0 + 1u] : 0u, p0 + 2u < nnz ? indices[p0 + 2u] : 0u, 0u};
+        if constexpr (kWeights) {
+          cd[u][0] = data[p0];
+          if (p0 + 1u < nnz) cd[u][1] = data[p0 + 1u];
+          if (p0 + 2u < nnz) cd[u][2] = data[p0 + 2u];
+        }
+      }
+    }
     F prod[U][4];  // (the vector's elements first, then the products: in F, as the reference forms them)
+    auto column = [&](int u, int t) {  // (beyond the step: element 0, unused)
+      const uint32_t p = 4u * (s0 / 4u + static_cast<uint32_t>(u) * kWave + lane) + static_cast<uint32_t>(t);
+      return p < s1 ? ci[u][t] : 0u;
+    };
+    if constexpr (STAGED) {
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const uint32_t p0 = 4u * (s0 / 4u + static_cast<uint32_t>(u) * kWave + lane);
-      const uint32_t c[4] = {ci[u].x, ci[u].y, ci[u].z, ci[u].w};
+      for (int u = 0; u < U; ++u) {
 #pragma unroll
-      for (int t = 0; t < 4; ++t) prod[u][t] = x[(p0 + t < s1) ? c[t] : 0u];  // (beyond the step: element 0, unused)
+        for (int t = 0; t < 4; ++t) {
+          const uint32_t c = column(u, t);
+          prod[u][t] = s_x[c < staged ? c : 0u];
+        }
+      }
+      if (staged < n_col) {  // (uniform)
+        // (all LDS reads first: without the empty statements each would be moved into the branch around the load)
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+#pragma unroll
+          for (int t = 0; t < 4; ++t) asm volatile("" : "+v"(prod[u][t]));
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+#pragma unroll
+          for (int t = 0; t < 4; ++t) {
+            const uint32_t c = column(u, t);
+            if (c >= staged) prod[u][t] = x[c];
+          }
+        }
+      }
+    } else {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) prod[u][t] = x[column(u, t)];
+      }
     }
     F cw[U][4];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
 #pragma unroll
-      for (int t = 0; t < 4; ++t) cw[u][t] = HETER ? cd[u][t] : w_homo;
+      for (int t = 0; t < 4; ++t) cw[u][t] = kWeights ? cd[u][t] : w_homo;
     }
     load_streams(s1, ci, cd);  // (a step at or beyond the end of the range loads nothing)
+    if constexpr (!kProducts) {
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
+      for (int u = 0; u < U; ++u) {
 #pragma unroll
-      for (int t = 0; t < 4; ++t) prod[u][t] = static_cast<F>(prod[u][t] * cw[u][t]);
+        for (int t = 0; t < 4; ++t) prod[u][t] = static_cast<F>(prod[u][t] * cw[u][t]);
+      }
     }
+    // (with products the elements of x are kept: this is the addend of the row's sum)
+    auto addend = [&](int u, int t) {
+      return static_cast<double>(kProducts ? static_cast<F>(prod[u][t] * cw[u][t]) : prod[u][t]);
+    };
     // windows of 64 rows from r on, until one reaches beyond the step
     for (;;) {
       s_ptr[lane] = ptr_lane;
+      if constexpr (kProducts) s_v[lane] = v_lane;
       if (lane == 0) s_ptr[kFlatRows] = ptr_last;
       __builtin_amdgcn_wave_barrier();
       const uint32_t lo = s_ptr[0], hi = ptr_last;  // this window takes the nonzeros [lo, hi) of the step
@@ -214,16 +303,33 @@ __global__ __launch_bounds__(kFlatThreads, 4) void csr_flat_gather_kernel(
         const uint32_t top = hi < s1 ? hi : s1;  // the window takes the nonzeros [lo, top)
         if (e2[u] > p0 + 3u || e1[u] >= top) {
           // one row, or two (what lies at e1 or behind belongs to row k + 1, unless that is the next window's)
-          double acc0 = 0.0, acc1 = 0.0;
+          if constexpr (kProducts) {
+            const F v0 = s_v[kq[u]], v1 = s_v[kq[u] + 1u];
+            F g[4];
 #pragma unroll
-          for (int t = 0; t < 4; ++t) {
-            const uint32_t p = p0 + static_cast<uint32_t>(t);
-            const double v = (p >= lo && p < top) ? static_cast<double>(prod[u][t]) : 0.0;
-            acc0 += p < e1[u] ? v : 0.0;
-            acc1 += p < e1[u] ? 0.0 : v;
+            for (int t = 0; t < 4; ++t) g[t] = (p0 + static_cast<uint32_t>(t) < e1[u] ? v0 : v1) * prod[u][t];
+            if (p0 >= lo && p0 + 3u < top) {
+              flat_store_quad(products + p0, g);
+            } else {
+#pragma unroll
+              for (int t = 0; t < 4; ++t) {
+                const uint32_t p = p0 + static_cast<uint32_t>(t);
+                if (p >= lo && p < top) products[p] = g[t];
+              }
+            }
           }
-          if (acc0 != 0.0) atomicAdd(&s_sum[kq[u]], acc0);
-          if (acc1 != 0.0) atomicAdd(&s_sum[kq[u] + 1u], acc1);
+          if constexpr (kSums) {
+            double acc0 = 0.0, acc1 = 0.0;
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+              const uint32_t p = p0 + static_cast<uint32_t>(t);
+              const double a = (p >= lo && p < top) ? addend(u, t) : 0.0;
+              acc0 += p < e1[u] ? a : 0.0;
+              acc1 += p < e1[u] ? 0.0 : a;
+            }
+            if (acc0 != 0.0) atomicAdd(&s_sum[kq[u]], acc0);
+            if (acc1 != 0.0) atomicAdd(&s_sum[kq[u] + 1u], acc1);
+          }
         } else if (p0 < top && p0 + 3u >= lo) {
           uint32_t k = kq[u];
           double acc = 0.0;
@@ -233,14 +339,17 @@ __global__ __launch_bounds__(kFlatThreads, 4) void csr_flat_gather_kernel(
             const uint32_t p = p0 + static_cast<uint32_t>(t);
             if (p >= lo && p < top) {
               while (s_ptr[k + 1u] <= p) ++k;  // (ends below 64: p < hi = s_ptr[64])
-              if (k != kacc) {
-                if (acc != 0.0) atomicAdd(&s_sum[kacc], acc);
-                acc = 0.0, kacc = k;
+              if constexpr (kProducts) products[p] = s_v[k] * prod[u][t];
+              if constexpr (kSums) {
+                if (k != kacc) {
+                  if (acc != 0.0) atomicAdd(&s_sum[kacc], acc);
+                  acc = 0.0, kacc = k;
+                }
+                acc += addend(u, t);
               }
-              acc += static_cast<double>(prod[u][t]);
             }
           }
-          if (acc != 0.0) atomicAdd(&s_sum[kacc], acc);
+          if (kSums && acc != 0.0) atomicAdd(&s_sum[kacc], acc);
         }
       }
       __builtin_amdgcn_wave_barrier();
@@ -249,17 +358,18 @@ __global__ __launch_bounds__(kFlatThreads, 4) void csr_flat_gather_kernel(
       const uint64_t row = static_cast<uint64_t>(r) + lane;
       const bool ended = row < n_row && s_ptr[lane + 1u] <= s1;
       const uint32_t n_ended = static_cast<uint32_t>(__popcll(__ballot(ended)));
-      if (ended) {
+      if (kSums && ended) {
         const double total = s_sum[lane];
         if (w != 0 && ptr_lane < begin) head[w] = total;
         else y[row] = static_cast<F>(total);
       }
-      const double open = n_ended < kFlatRows ? s_sum[n_ended] : 0.0;  // (wave uniform address: a broadcast)
+      double open = 0.0;
+      if constexpr (kSums) open = n_ended < kFlatRows ? s_sum[n_ended] : 0.0;  // (wave uniform address: a broadcast)
       __builtin_amdgcn_wave_barrier();
-      s_sum[lane] = 0.0;
+      if constexpr (kSums) s_sum[lane] = 0.0;
       r += n_ended;
       if (n_ended < kFlatRows || r >= n_row) {
-        if (lane == 0) s_sum[0] = open;
+        if (kSums && lane == 0) s_sum[0] = open;
         break;
       }
       load_window();
@@ -267,7 +377,7 @@ __global__ __launch_bounds__(kFlatThreads, 4) void csr_flat_gather_kernel(
     __builtin_amdgcn_wave_barrier();
   }
   // the row that is still open at the end of the range (if it has nonzeros in it)
-  if (lane == 0 && r < n_row) {
+  if (kSums && lane == 0 && r < n_row) {
     const uint32_t rs = indptr[r];
     if (rs < end) {
       if (w != 0 && rs < begin) head[w] = s_sum[0];
@@ -280,18 +390,17 @@ __global__ __launch_bounds__(kFlatThreads, 4) void csr_flat_gather_kernel(
 // it runs through, in a fixed order.
 template <typename F>
 __global__ __launch_bounds__(kWave) void csr_flat_finish_kernel(const uint32_t *__restrict__ indptr, F *__restrict__ y,
-                                                                uint32_t n_row, uint32_t min_mean, uint32_t max_mean,
+                                                                uint32_t n_row, uint32_t min_mean,
                                                                 uint32_t waves, const double *__restrict__ head,
                                                                 const double *__restrict__ tail,
-                                                                const uint32_t *__restrict__ tail_row) {
-  constexpr uint32_t kStepQuads = FlatQuads<F>::value * kWave;
+                                                                const uint32_t *__restrict__ tail_row, uint32_t unit) {
   const uint32_t nnz = indptr[n_row];
   const uint32_t mean = nnz / n_row;
-  if (mean < min_mean || mean >= max_mean || nnz > kFlatMaxNnz) return;
+  if (mean < min_mean || nnz > kFlatMaxNnz) return;
   const uint32_t w = blockIdx.x, lane = threadIdx.x;
   const uint32_t row = tail_row[w];
   if (row == kNoRow) return;
-  const uint32_t per = flat_quads_per_wave(nnz, waves, kStepQuads);
+  const uint32_t per = flat_quads_per_wave(nnz, waves, unit);
   const uint32_t last = ((indptr[row + 1u] - 1u) / 4u) / per;  // the range the row's last nonzero lies in
   double acc = 0.0;
   for (uint32_t v = w + 1u + lane; v <= last && v < waves; v += kWave) acc += head[v];
@@ -301,35 +410,110 @@ __global__ __launch_bounds__(kWave) void csr_flat_finish_kernel(const uint32_t *
 
 }  // namespace
 
+// Whether the walk keeps the first elements of x in LDS: while at least a quarter of them fit.  What a gather from L2 costs
+// is the 128-byte line it moves (about 29 TB/s from all L2s, 230 G gathers/s): staging takes its share of them away,
+// 120,000 floats and 2e7 nonzeros in rows of 100: 97 us, 155 us gathered from L2 alone.
 template <typename F>
-FlatGather csr_flat_gather(const char *target, hipStream_t stream, const F *data, bool heter, const uint32_t *indices,
-                     const uint32_t *indptr, const F *x, F *y, uint32_t n_row, uint32_t min_mean, uint32_t max_mean) {
-  if (n_row == 0) return FlatGather::kEnqueued;
-  // 16-byte loads of the streams
-  if ((reinterpret_cast<uintptr_t>(indices) & 15u) != 0 || (heter && (reinterpret_cast<uintptr_t>(data) & 15u) != 0))
-    return FlatGather::kNotApplicable;
-  const unsigned grid = static_cast<unsigned>(device_info().num_cu) * kFlatPerCu;
-  const uint32_t waves = grid * kFlatWaves;
-  // [head: waves doubles][tail: waves doubles][tail_row: waves words]
-  unsigned char *ws = static_cast<unsigned char *>(stream_workspace(stream, static_cast<size_t>(waves) * 20u));
-  if (ws == nullptr) return FlatGather::kFailed;
-  double *head = reinterpret_cast<double *>(ws), *tail = head + waves;
-  uint32_t *tail_row = reinterpret_cast<uint32_t *>(tail + waves);
-  if (heter)
-    hipLaunchKernelGGL((csr_flat_gather_kernel<F, true>), dim3(grid), dim3(kFlatThreads), 0, stream, data, indices, indptr,
-                       x, y, n_row, min_mean, max_mean, head, tail, tail_row);
-  else
-    hipLaunchKernelGGL((csr_flat_gather_kernel<F, false>), dim3(grid), dim3(kFlatThreads), 0, stream, data, indices,
-                       indptr, x, y, n_row, min_mean, max_mean, head, tail, tail_row);
-  hipLaunchKernelGGL(csr_flat_finish_kernel<F>, dim3(waves), dim3(kWave), 0, stream, indptr, y, n_row, min_mean, max_mean,
-                     waves, static_cast<const double *>(head), static_cast<const double *>(tail),
-                     static_cast<const uint32_t *>(tail_row));
-  return check_launch(target) ? FlatGather::kEnqueued : FlatGather::kFailed;
+bool flat_stages(uint32_t n_col) {
+  return static_cast<uint64_t>(n_col) * sizeof(F) <= 4ull * kFlatStagedBytes;
 }
 
-template FlatGather csr_flat_gather<float>(const char *, hipStream_t, const float *, bool, const uint32_t *, const uint32_t *,
+template <typename F, bool HETER, int OUT, bool STAGED>
+static bool launch_flat(const char *target, hipStream_t stream, const F *data, const uint32_t *indices,
+                        const uint32_t *indptr, const F *x, F *y, uint32_t n_row, uint32_t n_col, uint32_t min_mean,
+                        const F *v, F *products) {
+  constexpr bool kSums = (OUT & kFlatSums) != 0;
+  const unsigned grid = static_cast<unsigned>(device_info().num_cu) * flat_per_cu(STAGED);
+  const uint32_t waves = grid * (flat_threads(STAGED) / kWave);
+  double *head = nullptr, *tail = nullptr;
+  uint32_t *tail_row = nullptr;
+  if (kSums) {
+    // [head: waves doubles][tail: waves doubles][tail_row: waves words]
+    unsigned char *ws = static_cast<unsigned char *>(stream_workspace(stream, static_cast<size_t>(waves) * 20u));
+    if (ws == nullptr) return false;
+    head = reinterpret_cast<double *>(ws), tail = head + waves;
+    tail_row = reinterpret_cast<uint32_t *>(tail + waves);
+  }
+  auto kernel = csr_flat_gather_kernel<F, HETER, OUT, STAGED>;
+  size_t lds = 0;
+  if (STAGED) {
+    lds = static_cast<size_t>(n_col) * sizeof(F) < kFlatStagedBytes ? static_cast<size_t>(n_col) * sizeof(F) : kFlatStagedBytes;
+    if (hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                            static_cast<int>(kFlatStagedBytes)) != hipSuccess) {
+      (void)hipGetLastError();
+      set_error("%s: the device does not give a workgroup %u bytes of LDS", target, kFlatStagedBytes);
+      return false;
+    }
+  }
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(flat_threads(STAGED)), lds, stream, data, indices, indptr, x, y, n_row,
+                     n_col, min_mean, head, tail, tail_row, v, products);
+  if (kSums)
+    hipLaunchKernelGGL(csr_flat_finish_kernel<F>, dim3(waves), dim3(kWave), 0, stream, indptr, y, n_row, min_mean,
+                       waves, static_cast<const double *>(head), static_cast<const double *>(tail),
+                       static_cast<const uint32_t *>(tail_row), flat_unit<F, OUT, STAGED>());
+  return check_launch(target);
+}
+
+template <typename F>
+bool csr_flat_gather(const char *target, hipStream_t stream, const F *data, bool heter, const uint32_t *indices,
+                     const uint32_t *indptr, const F *x, F *y, uint32_t n_row, uint32_t n_col, uint32_t min_mean) {
+  if (n_row == 0) return true;
+  auto launch = [&](auto h, auto staged) {
+    return launch_flat<F, decltype(h)::value, kFlatSums, decltype(staged)::value>(
+      target, stream, data, indices, indptr, x, y, n_row, n_col, min_mean, nullptr, nullptr);
+  };
+  if (flat_stages<F>(n_col)) return heter ? launch(std::true_type(), std::true_type()) : launch(std::false_type(), std::true_type());
+  return heter ? launch(std::true_type(), std::false_type()) : launch(std::false_type(), std::false_type());
+}
+
+template <typename F>
+bool csr_gradient(const char *target, hipStream_t stream, const F *data, const uint32_t *indices, const uint32_t *indptr,
+                  const F *v, const F *x, F *products, F *sums, uint32_t n_row, uint32_t n_col, uint32_t nnz) {
+  if (n_row == 0) return true;
+  if (nnz > kFlatMaxNnz) {
+    set_error("%s: %u nonzeros are more than the walk's positions can number", target, nnz);
+    return false;
+  }
+  const bool staged = flat_stages<F>(n_col);
+  if (sums != nullptr)
+    return staged ? launch_flat<F, true, kFlatSums | kFlatProducts, true>(target, stream, data, indices, indptr, x, sums, n_row,
+                                                                          n_col, 0u, v, products)
+                  : launch_flat<F, true, kFlatSums | kFlatProducts, false>(target, stream, data, indices, indptr, x, sums,
+                                                                           n_row, n_col, 0u, v, products);
+  return staged ? launch_flat<F, true, kFlatProducts, true>(target, stream, data, indices, indptr, x, sums, n_row, n_col, 0u,
+                                                            v, products)
+                : launch_flat<F, true, kFlatProducts, false>(target, stream, data, indices, indptr, x, sums, n_row, n_col,
+                                                             0u, v, products);
+}
+
+// csr_matvec_gradient: buffers = [data, indices, indptr, row vector, column vector, products, sums (or null)]
+template <typename F>
+static void csr_matvec_gradient_entry(const char *target, hipStream_t stream, void **buffers, const char *opaque,
+                                      size_t opaque_len) {
+  bpl_csr_transpose_descriptor d;
+  if (!unpack(target, opaque, opaque_len, &d)) return;
+  if (buffers == nullptr) {
+    set_error("%s: null buffer table", target);
+    return;
+  }
+  csr_gradient<F>(target, stream, static_cast<const F *>(buffers[0]), static_cast<const uint32_t *>(buffers[1]),
+                  static_cast<const uint32_t *>(buffers[2]), static_cast<const F *>(buffers[3]),
+                  static_cast<const F *>(buffers[4]), static_cast<F *>(buffers[5]), static_cast<F *>(buffers[6]), d.n_row,
+                  d.n_col, d.nnz);
+}
+
+template bool flat_stages<float>(uint32_t);
+template bool flat_stages<double>(uint32_t);
+template bool csr_flat_gather<float>(const char *, hipStream_t, const float *, bool, const uint32_t *, const uint32_t *,
                                      const float *, float *, uint32_t, uint32_t, uint32_t);
-template FlatGather csr_flat_gather<double>(const char *, hipStream_t, const double *, bool, const uint32_t *,
-                                      const uint32_t *, const double *, double *, uint32_t, uint32_t, uint32_t);
+template bool csr_flat_gather<double>(const char *, hipStream_t, const double *, bool, const uint32_t *, const uint32_t *,
+                                      const double *, double *, uint32_t, uint32_t, uint32_t);
 
 }  // namespace bpl
+
+extern "C" void csr_matvec_gradient_float(bpl_stream_t stream, void **buffers, const char *opaque, size_t opaque_len) {
+  bpl::csr_matvec_gradient_entry<float>(__func__, static_cast<hipStream_t>(stream), buffers, opaque, opaque_len);
+}
+extern "C" void csr_matvec_gradient_double(bpl_stream_t stream, void **buffers, const char *opaque, size_t opaque_len) {
+  bpl::csr_matvec_gradient_entry<double>(__func__, static_cast<hipStream_t>(stream), buffers, opaque, opaque_len);
+}

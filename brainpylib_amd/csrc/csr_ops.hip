@@ -651,16 +651,6 @@ __device__ __forceinline__ void event_hits(const uint32_t *s_bits, const VT *__r
   }
 }
 
-// Element `col` of the dense vector.  BITS == 2: its first `lds_n` elements are staged in LDS
-// (`s_x`), the rest is gathered from global memory.
-template <typename VT, int BITS>
-__device__ __forceinline__ VT dense_element(const VT *__restrict__ x, const uint32_t *s_x, uint32_t lds_n, uint32_t col) {
-  if constexpr (BITS == 2) {
-    if (col < lds_n) return reinterpret_cast<const VT *>(s_x)[col];
-  }
-  return x[col];
-}
-
 typedef uint32_t row_u32x4 __attribute__((ext_vector_type(4), aligned(4)));  // (a row begins at any nonzero)
 typedef float row_f32x4 __attribute__((ext_vector_type(4), aligned(4)));
 template <typename F, typename VT, bool HETER, int MODE, int BITS, int G, int U>
@@ -770,7 +760,7 @@ __device__ __forceinline__ void gather_rows(const F *__restrict__ data, const ui
         if constexpr (kWeightRuns) d = wgt[u];
         else if constexpr (HETER) d = data[ok ? j : (end ? end - 1 : 0u)];
         // product formed in F, then widened (the reference multiplies two F values)
-        val[u] = static_cast<F>(static_cast<F>(dense_element<VT, BITS>(x, s_bits, coarse_g, col[u])) * d);
+        val[u] = static_cast<F>(static_cast<F>(x[col[u]]) * d);
       }
     }
     // indices of the next step, and the row bounds one row further ahead
@@ -858,7 +848,7 @@ __device__ __forceinline__ void gather_rows_wave(const F *__restrict__ data, con
         if (ok[u]) {
           const F d = HETER ? stream_load(dp + off) : w_homo;
           // product formed in F, then widened (the reference multiplies two F values)
-          val[u] = static_cast<F>(static_cast<F>(dense_element<VT, BITS>(x, s_bits, coarse_g, col[u])) * d);
+          val[u] = static_cast<F>(static_cast<F>(x[col[u]]) * d);
         }
       }
     }
@@ -964,7 +954,7 @@ __device__ __forceinline__ void gather_hub_rows(const F *__restrict__ data, cons
               }
             } else {
               const F d = HETER ? data[start + j] : w_homo;
-              acc += static_cast<double>(static_cast<F>(static_cast<F>(dense_element<VT, BITS>(x, s_bits, coarse_g, col[u])) * d));
+              acc += static_cast<double>(static_cast<F>(static_cast<F>(x[col[u]]) * d));
             }
           }
 #pragma unroll
@@ -1264,12 +1254,8 @@ __global__ __launch_bounds__(1024, (MODE == kEvent && BITS == 1) ? 8 : 4) void c
   if constexpr (MODE == kDense) {
     // BITS == 1: the dense vector itself is staged in LDS (the host checked that it fits), so the
     // per-nonzero gather is an LDS read instead of an L2 request and the kernel streams at HBM speed
-    // BITS == 2: as much of it as fits; the kernel gathers the rest from L2 as without LDS
-    if constexpr (BITS == 1 || BITS == 2) {
-      VT *s_x = reinterpret_cast<VT *>(s_bits);
-      const uint32_t fits = static_cast<uint32_t>(kLdsBitmapCap / sizeof(VT));
-      coarse_g = n_col < fits ? n_col : fits;  // (the walks take it as the number of staged elements)
-      for (uint32_t i = threadIdx.x; i < coarse_g; i += blockDim.x) s_x[i] = x[i];
+    if constexpr (BITS == 1) {
+      copy_to_lds(reinterpret_cast<VT *>(s_bits), x, n_col);
       __syncthreads();
     }
   } else if constexpr (BITS == 3) {
@@ -1297,10 +1283,6 @@ __global__ __launch_bounds__(1024, (MODE == kEvent && BITS == 1) ? 8 : 4) void c
     // (rows of `skip_mean` nonzeros or more on average: the launcher's other kernel has taken this matrix)
     if (skip_mean != 0 && mean >= skip_mean && nnz <= kFlatMaxNnz) return;
   }
-  if constexpr (MODE == kDense && BITS == 2) {
-    // (rows of 4 nonzeros or more but fewer than `skip_mean` on average: the flat walk has taken this matrix)
-    if (skip_mean != 0 && mean >= 4u && mean < skip_mean && nnz <= kFlatMaxNnz) return;
-  }
   if constexpr (MODE == kDense && BITS == 1) {
     // (nothing left to hide but the index and weight streams: the walks of the event gather)
     const VT *xs = reinterpret_cast<const VT *>(s_bits);
@@ -1308,10 +1290,6 @@ __global__ __launch_bounds__(1024, (MODE == kEvent && BITS == 1) ? 8 : 4) void c
     else if (mean >= 24) { gather_rows<F, VT, HETER, MODE, BITS, 8, 8>(data, indices, indptr, xs, y, n_row, s_bits, coarse_g); gpb = blockDim.x / 8; hub_len = kHubSteps * 8 * 8; }
     else if (mean >= 12) { gather_rows<F, VT, HETER, MODE, BITS, 4, 8>(data, indices, indptr, xs, y, n_row, s_bits, coarse_g); gpb = blockDim.x / 4; hub_len = kHubSteps * 8 * 4; }
     else { gather_rows<F, VT, HETER, MODE, BITS, 4, 4>(data, indices, indptr, xs, y, n_row, s_bits, coarse_g); gpb = blockDim.x / 4; hub_len = kHubSteps * 4 * 4; }
-  } else if constexpr (MODE == kDense && BITS == 2) {
-    if (mean >= 384) { gather_rows_wave<F, VT, HETER, MODE, BITS, 8>(data, indices, indptr, x, y, n_row, s_bits, coarse_g); gpb = 1; hub_len = kHubSteps * 8 * kWave; }
-    else if (mean >= 24) { gather_rows<F, VT, HETER, MODE, BITS, 8, 8>(data, indices, indptr, x, y, n_row, s_bits, coarse_g); gpb = blockDim.x / 8; hub_len = kHubSteps * 8 * 8; }
-    else { gather_rows<F, VT, HETER, MODE, BITS, 4, 8>(data, indices, indptr, x, y, n_row, s_bits, coarse_g); gpb = blockDim.x / 4; hub_len = kHubSteps * 8 * 4; }
   } else if constexpr (MODE == kEvent && (BITS == 2 || BITS == 3)) {
     // An event bitmap above 80 KB leaves room for one workgroup (16 waves) per CU only: every lane
     // then keeps 16 (rows under 48 nonzeros: 8) loads in flight instead of 2 to 8, in groups of
@@ -1739,9 +1717,12 @@ bool launch_gather_impl(const char *target, hipStream_t stream, const F *data, c
   return check_launch(target);
 }
 
+constexpr uint32_t kUnknownNnz = 0xffffffffu;
+
+// nnz: the number of nonzeros, if the caller's descriptor carries it (used for a dense vector only)
 template <typename F, typename VT, bool HETER, int MODE>
 void launch_gather(const char *target, const ScratchSource &src, const F *data, const uint32_t *indices,
-                   const uint32_t *indptr, const VT *x, F *y, uint32_t n_row, uint32_t n_col) {
+                   const uint32_t *indptr, const VT *x, F *y, uint32_t n_row, uint32_t n_col, uint32_t nnz = kUnknownNnz) {
   hipStream_t stream = src.stream;
   if (n_row == 0) return;
   if constexpr (MODE == kEvent && !std::is_same<VT, PackedBits>::value) {
@@ -1815,46 +1796,32 @@ void launch_gather(const char *target, const ScratchSource &src, const F *data, 
                                                     lds_bytes))
         return;
       bpl_clear_error();
-    } else if (n_row >= 16384 && lds_bytes <= 4 * kLdsBitmapCap) {
-      // up to four times that: the part that fits is staged (one workgroup per CU), which takes a
-      // quarter or more of the gathers off the L2.  Its walk is row-wise: rows of 4 to 23 nonzeros on average
-      // go to the flat walk over the nonzeros instead (the mean is known on the device only: both are enqueued).
-      constexpr uint32_t kStagedMinMean = 24;
-      bool flat_takes_short_rows = false;
-      if constexpr (std::is_same<F, VT>::value) {
-        const FlatGather flat = csr_flat_gather<F>(target, stream, data, HETER, indices, indptr, x, y, n_row, 4u, kStagedMinMean);
-        if (flat == FlatGather::kFailed) {
-          if (scratch_refused_by_capture()) return ensure_error(target, "nothing was enqueued: the path that the scratch memory at hand allows could not be launched");  // (the error stands: a graph must not record a slower path)
-          bpl_clear_error();
-        }
-        flat_takes_short_rows = flat == FlatGather::kEnqueued;
-      }
-      if (launch_gather_impl<F, VT, HETER, MODE, 2>(target, stream, data, indices, indptr, x, y, n_row, n_col,
-                                                    kLdsBitmapCap, flat_takes_short_rows ? kStagedMinMean : 0u))
-        return;
-      bpl_clear_error();
     }
     if constexpr (std::is_same<F, VT>::value) {
-      // A longer vector is gathered from L2.  Rows of 4 nonzeros or more on average: the flat walk over the
-      // nonzeros with 16-byte loads of the index and weight streams (csr_flat_gather.hip; 4,000,000 rows of 8:
-      // 224 against 304 us, 2,000,000 rows of 20: 255 against 348 us); shorter ones: the walks below.  The
-      // mean is known on the device only, so both are enqueued and one returns at once.  (Under 16,384 rows
-      // the walks below stay: with 2,000 rows of 40,000 and a vector of 12 MB the walk that keeps a row's
-      // gathers together takes 507 us, the flat one 835; only matrices of a few hundred rows that are
-      // nearly dense would gain, and small ones would pay for a launch that returns at once.)
-      constexpr uint32_t kFlatMinMean = 4;
-      if (n_row >= 16384 && n_col > 0) {
-        const FlatGather flat =
-          csr_flat_gather<F>(target, stream, data, HETER, indices, indptr, x, y, n_row, kFlatMinMean, 0xffffffffu);
-        if (flat == FlatGather::kEnqueued) {
-          launch_gather_impl<F, VT, HETER, MODE, 0>(target, stream, data, indices, indptr, x, y, n_row, n_col, 0,
-                                                    kFlatMinMean);
+      // A longer vector is gathered from L2 (up to four times what fits in LDS: less the part that does).
+      // Rows of 4 nonzeros or more on average: the flat walk over the nonzeros with 16-byte loads of the index and
+      // weight streams (csr_flat_gather.hip; 4,000,000 rows of 8: 224 against 304 us, 2,000,000 rows of 20: 255
+      // against 348 us); shorter ones: the walks below.  Where the number of nonzeros is known on the device only,
+      // both are enqueued and one returns at once (4.5 us).
+      // Under 16,384 rows only with a part of the vector staged (300 rows of 10,000 and 140,000 columns: 116 -> 21 us,
+      // 10,000 rows of 1,300 and 43,818 columns: 58 -> 43 us): with 2,000 rows of 40,000 and a vector of 12 MB the
+      // walk that keeps a row's gathers together takes 507 us, the flat one 835.
+      // Under a million nonzeros the row-wise walk, one launch and nothing to stage (20,000 rows of 10 to 30 and 60,000
+      // columns: 9 us against 14; 50,000 uneven rows of 20: 16.6 against 17.1).
+      constexpr uint32_t kFlatMinMean = 4, kFlatMinNnz = 1u << 20;
+      const bool known = nnz != kUnknownNnz;
+      const bool flat = known ? nnz >= kFlatMinNnz && nnz <= kFlatMaxNnz && nnz / n_row >= kFlatMinMean &&
+                                  (n_row >= 16384 || flat_stages<F>(n_col))
+                              : n_row >= 16384;
+      if (flat && n_col > 0) {
+        if (csr_flat_gather<F>(target, stream, data, HETER, indices, indptr, x, y, n_row, n_col, known ? 0u : kFlatMinMean)) {
+          if (!known)
+            launch_gather_impl<F, VT, HETER, MODE, 0>(target, stream, data, indices, indptr, x, y, n_row, n_col, 0,
+                                                      kFlatMinMean);
           return;
         }
-        if (flat == FlatGather::kFailed) {
-          if (scratch_refused_by_capture()) return ensure_error(target, "nothing was enqueued: the path that the scratch memory at hand allows could not be launched");  // (the error stands: a graph must not record a slower path)
-          bpl_clear_error();
-        }
+        if (scratch_refused_by_capture()) return ensure_error(target, "nothing was enqueued: the path that the scratch memory at hand allows could not be launched");  // (the error stands: a graph must not record a slower path)
+        bpl_clear_error();
       }
     }
   }
@@ -1889,9 +1856,9 @@ template <typename F, bool HETER, bool TRANSPOSE>
 void csr_matvec_entry(const char *target, hipStream_t stream, void **buffers, const char *opaque,
                       size_t opaque_len, int vector_slot) {
   bpl_double_size_descriptor d;
-  uint32_t nnz = 0;  // known only to the transposed targets' longer descriptor
+  uint32_t nnz = TRANSPOSE ? 0u : kUnknownNnz;  // known only to the longer descriptor
   begin_call();
-  if (TRANSPOSE && opaque != nullptr && opaque_len == sizeof(bpl_csr_transpose_descriptor)) {
+  if (opaque != nullptr && opaque_len == sizeof(bpl_csr_transpose_descriptor)) {
     bpl_csr_transpose_descriptor t;
     std::memcpy(&t, opaque, sizeof(t));
     d.n_row = t.n_row, d.n_col = t.n_col, nnz = t.nnz;
@@ -1926,7 +1893,7 @@ void csr_matvec_entry(const char *target, hipStream_t stream, void **buffers, co
     launch_scatter<F, F, HETER, kDense>(ScratchSource{stream}, data, indices, indptr, vec, out, d.n_row, d.n_col);
     check_launch(target);
   } else {
-    launch_gather<F, F, HETER, kDense>(target, ScratchSource{stream}, data, indices, indptr, vec, out, d.n_row, d.n_col);
+    launch_gather<F, F, HETER, kDense>(target, ScratchSource{stream}, data, indices, indptr, vec, out, d.n_row, d.n_col, nnz);
   }
 }
 

@@ -29,7 +29,9 @@
   X(csr_matvec_transpose_heter_float)       \
   X(csr_matvec_transpose_heter_double)      \
   X(csr_matvec_transpose_homo_float)        \
-  X(csr_matvec_transpose_homo_double)
+  X(csr_matvec_transpose_homo_double)       \
+  X(csr_matvec_gradient_float)              \
+  X(csr_matvec_gradient_double)
 
 #define BPL_JITCONN_TARGETS(X) \
   X(gpu_event_matvec_prob_homo_v2_float_bool) \

@@ -114,17 +114,19 @@ class _EventCSRMatvec(torch.autograd.Function):
     g_data = g_events = None
     if ct is not None:
       ct = ct.contiguous()
-      if ctx.needs_input_grad[3]:
-        g_events = sparse_ops._launch(data.detach(), indices, indptr, ct, ctx.shape, not ctx.transpose)
       if ctx.needs_input_grad[0]:
+        ev = events.detach()
         if data.shape[0] == 1:
           ones = torch.ones(1, dtype=data.dtype, device=ct.device)
-          g_data = torch.inner(ct, _launch(ones, indices, indptr, events.detach(), ctx.shape, ctx.transpose)).reshape(1)
+          g_data = torch.inner(ct, _launch(ones, indices, indptr, ev, ctx.shape, ctx.transpose)).reshape(1)
+        elif ctx.transpose:
+          # (the events' gradient is a sum over the rows of what the walk for the weights gathers anyway)
+          g_data, g_events = sparse_ops._gradients(data, indices, indptr, ev.to(data.dtype), ct, ctx.shape,
+                                                   ctx.needs_input_grad[3])
         else:
-          row, col = sparse_ops.csr_to_coo(indices, indptr)
-          row, col = sparse_ops._int64(row), sparse_ops._int64(col)
-          ev = events.detach().to(data.dtype)
-          g_data = ev[row] * ct[col] if ctx.transpose else ev[col] * ct[row]
+          g_data, _ = sparse_ops._gradients(data, indices, indptr, ct, ev.to(data.dtype), ctx.shape, False)
+      if ctx.needs_input_grad[3] and g_events is None:
+        g_events = sparse_ops._launch(data.detach(), indices, indptr, ct, ctx.shape, not ctx.transpose)
     return g_data, None, None, g_events, None, None
 
   @staticmethod

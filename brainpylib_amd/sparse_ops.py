@@ -118,10 +118,10 @@ def _launch(data, indices, indptr, vector, shape, transpose, method='vector'):
   device, data, indices, indptr, vector = _move(data, indices, indptr, vector)
   type_name = 'float' if data.dtype == torch.float32 else 'double'
   data_name = 'homo' if data.shape[0] == 1 else 'heter'
-  opaque = _lib.build_double_size_descriptor(shape[0], shape[1])
+  # (the longer descriptor, for both orientations: with the number of nonzeros the library picks one kernel)
+  opaque = _lib.build_csr_transpose_descriptor(shape[0], shape[1], indices.shape[0])
   out = torch.empty(shape[1] if transpose else shape[0], dtype=data.dtype, device=device)
   if transpose:
-    opaque = _lib.build_csr_transpose_descriptor(shape[0], shape[1], indices.shape[0])
     _lib.custom_call('csr_matvec_transpose_' + data_name + '_' + type_name, [data, indices, indptr, vector, out],
                      opaque)
     return out
@@ -145,6 +145,25 @@ def _wants_grad(*tensors):
     if t.is_floating_point() and torch.autograd.forward_ad.unpack_dual(t).tangent is not None:
       return True
   return False
+
+
+_GRADIENT_MAX_NNZ = 2 ** 32 - 8193  # what the gradient target's 32-bit positions can number
+
+
+def _gradients(data, indices, indptr, row_vector, col_vector, shape, want_sums):
+  """(products, sums): ``row_vector[row] * col_vector[col]`` per nonzero and, if wanted, the product of the matrix
+  with ``col_vector``, in one walk over the nonzeros (sums is None where it was not computed)."""
+  nnz = indices.shape[0]
+  differentiated = torch.is_grad_enabled() and (row_vector.requires_grad or col_vector.requires_grad)
+  if nnz > _GRADIENT_MAX_NNZ or differentiated:  # (create_graph: the products stay differentiable)
+    row, col = csr_to_coo(indices, indptr)
+    return row_vector[_int64(row)] * col_vector[_int64(col)], None
+  products = torch.empty(nnz, dtype=data.dtype, device=data.device)
+  sums = torch.empty(shape[0] if want_sums else 0, dtype=data.dtype, device=data.device)
+  _lib.custom_call('csr_matvec_gradient_' + ('float' if data.dtype == torch.float32 else 'double'),
+                   [data.detach(), indices, indptr, row_vector.detach(), col_vector.detach(), products, sums],
+                   _lib.build_csr_transpose_descriptor(shape[0], shape[1], nnz))
+  return products, sums if want_sums else None
 
 
 class _CSRMatvec(torch.autograd.Function):
@@ -171,17 +190,16 @@ class _CSRMatvec(torch.autograd.Function):
     g_data = g_vector = None
     if ct is not None:
       ct = ct.contiguous()
-      if ctx.needs_input_grad[3]:
-        g_vector = _launch(data.detach(), indices, indptr, ct, ctx.shape, not ctx.transpose)
       if ctx.needs_input_grad[0]:
         if data.shape[0] == 1:
           ones = torch.ones(1, dtype=data.dtype, device=ct.device)
           g_data = torch.inner(ct, _launch(ones, indices, indptr, vector.detach(), ctx.shape, ctx.transpose)).reshape(1)
+        elif ctx.transpose:  # the vector's gradient is a sum over the rows of what the walk gathers anyway
+          g_data, g_vector = _gradients(data, indices, indptr, vector.detach(), ct, ctx.shape, ctx.needs_input_grad[3])
         else:
-          row, col = csr_to_coo(indices, indptr)
-          row, col = _int64(row), _int64(col)
-          v = vector.detach()
-          g_data = v[row] * ct[col] if ctx.transpose else v[col] * ct[row]
+          g_data, _ = _gradients(data, indices, indptr, ct, vector.detach(), ctx.shape, False)
+      if ctx.needs_input_grad[3] and g_vector is None:
+        g_vector = _launch(data.detach(), indices, indptr, ct, ctx.shape, not ctx.transpose)
     return g_data, None, None, g_vector, None, None, None
 
   @staticmethod

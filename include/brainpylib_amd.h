@@ -365,7 +365,9 @@ BPL_TARGET(gpu_csr_event_prod_heter_f64_i64);
  *   scalar / vector: buffers = [data, indices, indptr, vector, out]
  *   adaptive:        buffers = [data, indices, indptr, row_blocks, vector, out]
  *                    (row_blocks is accepted for layout compatibility and not read)
- *   opaque = bpl_double_size_descriptor;  out[r] = sum_j data[j] * vector[indices[j]], F[n_row].
+ *   opaque = bpl_double_size_descriptor, or bpl_csr_transpose_descriptor, with whose nonzero count the
+ *   library enqueues one kernel where it must else enqueue two and let one return at once;
+ *   out[r] = sum_j data[j] * vector[indices[j]], F[n_row].
  *   The three method names select the same kernel family here: the lanes-per-row mode is
  *   picked on the device from the mean row length.
  * ---------------------------------------------------------------------------------------- */
@@ -392,6 +394,17 @@ BPL_TARGET(csr_matvec_transpose_heter_float);
 BPL_TARGET(csr_matvec_transpose_heter_double);
 BPL_TARGET(csr_matvec_transpose_homo_float);
 BPL_TARGET(csr_matvec_transpose_homo_double);
+
+/* Gradients of a product with a matrix of one weight per nonzero (own targets: the reference's
+ * differentiation rules, brainpylib/_src/sparse_ops/cusparse_matvec.py:281-308, are composed of
+ * gathers over an expanded list of the nonzeros' rows).
+ *   products[j] = row_vector[row of j] * column_vector[column of j] for every nonzero j,
+ *   sums = A @ column_vector (not computed if its pointer is null; `data` is read for it only).
+ *   buffers = [data, indices, indptr, row_vector(F[n_row]), column_vector(F[n_col]),
+ *              products(F[nnz]), sums(F[n_row]) or null],
+ *   opaque = bpl_csr_transpose_descriptor; nnz at most 2^32 - 8193. */
+BPL_TARGET(csr_matvec_gradient_float);
+BPL_TARGET(csr_matvec_gradient_double);
 
 /* ------------------------------------------------------------------------------------------
  * jitconn (event) matvec, version 2 kernels: y = M @ x with M regenerated on the fly.

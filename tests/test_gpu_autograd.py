@@ -6,6 +6,7 @@ import pytest
 import torch
 import torch.autograd.forward_ad as fwAD
 
+import benchdata as synth
 import brainpylib_amd as bpl
 from util import random_csr
 
@@ -99,6 +100,50 @@ def test_csr_matvec_gradients(cuda, shape, transpose, homo):
   Md = Md.T if transpose else Md
   want = Md @ torch.tensor(v_np) + M.detach() @ torch.tensor(v_dot)
   torch.testing.assert_close(tangent.cpu(), want, rtol=1e-10, atol=1e-10)
+
+
+# rows, columns, mean row length: one partial step; rows shorter than a quad (windows of more than 64 rows to a step);
+# vectors that just fit the 138 KB staged in LDS (35,328 floats, 17,664 doubles), one element more, four times as many
+# (the last staged size) and one more (gathered from L2 only); rows that run through many waves' ranges
+@pytest.mark.parametrize("n_row,n_col,mean", [(3, 9, 2), (9000, 200, 1), (300, 35_328, 900), (2000, 35_329, 300),
+                                              (900, 17_664, 10), (20_000, 141_312, 40), (700, 141_313, 800),
+                                              (10, 300_000, 20_000)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("transpose", [False, True])
+def test_gradients_of_weights_and_vector_from_one_walk(cuda, n_row, n_col, mean, dtype, transpose):
+  rng = np.random.default_rng(n_row)
+  counts = np.minimum(rng.poisson(mean * np.exp(rng.standard_normal(n_row) - 0.5)), n_col)
+  counts[rng.random(n_row) < 0.2] = 0
+  counts[-1] = 0  # (rows without nonzeros, the last one among them)
+  counts[0] = max(counts[0], 2)
+  idx, ptr = synth.counted_csr(counts, n_col, seed=n_row)
+  row = torch.from_numpy(np.repeat(np.arange(n_row), counts))
+  col = torch.from_numpy(idx.astype(np.int64))
+  print("case", n_row, n_col, dtype, transpose, idx.shape[0], flush=True)
+  n_in, n_out = (n_row, n_col) if transpose else (n_col, n_row)
+  g = torch.Generator().manual_seed(n_col)
+  data, vec, ct = (torch.randn(n, dtype=dtype, generator=g) for n in (idx.shape[0], n_in, n_out))
+  src, dst = (row, col) if transpose else (col, row)
+  want = vec[src] * ct[dst]  # one product per weight: the same bits
+  addend = (data * ct[dst]).to(torch.float64)  # the sums' addends, rounded once each as the kernels round them
+  want_vec = torch.zeros(n_in, dtype=torch.float64).index_add_(0, src, addend)
+  mag = torch.zeros(n_in, dtype=torch.float64).index_add_(0, src, addend.abs())
+  # (second round: index and weight arrays that do not begin at a multiple of 16 bytes)
+  for first in (0, 1):
+    d = torch.cat([torch.zeros(first, dtype=dtype), data]).cuda()[first:].requires_grad_()
+    i = torch.cat([torch.zeros(first, dtype=torch.int32), torch.from_numpy(idx)]).cuda()[first:]
+    v = vec.cuda().requires_grad_()
+    y = bpl.cusparse_csr_matvec(d, i, torch.from_numpy(ptr).cuda(), v, shape=(n_row, n_col), transpose=transpose)
+    got, got_vec = torch.autograd.grad(y, (d, v), ct.cuda())
+    assert torch.equal(got.cpu(), want)
+    # transposed: the walk's float64 sums in another order, rounded once to dtype; else the transposed product, whose
+    # partial sums are of dtype (the bound of two orders of summation in that precision)
+    order = torch.float64 if transpose else dtype
+    bound = torch.finfo(dtype).eps * want_vec.abs() + 4 * torch.finfo(order).eps * mag
+    assert bool(((got_vec.cpu().to(torch.float64) - want_vec).abs() <= bound).all())
+    # the weights' gradient alone (no sums), of float events; the events' values enter it
+    y = bpl.event_csr_matvec(d, i, torch.from_numpy(ptr).cuda(), v.detach(), shape=(n_row, n_col), transpose=transpose)
+    assert torch.equal(torch.autograd.grad(y, d, ct.cuda())[0].cpu(), want)
 
 
 @pytest.mark.parametrize("kind", ["homo", "uniform", "normal"])

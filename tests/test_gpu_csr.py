@@ -10,6 +10,7 @@ import pytest
 import torch
 
 import brainpylib_amd as bpl
+from brainpylib_amd import _lib
 import benchdata as synth
 from util import CSR_SHAPES, assert_close, assert_close_reordered, random_csr
 
@@ -1125,3 +1126,48 @@ def test_csr_matvec_flat_walk_over_the_nonzeros(cuda, oracle_mod, kind):
   want = oracle_mod.csr_matvec(data, indices, indptr, v, shape=(n_row, n_col))
   got = bpl.csr_matvec(data, indices, indptr, v, shape=(n_row, n_col)).cpu().numpy()
   assert_close(got, want, what="flat walk " + kind)
+
+
+# vectors one element longer than what a workgroup stages whole, up to the last partly staged size and one beyond (gathered
+# from L2 only); below and above 16,384 rows; just below and above a million nonzeros (a row-wise walk below)
+@pytest.mark.parametrize("n_row,n_col,mean", [(20_000, 35_329, 56), (3000, 35_329, 500), (300, 141_312, 4000),
+                                              (20_000, 141_312, 50), (20_000, 141_313, 60), (400_000, 40_705, 4)])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("homo", [False, True])
+def test_csr_matvec_with_a_part_of_the_vector_in_lds(cuda, n_row, n_col, mean, dtype, homo):
+  if dtype == np.float64:
+    n_col //= 2
+  rng = np.random.default_rng(n_row + n_col)
+  counts = np.minimum(rng.poisson(mean * np.exp(0.5 * rng.standard_normal(n_row))), n_col // 2)
+  counts[:3] = counts[-3:] = 0
+  indices, indptr = synth.counted_csr(counts, n_col, seed=n_row)
+  nnz = indices.shape[0]
+  data = rng.standard_normal(1 if homo else nnz).astype(dtype)
+  v = rng.standard_normal(n_col).astype(dtype)
+  print("case", n_row, n_col, dtype.__name__, homo, "nnz", nnz, flush=True)
+  addend = (v[indices] * data).astype(np.float64)  # rounded once each, as the kernels round them
+  want = np.bincount(np.repeat(np.arange(n_row), counts), weights=addend, minlength=n_row)
+  mag = np.bincount(np.repeat(np.arange(n_row), counts), weights=np.abs(addend), minlength=n_row)
+  # float64 sums in another order, rounded once to the result's type
+  bound = np.finfo(dtype).eps * np.abs(want) + 4 * np.finfo(np.float64).eps * np.maximum(counts, 1) ** 0.5 * mag
+  # first the host's count of the nonzeros decides the kernel, then (a descriptor without it) the device's
+  got = bpl.csr_matvec(data, indices, indptr, v, shape=(n_row, n_col)).cpu().numpy()
+  assert (np.abs(got - want) <= bound).all()
+  dev = [torch.from_numpy(a).cuda() for a in (data, indices, indptr, v)]
+  out = torch.empty(n_row, dtype=dev[0].dtype, device="cuda")
+  name = "csr_matvec_%s_vector_%s" % ("homo" if homo else "heter", "float" if dtype == np.float32 else "double")
+  _lib.custom_call(name, dev + [out], _lib.build_double_size_descriptor(n_row, n_col))
+  assert (np.abs(out.cpu().numpy() - want) <= bound).all()
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_csr_matvec_padded_index_arrays(cuda, dtype):
+  # arrays longer than indptr says: the matrix ends where indptr ends, whatever kernel the array's length picks
+  n_row, n_col = 20_000, 50_000
+  indptr = np.zeros(n_row + 1, np.int32)
+  indices, data = np.zeros(1 << 21, np.int32), np.ones(1 << 21, dtype)
+  got = bpl.csr_matvec(data, indices, indptr, np.ones(n_col, dtype), shape=(n_row, n_col)).cpu().numpy()
+  assert not got.any()
+  indptr[5:] = 3
+  got = bpl.csr_matvec(data, indices, indptr, np.ones(n_col, dtype), shape=(n_row, n_col)).cpu().numpy()
+  assert got[4] == 3 and got.sum() == 3
