@@ -137,6 +137,7 @@ bool flat_window_scatter(const char *target, hipStream_t stream, const F *data, 
 // = batch * columns, and `active_colbase` = what to add to the columns of each listed row (its
 // batch entry * columns); n_row stays the matrix's row count (indptr has n_row + 1 entries).
 constexpr size_t kBinEventFillBytes = 131072;
+constexpr uint64_t kMostRunPairs = 1ull << 27;  // pairs that the runs hold together at most
 template <typename F>
 bool bin_event_scatter_usable(uint32_t n_col);
 template <typename F>

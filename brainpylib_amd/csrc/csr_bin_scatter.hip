@@ -1267,7 +1267,7 @@ inline uint32_t event_window_shift(uint32_t n_out) {
 inline uint64_t event_run_pairs(uint32_t n_row, uint32_t n_col) {
   uint64_t t = 4096ull * (n_row > n_col ? n_row : n_col);
   if (t < (1ull << 24)) t = 1ull << 24;
-  if (t > (1ull << 27)) t = 1ull << 27;
+  if (t > kMostRunPairs) t = kMostRunPairs;
   return t;
 }
 

@@ -289,14 +289,14 @@ void launch_collect(hipStream_t stream, const I *indptr, const VT *x, uint32_t n
 // virtual row v = entry * n_row + r; `colbase` receives entry * n_col for every listed row.
 // events: [events_batch][n_row]; entry bi of this launch is entry first_entry + bi of the whole
 // batch and reads row (first_entry + bi) % events_batch.
-template <typename F, typename VT>
+// kPer virtual rows per thread; `batch` * n_row is below 2^31.
+template <typename F, typename VT, int kPer>
 __global__ __launch_bounds__(kWinThreads) void collect_active_rows_batched_kernel(
     const uint32_t *__restrict__ indptr, const VT *__restrict__ events, uint32_t n_row, uint32_t n_col,
     uint32_t batch, uint32_t events_batch, uint32_t first_entry, uint32_t *__restrict__ counter,
     uint2 *__restrict__ list,
     uint32_t *__restrict__ colbase, uint32_t *__restrict__ clear, uint32_t n_clear, F *__restrict__ zero,
     uint64_t n_zero) {
-  constexpr int kPer = 8;
   __shared__ uint32_t s_count, s_base;
   const uint32_t tid = threadIdx.x, lane = tid % kWave;
   if (tid == 0) s_count = 0;
@@ -305,24 +305,29 @@ __global__ __launch_bounds__(kWinThreads) void collect_active_rows_batched_kerne
        i += static_cast<uint64_t>(gridDim.x) * kWinThreads)
     zero[i] = F(0);
   __syncthreads();
-  const uint64_t total = static_cast<uint64_t>(batch) * n_row;
-  const uint64_t v0 = static_cast<uint64_t>(blockIdx.x) * (kWinThreads * kPer) + tid;
+  const uint32_t total = batch * n_row;
+  const uint32_t v0 = blockIdx.x * (kWinThreads * kPer) + tid;
   bool on[kPer];
-  uint32_t start[kPer], len[kPer], at[kPer], base_col[kPer];
+  uint32_t start[kPer], len[kPer], at[kPer], base_col[kPer], row[kPer];
 #pragma unroll
   for (int e = 0; e < kPer; ++e) {
-    const uint64_t v = v0 + static_cast<uint64_t>(e) * kWinThreads;
+    const uint32_t v = v0 + e * kWinThreads;
     on[e] = false;
-    start[e] = len[e] = at[e] = base_col[e] = 0;
+    base_col[e] = row[e] = 0;
     if (v < total) {
-      const uint32_t bi = static_cast<uint32_t>(v / n_row), r = static_cast<uint32_t>(v % n_row);
-      on[e] = is_event(events[static_cast<size_t>((first_entry + bi) % events_batch) * n_row + r]);
-      if (on[e]) {
-        start[e] = indptr[r];
-        len[e] = indptr[r + 1] - start[e];
-        on[e] = len[e] != 0;
-        base_col[e] = bi * n_col;
-      }
+      const uint32_t bi = v / n_row;
+      row[e] = v - bi * n_row;
+      on[e] = is_event(events[static_cast<size_t>((first_entry + bi) % events_batch) * n_row + row[e]]);
+      base_col[e] = bi * n_col;
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < kPer; ++e) {
+    start[e] = len[e] = at[e] = 0;
+    if (on[e]) {
+      start[e] = indptr[row[e]];
+      len[e] = indptr[row[e] + 1] - start[e];
+      on[e] = len[e] != 0;
     }
   }
 #pragma unroll
@@ -2211,12 +2216,18 @@ void event_csr_batching_entry(const char *target, hipStream_t stream, void **buf
                                                 d.batch_size, 0);
     return;
   }
-  // Transposed, one matrix for all entries: groups of up to 8 entries go through ONE sorted scatter
-  // over a virtual output of group * n_col columns (entry g's columns shifted by g * n_col), fed by
-  // one list of the active rows of the group's entries.  (Larger groups gain nothing more and
-  // overflow the runs of the sort sooner.)
+  // Transposed, one matrix for all entries: groups of entries go through ONE sorted scatter over a virtual output of
+  // group * n_col columns (entry g's columns shifted by g * n_col), fed by one list of the active rows of the
+  // group's entries.  A group is a chain of three launches whatever its size, so it takes as many entries as keep
+  // the virtual output within windows that are added in one slice (2^21 columns) and the pairs of a sixth of
+  // all nonzeros within the runs of the sort (20 entries of 8e6 nonzeros in one group instead of three: 105 -> 52 us);
+  // up to 8 entries beyond those bounds (1e8 nonzeros: larger groups gain nothing and overflow the runs sooner).
+  // Groups of equal size.
   if (d.transpose && shared_matrix && d.batch_size > 1 && d.n_row > 0 && d.n_col > 0) {
-    uint32_t group = d.batch_size < 8 ? d.batch_size : 8;
+    const uint64_t by_columns = (1ull << 21) / d.n_col, by_pairs = 6ull * kMostRunPairs / (d.nnz ? d.nnz : 1u);
+    const uint64_t fits = by_columns < by_pairs ? by_columns : by_pairs;
+    const uint32_t most = fits < 8 ? 8u : fits < d.batch_size ? static_cast<uint32_t>(fits) : d.batch_size;
+    uint32_t group = div_up(d.batch_size, div_up(d.batch_size, most));
     while (group > 1 && (static_cast<uint64_t>(group) * d.n_col >= (1ull << 24) ||
                          static_cast<uint64_t>(group) * d.n_row >= (1ull << 31)))
       --group;
@@ -2237,8 +2248,10 @@ void event_csr_batching_entry(const char *target, hipStream_t stream, void **buf
           const uint32_t g = (d.batch_size - b0 < group) ? d.batch_size - b0 : group;
           // entry b0 + i reads event vector (b0 + i) % events_batch: hand the kernel the rotation
           F *o = out + static_cast<size_t>(b0) * d.n_col;
-          hipLaunchKernelGGL((collect_active_rows_batched_kernel<F, VT>),
-                             dim3(div_up(static_cast<uint64_t>(g) * d.n_row, 8 * kWinThreads)), dim3(kWinThreads), 0,
+          // (few virtual rows: one per thread, or most of the device has none: 160,000 of them 10 -> 4 us)
+          const uint64_t listed = static_cast<uint64_t>(g) * d.n_row;
+          auto collect = listed > 524288u ? collect_active_rows_batched_kernel<F, VT, 8> : collect_active_rows_batched_kernel<F, VT, 1>;
+          hipLaunchKernelGGL(collect, dim3(div_up(listed, (listed > 524288u ? 8 : 1) * kWinThreads)), dim3(kWinThreads), 0,
                              stream, indptr, events, d.n_row, d.n_col, g, d.events_batch, b0, counters, list, colbase,
                              reinterpret_cast<uint32_t *>(scratch),
                              static_cast<uint32_t>(kBinEventFillBytes / sizeof(uint32_t)), o,

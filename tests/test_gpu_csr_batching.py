@@ -145,3 +145,22 @@ def test_full_size_batching_rows_equal_single_operator(cuda):
     assert_close(het[bi].cpu().numpy(), single.cpu().numpy(), what="heter entry %d" % bi)
     single = bpl.event_csr_matvec(w[0], indices, indptr, events[bi], shape=shape)
     assert torch.equal(hom[bi], single)
+
+
+# one group of all entries (listed one virtual row per thread, then eight per thread); groups bounded by the width of the
+# virtual output (33 entries of 100,000 columns: two groups) and a last group of fewer entries; events shared by entries
+@pytest.mark.parametrize("n_row,n_col,mean,batch,eb", [(900, 700, 40, 33, 33), (30_000, 3000, 5, 21, 21),
+                                                       (500, 100_000, 60, 33, 11), (40, 9000, 30, 23, 23)])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_batching_transposed_in_groups(cuda, oracle_mod, n_row, n_col, mean, batch, eb, dtype):
+  rng = np.random.default_rng(n_row)
+  counts = np.minimum(rng.poisson(mean, size=n_row), n_col)
+  indices, indptr = synth.counted_csr(counts, n_col, seed=n_row)
+  data = rng.standard_normal(indices.shape[0]).astype(dtype)
+  print("case", n_row, n_col, batch, eb, dtype.__name__, flush=True)
+  for rate in (0.02, 0.6):
+    events = rng.random((eb, n_row)) < rate
+    _check(oracle_mod, data[None], indices[None], indptr[None], events, batch, (n_row, n_col), True, "heter")
+    one = np.full((1, 1), 0.7, dtype=dtype)
+    got, want = _check(oracle_mod, one, indices[None], indptr[None], events, batch, (n_row, n_col), True, "homo")
+    assert np.array_equal(got, want)  # (counts: the reference's bits whatever the order)
