@@ -72,17 +72,22 @@ __global__ __launch_bounds__(256) void jitconn_matmat_kernel(const T1 *__restric
   constexpr int kWaves = 4;
   constexpr int kWords = StreamLds<T1, W>::words;
   __shared__ __attribute__((aligned(8))) uint32_t s_state[kWaves * kWords];
-  __shared__ Synapse<T1> s_syn[kWaves * kWave];
+  constexpr int kSlots = W == kNormal ? 2 * kWave : kWave;  // normal weights come two to a lane
+  __shared__ __attribute__((aligned(16))) Synapse<T1> s_syn[kWaves * kSlots];
   const int lane = lane_id();
   const uint32_t wave = threadIdx.x / kWave;
   uint32_t *st = s_state + wave * kWords;
-  Synapse<T1> *syn = s_syn + wave * kWave;
+  Synapse<T1> *syn = s_syn + wave * kSlots;
   const uint32_t row_base = pass * (MT * kWave);  // first row of Y of this pass
   // byte offsets into the pass's slice of XT fit 32 bits (checked by the host): one add per synapse instead of a
   // 64-bit product
   constexpr uint32_t row_bytes = MT * kWave * static_cast<uint32_t>(sizeof(T1));
   // (a wave-uniform base and a 32-bit offset per lane: one address add per synapse and the base in scalar registers)
   const char *xt_base = reinterpret_cast<const char *>(XT + static_cast<size_t>(pass) * k * (MT * kWave));
+  // lane l accumulates rows MT l .. MT l + MT - 1 of the pass: one load per synapse, MT entries wide
+  struct __attribute__((aligned(MT * sizeof(T1)))) Rows {
+    T1 x[MT];
+  };
   const uint32_t lane_bytes = static_cast<uint32_t>(lane) * static_cast<uint32_t>(sizeof(T1));
 
   // columns first .. first + count - 1 of M, their generators seeded ahead: states[c] for column first + c
@@ -92,21 +97,11 @@ __global__ __launch_bounds__(256) void jitconn_matmat_kernel(const T1 *__restric
 #pragma unroll
     for (int t = 0; t < MT; ++t) acc[t] = T1(0);
     const uint32_t *pre = states != nullptr ? states + static_cast<size_t>(c) * kMtN : nullptr;
-    walk_stream<T1, W>(st, lane, seed + j, pre, k, log_p, wa, wb, [&](uint32_t idx, T1 w, bool valid) {
-      // Every valid lane leaves its synapse (the byte offset of its row of XT, its weight) in the
-      // wave's LDS slots, in lane order (which is stream order); every lane then reads the slots
-      // one after the other (one address per read: a broadcast), so a synapse costs one LDS read,
-      // one address add, MT loads and MT multiply-adds, with U synapses' loads in flight.
-      const uint64_t mask = __ballot(valid);
-      const uint32_t count = static_cast<uint32_t>(__popcll(mask));
-      const uint32_t slot = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(mask >> 32),
-                                                      __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(mask), 0u));
-      __builtin_amdgcn_wave_barrier();  // the reads of the batch before are done
-      if (valid) {
-        syn[slot].off = idx * row_bytes;
-        syn[slot].w = w;
-      }
-      __builtin_amdgcn_wave_barrier();
+    // Every valid lane leaves its synapses (the byte offset of their rows of XT, their weights) in the
+    // wave's LDS slots, in lane order (which is stream order); every lane then reads the slots
+    // one after the other (one address per read: a broadcast), so a synapse costs one LDS read,
+    // one address add, one load and MT multiply-adds, with U synapses' loads in flight.
+    auto take = [&](uint32_t count) {
       constexpr int U = 8;
       uint32_t i = 0;
       for (; i + U <= count; i += U) {
@@ -132,7 +127,30 @@ __global__ __launch_bounds__(256) void jitconn_matmat_kernel(const T1 *__restric
 #pragma unroll
         for (int t = 0; t < MT; ++t) acc[t] = add_rn(acc[t], mul_rn(e.w, row[t * kWave]));
       }
-    });
+    };
+    auto put = [&](uint32_t slot, uint32_t idx, T1 w) {
+      syn[slot].off = idx * row_bytes;
+      syn[slot].w = w;
+    };
+    if constexpr (W == kNormal) {
+      walk_stream<T1, W>(st, lane, seed + j, pre, k, log_p, wa, wb,
+                         [&](uint32_t idx0, T1 w0, bool valid0, uint32_t idx1, T1 w1, bool valid1) {
+        __builtin_amdgcn_wave_barrier();  // the reads of the batch before are done
+        if (valid0) {
+          put(2u * static_cast<uint32_t>(lane), idx0, w0);
+          put(2u * static_cast<uint32_t>(lane) + 1u, idx1, w1);  // (not counted where only the first is valid)
+        }
+        __builtin_amdgcn_wave_barrier();
+        take(static_cast<uint32_t>(__popcll(__ballot(valid0)) + __popcll(__ballot(valid1))));
+      });
+    } else {
+      walk_stream<T1, W>(st, lane, seed + j, pre, k, log_p, wa, wb, [&](uint32_t idx, T1 w, bool valid) {
+        __builtin_amdgcn_wave_barrier();
+        if (valid) put(static_cast<uint32_t>(lane), idx, w);
+        __builtin_amdgcn_wave_barrier();
+        take(static_cast<uint32_t>(__popcll(__ballot(valid))));
+      });
+    }
 #pragma unroll
     for (int t = 0; t < MT; ++t) {
       const uint32_t r = row_base + t * kWave + lane;

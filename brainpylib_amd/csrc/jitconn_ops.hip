@@ -33,10 +33,15 @@ namespace {
 // LDS the row walk gives to an event bitmap when it wants two 16-wave workgroups per CU (each wave
 // can issue one instruction every four cycles, so the number of resident waves bounds the VALU
 // utilisation: 32 waves per CU walk 290 G synapses/s, the 15 that fit beside a 125 KB bitmap 228).
-constexpr uint32_t kRowwalkCoarseBytes = 38912;
+// What two workgroups leave of a CU's 160 KB beside their 16 waves' states and queues.
+template <typename T1, int W>
+constexpr uint32_t rowwalk_coarse_bytes() {
+  const uint32_t left = (80u * 1024u - 16u * 4u * StreamLds<T1, W>::words - 64u) / 256u * 256u;
+  return left < 38912u ? left : 38912u;
+}
 
 // BITS: where the event probes go.  0: the event vector in global memory; 1: its bitmap in LDS;
-// 2: a coarse bitmap in LDS (one bit per 2^g inputs, at most kRowwalkCoarseBytes) and, where its
+// 2: a coarse bitmap in LDS (one bit per 2^g inputs, at most rowwalk_coarse_bytes<T1, W>()) and, where its
 // bit is set, the exact packed bitmap in global memory (`in`, the coarse one behind it).
 // (With the coarse bitmap two 16-wave workgroups are meant to share a CU: 8 waves per SIMD, which
 // the register allocation has to leave room for; the normal-weight walk needs 66 otherwise.)
@@ -68,7 +73,7 @@ __global__ __launch_bounds__(1024, (BITS == 2 || (W == kNormal && sizeof(T1) == 
   uint32_t coarse_g = 0, coarse_g5 = 5;
   if constexpr (BITS == 2) {
     uint32_t *wbits = smem + nwaves * kWords;
-    coarse_g = coarse_shift(n_in, kRowwalkCoarseBytes);
+    coarse_g = coarse_shift(n_in, rowwalk_coarse_bytes<T1, W>());
     coarse_g5 = coarse_g + 5u;
     const uint32_t words = (coarse_bits(n_in, coarse_g) + 31u) >> 5;
     const uint32_t *coarse = reinterpret_cast<const uint32_t *>(in) + coarse_offset_words(n_in);
@@ -382,31 +387,26 @@ __global__ __launch_bounds__(kColBinThreads, sizeof(T1) == 4 ? 8 : 4) void jitco
     }
     walk_stream<T1, W>(st, lane, seed + col, pre, n_out, log_p, wa, wb, [&](uint32_t idx, T1 w, bool valid) {
       const uint32_t b = idx >> shift;
-      uint32_t slot = 0;
-      if constexpr (W != kNormal) {
-        // The positions rise from lane to lane and the lanes that hold a synapse are the first ones of the
-        // wave, so the lanes of a batch that meet in one window are neighbours (sixteen of them with
-        // 16,384-output windows and conn_prob 0.001, all 64 with a dense matrix).  A returning addition
-        // of several lanes to ONE counter occupies the CU's LDS for 64 cycles (measured; 7 when every lane
-        // has a counter of its own), so the first lane of every run of equal windows reserves the places
-        // of the whole run and the others fetch its answer (12 cycles with the shuffle): 3 to 6 % of the
-        // walk, whose larger cost is the scattered stores of the pairs.  Lanes 0 and 32 begin runs of their
-        // own, which keeps the masks at 32 bits.
-        const uint32_t n_valid = static_cast<uint32_t>(__popcll(__ballot(valid)));
-        const uint64_t heads = __ballot(b != wave_shift_up1(b)) | 0x100000001ull;
-        const uint32_t half = lane < 32 ? static_cast<uint32_t>(heads) : static_cast<uint32_t>(heads >> 32);
-        const uint32_t up = 31u - (static_cast<uint32_t>(lane) & 31u);  // lanes above this one in its half
-        const uint32_t rank = static_cast<uint32_t>(__builtin_clz(half << up));  // lanes from the run's first to this one
-        // the next run begins `run` lanes above this one (a run ends with its half at the latest)
-        const uint32_t above = ((half >> 1) >> (31u - up)) | (0x80000000u >> (31u - up));
-        uint32_t run = static_cast<uint32_t>(__builtin_ctz(above)) + 1u;
-        if (run > n_valid - static_cast<uint32_t>(lane)) run = n_valid - static_cast<uint32_t>(lane);
-        uint32_t first_slot = 0;
-        if (valid && rank == 0u) first_slot = atomicAdd(&s_cnt[b], run);
-        slot = static_cast<uint32_t>(__shfl(static_cast<int>(first_slot), lane - static_cast<int>(rank))) + rank;
-      } else if (valid) {
-        slot = atomicAdd(&s_cnt[b], 1u);  // (normal weights: the lanes that hold a synapse are not neighbours)
-      }
+      // The positions rise from lane to lane and the lanes that hold a synapse are the first ones of the
+      // wave, so the lanes of a batch that meet in one window are neighbours (sixteen of them with
+      // 16,384-output windows and conn_prob 0.001, all 64 with a dense matrix).  A returning addition
+      // of several lanes to ONE counter occupies the CU's LDS for 64 cycles (measured; 7 when every lane
+      // has a counter of its own), so the first lane of every run of equal windows reserves the places
+      // of the whole run and the others fetch its answer (12 cycles with the shuffle): 3 to 6 % of the
+      // walk, whose larger cost is the scattered stores of the pairs.  Lanes 0 and 32 begin runs of their
+      // own, which keeps the masks at 32 bits.
+      const uint32_t n_valid = static_cast<uint32_t>(__popcll(__ballot(valid)));
+      const uint64_t heads = __ballot(b != wave_shift_up1(b)) | 0x100000001ull;
+      const uint32_t half = lane < 32 ? static_cast<uint32_t>(heads) : static_cast<uint32_t>(heads >> 32);
+      const uint32_t up = 31u - (static_cast<uint32_t>(lane) & 31u);  // lanes above this one in its half
+      const uint32_t rank = static_cast<uint32_t>(__builtin_clz(half << up));  // lanes from the run's first to this one
+      // the next run begins `run` lanes above this one (a run ends with its half at the latest)
+      const uint32_t above = ((half >> 1) >> (31u - up)) | (0x80000000u >> (31u - up));
+      uint32_t run = static_cast<uint32_t>(__builtin_ctz(above)) + 1u;
+      if (run > n_valid - static_cast<uint32_t>(lane)) run = n_valid - static_cast<uint32_t>(lane);
+      uint32_t first_slot = 0;
+      if (valid && rank == 0u) first_slot = atomicAdd(&s_cnt[b], run);
+      const uint32_t slot = static_cast<uint32_t>(__shfl(static_cast<int>(first_slot), lane - static_cast<int>(rank))) + rank;
       if (valid) {
         T1 add;
         if (IN == kInDense) add = (W == kHomo) ? val : static_cast<T1>(w * val);
@@ -645,12 +645,12 @@ void launch_rowwalk(hipStream_t stream, const VT *in, T1 *out, uint32_t n_out, u
   // An event bitmap that would leave room for fewer than two 16-wave workgroups per CU: two levels
   // instead, the exact bitmap packed into global memory and a coarse one made for LDS.  Wide event
   // types: the vector is packed to one bit per element once, instead of once per workgroup.
-  const bool two_level = kEvents && words * 4 > kRowwalkCoarseBytes;
+  const bool two_level = kEvents && words * 4 > rowwalk_coarse_bytes<T1, W>();
   const bool packed = kEvents && (two_level || sizeof(VT) > 1);
   uint32_t g = 0, off = 0, c_words = 0;
   size_t bitmap_ws = 0;
   if (two_level) {
-    g = coarse_shift(n_in, kRowwalkCoarseBytes);
+    g = coarse_shift(n_in, rowwalk_coarse_bytes<T1, W>());
     off = coarse_offset_words(n_in);
     c_words = (coarse_bits(n_in, g) + 31u) / 32u;
     bitmap_ws = (static_cast<size_t>(off) + c_words + 1) * sizeof(uint32_t);

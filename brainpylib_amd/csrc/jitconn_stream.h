@@ -3,6 +3,7 @@
 #pragma once
 
 #include <cmath>
+#include <type_traits>
 
 #include "common.h"
 #include "mt_wave.h"
@@ -28,10 +29,27 @@ struct WeightWords {
   static constexpr int value = sizeof(T1) == 4 ? 1 : 2;  // mt19937 words per uniform weight
 };
 
-// LDS words one wave needs: the generator state.
+// Normal weights: a wave queues the accepted polar attempts and the positions of their synapses in LDS and
+// works the attempts off `drain` at a time, a lane each (the logarithm, division and square root of a weight
+// are two thirds of the instructions of a unit, and three units of ten are accepted attempts: evaluated in
+// place they ran for all 64 lanes of every batch: matvec and its gradient over 1.5e8 synapses 2.35 ms, now
+// 1.87; matmat of 128 rows with 1e7 synapses 234 -> 214 us).  A batch of 64 units accepts at most 22 attempts (an
+// attempt and its two skips are three units; of double coordinates four, 17), and the positions lag behind the
+// attempts by two at most.  `drain` in double is what leaves 16 waves their 64 KB of static LDS.
+template <typename T1>
+struct NormalQueue {
+  static constexpr uint32_t drain = sizeof(T1) == 4 ? 64 : 40;           // attempts worked off together
+  static constexpr uint32_t attempts = drain + (sizeof(T1) == 4 ? 24 : 18);  // slots
+  static constexpr uint32_t spill = 2 * (attempts - drain);             // positions that may outlast a drain
+  static constexpr int words = static_cast<int>(attempts * (2 * sizeof(T1) / 4 + 2));
+  static_assert(spill <= kWave && 2 * drain <= 2 * kWave, "one lane per attempt and per position moved");
+};
+
+// LDS words one wave needs: the generator state and, for normal weights, the queue behind it.
 template <typename T1, int W>
 struct StreamLds {
-  static constexpr int words = kMtStateWords;
+  static constexpr int words = kMtStateWords + (W == kNormal ? NormalQueue<T1>::words : 0);
+  static_assert(words % 2 == 0, "the queue of the next wave stays aligned");
 };
 
 __device__ __forceinline__ double read_lane_f64(double v, int l) {
@@ -72,72 +90,70 @@ __device__ __forceinline__ PolarF32 polar_attempt(uint32_t w0, uint32_t w1) {
   return a;
 }
 
-// Roles of the 64 two-word units of one batch of a normal-weight stream.  Which units are polar
-// attempts and which are skips follows from a small automaton over the units' "this attempt
-// would be accepted" bits; it runs on the scalar unit eight units at a time through a table:
-// entry [byte of accept bits] holds, for every state the automaton can enter the eight units in
-// (one byte per state), the units at which an attempt is accepted and 8 x the state it leaves in.
-struct RoleEntry {
-  uint32_t accept, next;
-};
-struct RoleTable {
-  RoleEntry e[256];
-};
-// float: 0 attempt expected, 1 first skip after an accepted attempt, 2 second skip.
-// double (kStates == 4; a unit is one coordinate): 0 X expected, 1 Y expected, 2 first skip, 3 second skip.
-template <int kStates>
-constexpr RoleTable make_role_table() {
-  RoleTable t{};
-  for (uint32_t b = 0; b < 256; ++b) {
-    uint32_t acc = 0, nxt = 0;
-    for (int s0 = 0; s0 < kStates; ++s0) {
-      int s = s0;
-      uint32_t e = 0;
-      for (int i = 0; i < 8; ++i) {
-        const bool ok = (b >> i) & 1u;
-        if (kStates == 3) {
-          if (s == 0) {
-            if (ok) e |= 1u << i, s = 1;
-          } else {
-            s = (s == 1) ? 2 : 0;
-          }
-        } else {
-          if (s == 0) s = 1;
-          else if (s == 1) {
-            if (ok) e |= 1u << i, s = 2;
-            else s = 0;
-          } else {
-            s = (s == 2) ? 3 : 0;
-          }
-        }
-      }
-      acc |= e << (8 * s0);
-      nxt |= static_cast<uint32_t>(8 * s) << (8 * s0);
-    }
-    t.e[b].accept = acc;
-    t.e[b].next = nxt;
-  }
-  return t;
+// Roles of the 64 two-word units of one batch of a normal-weight stream: which are polar attempts and which
+// are skips follows from a small automaton over the units' "this attempt would be accepted" bits.  A unit is a
+// map of the automaton's four states, one byte per state, and one byte permutation composes two maps, so a
+// prefix scan over the lanes gives every lane the state behind its unit.  (On the scalar unit, eight units at
+// a time through a table, the automaton took 64 scalar instructions a batch; a CU issues one of those a cycle
+// for its 32 waves, as many as vector instructions: matvec and its gradient over 1.5e8 synapses 2.58 ms, with
+// the scan 1.87.)
+// float: 0 attempt expected (the last one was rejected), 1 first skip expected, 2 second skip expected, 3 attempt expected
+// (the second skip was the last unit).
+// double (a unit is one coordinate): 0 X expected, 1 Y expected, 2 first skip, 3 second skip expected.
+constexpr uint32_t state_map(uint32_t from0, uint32_t from1, uint32_t from2, uint32_t from3) {
+  return from0 | from1 << 8 | from2 << 16 | from3 << 24;
 }
-static __constant__ const RoleTable kRolesF32 = make_role_table<3>();
-static __constant__ const RoleTable kRolesF64 = make_role_table<4>();
+template <bool kWide>
+struct UnitMaps {
+  static constexpr uint32_t accepts = kWide ? state_map(1, 2, 3, 0) : state_map(1, 2, 3, 1);
+  static constexpr uint32_t rejects = kWide ? state_map(1, 0, 3, 0) : state_map(0, 2, 3, 0);
+};
+template <int kDpp, int kRows>
+__device__ __forceinline__ uint32_t compose_behind(uint32_t map) {
+  const uint32_t before = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(
+    static_cast<int>(state_map(0, 1, 2, 3)), static_cast<int>(map), kDpp, kRows, 0xf, false));
+  return __builtin_amdgcn_perm(map, map, before);
+}
+// the state behind this lane's unit; `entered` is the state in front of lane 0's and becomes the one behind lane 63's
+template <bool kWide>
+__device__ __forceinline__ uint32_t state_behind(bool ok, uint32_t &entered) {
+  uint32_t map = ok ? UnitMaps<kWide>::accepts : UnitMaps<kWide>::rejects;
+  map = compose_behind<0x111, 0xf>(map);  // row_shr:1, 2, 4, 8, then the rows' totals (wave_inclusive_scan_u32)
+  map = compose_behind<0x112, 0xf>(map);
+  map = compose_behind<0x114, 0xf>(map);
+  map = compose_behind<0x118, 0xf>(map);
+  map = compose_behind<0x142, 0xa>(map);
+  map = compose_behind<0x143, 0xc>(map);
+  const uint32_t state = __builtin_amdgcn_ubfe(map, 8u * entered, 8u);
+  entered = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(state), kWave - 1));
+  return state;
+}
 
-// accept mask of a batch; `state8` = 8 x automaton state, carried from batch to batch
-__device__ __forceinline__ uint64_t accepted_units(const RoleTable &tab, uint64_t okm, uint32_t &state8) {
-  uint64_t acc = 0;
-  uint32_t sh = state8;
-#pragma unroll
-  for (int c = 0; c < 8; ++c) {
-    const RoleEntry t = tab.e[static_cast<uint32_t>(okm >> (8 * c)) & 0xffu];
-    acc |= static_cast<uint64_t>((t.accept >> sh) & 0xffu) << (8 * c);
-    sh = (t.next >> sh) & 0xffu;
-  }
-  state8 = sh;
-  return acc;
+// The two weights of an accepted attempt (libstdc++: y * mult first, then the saved x * mult)
+__device__ __forceinline__ void polar_weights(float x, float y, float mean, float sigma, float &w_first, float &w_second) {
+  const float r2 = __fadd_rn(__fmul_rn(x, x), __fmul_rn(y, y));
+  const float mult = __fsqrt_rn(__fdiv_rn(__fmul_rn(-2.0f, logf(r2)), r2));
+  w_first = __fadd_rn(__fmul_rn(__fmul_rn(y, mult), sigma), mean);
+  w_second = __fadd_rn(__fmul_rn(__fmul_rn(x, mult), sigma), mean);
+}
+__device__ __forceinline__ void polar_weights(double x, double y, double mean, double sigma, double &w_first, double &w_second) {
+  const double r2 = __dadd_rn(__dmul_rn(x, x), __dmul_rn(y, y));
+  const double mult = sqrt(-2 * log(r2) / r2);
+  w_first = __dadd_rn(__dmul_rn(__dmul_rn(y, mult), sigma), mean);
+  w_second = __dadd_rn(__dmul_rn(__dmul_rn(x, mult), sigma), mean);
+}
+
+// number of lanes below this one in `mask`, plus `base`
+__device__ __forceinline__ uint32_t lanes_below(uint64_t mask, uint32_t base) {
+  return __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(mask >> 32),
+                                   __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(mask), base));
 }
 
 // Walks stream std::mt19937{stream_seed} over [0, n): calls f(index, weight, valid) once per
-// batch with the whole wave converged; `valid` marks the lanes that hold a synapse of the row.
+// batch with the whole wave converged; `valid` marks the lanes that hold a synapse of the row: the first
+// lanes of the wave, their indices rising from lane to lane.  Normal weights come two at a time: synapses
+// 2 l and 2 l + 1 of a group are lane l's.  f is called for the first and then for the second ones, or, if
+// it can be called so, f(index, weight, valid, index, weight, valid) for both.
 //
 // `pre` points at the stream's 624 seeded state words when they were prepared by
 // launch_seed_streams(); with nullptr the wave seeds the generator itself on the scalar unit.
@@ -196,109 +212,99 @@ __device__ __forceinline__ void walk_stream(uint32_t *st, int lane, uint32_t str
       if (done) break;
       carry += __builtin_amdgcn_readlane(incl, kWave - 1);
     }
-  } else if constexpr (W == kNormal && sizeof(T1) == 4) {
-    // stream in 2-word units: K  (A..A K) (K) (A..A K) (K) ...   A = polar attempt (x word, y word),
-    // the last A of a group is the accepted one; the first K after it belongs to the synapse
-    // that receives y*mult, the second K to the synapse that receives the cached x*mult.
-    // Every lane evaluates its unit both ways; accepted_units() assigns the roles.
-    uint32_t w0[2] = {1u, 1u};
-    mt_generate<2>(st, pos, lane, 1, w0);
-    uint32_t carry = __builtin_amdgcn_readfirstlane(skip_from_words(w0[0], w0[1], log_p));
-    uint32_t state8 = 0;
-    float prev_x62 = 0.f, prev_x63 = 0.f, prev_y63 = 0.f;
-    for (uint32_t b = 0; b < max_batches; ++b) {
-      uint32_t w[2] = {1u, 1u};
-      mt_generate<2>(st, pos, lane, kWave, w);
-      const PolarF32 a = polar_attempt(w[0], w[1]);
-      const uint64_t okm = __ballot(a.ok);
-      // An accepted attempt at unit q makes q + 1 the first and q + 2 the second skip; a role
-      // that falls past unit 63 belongs to the next batch and comes back through `state8`.
-      const uint32_t entered = state8;
-      const uint64_t acc = accepted_units(kRolesF32, okm, state8);
-      const uint64_t k1 = (acc << 1) | (entered == 8u ? 1ull : 0ull);
-      const uint64_t k2 = (acc << 2) | (entered == 8u ? 2ull : entered == 16u ? 1ull : 0ull);
-      const bool is_k1 = (k1 >> lane) & 1ull;
-      const bool is_k2 = (k2 >> lane) & 1ull;
-      const bool is_k = is_k1 || is_k2;
-      float xw = 0.f, yw = 0.f;
-      if (a.ok) {
-        const float mult = __fsqrt_rn(__fdiv_rn(__fmul_rn(-2.0f, logf(a.r2)), a.r2));
-        xw = __fmul_rn(a.x, mult);
-        yw = __fmul_rn(a.y, mult);
-      }
-      float y_m1 = wave_shift_up1(yw);
-      float x_m2 = wave_shift_up1(wave_shift_up1(xw));
-      if (lane == 0) y_m1 = prev_y63, x_m2 = prev_x62;
-      if (lane == 1) x_m2 = prev_x63;
-      const float raw = is_k1 ? y_m1 : x_m2;
-      const T1 weight = static_cast<T1>(__fadd_rn(__fmul_rn(raw, static_cast<float>(wb)), static_cast<float>(wa)));
-      const uint32_t skip_any = skip_from_words(w[0], w[1], log_p);  // wave-converged call
-      const uint32_t skip = is_k ? skip_any : 0u;
-      const uint32_t incl = wave_inclusive_scan_u32(skip);
-      const uint32_t idx = carry + incl - skip;
-      const uint64_t done = __ballot(is_k && idx >= n);
-      const int first = done ? (__ffsll(static_cast<unsigned long long>(done)) - 1) : kWave;
-      f(idx, weight, is_k && lane < first);
-      if (done) break;
-      carry += __builtin_amdgcn_readlane(incl, kWave - 1);
-      prev_x62 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, xw), 62));
-      prev_x63 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, xw), 63));
-      prev_y63 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, yw), 63));
-    }
   } else {
-    // std::normal_distribution<double>: every draw is one canonical double, so the stream again
-    // consists of 2-word units:  K  (X Y .. X Y K) (K) (X Y .. X Y K) (K) ...   X, Y = the two
-    // coordinates of a polar attempt, the last pair of a group is the accepted one; the first K
-    // after it belongs to the synapse that receives y*mult, the second K to the synapse that
-    // receives the cached x*mult.  Every lane evaluates its unit as a coordinate (and, with its
-    // left neighbour's, as the end of an attempt) and as a skip; accepted_units() assigns the roles.
+    // float: the stream in 2-word units is  K  (A..A K) (K) (A..A K) (K) ...   A = polar attempt (x word, y
+    // word), the last A of a group is the accepted one.  double: every draw is one canonical double, so the
+    // units are  K  (X Y .. X Y K) (K) ...   X, Y = the two coordinates of an attempt.  The first K after an
+    // accepted attempt belongs to the synapse that receives y*mult, the second K to the one that receives the
+    // saved x*mult.  Every lane evaluates its unit both ways; state_behind() assigns the roles.  Synapses 2 a
+    // and 2 a + 1 of the stream so belong to its accepted attempt a.
+    using Q = NormalQueue<T1>;
+    constexpr bool kWide = sizeof(T1) == 8;
+    T1 *const q_attempt = reinterpret_cast<T1 *>(st + kMtStateWords);           // x, y of the attempts queued
+    uint32_t *const q_pos = st + kMtStateWords + Q::attempts * (2 * sizeof(T1) / 4);  // their synapses' positions
+    uint32_t n_attempt = 0, n_pos = 0;
     uint32_t w0[2] = {1u, 1u};
     mt_generate<2>(st, pos, lane, 1, w0);
     uint32_t carry = __builtin_amdgcn_readfirstlane(skip_from_words(w0[0], w0[1], log_p));
-    uint32_t state8 = 0;
-    double prev_v63 = 0.0, prev_x62 = 0.0, prev_x63 = 0.0, prev_y63 = 0.0;
+    uint32_t entered = 0;
+    double prev_v63 = 0.0;
     for (uint32_t b = 0; b < max_batches; ++b) {
       uint32_t w[2] = {1u, 1u};
       mt_generate<2>(st, pos, lane, kWave, w);
-      const double v = __dsub_rn(__dmul_rn(2.0, canonical_f64(w[0], w[1])), 1.0);
-      double v_m1 = wave_shift_up1(v);
-      if (lane == 0) v_m1 = prev_v63;
-      const double r2 = __dadd_rn(__dmul_rn(v_m1, v_m1), __dmul_rn(v, v));
-      const bool ok = !(r2 > 1.0 || r2 == 0.0);  // an attempt (lane - 1, lane) would be accepted
-      const uint64_t okm = __ballot(ok);
-      // unit 0 may complete the attempt begun by the previous batch's last unit (state 1)
-      const uint32_t entered = state8;
-      const uint64_t acc = accepted_units(kRolesF64, okm, state8);
-      const uint64_t k1 = (acc << 1) | (entered == 16u ? 1ull : 0ull);
-      const uint64_t k2 = (acc << 2) | (entered == 16u ? 2ull : entered == 24u ? 1ull : 0ull);
-      const bool is_k1 = (k1 >> lane) & 1ull;
-      const bool is_k2 = (k2 >> lane) & 1ull;
-      const bool is_k = is_k1 || is_k2;
-      double xw = 0.0, yw = 0.0;
-      if (ok) {
-        const double mult = sqrt(-2 * log(r2) / r2);
-        xw = __dmul_rn(v_m1, mult);
-        yw = __dmul_rn(v, mult);
+      T1 x, y;
+      bool ok;
+      if constexpr (!kWide) {
+        const PolarF32 a = polar_attempt(w[0], w[1]);
+        x = a.x, y = a.y, ok = a.ok;
+      } else {
+        y = __dsub_rn(__dmul_rn(2.0, canonical_f64(w[0], w[1])), 1.0);
+        x = wave_shift_up1(y);
+        if (lane == 0) x = prev_v63;
+        prev_v63 = read_lane_f64(y, kWave - 1);
+        const double r2 = __dadd_rn(__dmul_rn(x, x), __dmul_rn(y, y));
+        ok = !(r2 > 1.0 || r2 == 0.0);  // an attempt (lane - 1, lane) would be accepted
       }
-      double y_m1 = wave_shift_up1(yw);
-      double x_m2 = wave_shift_up1(wave_shift_up1(xw));
-      if (lane == 0) y_m1 = prev_y63, x_m2 = prev_x62;
-      if (lane == 1) x_m2 = prev_x63;
-      const double raw = is_k1 ? y_m1 : x_m2;
-      const T1 weight = static_cast<T1>(__dadd_rn(__dmul_rn(raw, static_cast<double>(wb)), static_cast<double>(wa)));
-      const uint32_t skip_any = skip_from_words(w[0], w[1], log_p);  // wave-converged call
+      const uint32_t before = entered;
+      const uint32_t state = state_behind<kWide>(ok, entered);
+      const bool accepted = state == (kWide ? 2u : 1u);
+      uint64_t skips;
+      if constexpr (kWide) {
+        const uint64_t k1 = __ballot(state == 3u);
+        skips = k1 | (k1 << 1) | (before == 3u ? 1ull : 0ull);
+      } else {
+        skips = __ballot(state >= 2u);
+      }
+      const bool is_k = __builtin_amdgcn_inverse_ballot_w64(skips);
+      const uint32_t skip_any = skip_from_words(w[0], w[1], log_p, skips);  // wave-converged call
       const uint32_t skip = is_k ? skip_any : 0u;
       const uint32_t incl = wave_inclusive_scan_u32(skip);
       const uint32_t idx = carry + incl - skip;
-      const uint64_t done = __ballot(is_k && idx >= n);
-      const int first = done ? (__ffsll(static_cast<unsigned long long>(done)) - 1) : kWave;
-      f(idx, weight, is_k && lane < first);
+      const uint64_t acc = __ballot(accepted);
+      if (accepted) {
+        T1 *const q = q_attempt + 2u * lanes_below(acc, n_attempt);
+        q[0] = x;
+        q[1] = y;
+      }
+      if (is_k) q_pos[lanes_below(skips, n_pos)] = idx;
+      const uint64_t done = __ballot(idx >= n) & skips;
+      // (the positions rise: the synapses of the row are the skips below the first one at or past n)
+      n_attempt += static_cast<uint32_t>(__popcll(acc));
+      n_pos += static_cast<uint32_t>(__popcll(done ? skips & (done ^ (done - 1u)) & ~done : skips));
+      while (n_pos >= 2u * Q::drain || (done && n_pos != 0u)) {
+        __builtin_amdgcn_wave_barrier();
+        const uint32_t at = static_cast<uint32_t>(lane);
+        const bool have = kWave == static_cast<int>(Q::drain) || at < Q::drain;
+        const bool valid0 = have && 2u * at < n_pos, valid1 = have && 2u * at + 1u < n_pos;
+        T1 first = T1(0), second = T1(0);
+        uint32_t idx0 = 0, idx1 = 0;
+        if (valid0) {
+          polar_weights(q_attempt[2u * at], q_attempt[2u * at + 1u], wa, wb, first, second);
+          idx0 = q_pos[2u * at], idx1 = q_pos[2u * at + 1u];
+          if (!valid1) idx1 = 0;
+        }
+        if constexpr (std::is_invocable_v<F &, uint32_t, T1, bool, uint32_t, T1, bool>) {
+          f(idx0, first, valid0, idx1, second, valid1);
+        } else {
+#pragma unroll kWide ? 1 : 2
+          for (int h = 0; h < 2; ++h) f(h ? idx1 : idx0, h ? second : first, h ? valid1 : valid0);
+        }
+        if (n_pos <= 2u * Q::drain && done) break;
+        // what the group left goes to the front
+        __builtin_amdgcn_wave_barrier();
+        if (at < Q::spill) {
+          const T1 a = q_attempt[2u * Q::drain + at];
+          const uint32_t p = q_pos[2u * Q::drain + at];
+          __builtin_amdgcn_wave_barrier();
+          q_attempt[at] = a;
+          q_pos[at] = p;
+        }
+        __builtin_amdgcn_wave_barrier();
+        n_attempt -= Q::drain;
+        n_pos -= 2u * Q::drain;
+      }
       if (done) break;
       carry += __builtin_amdgcn_readlane(incl, kWave - 1);
-      prev_v63 = read_lane_f64(v, kWave - 1);
-      prev_x62 = read_lane_f64(xw, kWave - 2);
-      prev_x63 = read_lane_f64(xw, kWave - 1);
-      prev_y63 = read_lane_f64(yw, kWave - 1);
     }
   }
 }

@@ -230,11 +230,12 @@ __device__ __forceinline__ uint32_t skip_fast(uint32_t lo, uint32_t hi, const Sk
 
 // If any lane of the wave is inside the band, the whole wave takes the exact path (a wave-uniform
 // branch); for conn_prob around 1e-3 that happens in a few per cent of the batches, for very sparse
-// matrices (guard >= 0.5) always.
-__device__ __forceinline__ uint32_t skip_from_words(uint32_t lo, uint32_t hi, const SkipParams &sp) {
+// matrices (guard >= 0.5) always.  Only the lanes in `needed` have to be right.
+__device__ __forceinline__ uint32_t skip_from_words(uint32_t lo, uint32_t hi, const SkipParams &sp,
+                                                    uint64_t needed = ~0ull) {
   bool safe;
   const uint32_t fast = skip_fast(lo, hi, sp, safe);
-  if (__ballot(!safe) == 0) return fast;
+  if ((__ballot(!safe) & needed) == 0) return fast;
   return skip_exact(lo, hi, sp);
 }
 

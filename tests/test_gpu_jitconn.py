@@ -611,6 +611,32 @@ def test_version_argument_of_the_dense_wrappers(cuda):
     _lib.custom_call("gpu_matvec_prob_homo_v1_float", [t, out], _lib.build_jitconn_prob_homo_descriptor(10, 10, 1, -0.5))
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n_syn", [1, 2, 3, 22, 79, 80, 81, 82, 127, 128, 129, 130, 159, 160, 161, 255, 256, 257, 1000])
+def test_normal_weights_worked_off_in_groups(cuda, oracle_mod, n_syn, dtype):
+  # A wave works the weights of 128 synapses (80 in double) off at a time.  With conn_prob 1 a stream holds
+  # every index once: streams that end just before, at and behind the end of a group, in every operator.
+  rng = np.random.default_rng(n_syn)
+  lp, m = oracle_mod.log_p_of(1.0), 37
+  vec = rng.uniform(0.5, 2.0, n_syn).astype(dtype)
+  ev = (rng.random(n_syn) < 0.3) | (np.arange(n_syn) == n_syn - 1)
+  kw = dict(w_kind="normal", w_a=0.5, w_b=2.0, log_p=lp, seed=11)
+  print("case", n_syn, dtype.__name__, flush=True)
+  for inp, dense in ((vec, True), (ev, False)):
+    want, mag = oracle_mod.jitconn_matvec(inp, n_row=m, n_col=n_syn, dense=dense, return_abs=True, out_dtype=dtype, **kw)
+    got = kernel_call(inp, n_row=m, n_col=n_syn, col_walk=False, dense=dense, out_dtype=dtype, **kw)
+    assert_close_reordered(got, want, mag, dtype, what="normal weights, row walk")
+  x = rng.uniform(0.5, 2.0, m).astype(dtype)
+  want, mag = oracle_mod.jitconn_matvec(x, n_row=n_syn, n_col=m, col_walk=True, dense=True, return_abs=True, **kw)
+  got = kernel_call(x, n_row=n_syn, n_col=m, col_walk=True, dense=True, **kw)
+  assert_close_reordered(got, want, mag, dtype, what="normal weights, column walk")
+  X = rng.uniform(0.5, 2.0, (70, n_syn)).astype(dtype)
+  want, mag = oracle_mod.jitconn_matmat(X, n=m, return_abs=True, **kw)
+  got = bpl.matmat_prob_conn_normal_weight(torch.from_numpy(X).cuda(), w_mu=0.5, w_sigma=2.0, conn_prob=1.0,
+                                           shape=(n_syn, m), seed=11).cpu().numpy()
+  assert_close_reordered(got, want, mag, dtype, what="normal weights, matmat")
+
+
 @pytest.mark.parametrize("n_out,n_in", [(8192, 3000), (10_007, 200_000), (20_000, 400_000), (70_001, 5000)])
 def test_row_walk_with_generators_seeded_inside_the_kernel(cuda, oracle_mod, n_out, n_in):
   # from 8,192 outputs the row walk seeds its generators itself, 64 streams at a time, into rings of
