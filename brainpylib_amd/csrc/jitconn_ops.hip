@@ -100,7 +100,7 @@ __global__ __launch_bounds__(1024, (BITS == 2 || (W == kNormal && sizeof(T1) == 
       if (W == kHomo) cnt += static_cast<uint32_t>(__popcll(late_coarse & __builtin_amdgcn_ballot_w64(bit)));
       else if (bit && late_lane) acc += static_cast<double>(late_w);
     };
-    walk_stream<T1, W>(st, lane, seed + o, pre, n_in, log_p, wa, wb, [&](uint32_t idx, T1 w, bool valid) {
+    walk_stream<T1, W, W != kNormal>(st, lane, seed + o, pre, n_in, log_p, wa, wb, [&](uint32_t idx, T1 w, bool valid) {
       if constexpr (IN == kInEvent && BITS == 2) {
         settle();
         // bit c = idx >> g of the coarse bitmap: word c >> 5, bit c & 31 (the bit-field extract takes the
@@ -864,14 +864,23 @@ __global__ __launch_bounds__(256) void check_skips_kernel(uint32_t seed, uint64_
     const uint32_t exact = skip_exact(lo, hi, sp);
     if (!safe) ++untrusted;
     else if (fast != exact) ++differ;
+    const uint32_t quick = skip_quick(hi, sp, safe);
+    if (sp.quick && safe && quick != exact) ++differ;
   }
   if (differ) atomicAdd(&counts[0], differ);
   if (untrusted) atomicAdd(&counts[1], untrusted);
 }
 
-// |hardware log2 - log2| over every fp32 in [0.5, 1): the largest, as the bits of a double
-__global__ __launch_bounds__(256) void check_log2_kernel(unsigned long long *__restrict__ worst) {
+// |hardware log2 - log2| over every fp32 in [0.5, 1): the largest, as the bits of a double; and over those in
+// [2^-10, 1) against what the quick path allows it, counted with the draws that differ
+__global__ __launch_bounds__(256) void check_log2_kernel(unsigned long long *__restrict__ worst,
+                                                         unsigned long long *__restrict__ differ) {
   const uint32_t t = blockIdx.x * 256u + threadIdx.x;  // < 2^23
+  for (uint32_t e = 0; e < 10u; ++e) {
+    const float u = __uint_as_float((0x3f000000u - (e << 23)) | t);
+    const double off = fabs(static_cast<double>(__builtin_amdgcn_logf(u)) - log2(static_cast<double>(u)));
+    if (!(off <= 9.6e-7)) atomicAdd(differ, 1ull);
+  }
   const float m = __uint_as_float(0x3f000000u | t);
   const double err = fabs(static_cast<double>(__log2f(m)) - log2(static_cast<double>(m)));
   double wave_worst = err;
@@ -899,7 +908,7 @@ extern "C" int bpl_selfcheck_jitconn_skips(bpl_stream_t stream, uint32_t seed, u
   hipStream_t s = static_cast<hipStream_t>(stream);
   unsigned long long *c = reinterpret_cast<unsigned long long *>(counts);
   hipLaunchKernelGGL(check_skips_kernel, dim3(2048), dim3(256), 0, s, seed, n_draws, near_boundaries ? 1 : 0, log_p, c);
-  hipLaunchKernelGGL(check_log2_kernel, dim3((1u << 23) / 256u), dim3(256), 0, s, c + 2);
+  hipLaunchKernelGGL(check_log2_kernel, dim3((1u << 23) / 256u), dim3(256), 0, s, c + 2, c);
   return check_launch("bpl_selfcheck_jitconn_skips") ? 0 : 1;
 }
 

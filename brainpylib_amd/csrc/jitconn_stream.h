@@ -158,11 +158,13 @@ __device__ __forceinline__ uint32_t lanes_below(uint64_t mask, uint32_t base) {
 // `pre` points at the stream's 624 seeded state words when they were prepared by
 // launch_seed_streams(); with nullptr the wave seeds the generator itself on the scalar unit.
 //
+// kQuick: skips are first tried on the upper words alone (skip_quick).
+//
 // `loaded()` is called once, when the generator state is in LDS and `pre` is no longer read.
 struct NoLoadHook {
   __device__ __forceinline__ void operator()() const {}
 };
-template <typename T1, int W, typename F, typename L = NoLoadHook>
+template <typename T1, int W, bool kQuick = false, typename F, typename L = NoLoadHook>
 __device__ __forceinline__ void walk_stream(uint32_t *st, int lane, uint32_t stream_seed, const uint32_t *pre,
                                             uint32_t n, double log_p_, T1 wa, T1 wb, F &&f, L &&loaded = L()) {
   const SkipParams log_p = make_skip_params(log_p_);
@@ -178,8 +180,8 @@ __device__ __forceinline__ void walk_stream(uint32_t *st, int lane, uint32_t str
     uint32_t carry = 0;
     for (uint32_t b = 0; b < max_batches; ++b) {
       uint32_t w[2] = {1u, 1u};
-      mt_generate<2>(st, pos, lane, kWave, w);
-      const uint32_t skip = skip_from_words(w[0], w[1], log_p);
+      mt_generate<2, kQuick ? 0 : -1>(st, pos, lane, kWave, w);
+      const uint32_t skip = skip_from_words<kQuick, !kQuick>(w[0], w[1], log_p);
       const uint32_t idx = carry + wave_inclusive_scan_u32(skip);
       // (the positions rise from lane to lane: the lanes of the row are exactly those below n)
       const bool over = idx >= n;
@@ -195,14 +197,14 @@ __device__ __forceinline__ void walk_stream(uint32_t *st, int lane, uint32_t str
     constexpr int NL = (K == 3) ? 64 : 56;  // K * NL <= 227
     uint32_t w0[2] = {1u, 1u};
     mt_generate<2>(st, pos, lane, 1, w0);
-    uint32_t carry = __builtin_amdgcn_readfirstlane(skip_from_words(w0[0], w0[1], log_p));
+    uint32_t carry = __builtin_amdgcn_readfirstlane(skip_from_words<false, true>(w0[0], w0[1], log_p, 1ull));
     for (uint32_t b = 0; b < max_batches; ++b) {
       uint32_t w[K];
 #pragma unroll
       for (int i = 0; i < K; ++i) w[i] = 1u;
-      mt_generate<K>(st, pos, lane, NL, w);
+      mt_generate<K, kQuick ? WW : -1>(st, pos, lane, NL, w);
       const T1 weight = uniform_weight(w, wa, wb);
-      uint32_t skip = skip_from_words(w[WW], w[WW + 1], log_p);
+      uint32_t skip = skip_from_words<kQuick, !kQuick>(w[WW], w[WW + 1], log_p, ~0ull >> (kWave - NL));
       if (lane >= NL) skip = 0;
       const uint32_t incl = wave_inclusive_scan_u32(skip);
       const uint32_t idx = carry + incl - skip;
@@ -226,7 +228,7 @@ __device__ __forceinline__ void walk_stream(uint32_t *st, int lane, uint32_t str
     uint32_t n_attempt = 0, n_pos = 0;
     uint32_t w0[2] = {1u, 1u};
     mt_generate<2>(st, pos, lane, 1, w0);
-    uint32_t carry = __builtin_amdgcn_readfirstlane(skip_from_words(w0[0], w0[1], log_p));
+    uint32_t carry = __builtin_amdgcn_readfirstlane(skip_from_words<false, true>(w0[0], w0[1], log_p, 1ull));
     uint32_t entered = 0;
     double prev_v63 = 0.0;
     for (uint32_t b = 0; b < max_batches; ++b) {
@@ -256,7 +258,7 @@ __device__ __forceinline__ void walk_stream(uint32_t *st, int lane, uint32_t str
         skips = __ballot(state >= 2u);
       }
       const bool is_k = __builtin_amdgcn_inverse_ballot_w64(skips);
-      const uint32_t skip_any = skip_from_words(w[0], w[1], log_p, skips);  // wave-converged call
+      const uint32_t skip_any = skip_from_words<false, true>(w[0], w[1], log_p, skips);  // wave-converged call
       const uint32_t skip = is_k ? skip_any : 0u;
       const uint32_t incl = wave_inclusive_scan_u32(skip);
       const uint32_t idx = carry + incl - skip;
