@@ -1,5 +1,6 @@
 """Argument plumbing shared by the operator wrappers: everything becomes a contiguous torch
 CUDA tensor (device memory is PyTorch-ROCm's; nothing is computed with torch)."""
+import inspect
 import struct
 
 import numpy as np
@@ -75,3 +76,11 @@ def _np_to_torch(dt):
 
 def is_index_dtype(dt):
   return dt in _INDEX_DTYPES
+
+
+def keep_signature(function):
+  """Class decorator for autograd functions: torch binds the arguments of one with a ``setup_context`` through
+  ``inspect.signature(forward)`` on every call and builds it anew each time; kept on ``forward`` it is only
+  looked up."""
+  function.forward.__signature__ = inspect.signature(function.forward)
+  return function

@@ -9,7 +9,7 @@ from typing import Tuple
 import torch
 
 from . import _lib, sparse_ops
-from ._tensors import FLOAT_DTYPES, as_tensor, device_of, is_index_dtype, to_device
+from ._tensors import FLOAT_DTYPES, as_tensor, device_of, is_index_dtype, keep_signature, to_device
 
 __all__ = ["event_csr_matvec", "event_csr_matvec_batching", "event_info"]
 
@@ -87,6 +87,7 @@ def _launch(data, indices, indptr, events, shape, transpose):
   return out
 
 
+@keep_signature
 class _EventCSRMatvec(torch.autograd.Function):
   """Differentiation rules of event_csr_matvec
   (brainpylib/_src/event_ops/event_csr_matvec.py:439-463).  Tangent of the weights: the same

@@ -15,7 +15,7 @@ import numpy as np
 import torch
 
 from . import _lib
-from ._tensors import FLOAT_DTYPES, as_tensor, device_of, to_device
+from ._tensors import FLOAT_DTYPES, as_tensor, device_of, keep_signature, to_device
 
 __all__ = [
   'event_matvec_prob_conn_homo_weight', 'event_matvec_prob_conn_uniform_weight',
@@ -98,6 +98,7 @@ def _launch(fn_prefix, w_kind, inp, out_dtype, suffix, *, conn_prob, shape, seed
   return out
 
 
+@keep_signature
 class _JitconnMatvec(torch.autograd.Function):
   """Differentiation rules of the jitconn matvec primitives with respect to the input vector
   (brainpylib/_src/jitconn_ops/event_matvec.py:242-273, matvec.py:371-409): the tangent goes

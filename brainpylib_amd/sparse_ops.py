@@ -11,7 +11,7 @@ from typing import Tuple
 import torch
 
 from . import _lib
-from ._tensors import FLOAT_DTYPES, as_tensor, device_of, is_index_dtype, to_device
+from ._tensors import FLOAT_DTYPES, as_tensor, device_of, is_index_dtype, keep_signature, to_device
 
 __all__ = ["csr_matvec", "cusparse_csr_matvec", "csr_to_coo", "coo_to_csr", "csr_to_dense", "check_csr"]
 
@@ -166,6 +166,7 @@ def _gradients(data, indices, indptr, row_vector, col_vector, shape, want_sums):
   return products, sums if want_sums else None
 
 
+@keep_signature
 class _CSRMatvec(torch.autograd.Function):
   """Differentiation rules of the CSR matrix-vector product
   (brainpylib/_src/sparse_ops/cusparse_matvec.py:281-308): tangents go through the same
