@@ -612,7 +612,17 @@ __global__ __launch_bounds__(256) void sum_partials_kernel(const F *__restrict__
 // gather
 // ------------------------------------------------------------------------------------------------
 
-constexpr uint32_t kHubSteps = 64;  // a row of more steps than this is left to the whole workgroup (gather_hub_rows)
+// A row of more nonzeros than this is left to gather_hub_rows(), `step` being what the walk takes of a row at once: one
+// of more than 4 steps and 4 times the mean (rows of one length with binomial scatter stay below that from 10 per row
+// on), or of more than 64 steps in any case.  A step is a chain of dependent loads, 0.7 us: with 64 steps alone the
+// longest rows of an uneven matrix were the last to end by far (17,683 rows of 150 on average, log-normal with
+// sigma 1, weights per nonzero, float: 51 us, now 26, with a dense vector 42 and 18; 2,493 rows of 1,735, double: 86 us,
+// now 39).
+constexpr uint32_t kHubSteps = 64;
+__device__ __forceinline__ uint32_t hub_length(uint32_t mean, uint32_t step) {
+  const uint32_t low = mean < 0x10000000u && 4u * mean > 4u * step ? 4u * mean : 4u * step;
+  return low < kHubSteps * step ? low : kHubSteps * step;
+}
 
 // G lanes walk the rows assigned to their group as ONE sequence of steps of U*G nonzeros: the
 // column indices of the next step (which may belong to the group's next row) are requested
@@ -662,7 +672,7 @@ template <typename F, typename VT, bool HETER, int MODE, int BITS, int G, int U>
 __device__ __forceinline__ void gather_rows(const F *__restrict__ data, const uint32_t *__restrict__ indices,
                                             const uint32_t *__restrict__ indptr, const VT *__restrict__ x,
                                             F *__restrict__ y, uint32_t n_row, const uint32_t *s_bits,
-                                            uint32_t coarse_g) {
+                                            uint32_t coarse_g, uint32_t hub_len) {
   const uint32_t groups_per_block = blockDim.x / G;
   const uint32_t gl = threadIdx.x % G;
   const uint32_t total_groups = gridDim.x * groups_per_block;
@@ -675,8 +685,7 @@ __device__ __forceinline__ void gather_rows(const F *__restrict__ data, const ui
   constexpr int Q = ((U == 4 || U == 8) && !(MODE == kDense && BITS == 1)) ? 4 : 1;
   auto slot = [&](int u) { return static_cast<uint32_t>(Q * ((u / Q) * G) + u % Q) + static_cast<uint32_t>(Q) * gl; };
   const uint32_t nnz = Q > 1 ? indptr[n_row] : 0u;  // (a run of Q is loaded whole only where the arrays hold all of it)
-  // A row of more than kHubSteps steps looks empty here: gather_hub_rows() gives it to the whole workgroup.
-  constexpr uint32_t hub_len = kHubSteps * U * G;
+  // A row of more than hub_len nonzeros looks empty here: gather_hub_rows() gives it to a wave or the whole workgroup.
   auto bounds = [&](uint32_t r, uint32_t &s, uint32_t &e) {
     s = indptr[r], e = indptr[r + 1];
     if (e - s > hub_len) e = s;
@@ -812,7 +821,7 @@ template <typename F, typename VT, bool HETER, int MODE, int BITS, int U>
 __device__ __forceinline__ void gather_rows_wave(const F *__restrict__ data, const uint32_t *__restrict__ indices,
                                                  const uint32_t *__restrict__ indptr, const VT *__restrict__ x,
                                                  F *__restrict__ y, uint32_t n_row, const uint32_t *s_bits,
-                                                 uint32_t coarse_g) {
+                                                 uint32_t coarse_g, uint32_t hub_len) {
   const uint32_t lane = static_cast<uint32_t>(lane_id());
   const uint32_t waves_per_block = blockDim.x / kWave;
   const uint32_t total_waves = gridDim.x * waves_per_block;
@@ -867,7 +876,7 @@ __device__ __forceinline__ void gather_rows_wave(const F *__restrict__ data, con
     const uint32_t urow = __builtin_amdgcn_readfirstlane(row);
     const uint32_t start = indptr[urow];
     const uint32_t len = indptr[urow + 1] - start;
-    if (len > kHubSteps * U * kWave) continue;  // (a whole workgroup takes it and stores it: gather_hub_rows())
+    if (len > hub_len) continue;  // (a whole workgroup takes it and stores it: gather_hub_rows())
     const uint32_t *ip = indices + start;
     const F *dp = data + (HETER ? start : 0u);
     double acc = 0.0;
@@ -893,14 +902,16 @@ __device__ __forceinline__ void gather_rows_wave(const F *__restrict__ data, con
 
 // Hub rows.  The walks above give a row to G lanes (or one wave), so one row that holds a large share
 // of the nonzeros would be walked by a handful of lanes while the rest of the device is done (a row of
-// 1e6 nonzeros among 20,000 of 50: 19 ms).  They treat a row of more than kHubSteps of their steps as
+// 1e6 nonzeros among 20,000 of 50: 19 ms).  They treat a row of more than hub_len nonzeros as
 // empty, and after its walk every workgroup looks through the bounds of the rows it was dealt again
-// (workgroup b: rows b * gpb + g + k * total_groups, g < gpb) and walks each such row with all its
-// threads: partial sums per lane, a wave sum, one float64 (or integer) LDS atomic per wave.
-// The walk with a wave per row skips such rows without storing anything, and they are dealt one by one
-// (gpb = 1: workgroup b looks at rows b, b + gridDim.x, ...): in a matrix of a few thousand rows that are
-// all this long, sixteen consecutive rows per workgroup would leave most of the device idle (2,000 rows of
+// (workgroup b: rows b * gpb + g + k * total_groups, g < gpb).  Its waves take the ones of up to kHubWave nonzeros
+// in turn, each by itself, and then all its threads the longer ones together: partial sums per lane, a wave sum,
+// one float64 (or integer) LDS atomic per wave.
+// The walk with a wave per row skips such rows without storing anything (they all go to the whole workgroup), and
+// they are dealt one by one (gpb = 1: workgroup b looks at rows b, b + gridDim.x, ...): in a matrix of a few thousand
+// rows that are all this long, sixteen consecutive rows per workgroup would leave most of the device idle (2,000 rows of
 // 50,000: an eighth of the workgroups had rows).
+constexpr uint32_t kHubWave = 4096;  // eight steps of a wave
 template <typename F, typename VT, bool HETER, int MODE, int BITS>
 __device__ __forceinline__ void gather_hub_rows(const F *__restrict__ data, const uint32_t *__restrict__ indices,
                                                 const uint32_t *__restrict__ indptr, const VT *__restrict__ x,
@@ -909,67 +920,88 @@ __device__ __forceinline__ void gather_hub_rows(const F *__restrict__ data, cons
   __shared__ unsigned long long s_mask[1024 / kWave];
   __shared__ double s_acc;
   __shared__ uint32_t s_hits;
-  const uint32_t tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave, nwaves = blockDim.x / kWave;
+  const uint32_t tid = threadIdx.x, lane = tid % kWave, nwaves = blockDim.x / kWave;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const uint32_t total_groups = gridDim.x * gpb;
   const uint32_t first = blockIdx.x * gpb;
   if (first >= n_row) return;
   const uint32_t count = ((n_row - first + total_groups - 1u) / total_groups) * gpb;  // rows dealt to this workgroup
   const F w_homo = HETER ? F(0) : data[0];
   auto row_of = [&](uint32_t i) { return (i / gpb) * total_groups + first + (i % gpb); };
+  // thread t of `team` of them: its part of a row (the sum over the wave)
+  auto walk = [&](uint32_t start, uint32_t len, uint32_t t, uint32_t team, double &acc, uint32_t &hits) {
+    constexpr uint32_t U = 4;  // loads in flight per lane and step; the next step's are requested before this one's are used
+    uint32_t col[U], ncol[U];
+    auto load_cols = [&](uint32_t j0, uint32_t (&c)[U]) {  // (beyond the row: its last index again)
+#pragma unroll
+      for (uint32_t u = 0; u < U; ++u) {
+        const uint32_t j = j0 + u * team;
+        c[u] = indices[start + (j < len ? j : len - 1u)];
+      }
+    };
+    load_cols(t, col);
+    for (uint32_t j0 = t; j0 < len; j0 += U * team) {
+      load_cols(j0 + U * team, ncol);
+#pragma unroll
+      for (uint32_t u = 0; u < U; ++u) {
+        const uint32_t j = j0 + u * team;
+        if (j >= len) continue;
+        if (MODE == kEvent) {
+          if (event_hit<BITS>(s_bits, x, col[u], coarse_g)) {
+            if (HETER) acc += static_cast<double>(data[start + j]);
+            else ++hits;
+          }
+        } else {
+          const F d = HETER ? data[start + j] : w_homo;
+          acc += static_cast<double>(static_cast<F>(static_cast<F>(x[col[u]]) * d));
+        }
+      }
+#pragma unroll
+      for (uint32_t u = 0; u < U; ++u) col[u] = ncol[u];
+    }
+    if (MODE == kEvent && !HETER) hits = wave_sum(hits);
+    else acc = wave_sum(acc);
+  };
   for (uint32_t i0 = 0; i0 < count; i0 += blockDim.x) {
-    bool hub = false;
+    uint32_t len = 0;
     if (i0 + tid < count) {
       const uint32_t r = row_of(i0 + tid);
-      if (r < n_row) hub = indptr[r + 1] - indptr[r] > hub_len;
+      if (r < n_row) len = indptr[r + 1] - indptr[r];
     }
-    const unsigned long long mine = __ballot(hub);
+    const bool hub = len > hub_len, alone = hub && (gpb == 1u || len > kHubWave);
+    const unsigned long long by_wave = __ballot(hub && !alone), by_all = __ballot(alone);
     if (!__syncthreads_or(hub)) continue;  // (the usual case: none)
-    if (lane == 0) s_mask[wave] = mine;
+    if (lane == 0) s_mask[wave] = by_wave;
+    __syncthreads();
+    uint32_t turn = 0;
+    for (uint32_t w = 0; w < nwaves; ++w) {
+      unsigned long long m = s_mask[w];
+      for (; m != 0; m &= m - 1ull, ++turn) {
+        if (turn % nwaves != wave) continue;
+        const uint32_t r = row_of(i0 + w * kWave + static_cast<uint32_t>(__ffsll(m) - 1));
+        const uint32_t start = indptr[r];
+        double acc = 0.0;
+        uint32_t hits = 0;
+        walk(start, indptr[r + 1] - start, lane, kWave, acc, hits);
+        if (lane == 0) y[r] = (MODE == kEvent && !HETER) ? gathered_sum(w_homo, hits) : static_cast<F>(acc);
+      }
+    }
+    __syncthreads();
+    if (lane == 0) s_mask[wave] = by_all;
     __syncthreads();
     for (uint32_t w = 0; w < nwaves; ++w) {
       unsigned long long m = s_mask[w];
-      while (m != 0) {
+      for (; m != 0; m &= m - 1ull) {
         const uint32_t r = row_of(i0 + w * kWave + static_cast<uint32_t>(__ffsll(m) - 1));
-        m &= m - 1ull;
         if (tid == 0) s_acc = 0.0, s_hits = 0u;
         __syncthreads();
-        const uint32_t start = indptr[r], len = indptr[r + 1] - start;
+        const uint32_t start = indptr[r];
         double acc = 0.0;
         uint32_t hits = 0;
-        constexpr uint32_t U = 4;  // loads in flight per lane and step; the next step's are requested before this one's are used
-        uint32_t col[U], ncol[U];
-        auto load_cols = [&](uint32_t j0, uint32_t (&c)[U]) {  // (beyond the row: its last index again)
-#pragma unroll
-          for (uint32_t u = 0; u < U; ++u) {
-            const uint32_t j = j0 + u * blockDim.x;
-            c[u] = indices[start + (j < len ? j : len - 1u)];
-          }
-        };
-        load_cols(tid, col);
-        for (uint32_t j0 = tid; j0 < len; j0 += U * blockDim.x) {
-          load_cols(j0 + U * blockDim.x, ncol);
-#pragma unroll
-          for (uint32_t u = 0; u < U; ++u) {
-            const uint32_t j = j0 + u * blockDim.x;
-            if (j >= len) continue;
-            if (MODE == kEvent) {
-              if (event_hit<BITS>(s_bits, x, col[u], coarse_g)) {
-                if (HETER) acc += static_cast<double>(data[start + j]);
-                else ++hits;
-              }
-            } else {
-              const F d = HETER ? data[start + j] : w_homo;
-              acc += static_cast<double>(static_cast<F>(static_cast<F>(x[col[u]]) * d));
-            }
-          }
-#pragma unroll
-          for (uint32_t u = 0; u < U; ++u) col[u] = ncol[u];
-        }
+        walk(start, indptr[r + 1] - start, tid, blockDim.x, acc, hits);
         if (MODE == kEvent && !HETER) {
-          hits = wave_sum(hits);
           if (lane == 0 && hits != 0u) atomicAdd(&s_hits, hits);
         } else {
-          acc = wave_sum(acc);
           if (lane == 0) atomicAdd(&s_acc, acc);
         }
         __syncthreads();
@@ -977,6 +1009,7 @@ __device__ __forceinline__ void gather_hub_rows(const F *__restrict__ data, cons
         __syncthreads();
       }
     }
+    __syncthreads();  // (the masks are written again)
   }
 }
 
@@ -1284,6 +1317,9 @@ __global__ __launch_bounds__(1024, (MODE == kEvent && BITS == 1) ? 8 : 4) void c
   // lanes per row from the mean row length
   const uint32_t mean = nnz / n_row;
   uint32_t gpb = 0, hub_len = 0;  // rows per workgroup and round of the walk chosen below, its longest row
+  // (counts of one double weight: their sum is formed by one thread of a workgroup that waits for it, which costs more
+  // than the longer walk: 60,000 rows of 700, log-normal: 88 us with steps of 512 here)
+  constexpr uint32_t kWaveStep = 8 * kWave * (MODE == kEvent && !HETER && sizeof(F) == 8 ? 4 : 1);
   if constexpr (MODE == kDense && BITS == 0) {
     // (rows of `skip_mean` nonzeros or more on average: the launcher's other kernel has taken this matrix)
     if (skip_mean != 0 && mean >= skip_mean && nnz <= kFlatMaxNnz) return;
@@ -1291,10 +1327,10 @@ __global__ __launch_bounds__(1024, (MODE == kEvent && BITS == 1) ? 8 : 4) void c
   if constexpr (MODE == kDense && BITS == 1) {
     // (nothing left to hide but the index and weight streams: the walks of the event gather)
     const VT *xs = reinterpret_cast<const VT *>(s_bits);
-    if (mean >= 384) { gather_rows_wave<F, VT, HETER, MODE, BITS, 8>(data, indices, indptr, xs, y, n_row, s_bits, coarse_g); gpb = 1; hub_len = kHubSteps * 8 * kWave; }
-    else if (mean >= 24) { gather_rows<F, VT, HETER, MODE, BITS, 8, 8>(data, indices, indptr, xs, y, n_row, s_bits, coarse_g); gpb = blockDim.x / 8; hub_len = kHubSteps * 8 * 8; }
-    else if (mean >= 12) { gather_rows<F, VT, HETER, MODE, BITS, 4, 8>(data, indices, indptr, xs, y, n_row, s_bits, coarse_g); gpb = blockDim.x / 4; hub_len = kHubSteps * 8 * 4; }
-    else { gather_rows<F, VT, HETER, MODE, BITS, 4, 4>(data, indices, indptr, xs, y, n_row, s_bits, coarse_g); gpb = blockDim.x / 4; hub_len = kHubSteps * 4 * 4; }
+    if (mean >= 384) { gpb = 1; hub_len = hub_length(mean, kWaveStep); gather_rows_wave<F, VT, HETER, MODE, BITS, 8>(data, indices, indptr, xs, y, n_row, s_bits, coarse_g, hub_len); }
+    else if (mean >= 24) { gpb = blockDim.x / 8; hub_len = hub_length(mean, 8 * 8); gather_rows<F, VT, HETER, MODE, BITS, 8, 8>(data, indices, indptr, xs, y, n_row, s_bits, coarse_g, hub_len); }
+    else if (mean >= 12) { gpb = blockDim.x / 4; hub_len = hub_length(mean, 8 * 4); gather_rows<F, VT, HETER, MODE, BITS, 4, 8>(data, indices, indptr, xs, y, n_row, s_bits, coarse_g, hub_len); }
+    else { gpb = blockDim.x / 4; hub_len = hub_length(mean, 4 * 4); gather_rows<F, VT, HETER, MODE, BITS, 4, 4>(data, indices, indptr, xs, y, n_row, s_bits, coarse_g, hub_len); }
   } else if constexpr (MODE == kEvent && (BITS == 2 || BITS == 3)) {
     // An event bitmap above 80 KB leaves room for one workgroup (16 waves) per CU only: every lane
     // then keeps 16 (rows under 48 nonzeros: 8) loads in flight instead of 2 to 8, in groups of
@@ -1308,9 +1344,9 @@ __global__ __launch_bounds__(1024, (MODE == kEvent && BITS == 1) ? 8 : 4) void c
         return;
       }
     }
-    if (mean >= 384) { gather_rows_wave<F, VT, HETER, MODE, BITS, 8>(data, indices, indptr, x, y, n_row, s_bits, coarse_g); gpb = 1; hub_len = kHubSteps * 8 * kWave; }
-    else if (mean >= 48) { gather_rows<F, VT, HETER, MODE, BITS, 8, 16>(data, indices, indptr, x, y, n_row, s_bits, coarse_g); gpb = blockDim.x / 8; hub_len = kHubSteps * 16 * 8; }
-    else { gather_rows<F, VT, HETER, MODE, BITS, 4, 8>(data, indices, indptr, x, y, n_row, s_bits, coarse_g); gpb = blockDim.x / 4; hub_len = kHubSteps * 8 * 4; }
+    if (mean >= 384) { gpb = 1; hub_len = hub_length(mean, kWaveStep); gather_rows_wave<F, VT, HETER, MODE, BITS, 8>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
+    else if (mean >= 48) { gpb = blockDim.x / 8; hub_len = hub_length(mean, 16 * 8); gather_rows<F, VT, HETER, MODE, BITS, 8, 16>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
+    else { gpb = blockDim.x / 4; hub_len = hub_length(mean, 8 * 4); gather_rows<F, VT, HETER, MODE, BITS, 4, 8>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
   } else {
     if constexpr (MODE == kEvent && BITS == 1 && HETER) {
       // The same walk within 64 registers, where the launcher left room for it behind the bitmap.  A wave's steps
@@ -1326,18 +1362,18 @@ __global__ __launch_bounds__(1024, (MODE == kEvent && BITS == 1) ? 8 : 4) void c
         return;
       }
     }
-    if (mean >= 384) { gather_rows_wave<F, VT, HETER, MODE, BITS, 8>(data, indices, indptr, x, y, n_row, s_bits, coarse_g); gpb = 1; hub_len = kHubSteps * 8 * kWave; }
+    if (mean >= 384) { gpb = 1; hub_len = hub_length(mean, kWaveStep); gather_rows_wave<F, VT, HETER, MODE, BITS, 8>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
     // (a dense vector is gathered from L2: for rows of 48 .. 191 nonzeros the pipelined 32-lane walk keeps more
     // of those gathers in flight than a wave per row does)
-    else if (MODE == kEvent && mean >= 48u) { gather_rows<F, VT, HETER, MODE, BITS, 8, 8>(data, indices, indptr, x, y, n_row, s_bits, coarse_g); gpb = blockDim.x / 8; hub_len = kHubSteps * 8 * 8; }
-    else if (MODE == kDense && mean >= 192u) { gather_rows_wave<F, VT, HETER, MODE, BITS, 2>(data, indices, indptr, x, y, n_row, s_bits, coarse_g); gpb = 1; hub_len = kHubSteps * 2 * kWave; }
-    else if (mean >= 48) { gather_rows<F, VT, HETER, MODE, BITS, 32, 4>(data, indices, indptr, x, y, n_row, s_bits, coarse_g); gpb = blockDim.x / 32; hub_len = kHubSteps * 4 * 32; }
-    else if (MODE == kEvent && mean >= 24) { gather_rows<F, VT, HETER, MODE, BITS, 8, 8>(data, indices, indptr, x, y, n_row, s_bits, coarse_g); gpb = blockDim.x / 8; hub_len = kHubSteps * 8 * 8; }
-    else if (MODE == kEvent && mean >= 12) { gather_rows<F, VT, HETER, MODE, BITS, 4, 8>(data, indices, indptr, x, y, n_row, s_bits, coarse_g); gpb = blockDim.x / 4; hub_len = kHubSteps * 8 * 4; }
-    else if (MODE == kEvent) { gather_rows<F, VT, HETER, MODE, BITS, 4, 4>(data, indices, indptr, x, y, n_row, s_bits, coarse_g); gpb = blockDim.x / 4; hub_len = kHubSteps * 4 * 4; }
-    else if (mean >= 24) { gather_rows<F, VT, HETER, MODE, BITS, 32, 2>(data, indices, indptr, x, y, n_row, s_bits, coarse_g); gpb = blockDim.x / 32; hub_len = kHubSteps * 2 * 32; }
-    else if (mean >= 12) { gather_rows<F, VT, HETER, MODE, BITS, 16, 2>(data, indices, indptr, x, y, n_row, s_bits, coarse_g); gpb = blockDim.x / 16; hub_len = kHubSteps * 2 * 16; }
-    else { gather_rows<F, VT, HETER, MODE, BITS, 8, 2>(data, indices, indptr, x, y, n_row, s_bits, coarse_g); gpb = blockDim.x / 8; hub_len = kHubSteps * 2 * 8; }
+    else if (MODE == kEvent && mean >= 48u) { gpb = blockDim.x / 8; hub_len = hub_length(mean, 8 * 8); gather_rows<F, VT, HETER, MODE, BITS, 8, 8>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
+    else if (MODE == kDense && mean >= 192u) { gpb = 1; hub_len = hub_length(mean, 2 * kWave); gather_rows_wave<F, VT, HETER, MODE, BITS, 2>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
+    else if (mean >= 48) { gpb = blockDim.x / 32; hub_len = hub_length(mean, 4 * 32); gather_rows<F, VT, HETER, MODE, BITS, 32, 4>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
+    else if (MODE == kEvent && mean >= 24) { gpb = blockDim.x / 8; hub_len = hub_length(mean, 8 * 8); gather_rows<F, VT, HETER, MODE, BITS, 8, 8>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
+    else if (MODE == kEvent && mean >= 12) { gpb = blockDim.x / 4; hub_len = hub_length(mean, 8 * 4); gather_rows<F, VT, HETER, MODE, BITS, 4, 8>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
+    else if (MODE == kEvent) { gpb = blockDim.x / 4; hub_len = hub_length(mean, 4 * 4); gather_rows<F, VT, HETER, MODE, BITS, 4, 4>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
+    else if (mean >= 24) { gpb = blockDim.x / 32; hub_len = hub_length(mean, 2 * 32); gather_rows<F, VT, HETER, MODE, BITS, 32, 2>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
+    else if (mean >= 12) { gpb = blockDim.x / 16; hub_len = hub_length(mean, 2 * 16); gather_rows<F, VT, HETER, MODE, BITS, 16, 2>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
+    else { gpb = blockDim.x / 8; hub_len = hub_length(mean, 2 * 8); gather_rows<F, VT, HETER, MODE, BITS, 8, 2>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
   }
   // the rows the walk left to the whole workgroup
   if constexpr (MODE == kDense && BITS == 1)

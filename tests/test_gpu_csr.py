@@ -1171,3 +1171,29 @@ def test_csr_matvec_padded_index_arrays(cuda, dtype):
   indptr[5:] = 3
   got = bpl.csr_matvec(data, indices, indptr, np.ones(n_col, dtype), shape=(n_row, n_col)).cpu().numpy()
   assert got[4] == 3 and got.sum() == 3
+
+
+@pytest.mark.parametrize("n_row,n_col,mean", [(300, 20_000, 8), (2500, 60_000, 20), (18_000, 30_000, 30), (2100, 40_000, 60),
+                                              (17_000, 700_000, 100), (2200, 150_000, 200), (2049, 90_000, 500)])
+def test_rows_left_to_a_wave_or_a_workgroup(cuda, oracle_mod, n_row, n_col, mean):
+  # rows of more than four steps of their walk and four times the mean are walked by a wave (up to 4,096 nonzeros)
+  # or a whole workgroup: lengths at and around every step multiple, at both lines and far above, first and last row
+  # among them, empty rows between.  Integer weights and vectors: every sum is exact.
+  rng = np.random.default_rng(n_row)
+  counts = np.full(n_row, mean)
+  special = [b + d for b in (64, 128, 256, 512, 1024, 2048, 4 * mean, 4096, 8192, 16_384) for d in (-1, 0, 1)] + [0, 0]
+  at = np.unique(np.concatenate([[0, n_row - 1], rng.choice(n_row, len(special) - 2, replace=False)]))
+  counts[at] = np.minimum(special[:at.size], n_col)
+  ptr = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+  idx = np.concatenate([np.arange(c) * (n_col // max(c, 1)) + rng.integers(0, n_col // max(c, 1)) for c in counts]).astype(np.int32)
+  w = rng.integers(-4, 5, idx.shape[0])
+  ev = rng.random(n_col) < 0.2
+  v = rng.integers(-4, 5, n_col)
+  print("case", n_row, n_col, mean, flush=True)
+  for dt in (np.float32, np.float64):
+    for data in (w.astype(dt), np.asarray([0.5], dtype=dt)):
+      kw = dict(shape=(n_row, n_col), transpose=False)
+      got = bpl.event_csr_matvec(data, idx, ptr, ev, **kw).cpu().numpy()
+      assert np.array_equal(got, oracle_mod.event_csr_matvec(data, idx, ptr, ev, **kw)), ("event", dt, data.shape)
+      got = bpl.csr_matvec(data, idx, ptr, v.astype(dt), shape=(n_row, n_col)).cpu().numpy()
+      assert np.array_equal(got, oracle_mod.csr_matvec(data, idx, ptr, v.astype(dt), shape=(n_row, n_col))), ("dense", dt, data.shape)
