@@ -147,6 +147,19 @@ def _wants_grad(*tensors):
   return False
 
 
+def _transformed(t):
+  """True for a tensor whose products must stay visible to a differentiation or batching transform."""
+  if torch.is_grad_enabled() and t.requires_grad:
+    return True
+  if torch.autograd.forward_ad.unpack_dual(t).tangent is not None:
+    return True
+  try:
+    t.data_ptr()
+  except RuntimeError:  # (the wrappers of vmap and torch.func have no storage of their own)
+    return True
+  return False
+
+
 _GRADIENT_MAX_NNZ = 2 ** 32 - 8193  # what the gradient target's 32-bit positions can number
 
 
@@ -154,10 +167,12 @@ def _gradients(data, indices, indptr, row_vector, col_vector, shape, want_sums):
   """(products, sums): ``row_vector[row] * col_vector[col]`` per nonzero and, if wanted, the product of the matrix
   with ``col_vector``, in one walk over the nonzeros (sums is None where it was not computed)."""
   nnz = indices.shape[0]
-  differentiated = torch.is_grad_enabled() and (row_vector.requires_grad or col_vector.requires_grad)
-  if nnz > _GRADIENT_MAX_NNZ or differentiated:  # (create_graph: the products stay differentiable)
+  # Composed of torch's own operators where a transform has to see through it: create_graph, a cotangent with a
+  # tangent (forward over reverse), a batch of cotangents (is_grads_batched).
+  if nnz > _GRADIENT_MAX_NNZ or _transformed(row_vector) or _transformed(col_vector):
     row, col = csr_to_coo(indices, indptr)
     return row_vector[_int64(row)] * col_vector[_int64(col)], None
+  _, data, indices, indptr, row_vector, col_vector = _move(data, indices, indptr, row_vector, col_vector)
   products = torch.empty(nnz, dtype=data.dtype, device=data.device)
   sums = torch.empty(shape[0] if want_sums else 0, dtype=data.dtype, device=data.device)
   _lib.custom_call('csr_matvec_gradient_' + ('float' if data.dtype == torch.float32 else 'double'),
