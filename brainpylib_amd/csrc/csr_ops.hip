@@ -1861,7 +1861,8 @@ void launch_gather(const char *target, const ScratchSource &src, const F *data, 
                                                       kFlatMinMean);
           return;
         }
-        if (scratch_refused_by_capture()) return ensure_error(target, "nothing was enqueued: the path that the scratch memory at hand allows could not be launched");  // (the error stands: a graph must not record a slower path)
+        // (under 16,384 rows a capture without scratch memory takes the row-wise walk, which needs none)
+        if (n_row >= 16384 && scratch_refused_by_capture()) return ensure_error(target, "nothing was enqueued: the path that the scratch memory at hand allows could not be launched");  // (the error stands: a graph must not record a slower path)
         bpl_clear_error();
       }
     }

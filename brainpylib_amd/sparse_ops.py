@@ -175,9 +175,17 @@ def _gradients(data, indices, indptr, row_vector, col_vector, shape, want_sums):
   _, data, indices, indptr, row_vector, col_vector = _move(data, indices, indptr, row_vector, col_vector)
   products = torch.empty(nnz, dtype=data.dtype, device=data.device)
   sums = torch.empty(shape[0] if want_sums else 0, dtype=data.dtype, device=data.device)
-  _lib.custom_call('csr_matvec_gradient_' + ('float' if data.dtype == torch.float32 else 'double'),
-                   [data.detach(), indices, indptr, row_vector.detach(), col_vector.detach(), products, sums],
-                   _lib.build_csr_transpose_descriptor(shape[0], shape[1], nnz))
+  name = 'csr_matvec_gradient_' + ('float' if data.dtype == torch.float32 else 'double')
+  opaque = _lib.build_csr_transpose_descriptor(shape[0], shape[1], nnz)
+  buffers = [data.detach(), indices, indptr, row_vector.detach(), col_vector.detach(), products, sums]
+  try:
+    _lib.custom_call(name, buffers, opaque)
+  except RuntimeError:
+    if not (want_sums and torch.cuda.is_current_stream_capturing()):
+      raise
+    # (captured on a stream without scratch memory, which only the sums need: nothing was enqueued)
+    want_sums = False
+    _lib.custom_call(name, buffers[:-1] + [sums[:0]], opaque)
   return products, sums if want_sums else None
 
 

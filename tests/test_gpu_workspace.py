@@ -8,7 +8,7 @@ import pytest
 import torch
 
 import brainpylib_amd as bpl
-from brainpylib_amd import _lib
+from brainpylib_amd import _lib, sparse_ops
 import benchdata as synth
 
 pytestmark = pytest.mark.gpu
@@ -102,3 +102,29 @@ def test_growth_is_refused_during_capture_and_works_after_a_warm_up(cuda, oracle
   g2.replay()
   torch.cuda.synchronize()
   assert torch.allclose(out, want, rtol=1e-5, atol=1e-6)
+
+
+def test_calls_that_did_without_scratch_memory_are_captured_on_a_cold_stream(cuda):
+  n_row, n_col = 2_000, 60_000
+  rng = np.random.default_rng(5)
+  indices, indptr = synth.fixed_count_csr(n_row, n_col, 600, seed=5)
+  data = torch.from_numpy(rng.integers(-3, 4, size=indices.shape[0]).astype(np.float32)).to(cuda)
+  idx, ptr = torch.from_numpy(indices).to(cuda), torch.from_numpy(indptr).to(cuda)
+  x = torch.zeros(n_col, dtype=torch.float32, device=cuda)
+  v = torch.zeros(n_row, dtype=torch.float32, device=cuda)
+  s = torch.cuda.Stream()
+  torch.cuda.synchronize()
+  g = torch.cuda.CUDAGraph()
+  with torch.cuda.graph(g, stream=s):
+    y = bpl.csr_matvec(data, idx, ptr, x, shape=(n_row, n_col))
+    products, sums = sparse_ops._gradients(data, idx, ptr, v, x, (n_row, n_col), True)
+  for i in range(3):  # (eager work between the replays; integers: exact sums)
+    x.copy_(torch.from_numpy(rng.integers(-4, 5, size=n_col).astype(np.float32)))
+    v.copy_(torch.from_numpy(rng.integers(-4, 5, size=n_row).astype(np.float32)))
+    torch.cuda.synchronize()
+    g.replay()
+    torch.cuda.synchronize()
+    want, want_sums = sparse_ops._gradients(data, idx, ptr, v, x, (n_row, n_col), True)
+    assert torch.equal(products, want), i
+    assert torch.equal(y, want_sums), i
+    assert sums is None or torch.equal(sums, want_sums)
