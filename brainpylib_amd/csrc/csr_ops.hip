@@ -21,6 +21,7 @@
 //
 // Reference boundary: lib/gpu_event_csr_matvec.cu:148-260, lib/gpu_csr_matvec.cu:84-135,195-246,
 // 505-621 (buffer order, descriptor, target names).
+#include <algorithm>
 #include <mutex>
 #include <type_traits>
 
@@ -2257,12 +2258,13 @@ void event_csr_batching_entry(const char *target, hipStream_t stream, void **buf
   // group * n_col columns (entry g's columns shifted by g * n_col), fed by one list of the active rows of the
   // group's entries.  A group is a chain of three launches whatever its size, so it takes as many entries as keep
   // the virtual output within windows that are added in one slice (2^21 columns) and the pairs of a sixth of
-  // all nonzeros within the runs of the sort (20 entries of 8e6 nonzeros in one group instead of three: 105 -> 52 us);
-  // up to 8 entries beyond those bounds (1e8 nonzeros: larger groups gain nothing and overflow the runs sooner).
-  // Groups of equal size.
+  // all nonzeros within the runs of the sort (20 entries of 8e6 nonzeros in one group instead of three: 105 -> 52 us),
+  // and the list of its active rows within 400 MB (2^25 rows); up to 8 entries beyond those bounds (1e8 nonzeros:
+  // larger groups gain nothing and overflow the runs sooner).  Groups of equal size.
   if (d.transpose && shared_matrix && d.batch_size > 1 && d.n_row > 0 && d.n_col > 0) {
     const uint64_t by_columns = (1ull << 21) / d.n_col, by_pairs = 6ull * kMostRunPairs / (d.nnz ? d.nnz : 1u);
-    const uint64_t fits = by_columns < by_pairs ? by_columns : by_pairs;
+    const uint64_t by_rows = (1ull << 25) / d.n_row;
+    const uint64_t fits = std::min(by_rows, std::min(by_columns, by_pairs));
     const uint32_t most = fits < 8 ? 8u : fits < d.batch_size ? static_cast<uint32_t>(fits) : d.batch_size;
     uint32_t group = div_up(d.batch_size, div_up(d.batch_size, most));
     while (group > 1 && (static_cast<uint64_t>(group) * d.n_col >= (1ull << 24) ||
@@ -2302,7 +2304,9 @@ void event_csr_batching_entry(const char *target, hipStream_t stream, void **buf
         check_launch(target);
         return;
       }
-      if (scratch_refused_by_capture()) return ensure_error(target, "nothing was enqueued: the path that the scratch memory at hand allows could not be launched");
+      // (small networks, whose entries one by one need no scratch memory, are captured without any)
+      const bool by_entry = static_cast<uint64_t>(d.batch_size < 8 ? d.batch_size : 8) * d.n_col <= 8192;
+      if (scratch_refused_by_capture() && !by_entry) return ensure_error(target, "nothing was enqueued: the path that the scratch memory at hand allows could not be launched");
       bpl_clear_error();
     }
   }

@@ -128,3 +128,24 @@ def test_calls_that_did_without_scratch_memory_are_captured_on_a_cold_stream(cud
     assert torch.equal(products, want), i
     assert torch.equal(y, want_sums), i
     assert sums is None or torch.equal(sums, want_sums)
+
+
+def test_batched_scatter_of_a_small_network_is_captured_on_a_cold_stream(cuda):
+  n, batch = 1_000, 20
+  rng = np.random.default_rng(6)
+  indices, indptr = synth.fixed_count_csr(n, n, 50, seed=6)
+  data = torch.from_numpy(rng.integers(-3, 4, size=indices.shape[0]).astype(np.float32)).to(cuda).reshape(1, -1)
+  idx, ptr = (torch.from_numpy(a).to(cuda).reshape(1, -1) for a in (indices, indptr))
+  events = torch.zeros((batch, n), dtype=torch.bool, device=cuda)
+  call = lambda: bpl.event_csr_matvec_batching(data, idx, ptr, events, batch_size=batch, shape=(n, n), transpose=True)
+  s = torch.cuda.Stream()
+  torch.cuda.synchronize()
+  g = torch.cuda.CUDAGraph()
+  with torch.cuda.graph(g, stream=s):
+    out = call()
+  for i in range(3):
+    events.copy_(torch.from_numpy(rng.random((batch, n)) < 0.1))
+    torch.cuda.synchronize()
+    g.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(out, call()), i  # (integers: exact in any order)
