@@ -25,7 +25,8 @@ template <typename F>
 bool flat_stages(uint32_t n_col);
 
 // The same walk for the gradients of a product with a matrix of one weight per nonzero:
-// products[j] = v[row of j] * x[column of j] and, if `sums` is given, sums = A x.
+// products[j] = v[row of j] * x[column of j] and, if `sums` is given, sums = A x.  `products` has nnz elements; those
+// beyond indptr[n_row], if that is less, become zero.
 template <typename F>
 bool csr_gradient(const char *target, hipStream_t stream, const F *data, const uint32_t *indices, const uint32_t *indptr,
                   const F *v, const F *x, F *products, F *sums, uint32_t n_row, uint32_t n_col, uint32_t nnz);

@@ -122,7 +122,7 @@ __global__ __launch_bounds__(flat_threads(STAGED), 4) void csr_flat_gather_kerne
     const F *__restrict__ data, const uint32_t *__restrict__ indices, const uint32_t *__restrict__ indptr,
     const F *__restrict__ x, F *__restrict__ y, uint32_t n_row, uint32_t n_col, uint32_t min_mean,
     double *__restrict__ head, double *__restrict__ tail, uint32_t *__restrict__ tail_row, const F *__restrict__ v,
-    F *__restrict__ products) {
+    F *__restrict__ products, uint32_t n_products) {
   constexpr int U = FlatQuads<F, OUT>::value;
   constexpr uint32_t kStepQuads = U * kWave;
   constexpr int kFlatWaves = flat_threads(STAGED) / kWave;
@@ -135,6 +135,11 @@ __global__ __launch_bounds__(flat_threads(STAGED), 4) void csr_flat_gather_kerne
   const uint32_t nnz = indptr[n_row];
   const uint32_t mean = nnz / n_row;
   if (mean < min_mean || nnz > kFlatMaxNnz) return;  // (the launcher's other kernel takes those matrices)
+  if constexpr (kProducts) {  // (index arrays longer than indptr says: nothing depends on what lies beyond)
+    for (uint64_t i = nnz + static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n_products;
+         i += gridDim.x * blockDim.x)
+      products[i] = F(0);
+  }
   if (kSums && nnz == 0) {
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n_row; i += gridDim.x * blockDim.x) y[i] = F(0);
   }
@@ -421,7 +426,7 @@ bool flat_stages(uint32_t n_col) {
 template <typename F, bool HETER, int OUT, bool STAGED>
 static bool launch_flat(const char *target, hipStream_t stream, const F *data, const uint32_t *indices,
                         const uint32_t *indptr, const F *x, F *y, uint32_t n_row, uint32_t n_col, uint32_t min_mean,
-                        const F *v, F *products) {
+                        const F *v, F *products, uint32_t n_products) {
   constexpr bool kSums = (OUT & kFlatSums) != 0;
   const unsigned grid = static_cast<unsigned>(device_info().num_cu) * flat_per_cu(STAGED);
   const uint32_t waves = grid * (flat_threads(STAGED) / kWave);
@@ -446,7 +451,7 @@ static bool launch_flat(const char *target, hipStream_t stream, const F *data, c
     }
   }
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(flat_threads(STAGED)), lds, stream, data, indices, indptr, x, y, n_row,
-                     n_col, min_mean, head, tail, tail_row, v, products);
+                     n_col, min_mean, head, tail, tail_row, v, products, n_products);
   if (kSums)
     hipLaunchKernelGGL(csr_flat_finish_kernel<F>, dim3(waves), dim3(kWave), 0, stream, indptr, y, n_row, min_mean,
                        waves, static_cast<const double *>(head), static_cast<const double *>(tail),
@@ -460,7 +465,7 @@ bool csr_flat_gather(const char *target, hipStream_t stream, const F *data, bool
   if (n_row == 0) return true;
   auto launch = [&](auto h, auto staged) {
     return launch_flat<F, decltype(h)::value, kFlatSums, decltype(staged)::value>(
-      target, stream, data, indices, indptr, x, y, n_row, n_col, min_mean, nullptr, nullptr);
+      target, stream, data, indices, indptr, x, y, n_row, n_col, min_mean, nullptr, nullptr, 0u);
   };
   if (flat_stages<F>(n_col)) return heter ? launch(std::true_type(), std::true_type()) : launch(std::false_type(), std::true_type());
   return heter ? launch(std::true_type(), std::false_type()) : launch(std::false_type(), std::false_type());
@@ -469,21 +474,22 @@ bool csr_flat_gather(const char *target, hipStream_t stream, const F *data, bool
 template <typename F>
 bool csr_gradient(const char *target, hipStream_t stream, const F *data, const uint32_t *indices, const uint32_t *indptr,
                   const F *v, const F *x, F *products, F *sums, uint32_t n_row, uint32_t n_col, uint32_t nnz) {
-  if (n_row == 0) return true;
+  if (n_row == 0) {
+    fill_zero(stream, products, nnz);
+    return check_launch(target);
+  }
   if (nnz > kFlatMaxNnz) {
     set_error("%s: %u nonzeros are more than the walk's positions can number", target, nnz);
     return false;
   }
-  const bool staged = flat_stages<F>(n_col);
-  if (sums != nullptr)
-    return staged ? launch_flat<F, true, kFlatSums | kFlatProducts, true>(target, stream, data, indices, indptr, x, sums, n_row,
-                                                                          n_col, 0u, v, products)
-                  : launch_flat<F, true, kFlatSums | kFlatProducts, false>(target, stream, data, indices, indptr, x, sums,
-                                                                           n_row, n_col, 0u, v, products);
-  return staged ? launch_flat<F, true, kFlatProducts, true>(target, stream, data, indices, indptr, x, sums, n_row, n_col, 0u,
-                                                            v, products)
-                : launch_flat<F, true, kFlatProducts, false>(target, stream, data, indices, indptr, x, sums, n_row, n_col,
-                                                             0u, v, products);
+  auto launch = [&](auto out, auto staged) {
+    return launch_flat<F, true, decltype(out)::value, decltype(staged)::value>(target, stream, data, indices, indptr, x, sums,
+                                                                               n_row, n_col, 0u, v, products, nnz);
+  };
+  using Products = std::integral_constant<int, kFlatProducts>;
+  using Both = std::integral_constant<int, kFlatSums | kFlatProducts>;
+  if (flat_stages<F>(n_col)) return sums != nullptr ? launch(Both(), std::true_type()) : launch(Products(), std::true_type());
+  return sums != nullptr ? launch(Both(), std::false_type()) : launch(Products(), std::false_type());
 }
 
 // csr_matvec_gradient: buffers = [data, indices, indptr, row vector, column vector, products, sums (or null)]

@@ -170,8 +170,16 @@ def _gradients(data, indices, indptr, row_vector, col_vector, shape, want_sums):
   # Composed of torch's own operators where a transform has to see through it: create_graph, a cotangent with a
   # tangent (forward over reverse), a batch of cotangents (is_grads_batched).
   if nnz > _GRADIENT_MAX_NNZ or _transformed(row_vector) or _transformed(col_vector):
-    row, col = csr_to_coo(indices, indptr)
-    return row_vector[_int64(row)] * col_vector[_int64(col)], None
+    if 0 in shape:
+      return torch.zeros(nnz, dtype=data.dtype, device=data.device), None
+    # (index arrays longer than indptr says: what lies beyond counts as one row more, with gradient zero)
+    ptr = _int64(indptr)
+    row = torch.repeat_interleave(torch.arange(shape[0] + 1, device=ptr.device),
+                                  torch.cat([ptr[1:] - ptr[:-1], nnz - ptr[-1:]]), output_size=nnz)
+    inside = row < shape[0]
+    row, col = row.clamp(max=shape[0] - 1), torch.where(inside, _int64(indices), 0)
+    products = row_vector[row] * col_vector[col]
+    return torch.where(inside, products, torch.zeros((), dtype=products.dtype, device=products.device)), None
   _, data, indices, indptr, row_vector, col_vector = _move(data, indices, indptr, row_vector, col_vector)
   products = torch.empty(nnz, dtype=data.dtype, device=data.device)
   sums = torch.empty(shape[0] if want_sums else 0, dtype=data.dtype, device=data.device)

@@ -398,7 +398,8 @@ BPL_TARGET(csr_matvec_transpose_homo_double);
 /* Gradients of a product with a matrix of one weight per nonzero (own targets: the reference's
  * differentiation rules, brainpylib/_src/sparse_ops/cusparse_matvec.py:281-308, are composed of
  * gathers over an expanded list of the nonzeros' rows).
- *   products[j] = row_vector[row of j] * column_vector[column of j] for every nonzero j,
+ *   products[j] = row_vector[row of j] * column_vector[column of j] for every nonzero j, and 0 for the
+ *                 elements from indptr[n_row] up to the descriptor's nnz,
  *   sums = A @ column_vector (not computed if its pointer is null; `data` is read for it only).
  *   buffers = [data, indices, indptr, row_vector(F[n_row]), column_vector(F[n_col]),
  *              products(F[nnz]), sums(F[n_row]) or null],

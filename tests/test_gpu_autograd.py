@@ -146,6 +146,38 @@ def test_gradients_of_weights_and_vector_from_one_walk(cuda, n_row, n_col, mean,
     assert torch.equal(torch.autograd.grad(y, d, ct.cuda())[0].cpu(), want)
 
 
+# arrays longer than indptr says, by less than a quad and by more than the walk has threads; a matrix without nonzeros and
+# one without rows.  Nothing depends on what lies beyond: its gradient is zero, whatever its columns are.
+@pytest.mark.parametrize("n_row,mean,extra", [(50, 7, 3), (2000, 40, 300_000), (2000, 0, 1000), (0, 0, 5)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("transpose", [False, True])
+@pytest.mark.parametrize("product", ["cusparse_csr_matvec", "event_csr_matvec"])
+def test_gradients_of_padded_index_arrays(cuda, n_row, mean, extra, dtype, transpose, product):
+  n_col = 900
+  rng = np.random.default_rng(extra)
+  counts = np.minimum(rng.poisson(mean, n_row), n_col)
+  idx, ptr = synth.counted_csr(counts, n_col, seed=extra) if n_row else (np.zeros(0, np.int32), np.zeros(1, np.int32))
+  nnz = idx.shape[0]
+  row, col = torch.from_numpy(np.repeat(np.arange(n_row), counts)), torch.from_numpy(idx.astype(np.int64))
+  g = torch.Generator().manual_seed(n_row)
+  data = torch.randn(nnz + extra, dtype=dtype, generator=g)
+  n_in, n_out = (n_row, n_col) if transpose else (n_col, n_row)
+  vec, ct = (torch.rand(n_in, generator=g) < 0.5).to(dtype), torch.randn(n_out, dtype=dtype, generator=g)
+  src, dst = (row, col) if transpose else (col, row)
+  d, v = data.cuda().requires_grad_(), vec.cuda().requires_grad_()
+  idx = torch.cat([torch.from_numpy(idx), torch.full((extra,), n_col - 1, dtype=torch.int32)]).cuda()
+  for wanted in ((d,), (d, v)):
+    y = getattr(bpl, product)(d, idx, torch.from_numpy(ptr).cuda(), v, shape=(n_row, n_col), transpose=transpose)
+    torch.full_like(d, float("nan"))  # (memory that an unwritten result would show)
+    got = torch.autograd.grad(y, wanted, ct.cuda())
+    assert torch.equal(got[0][:nnz].cpu(), vec[src] * ct[dst]) and not got[0][nnz:].any()
+  want = torch.zeros(n_in, dtype=torch.float64).index_add_(0, src, (data[:nnz] * ct[dst]).to(torch.float64))
+  mag = torch.zeros(n_in, dtype=torch.float64).index_add_(0, src, (data[:nnz] * ct[dst]).abs().to(torch.float64))
+  # (two orders of summation in the result's precision)
+  bound = torch.finfo(dtype).eps * want.abs() + 4 * torch.finfo(dtype).eps * mag
+  assert bool(((got[1].cpu().to(torch.float64) - want).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("kind", ["homo", "uniform", "normal"])
 @pytest.mark.parametrize("transpose", [False, True])
 @pytest.mark.parametrize("outdim_parallel", [False, True])

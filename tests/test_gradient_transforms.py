@@ -69,3 +69,18 @@ def test_derivative_by_the_cotangent(product, transpose):
   assert torch.equal(got.detach(), want[0])
   second, = torch.autograd.grad(got.sum(), ct)
   torch.testing.assert_close(second, torch.zeros_like(second).index_add_(0, dst, vec[src]), rtol=1e-14, atol=1e-14)
+
+
+@pytest.mark.parametrize("transpose", [False, True])
+def test_padded_index_arrays(product, transpose, monkeypatch):
+  # arrays longer than indptr says: the matrix ends where indptr ends, and what lies beyond has gradient zero
+  shape, idx, ptr, data, vec, ct, want, _, _ = _problem(transpose)
+  launch = sparse_ops._launch
+  nnz, extra = idx.shape[0], 4
+  monkeypatch.setattr(sparse_ops, "_launch", lambda d, i, *a: launch(d[:nnz], i[:nnz], *a))
+  monkeypatch.setattr(event_ops, "_launch", lambda d, i, *a: launch(d[:nnz], i[:nnz], *a))
+  data = torch.cat([data.detach(), torch.ones(extra, dtype=data.dtype)]).requires_grad_()
+  idx = torch.cat([idx, torch.full((extra,), 2 ** 31 - 1, dtype=idx.dtype)])
+  out = product(data, idx, ptr, vec, shape, transpose)
+  got, = torch.autograd.grad(out, data, ct, is_grads_batched=True)
+  assert torch.equal(got[:, :nnz], want) and not got[:, nnz:].any()
