@@ -14,7 +14,7 @@ constexpr uint32_t kFlatMaxNnz = 0xffffffffu - 8192u;
 // y = A x, walked flat: every wave owns a contiguous range of the nonzeros and tells the rows apart through
 // windows of indptr in LDS.  For matrices with min_mean <= nnz / n_row and nnz <= kFlatMaxNnz; for others the kernels
 // return at once and write nothing (the mean is known on the device only, so the caller enqueues its kernel
-// for short rows behind this one).  x must have at least one element.  Takes 20 bytes of the stream's scratch
+// for short rows behind this one).  x must have at least one element.  Takes 24 bytes of the stream's scratch
 // memory per wave of its launch.  false: no scratch memory, or the launch failed (error recorded).
 template <typename F>
 bool csr_flat_gather(const char *target, hipStream_t stream, const F *data, bool heter, const uint32_t *indices,

@@ -24,8 +24,8 @@
 // Rows across the ranges of two or more waves: a wave never stores a row that began before its range; it
 // leaves that row's partial sum in head[wave], and the partial sum of the row still open at the end of its
 // range in tail[wave] with the row's number.  A second, small kernel adds tail[w] and the heads of the waves
-// that follow, up to the wave the row ends in, and stores the row.  Both arrays hold one entry per wave of the
-// launch (the nonzero count is known on the device only; the number of waves is the launcher's).
+// that follow, as far as their ranges begin within the row, and stores the row.  The arrays hold one entry per wave of
+// the launch (the nonzero count is known on the device only; the number of waves is the launcher's).
 //
 // OUT: what the walk leaves behind.  kFlatSums: y = A x.  kFlatProducts: products[j] = v[row of j] * x[column of j]
 // for every nonzero j (the gradient of the weights), stored with the quads' own 16-byte width; the rows of the
@@ -65,18 +65,11 @@ struct FlatQuads {
   static constexpr int value = sizeof(F) == 4 && OUT != (kFlatSums | kFlatProducts) ? 4 : 2;
 };
 
-// Quads a wave owns: the same on the device (both kernels) from the nonzero count and the number of waves, a multiple
-// of `unit`.  Whole wavefronts of quads: with 1e7 nonzeros and 4,096 waves a wave has two and a half steps, and three
-// for each would leave a fifth of the waves without any.  (The plain sums of x in L2 keep whole steps: that walk is at
-// 126 registers, and spills two if its steps may end anywhere.)
-__device__ __forceinline__ uint32_t flat_quads_per_wave(uint32_t nnz, uint32_t waves, uint32_t unit) {
-  const uint32_t quads = nnz / 4u + (nnz % 4u ? 1u : 0u);
-  const uint32_t per = quads / waves + (quads % waves ? 1u : 0u);
-  return (per + unit - 1u) / unit * unit;
-}
+// The least a wave takes, in nonzeros and rows: a wavefront of quads.  (The plain sums of x in L2 whole steps: a gather
+// costs the address unit the same however many of its lanes hold a nonzero.)
 template <typename F, int OUT, bool STAGED>
-constexpr uint32_t flat_unit() {
-  return (OUT == kFlatSums && !STAGED) ? FlatQuads<F, OUT>::value * kWave : kWave;
+constexpr uint32_t flat_min_share() {
+  return 4u * kWave * ((OUT == kFlatSums && !STAGED) ? FlatQuads<F, OUT>::value : 1);
 }
 
 // Four consecutive indices / weights, whole quad q of the array.
@@ -100,29 +93,59 @@ __device__ __forceinline__ void flat_store_quad(double *__restrict__ p, const do
   __builtin_nontemporal_store(f64x2{v[2], v[3]}, reinterpret_cast<f64x2 *>(p) + 1);
 }
 
-// The last row r in [0, n_row) with indptr[r] <= pos, for pos < indptr[n_row]: the wave searches together,
-// 64 probes a round (four rounds for a million rows).
-__device__ __forceinline__ uint32_t flat_row_of(const uint32_t *__restrict__ indptr, uint32_t n_row, uint32_t pos,
-                                                uint32_t lane) {
-  uint32_t lo = 0, hi = n_row;  // indptr[lo] <= pos < indptr[hi]
-  while (hi - lo > 1u) {
-    const uint32_t span = hi - lo;
-    const uint32_t stride = span / kWave + (span % kWave ? 1u : 0u);
-    const uint64_t probe = static_cast<uint64_t>(lo) + static_cast<uint64_t>(lane) * stride;
-    const bool below = probe < hi && indptr[probe] <= pos;  // (true for lane 0; true lanes form a prefix)
-    const uint32_t cnt = static_cast<uint32_t>(__popcll(__ballot(below)));
-    lo += (cnt - 1u) * stride;
-    hi = (hi - lo > stride) ? lo + stride : hi;
+// Where the waves' ranges begin.  Rows and nonzeros are one list, each row's end behind its nonzeros, and a wave takes
+// an equal piece of that list: a range balanced by nonzeros alone leaves a long block of empty or nearly empty rows to
+// one wave, a window of 64 rows after the other (1,000,000 rows and 5e6 nonzeros, all in the first tenth of the rows: 21 ms,
+// now 70 us; 2,000 rows of 20,000 among as many of 0.1: 5.8 ms, now 0.61; the weights' gradient with 100 nonzeros: 26 ms,
+// now 80 us).  Even matrices: 0.91 to 1.02 of the time before, 1.05 with doubles of 30,000 columns and ten per row.
+// row, pos: of the first `diag` entries of the list, how many are rows (= the row the next nonzero belongs to or the next
+// end is of) and how many nonzeros; two places side by side, 64 probes a round (four rounds for a million rows).
+// A place moves back to a multiple of 32 nonzeros (a line of indices) where the row that holds that one is among the
+// last round's probes: the loads of a wave then cover whole lines.  (A function of `diag` alone and monotone in it: the
+// last round's probes are a fixed division of the rows.)
+__device__ __forceinline__ void flat_split(const uint32_t *__restrict__ indptr, uint32_t n_row, uint32_t nnz,
+                                           const uint64_t (&diag)[2], uint32_t lane, uint32_t (&row)[2],
+                                           uint32_t (&pos)[2]) {
+  const uint64_t total = static_cast<uint64_t>(n_row) + nnz;
+  uint32_t lo[2] = {0, 0}, first[2], ptr[2];
+  uint64_t hi[2] = {n_row, n_row};
+  for (uint32_t stride = n_row / kWave + (n_row % kWave ? 1u : 0u);; stride = stride / kWave + (stride % kWave ? 1u : 0u)) {
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const uint64_t probe = static_cast<uint64_t>(lo[k]) + static_cast<uint64_t>(lane) * stride;
+      ptr[k] = probe < hi[k] ? indptr[probe] : 0xffffffffu;
+    }
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const uint64_t probe = static_cast<uint64_t>(lo[k]) + static_cast<uint64_t>(lane) * stride;
+      const bool below = lane == 0 || (probe < hi[k] && probe + ptr[k] <= diag[k]);  // (a prefix of the lanes)
+      first[k] = lo[k];
+      lo[k] += (static_cast<uint32_t>(__popcll(__ballot(below))) - 1u) * stride;
+      const uint64_t top = static_cast<uint64_t>(lo[k]) + stride;
+      hi[k] = top < hi[k] ? top : hi[k];
+    }
+    if (stride == 1u) break;
   }
-  return lo;
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    if (diag[k] >= total) {
+      row[k] = n_row, pos[k] = nnz;
+      continue;
+    }
+    const uint64_t p = diag[k] - lo[k];
+    row[k] = lo[k], pos[k] = p < nnz ? static_cast<uint32_t>(p) : nnz;
+    const uint32_t back = pos[k] & ~31u;
+    const uint32_t rows = static_cast<uint32_t>(__popcll(__ballot(lane <= lo[k] - first[k] && ptr[k] <= back)));
+    if (rows != 0u) row[k] = first[k] + rows - 1u, pos[k] = back;
+  }
 }
 
 template <typename F, bool HETER, int OUT, bool STAGED>
 __global__ __launch_bounds__(flat_threads(STAGED), 4) void csr_flat_gather_kernel(
     const F *__restrict__ data, const uint32_t *__restrict__ indices, const uint32_t *__restrict__ indptr,
     const F *__restrict__ x, F *__restrict__ y, uint32_t n_row, uint32_t n_col, uint32_t min_mean,
-    double *__restrict__ head, double *__restrict__ tail, uint32_t *__restrict__ tail_row, const F *__restrict__ v,
-    F *__restrict__ products, uint32_t n_products) {
+    double *__restrict__ head, double *__restrict__ tail, uint32_t *__restrict__ tail_row, uint32_t *__restrict__ range,
+    const F *__restrict__ v, F *__restrict__ products, uint32_t n_products) {
   constexpr int U = FlatQuads<F, OUT>::value;
   constexpr uint32_t kStepQuads = U * kWave;
   constexpr int kFlatWaves = flat_threads(STAGED) / kWave;
@@ -140,10 +163,7 @@ __global__ __launch_bounds__(flat_threads(STAGED), 4) void csr_flat_gather_kerne
          i += gridDim.x * blockDim.x)
       products[i] = F(0);
   }
-  if (kSums && nnz == 0) {
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n_row; i += gridDim.x * blockDim.x) y[i] = F(0);
-  }
-  const uint32_t lane = static_cast<uint32_t>(lane_id()), wv = threadIdx.x / kWave;
+  const uint32_t lane = static_cast<uint32_t>(lane_id()), wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   uint32_t *s_ptr = s_ptr_all[wv];
   double *s_sum = s_sum_all[kSums ? wv : 0];
   F *s_v = s_v_all[kProducts ? wv : 0];
@@ -156,18 +176,23 @@ __global__ __launch_bounds__(flat_threads(STAGED), 4) void csr_flat_gather_kerne
     __syncthreads();
   }
   const uint32_t waves = gridDim.x * kFlatWaves, w = blockIdx.x * kFlatWaves + wv;
-  const uint32_t per = flat_quads_per_wave(nnz, waves, flat_unit<F, OUT, STAGED>());
-  if (kSums && lane == 0) head[w] = 0.0, tail[w] = 0.0, tail_row[w] = kNoRow;
-  const uint64_t first_quad = static_cast<uint64_t>(w) * per;
-  if (4u * first_quad >= nnz) return;
-  const uint32_t begin = static_cast<uint32_t>(4u * first_quad);  // the wave owns the nonzeros [begin, end)
-  const uint32_t end = (4u * (first_quad + per) < nnz) ? static_cast<uint32_t>(4u * (first_quad + per)) : nnz;
+  // the wave owns the nonzeros [begin, end) and stores the rows [r, row_end), but for one that began before `begin`
+  uint32_t share = nnz / waves + n_row / waves + 2u;
+  if (share < flat_min_share<F, OUT, STAGED>()) share = flat_min_share<F, OUT, STAGED>();
+  const uint64_t diag[2] = {static_cast<uint64_t>(w) * share, (static_cast<uint64_t>(w) + 1u) * share};
+  uint32_t split_row[2], split_pos[2];
+  if (diag[0] >= static_cast<uint64_t>(n_row) + nnz) {
+    if (kSums && lane == 0) head[w] = 0.0, tail[w] = 0.0, tail_row[w] = kNoRow, range[w] = nnz;
+    return;
+  }
+  flat_split(indptr, n_row, nnz, diag, lane, split_row, split_pos);
+  const uint32_t begin = split_pos[0], end = split_pos[1], row_end = split_row[1];
+  if (kSums && lane == 0) head[w] = 0.0, tail[w] = 0.0, tail_row[w] = kNoRow, range[w] = begin;
   const F w_homo = (HETER || !kSums) ? F(0) : data[0];
 
-  // Invariant at the start of a step [s0, s1): r is the row that holds nonzero s0 or begins there (rows that
-  // end at s0 or before are stored or left to the wave before); s_sum[0] holds what row r has gathered in
-  // this wave so far, s_sum[1..63] are zero.  Wave 0 begins at row 0, so that leading empty rows are stored.
-  uint32_t r = (w == 0) ? 0u : flat_row_of(indptr, n_row, begin, lane);
+  // Invariant at the start of a step [s0, s1): r is the first row whose end is not behind the wave; s_sum[0] holds what
+  // row r has gathered in this wave so far, s_sum[1..63] are zero.
+  uint32_t r = split_row[0];
   if (kSums) s_sum[lane] = 0.0;
   if (lane == 0) s_ptr[kFlatRows + 1] = 0xffffffffu;
 
@@ -198,8 +223,9 @@ __global__ __launch_bounds__(flat_threads(STAGED), 4) void csr_flat_gather_kerne
   };
   u32x4 ci[U] = {};
   F cd[U][4] = {};
-  load_streams(begin, ci, cd);
-  for (uint32_t s0 = begin; s0 < end; s0 += kStep) {
+  load_streams(begin & ~3u, ci, cd);
+  // (a range without nonzeros has one step, for its rows)
+  for (uint32_t s0 = begin & ~3u;; s0 += kStep) {
     const uint32_t s1 = (end - s0 > kStep) ? s0 + kStep : end;
     uint32_t ptr_lane, ptr_last;
     F v_lane = F(0);
@@ -207,10 +233,13 @@ __global__ __launch_bounds__(flat_threads(STAGED), 4) void csr_flat_gather_kerne
       const uint64_t k = static_cast<uint64_t>(r) + lane;
       if constexpr (kProducts) v_lane = k < n_row ? v[k] : F(0);
       ptr_lane = k <= n_row ? indptr[k] : 0xffffffffu;
-      ptr_last = static_cast<uint64_t>(r) + kFlatRows <= n_row ? indptr[r + kFlatRows] : 0xffffffffu;
+      // (a load of the vector unit: one of the scalar unit would be waited for together with every LDS read)
+      uint32_t last = r + kFlatRows;
+      asm volatile("" : "+v"(last));
+      ptr_last = static_cast<uint64_t>(r) + kFlatRows <= n_row ? indptr[last] : 0xffffffffu;
     };
     load_window();
-    if (s1 == nnz && (nnz & 3u) != 0u) {  // (the wave that ends the array: its last one to three nonzeros)
+    if (s1 > 4u * whole) {  // (the array's last one to three nonzeros)
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         if (s0 / 4u + static_cast<uint32_t>(u) * kWave + lane != whole) continue;
@@ -284,13 +313,13 @@ __global__ __launch_bounds__(flat_threads(STAGED), 4) void csr_flat_gather_kerne
       if constexpr (kProducts) s_v[lane] = v_lane;
       if (lane == 0) s_ptr[kFlatRows] = ptr_last;
       __builtin_amdgcn_wave_barrier();
-      const uint32_t lo = s_ptr[0], hi = ptr_last;  // this window takes the nonzeros [lo, hi) of the step
+      const uint32_t lo = s_ptr[0] > begin ? s_ptr[0] : begin, hi = ptr_last;  // this window takes [lo, hi) of the step
       // The row of every quad's first nonzero and the ends of that row and of the next one, for the U quads
       // together (the LDS reads of different quads do not wait for each other); then, without a branch, the
       // quads that lie in one row or in two; a loop only for quads that meet three rows or more.
       uint32_t kq[U], e1[U], e2[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) kq[u] = 0;  // the last k < 64 with s_ptr[k] <= max(p0, lo) (s_ptr[0] = lo)
+      for (int u = 0; u < U; ++u) kq[u] = 0;  // the last k < 64 with s_ptr[k] <= max(p0, lo) (s_ptr[0] <= lo)
 #pragma unroll
       for (uint32_t step = kFlatRows / 2; step != 0; step >>= 1) {
 #pragma unroll
@@ -361,11 +390,11 @@ __global__ __launch_bounds__(flat_threads(STAGED), 4) void csr_flat_gather_kerne
       // rows of the window that end inside the step (a prefix of the window): stored, or, the one that began
       // before this wave's range, left in head[]
       const uint64_t row = static_cast<uint64_t>(r) + lane;
-      const bool ended = row < n_row && s_ptr[lane + 1u] <= s1;
+      const bool ended = lane < row_end - r && s_ptr[lane + 1u] <= s1;
       const uint32_t n_ended = static_cast<uint32_t>(__popcll(__ballot(ended)));
       if (kSums && ended) {
         const double total = s_sum[lane];
-        if (w != 0 && ptr_lane < begin) head[w] = total;
+        if (ptr_lane < begin) head[w] = total;
         else y[row] = static_cast<F>(total);
       }
       double open = 0.0;
@@ -380,12 +409,13 @@ __global__ __launch_bounds__(flat_threads(STAGED), 4) void csr_flat_gather_kerne
       load_window();
     }
     __builtin_amdgcn_wave_barrier();
+    if (s1 == end) break;
   }
   // the row that is still open at the end of the range (if it has nonzeros in it)
   if (kSums && lane == 0 && r < n_row) {
     const uint32_t rs = indptr[r];
     if (rs < end) {
-      if (w != 0 && rs < begin) head[w] = s_sum[0];
+      if (rs < begin) head[w] = s_sum[0];
       else tail[w] = s_sum[0], tail_row[w] = r;
     }
   }
@@ -398,17 +428,17 @@ __global__ __launch_bounds__(kWave) void csr_flat_finish_kernel(const uint32_t *
                                                                 uint32_t n_row, uint32_t min_mean,
                                                                 uint32_t waves, const double *__restrict__ head,
                                                                 const double *__restrict__ tail,
-                                                                const uint32_t *__restrict__ tail_row, uint32_t unit) {
+                                                                const uint32_t *__restrict__ tail_row,
+                                                                const uint32_t *__restrict__ range) {
   const uint32_t nnz = indptr[n_row];
   const uint32_t mean = nnz / n_row;
   if (mean < min_mean || nnz > kFlatMaxNnz) return;
   const uint32_t w = blockIdx.x, lane = threadIdx.x;
   const uint32_t row = tail_row[w];
   if (row == kNoRow) return;
-  const uint32_t per = flat_quads_per_wave(nnz, waves, unit);
-  const uint32_t last = ((indptr[row + 1u] - 1u) / 4u) / per;  // the range the row's last nonzero lies in
+  const uint32_t row_end = indptr[row + 1u];
   double acc = 0.0;
-  for (uint32_t v = w + 1u + lane; v <= last && v < waves; v += kWave) acc += head[v];
+  for (uint32_t v = w + 1u + lane; v < waves && range[v] < row_end; v += kWave) acc += head[v];
   acc = wave_sum(acc);
   if (lane == 0) y[row] = static_cast<F>(tail[w] + acc);
 }
@@ -431,13 +461,13 @@ static bool launch_flat(const char *target, hipStream_t stream, const F *data, c
   const unsigned grid = static_cast<unsigned>(device_info().num_cu) * flat_per_cu(STAGED);
   const uint32_t waves = grid * (flat_threads(STAGED) / kWave);
   double *head = nullptr, *tail = nullptr;
-  uint32_t *tail_row = nullptr;
+  uint32_t *tail_row = nullptr, *range = nullptr;
   if (kSums) {
-    // [head: waves doubles][tail: waves doubles][tail_row: waves words]
-    unsigned char *ws = static_cast<unsigned char *>(stream_workspace(stream, static_cast<size_t>(waves) * 20u));
+    // [head: waves doubles][tail: waves doubles][tail_row: waves words][range: waves words]
+    unsigned char *ws = static_cast<unsigned char *>(stream_workspace(stream, static_cast<size_t>(waves) * 24u));
     if (ws == nullptr) return false;
     head = reinterpret_cast<double *>(ws), tail = head + waves;
-    tail_row = reinterpret_cast<uint32_t *>(tail + waves);
+    tail_row = reinterpret_cast<uint32_t *>(tail + waves), range = tail_row + waves;
   }
   auto kernel = csr_flat_gather_kernel<F, HETER, OUT, STAGED>;
   size_t lds = 0;
@@ -451,11 +481,11 @@ static bool launch_flat(const char *target, hipStream_t stream, const F *data, c
     }
   }
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(flat_threads(STAGED)), lds, stream, data, indices, indptr, x, y, n_row,
-                     n_col, min_mean, head, tail, tail_row, v, products, n_products);
+                     n_col, min_mean, head, tail, tail_row, range, v, products, n_products);
   if (kSums)
     hipLaunchKernelGGL(csr_flat_finish_kernel<F>, dim3(waves), dim3(kWave), 0, stream, indptr, y, n_row, min_mean,
                        waves, static_cast<const double *>(head), static_cast<const double *>(tail),
-                       static_cast<const uint32_t *>(tail_row), flat_unit<F, OUT, STAGED>());
+                       static_cast<const uint32_t *>(tail_row), static_cast<const uint32_t *>(range));
   return check_launch(target);
 }
 

@@ -1173,6 +1173,70 @@ def test_csr_matvec_padded_index_arrays(cuda, dtype):
   assert got[4] == 3 and got.sum() == 3
 
 
+def _uneven_blocks(kind, rng):
+  """Row lengths of a matrix whose nonzeros lie in a small part of the rows."""
+  counts = np.zeros(400_000, np.int64)
+  if kind == "first":
+    counts[:20_000] = rng.poisson(100, 20_000)
+  elif kind == "last":
+    counts[-20_000:] = rng.poisson(100, 20_000)
+  elif kind == "thin":  # a few thousand long rows in the middle, one nonzero in ten rows elsewhere
+    counts[:] = rng.random(counts.shape[0]) < 0.1
+    counts[200_000:202_000] = 900
+  elif kind == "few":  # far fewer nonzeros than rows
+    counts[::9973] = 1
+  elif kind == "long":  # rows that run through many waves' ranges, empty rows between them
+    counts[[0, 1, 150_000, 150_001, 399_999]] = [600_000, 3, 500_000, 700_001, 1]
+  return counts
+
+
+# The walk over the nonzeros shares rows as well as nonzeros among its waves: no wave is left with all the rows that have
+# (nearly) none.  60,000 columns: a part of the vector in LDS; 200,000: gathered from L2 (doubles: half of that).
+@pytest.mark.parametrize("kind", ["first", "last", "thin", "few", "long"])
+@pytest.mark.parametrize("n_col", [60_000, 200_000])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_csr_walk_over_blocks_of_empty_rows(cuda, kind, n_col, dtype):
+  if dtype == np.float64:
+    n_col //= 2
+  rng = np.random.default_rng(n_col)
+  counts = _uneven_blocks(kind, rng)
+  n_row, nnz = counts.shape[0], int(counts.sum())
+  print("case", kind, n_col, dtype.__name__, nnz, flush=True)
+  indptr = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+  indices = rng.integers(0, n_col, nnz).astype(np.int32)  # (not sorted, some twice: the walk needs neither)
+  data, v, ct = (rng.standard_normal(n).astype(dtype) for n in (nnz, n_col, n_row))
+  rows = np.repeat(np.arange(n_row), counts)
+  addend = (v[indices] * data).astype(np.float64)
+  want = np.bincount(rows, weights=addend, minlength=n_row)
+  mag = np.bincount(rows, weights=np.abs(addend), minlength=n_row)
+  # float64 sums in another order, rounded once to the result's type
+  bound = np.finfo(dtype).eps * np.abs(want) + 4 * np.finfo(np.float64).eps * np.sqrt(np.maximum(counts, 1)) * mag
+  dev = [torch.from_numpy(a).cuda() for a in (data, indices, indptr, v, ct)]
+  forward = lambda: bpl.csr_matvec(dev[0], dev[1], dev[2], dev[3], shape=(n_row, n_col))
+  assert (np.abs(forward().cpu().numpy() - want) <= bound).all()
+  d = dev[0].clone().requires_grad_()
+  y = bpl.cusparse_csr_matvec(d, dev[1], dev[2], dev[3], shape=(n_row, n_col))
+  products = lambda: torch.autograd.grad(y, d, dev[4], retain_graph=True)
+  assert np.array_equal(products()[0].cpu().numpy(), ct[rows] * v[indices])
+  t = dev[4].clone().requires_grad_()
+  z = bpl.cusparse_csr_matvec(d, dev[1], dev[2], t, shape=(n_row, n_col), transpose=True)
+  both = lambda: torch.autograd.grad(z, (d, t), dev[3], retain_graph=True)
+  got, got_sums = (g.cpu().numpy() for g in both())
+  assert np.array_equal(got, ct[rows] * v[indices]) and (np.abs(got_sums - want) <= bound).all()
+  # 1.3e6 nonzeros and 400,000 rows are 20 to 60 us' work; one wave that takes 380,000 rows 64 at a time needs 3 ms and more
+  # ("few", forward: another walk)
+  for call in (forward, products, both):
+    times = []
+    for _ in range(5):
+      a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+      a.record()
+      call()
+      b.record()
+      b.synchronize()
+      times.append(a.elapsed_time(b))
+    assert min(times) < 1.0, times
+
+
 @pytest.mark.parametrize("n_row,n_col,mean", [(300, 20_000, 8), (2500, 60_000, 20), (18_000, 30_000, 30), (2100, 40_000, 60),
                                               (17_000, 700_000, 100), (2200, 150_000, 200), (2049, 90_000, 500)])
 def test_rows_left_to_a_wave_or_a_workgroup(cuda, oracle_mod, n_row, n_col, mean):
