@@ -137,7 +137,16 @@ bool flat_window_scatter(const char *target, hipStream_t stream, const F *data, 
 // = batch * columns, and `active_colbase` = what to add to the columns of each listed row (its
 // batch entry * columns); n_row stays the matrix's row count (indptr has n_row + 1 entries).
 constexpr size_t kBinEventFillBytes = 131072;
-constexpr uint64_t kMostRunPairs = 1ull << 27;  // pairs that the runs hold together at most
+// How many entries of a batch (one matrix of nnz nonzeros, entries' columns side by side) such a chain takes, and how many
+// pairs its runs are to hold.
+struct EventGroup {
+  uint32_t entries;
+  uint64_t run_pairs;
+};
+template <typename F>
+EventGroup bin_event_group(uint32_t n_row, uint32_t n_col, uint32_t nnz, uint32_t batch);
+template <typename F>
+size_t bin_event_group_bytes(uint32_t n_col, uint64_t run_pairs);
 template <typename F>
 bool bin_event_scatter_usable(uint32_t n_col);
 template <typename F>

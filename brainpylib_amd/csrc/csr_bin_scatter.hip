@@ -1267,7 +1267,7 @@ inline uint32_t event_window_shift(uint32_t n_out) {
 inline uint64_t event_run_pairs(uint32_t n_row, uint32_t n_col) {
   uint64_t t = 4096ull * (n_row > n_col ? n_row : n_col);
   if (t < (1ull << 24)) t = 1ull << 24;
-  if (t > kMostRunPairs) t = kMostRunPairs;
+  if (t > (1ull << 27)) t = 1ull << 27;
   return t;
 }
 
@@ -1366,9 +1366,38 @@ bool bin_event_scatter_usable(uint32_t n_col) {
 
 template <typename F>
 size_t bin_event_scatter_bytes(uint32_t n_row, uint32_t n_col) {
+  return bin_event_group_bytes<F>(n_col, event_run_pairs(n_row, n_col));
+}
+
+template <typename F>
+size_t bin_event_group_bytes(uint32_t n_col, uint64_t run_pairs) {
   const uint32_t n_win = div_up(n_col, 1u << event_window_shift(n_col));
-  const uint64_t cap = event_run_pairs(n_row, n_col) / (n_win * kSubRuns);
+  const uint64_t cap = run_pairs / (n_win * kSubRuns);
   return kBinEventFillBytes + static_cast<size_t>(cap) * n_win * kSubRuns * sizeof(BinPair<F>);
+}
+
+// A group is a chain of three launches whatever its size, so it takes as many entries as keep the virtual output within
+// windows that are added in one slice (2^21 columns), the list of its active rows within 400 MB (2^25 rows) and every
+// pair of all its nonzeros within runs of 2 GB (with half of their number to spare: a producer's pairs go to one of the
+// eight parts of a window's run, a few producers to an entry): at whatever activity nothing of a group of more than 8
+// entries goes through direct atomics.  Up to 8 entries beyond those bounds.  Groups of equal size.  20 entries of 8e6
+// nonzeros at 3 / 60 / 100 % events, one group: 55 / 620 / 1,010 us (three groups of 7: 107 / 663 / 1,097); 64 of 1e7 at 100 %,
+// four groups of 16: 4,300 us (groups of 8: 4,528; of 64, whose pairs find the runs full from 20 % on: 21,950).
+constexpr uint64_t kMostGroupRunBytes = 1ull << 31;
+template <typename F>
+EventGroup bin_event_group(uint32_t n_row, uint32_t n_col, uint32_t nnz, uint32_t batch) {
+  const uint64_t by_pairs = 2ull * (kMostGroupRunBytes / sizeof(BinPair<F>)) / (3ull * (nnz ? nnz : 1u));
+  uint64_t fits = (1ull << 21) / n_col;
+  if (fits > (1ull << 25) / n_row) fits = (1ull << 25) / n_row;
+  if (fits > by_pairs) fits = by_pairs;
+  const uint32_t most = fits < 8 ? 8u : fits < batch ? static_cast<uint32_t>(fits) : batch;
+  uint32_t group = div_up(batch, div_up(batch, most));
+  while (group > 1 && (static_cast<uint64_t>(group) * n_col >= (1ull << 24) || static_cast<uint64_t>(group) * n_row >= (1ull << 31)))
+    --group;
+  const uint64_t all = static_cast<uint64_t>(group) * nnz;
+  uint64_t pairs = event_run_pairs(n_row, group * n_col);
+  if (group > 8 && pairs < all + all / 2) pairs = all + all / 2;
+  return EventGroup{group, pairs};
 }
 
 // at least kMinRunPairs pairs per run
@@ -1576,6 +1605,10 @@ template bool bin_event_scatter_usable<float>(uint32_t);
 template bool bin_event_scatter_usable<double>(uint32_t);
 template size_t bin_event_scatter_bytes<float>(uint32_t, uint32_t);
 template size_t bin_event_scatter_bytes<double>(uint32_t, uint32_t);
+template size_t bin_event_group_bytes<float>(uint32_t, uint64_t);
+template size_t bin_event_group_bytes<double>(uint32_t, uint64_t);
+template EventGroup bin_event_group<float>(uint32_t, uint32_t, uint32_t, uint32_t);
+template EventGroup bin_event_group<double>(uint32_t, uint32_t, uint32_t, uint32_t);
 template size_t bin_event_scatter_min_bytes<float>(uint32_t);
 template size_t bin_event_scatter_min_bytes<double>(uint32_t);
 template bool bin_event_scatter<float, uint32_t>(hipStream_t, const float *, bool, const uint32_t *, const uint32_t *, float *,
@@ -1602,3 +1635,13 @@ template bool bin_scatter<double>(const char *, hipStream_t, const double *, boo
                                   const double *, double *, uint32_t, uint32_t, uint32_t);
 
 }  // namespace bpl
+
+extern "C" void bpl_batched_scatter_plan(uint32_t n_row, uint32_t n_col, uint32_t nnz, uint32_t batch_size,
+                                         uint32_t value_bytes, uint32_t *entries, uint64_t *run_pairs) {
+  bpl::EventGroup plan = {0, 0};
+  if (n_row != 0 && n_col != 0 && batch_size != 0)
+    plan = value_bytes == 8 ? bpl::bin_event_group<double>(n_row, n_col, nnz, batch_size)
+                            : bpl::bin_event_group<float>(n_row, n_col, nnz, batch_size);
+  if (entries != nullptr) *entries = plan.entries;
+  if (run_pairs != nullptr) *run_pairs = plan.run_pairs;
+}

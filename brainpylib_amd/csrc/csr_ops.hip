@@ -21,7 +21,6 @@
 //
 // Reference boundary: lib/gpu_event_csr_matvec.cu:148-260, lib/gpu_csr_matvec.cu:84-135,195-246,
 // 505-621 (buffer order, descriptor, target names).
-#include <algorithm>
 #include <mutex>
 #include <type_traits>
 
@@ -2254,29 +2253,19 @@ void event_csr_batching_entry(const char *target, hipStream_t stream, void **buf
                                                 d.batch_size, 0);
     return;
   }
-  // Transposed, one matrix for all entries: groups of entries go through ONE sorted scatter over a virtual output of
-  // group * n_col columns (entry g's columns shifted by g * n_col), fed by one list of the active rows of the
-  // group's entries.  A group is a chain of three launches whatever its size, so it takes as many entries as keep
-  // the virtual output within windows that are added in one slice (2^21 columns) and the pairs of a sixth of
-  // all nonzeros within the runs of the sort (20 entries of 8e6 nonzeros in one group instead of three: 105 -> 52 us),
-  // and the list of its active rows within 400 MB (2^25 rows); up to 8 entries beyond those bounds (1e8 nonzeros:
-  // larger groups gain nothing and overflow the runs sooner).  Groups of equal size.
+  // Transposed, one matrix for all entries: groups of entries (bin_event_group()) go through ONE sorted scatter over a
+  // virtual output of group * n_col columns (entry g's columns shifted by g * n_col), fed by one list of the active rows
+  // of the group's entries.
   if (d.transpose && shared_matrix && d.batch_size > 1 && d.n_row > 0 && d.n_col > 0) {
-    const uint64_t by_columns = (1ull << 21) / d.n_col, by_pairs = 6ull * kMostRunPairs / (d.nnz ? d.nnz : 1u);
-    const uint64_t by_rows = (1ull << 25) / d.n_row;
-    const uint64_t fits = std::min(by_rows, std::min(by_columns, by_pairs));
-    const uint32_t most = fits < 8 ? 8u : fits < d.batch_size ? static_cast<uint32_t>(fits) : d.batch_size;
-    uint32_t group = div_up(d.batch_size, div_up(d.batch_size, most));
-    while (group > 1 && (static_cast<uint64_t>(group) * d.n_col >= (1ull << 24) ||
-                         static_cast<uint64_t>(group) * d.n_row >= (1ull << 31)))
-      --group;
+    const EventGroup plan = bin_event_group<F>(d.n_row, d.n_col, d.nnz, d.batch_size);
+    const uint32_t group = plan.entries;
     const uint32_t vcols = group * d.n_col;
     if (group > 1 && vcols > 8192 && bin_event_scatter_usable<F>(vcols)) {
       auto round_up = [](size_t v) { return (v + 255) / 256 * 256; };
       const size_t vrows = static_cast<size_t>(group) * d.n_row;
       const size_t list_sz = round_up(vrows * sizeof(uint2));
       const size_t base_sz = round_up(vrows * sizeof(uint32_t));
-      const size_t scratch_bytes = bin_event_scatter_bytes<F>(d.n_row, vcols);
+      const size_t scratch_bytes = bin_event_group_bytes<F>(vcols, plan.run_pairs);
       unsigned char *ws = static_cast<unsigned char *>(stream_workspace(stream, list_sz + base_sz + scratch_bytes));
       uint32_t *counters = ws ? stream_counters(stream) : nullptr;
       if (ws != nullptr && counters != nullptr) {

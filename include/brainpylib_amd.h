@@ -204,6 +204,12 @@ const char *bpl_version(void);
  * three pointers may be NULL. */
 int bpl_stream_workspace_query(bpl_stream_t stream, void **ptr, size_t *bytes, size_t *retired_bytes);
 
+/* How event_csr_matvec_batching_* with transpose set divides a batch that shares one matrix: at most
+ * `entries` of them go through one chain of launches, whose scratch memory holds `run_pairs` pairs of
+ * value_bytes (4 or 8) each with their columns.  No device is touched. */
+void bpl_batched_scatter_plan(uint32_t n_row, uint32_t n_col, uint32_t nnz, uint32_t batch_size, uint32_t value_bytes,
+                              uint32_t *entries, uint64_t *run_pairs);
+
 /* Self-check of the jitconn operators' skip computation (no counterpart in the reference, whose
  * kernels call log() per synapse, lib/gpu_jitconn_event_matvec.cu:94-110).  The kernels compute
  * ceil(log(U) / log_p) on a fast path (hardware fp32 log2) wherever the quotient is further from an

@@ -164,3 +164,38 @@ def test_batching_transposed_in_groups(cuda, oracle_mod, n_row, n_col, mean, bat
     one = np.full((1, 1), 0.7, dtype=dtype)
     got, want = _check(oracle_mod, one, indices[None], indptr[None], events, batch, (n_row, n_col), True, "homo")
     assert np.array_equal(got, want)  # (counts: the reference's bits whatever the order)
+
+
+def test_batching_transposed_with_every_event_set(cuda):
+  # 40 entries of 8e6 nonzeros: one group of them has 3.2e8 pairs, more than the runs of the sort hold; what finds them full
+  # goes through atomics on device memory, which is right but takes five times as long.  Integer weights: exact sums.
+  n_row, n_col, batch = 20_000, 20_000, 40
+  rng = np.random.default_rng(3)
+  indptr = np.arange(n_row + 1, dtype=np.int32) * 400
+  indices = rng.integers(0, n_col, n_row * 400).astype(np.int32)
+  data = rng.integers(-3, 4, indices.shape[0]).astype(np.float32)
+  events = np.ones((batch, n_row), bool)
+  events[5], events[17, ::2] = False, False
+  dev = [torch.from_numpy(a).to(cuda) for a in (data[None], indices[None], indptr[None], events)]
+  call = lambda b: bpl.event_csr_matvec_batching(*dev[:3], dev[3][:b], batch_size=b, shape=(n_row, n_col), transpose=True)
+  got = call(batch).cpu().numpy()
+  want = np.bincount(indices, weights=data, minlength=n_col)
+  half = np.repeat(np.arange(n_row) % 2 == 1, 400)
+  for b in range(batch):
+    if b == 5:
+      assert not got[b].any()
+    elif b == 17:
+      assert np.array_equal(got[b], np.bincount(indices[half], weights=data[half], minlength=n_col))
+    else:
+      assert np.array_equal(got[b], want)
+  times = {}
+  for b in (8, batch):  # (eight entries' pairs fit in any case)
+    times[b] = []
+    for _ in range(4):
+      t0, t1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+      t0.record()
+      call(b)
+      t1.record()
+      t1.synchronize()
+      times[b].append(t0.elapsed_time(t1) / b)
+  assert min(times[batch]) < 2.0 * min(times[8]), times
