@@ -1364,6 +1364,9 @@ bool bin_event_scatter_usable(uint32_t n_col) {
   return n_win >= 2 && n_win <= kMaxWindows;
 }
 
+// at least kMinRunPairs pairs per run
+constexpr uint32_t kMinRunPairs = 1024;
+
 template <typename F>
 size_t bin_event_scatter_bytes(uint32_t n_row, uint32_t n_col) {
   return bin_event_group_bytes<F>(n_col, event_run_pairs(n_row, n_col));
@@ -1381,8 +1384,9 @@ size_t bin_event_group_bytes(uint32_t n_col, uint64_t run_pairs) {
 // pair of all its nonzeros within runs of 2 GB (with half of their number to spare: a producer's pairs go to one of the
 // eight parts of a window's run, a few producers to an entry): at whatever activity nothing of a group of more than 8
 // entries goes through direct atomics.  Up to 8 entries beyond those bounds.  Groups of equal size.  20 entries of 8e6
-// nonzeros at 3 / 60 / 100 % events, one group: 55 / 620 / 1,010 us (three groups of 7: 107 / 663 / 1,097); 64 of 1e7 at 100 %,
-// four groups of 16: 4,300 us (groups of 8: 4,528; of 64, whose pairs find the runs full from 20 % on: 21,950).
+// nonzeros at 3 / 30 / 100 % events: one group 54 / 345 / 1,240 us, three of 7 107 / 352 / 1,100.  64 of 1e7 at 3 / 60 / 100 %:
+// four groups of 16 201 / 2,730 / 4,800 us, eight of 8 323 / 2,730 / 4,530; one of 64, whose pairs find the runs full from
+// 20 % on, 159 / 11,660 / 21,950.
 constexpr uint64_t kMostGroupRunBytes = 1ull << 31;
 template <typename F>
 EventGroup bin_event_group(uint32_t n_row, uint32_t n_col, uint32_t nnz, uint32_t batch) {
@@ -1397,11 +1401,17 @@ EventGroup bin_event_group(uint32_t n_row, uint32_t n_col, uint32_t nnz, uint32_
   const uint64_t all = static_cast<uint64_t>(group) * nnz;
   uint64_t pairs = event_run_pairs(n_row, group * n_col);
   if (group > 8 && pairs < all + all / 2) pairs = all + all / 2;
+  // (nor more than there can be: every nonzero of the entries that meet in a window in that window, for all windows, and a
+  // producer more than its share of them in each eighth of a run; 20 entries of 1,000 x 1,000 with 50 per row hold 42 MB)
+  const uint32_t shift = event_window_shift(group * n_col), n_win = div_up(group * n_col, 1u << shift);
+  const uint64_t meet = static_cast<uint64_t>(div_up(1u << shift, n_col)) * n_win * nnz;
+  const uint64_t most_pairs = meet + meet / 64u * (group < n_win ? group : n_win);
+  const uint64_t least_pairs = static_cast<uint64_t>(kMinRunPairs) * n_win * kSubRuns;
+  if (pairs > most_pairs) pairs = most_pairs;
+  if (pairs < least_pairs) pairs = least_pairs;
   return EventGroup{group, pairs};
 }
 
-// at least kMinRunPairs pairs per run
-constexpr uint32_t kMinRunPairs = 1024;
 template <typename F>
 size_t bin_event_scatter_min_bytes(uint32_t n_col) {
   const uint32_t n_win = div_up(n_col, 1u << event_window_shift(n_col));

@@ -35,5 +35,21 @@ def test_every_pair_of_a_large_group_finds_room(value_bytes, per_row):
         assert entries >= min(batch, 8) or -(-batch // entries) == -(-batch // 8), what
 
 
+@pytest.mark.parametrize("value_bytes", [4, 8])
+def test_small_networks_take_little_scratch_memory(value_bytes):
+  # 20 entries of a 1,000 x 1,000 network of 50,000 nonzeros: every nonzero of an entry may lie in one of the four windows that
+  # an entry spans, which makes five times the 1e6 pairs there are at most
+  entries, pairs = _plan(1000, 1000, 50_000, 20, value_bytes)
+  assert entries == 20 and 1_000_000 * 4 <= pairs <= 1_000_000 * 6
+  for n_row, n_col in SHAPES:
+    for per_row in (1, 3, 50):
+      nnz = n_row * per_row
+      for batch in (2, 8, 20, 500):
+        entries, pairs = _plan(n_row, n_col, nnz, batch, value_bytes)
+        # never more than every nonzero of every entry in each of at most 128 windows, twice, but for the least the sort
+        # works with (1,024 pairs in each of the eight parts of a window's run)
+        assert pairs <= max(2 * 128 * entries * nnz, 128 * 8 * 1024), (n_row, n_col, nnz, entries, pairs)
+
+
 def test_no_matrix():
   assert _plan(0, 5, 0, 3, 4) == _plan(5, 0, 0, 3, 4) == _plan(5, 5, 9, 0, 4) == (0, 0)

@@ -149,3 +149,21 @@ def test_batched_scatter_of_a_small_network_is_captured_on_a_cold_stream(cuda):
     g.replay()
     torch.cuda.synchronize()
     assert torch.equal(out, call()), i  # (integers: exact in any order)
+
+
+def test_scratch_memory_of_a_batch_of_a_small_network(cuda):
+  # the batching descriptor says how many nonzeros there are: 20 entries of 1,000 x 1,000 with 50 per row hold 42 MB of runs
+  # and a quarter of head room, not what 4,096 pairs for every column would take (655 MB)
+  s = torch.cuda.Stream()
+  rng = np.random.default_rng(8)
+  indices = torch.from_numpy(rng.integers(0, 1000, (1, 50_000)).astype(np.int32)).to(cuda)
+  indptr = (torch.arange(1001, dtype=torch.int32) * 50)[None].to(cuda)
+  data = torch.ones((1, 50_000), device=cuda)
+  events = torch.ones((20, 1000), dtype=torch.bool, device=cuda)
+  torch.cuda.synchronize()
+  with torch.cuda.stream(s):
+    out = bpl.event_csr_matvec_batching(data, indices, indptr, events, batch_size=20, shape=(1000, 1000), transpose=True)
+    has, _, size, _ = _query(s.cuda_stream)
+  s.synchronize()
+  assert has and size < 60e6, size
+  assert torch.equal(out.cpu(), torch.bincount(indices[0].cpu(), minlength=1000).to(torch.float32).expand(20, -1))
