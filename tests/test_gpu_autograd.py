@@ -103,11 +103,13 @@ def test_csr_matvec_gradients(cuda, shape, transpose, homo):
 
 
 # rows, columns, mean row length: one partial step; rows shorter than a quad (windows of more than 64 rows to a step);
-# vectors that just fit the 138 KB staged in LDS (35,328 floats, 17,664 doubles), one element more, four times as many
-# (the last staged size) and one more (gathered from L2 only); rows that run through many waves' ranges
+# vectors that fit the 139 to 151 KB staged in LDS, one element more than what fits (beside sums and products 36,608 floats
+# or 17,792 doubles, beside products alone 38,656 or 18,816), the last staged size and one more (gathered from L2 only);
+# rows that run through many waves' ranges
 @pytest.mark.parametrize("n_row,n_col,mean", [(3, 9, 2), (9000, 200, 1), (300, 35_328, 900), (2000, 35_329, 300),
                                               (900, 17_664, 10), (20_000, 141_312, 40), (700, 141_313, 800),
-                                              (10, 300_000, 20_000)])
+                                              (10, 300_000, 20_000), (500, 36_609, 40), (500, 38_657, 40),
+                                              (500, 17_793, 40), (500, 18_817, 40)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
 @pytest.mark.parametrize("transpose", [False, True])
 def test_gradients_of_weights_and_vector_from_one_walk(cuda, n_row, n_col, mean, dtype, transpose):
