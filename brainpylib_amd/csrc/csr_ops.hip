@@ -617,10 +617,11 @@ __global__ __launch_bounds__(256) void sum_partials_kernel(const F *__restrict__
 // on), or of more than 64 steps in any case.  A step is a chain of dependent loads, 0.7 us: with 64 steps alone the
 // longest rows of an uneven matrix were the last to end by far (17,683 rows of 150 on average, log-normal with
 // sigma 1, weights per nonzero, float: 51 us, now 26, with a dense vector 42 and 18; 2,493 rows of 1,735, double: 86 us,
-// now 39).
+// now 39).  `least`: none is shorter than this.
 constexpr uint32_t kHubSteps = 64;
-__device__ __forceinline__ uint32_t hub_length(uint32_t mean, uint32_t step) {
-  const uint32_t low = mean < 0x10000000u && 4u * mean > 4u * step ? 4u * mean : 4u * step;
+__device__ __forceinline__ uint32_t hub_length(uint32_t mean, uint32_t step, uint32_t least = 0) {
+  uint32_t low = mean < 0x10000000u && 4u * mean > 4u * step ? 4u * mean : 4u * step;
+  if (least > low) low = least;
   return low < kHubSteps * step ? low : kHubSteps * step;
 }
 
@@ -1317,9 +1318,22 @@ __global__ __launch_bounds__(1024, (MODE == kEvent && BITS == 1) ? 8 : 4) void c
   // lanes per row from the mean row length
   const uint32_t mean = nnz / n_row;
   uint32_t gpb = 0, hub_len = 0;  // rows per workgroup and round of the walk chosen below, its longest row
-  // (counts of one double weight: their sum is formed by one thread of a workgroup that waits for it, which costs more
-  // than the longer walk: 60,000 rows of 700, log-normal: 88 us with steps of 512 here)
-  constexpr uint32_t kWaveStep = 8 * kWave * (MODE == kEvent && !HETER && sizeof(F) == 8 ? 4 : 1);
+  // (counts of one weight: a step is cheap, and the sum of double is formed by one thread of a workgroup that waits for
+  // it: 60,000 rows of 700, log-normal, double: 88 us with 512 here; 50,000 rows of 200, a tenth of 2,600: 54 -> 29 us)
+  constexpr uint32_t kWaveStep = 8 * kWave * (MODE == kEvent && !HETER ? 4 : 1);
+  // A hub row costs its workgroup 2.4 us whatever its length (three barriers, a chain of loads), a step in the wave walk
+  // 0.4 to 0.7 us with a dense vector or one weight and up to 1.8 with weights per nonzero.  So a workgroup of 256 threads
+  // leaves rows of up to eight (dense), six or, above, sixteen steps to their waves (5,000 rows of 100, every fifth of 3,000, weights
+  // per nonzero 24 -> 21 us, 300 uneven rows of 500 12.5 -> 10.3), and with a dense vector a row of up to twice a wave's
+  // share of the nonzeros is none (20,000 x 30,000, a tenth of the rows of 4,000, the others of 100: 60 -> 34 us).
+  uint32_t wave_least = 0;
+  if constexpr (MODE == kDense) {
+    const uint32_t share = nnz / (gridDim.x * (blockDim.x / kWave));
+    wave_least = blockDim.x < 1024u ? 8u * kWaveStep : 0u;
+    if (share < 0x10000000u && 2u * share > wave_least) wave_least = 2u * share;
+  } else if (HETER) {
+    wave_least = blockDim.x < 1024u ? 6u * kWaveStep : 0u;
+  }
   if constexpr (MODE == kDense && BITS == 0) {
     // (rows of `skip_mean` nonzeros or more on average: the launcher's other kernel has taken this matrix)
     if (skip_mean != 0 && mean >= skip_mean && nnz <= kFlatMaxNnz) return;
@@ -1327,7 +1341,7 @@ __global__ __launch_bounds__(1024, (MODE == kEvent && BITS == 1) ? 8 : 4) void c
   if constexpr (MODE == kDense && BITS == 1) {
     // (nothing left to hide but the index and weight streams: the walks of the event gather)
     const VT *xs = reinterpret_cast<const VT *>(s_bits);
-    if (mean >= 384) { gpb = 1; hub_len = hub_length(mean, kWaveStep); gather_rows_wave<F, VT, HETER, MODE, BITS, 8>(data, indices, indptr, xs, y, n_row, s_bits, coarse_g, hub_len); }
+    if (mean >= 384) { gpb = 1; hub_len = hub_length(mean, kWaveStep, wave_least); gather_rows_wave<F, VT, HETER, MODE, BITS, 8>(data, indices, indptr, xs, y, n_row, s_bits, coarse_g, hub_len); }
     else if (mean >= 24) { gpb = blockDim.x / 8; hub_len = hub_length(mean, 8 * 8); gather_rows<F, VT, HETER, MODE, BITS, 8, 8>(data, indices, indptr, xs, y, n_row, s_bits, coarse_g, hub_len); }
     else if (mean >= 12) { gpb = blockDim.x / 4; hub_len = hub_length(mean, 8 * 4); gather_rows<F, VT, HETER, MODE, BITS, 4, 8>(data, indices, indptr, xs, y, n_row, s_bits, coarse_g, hub_len); }
     else { gpb = blockDim.x / 4; hub_len = hub_length(mean, 4 * 4); gather_rows<F, VT, HETER, MODE, BITS, 4, 4>(data, indices, indptr, xs, y, n_row, s_bits, coarse_g, hub_len); }
@@ -1344,7 +1358,7 @@ __global__ __launch_bounds__(1024, (MODE == kEvent && BITS == 1) ? 8 : 4) void c
         return;
       }
     }
-    if (mean >= 384) { gpb = 1; hub_len = hub_length(mean, kWaveStep); gather_rows_wave<F, VT, HETER, MODE, BITS, 8>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
+    if (mean >= 384) { gpb = 1; hub_len = hub_length(mean, kWaveStep, wave_least); gather_rows_wave<F, VT, HETER, MODE, BITS, 8>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
     else if (mean >= 48) { gpb = blockDim.x / 8; hub_len = hub_length(mean, 16 * 8); gather_rows<F, VT, HETER, MODE, BITS, 8, 16>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
     else { gpb = blockDim.x / 4; hub_len = hub_length(mean, 8 * 4); gather_rows<F, VT, HETER, MODE, BITS, 4, 8>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
   } else {
@@ -1362,7 +1376,7 @@ __global__ __launch_bounds__(1024, (MODE == kEvent && BITS == 1) ? 8 : 4) void c
         return;
       }
     }
-    if (mean >= 384) { gpb = 1; hub_len = hub_length(mean, kWaveStep); gather_rows_wave<F, VT, HETER, MODE, BITS, 8>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
+    if (mean >= 384) { gpb = 1; hub_len = hub_length(mean, kWaveStep, wave_least); gather_rows_wave<F, VT, HETER, MODE, BITS, 8>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
     // (a dense vector is gathered from L2: for rows of 48 .. 191 nonzeros the pipelined 32-lane walk keeps more
     // of those gathers in flight than a wave per row does)
     else if (MODE == kEvent && mean >= 48u) { gpb = blockDim.x / 8; hub_len = hub_length(mean, 8 * 8); gather_rows<F, VT, HETER, MODE, BITS, 8, 8>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
@@ -1721,7 +1735,10 @@ bool launch_gather_impl(const char *target, hipStream_t stream, const F *data, c
   // Small problems: 256-thread workgroups, one wave per row at most.  Large ones: 1024-thread
   // persistent workgroups so that few copies of the event bitmap are built.
   // (Few rows over many columns, or an LDS image of more than 16 KB per workgroup: the large ones too.)
-  const bool wide = n_col > kHubSteps * 8 * kWave;  // rows can be long enough to go to whole workgroups
+  // (Few rows that can be longer than 64 steps of a wave.  Rows go to whole workgroups from 2,048 to 4,096 nonzeros on, but
+  // 1,024 threads a row for so short ones cost more than 256: 1,000 uneven rows of 500 over 20,000 columns 13.3 -> 14.6 us,
+  // dense 11.6 -> 14.3, 300 of 1,500 21 -> 28.)
+  const bool wide = n_col > kHubSteps * 8 * kWave;
   const int block = (n_row >= 16384 || lds_bytes > 16 * 1024 || (wide && n_row < 2048)) ? 1024 : 256;
   // The occupancy query is the same for every call with the same LDS size: remember the last one.
   struct Cached {

@@ -1239,14 +1239,15 @@ def test_csr_walk_over_blocks_of_empty_rows(cuda, kind, n_col, dtype):
 
 
 @pytest.mark.parametrize("n_row,n_col,mean", [(300, 20_000, 8), (2500, 60_000, 20), (18_000, 30_000, 30), (2100, 40_000, 60),
-                                              (17_000, 700_000, 100), (2200, 150_000, 200), (2049, 90_000, 500)])
+                                              (17_000, 700_000, 100), (2200, 150_000, 200), (2049, 90_000, 500),
+                                              (700, 20_000, 420)])
 def test_rows_left_to_a_wave_or_a_workgroup(cuda, oracle_mod, n_row, n_col, mean):
   # rows of more than four steps of their walk and four times the mean are walked by a wave (up to 4,096 nonzeros)
   # or a whole workgroup: lengths at and around every step multiple, at both lines and far above, first and last row
   # among them, empty rows between.  Integer weights and vectors: every sum is exact.
   rng = np.random.default_rng(n_row)
   counts = np.full(n_row, mean)
-  special = [b + d for b in (64, 128, 256, 512, 1024, 2048, 4 * mean, 4096, 8192, 16_384) for d in (-1, 0, 1)] + [0, 0]
+  special = [b + d for b in (64, 128, 256, 512, 1024, 2048, 3072, 4 * mean, 4096, 8192, 16_384) for d in (-1, 0, 1)] + [0, 0]
   at = np.unique(np.concatenate([[0, n_row - 1], rng.choice(n_row, len(special) - 2, replace=False)]))
   counts[at] = np.minimum(special[:at.size], n_col)
   ptr = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
@@ -1262,3 +1263,37 @@ def test_rows_left_to_a_wave_or_a_workgroup(cuda, oracle_mod, n_row, n_col, mean
       assert np.array_equal(got, oracle_mod.event_csr_matvec(data, idx, ptr, ev, **kw)), ("event", dt, data.shape)
       got = bpl.csr_matvec(data, idx, ptr, v.astype(dt), shape=(n_row, n_col)).cpu().numpy()
       assert np.array_equal(got, oracle_mod.csr_matvec(data, idx, ptr, v.astype(dt), shape=(n_row, n_col))), ("dense", dt, data.shape)
+
+
+@pytest.mark.parametrize("n_row,n_col,long,short,events", [(20_000, 30_000, 4000, 100, False), (50_000, 100_000, 2600, 200, True)])
+def test_many_long_rows_cost_what_their_nonzeros_cost(cuda, n_row, n_col, long, short, events):
+  # a tenth of the rows long: no longer than 1.6 times what as many nonzeros in rows of one length take (a whole workgroup
+  # for every long row: 2.0 times; measured 1.2)
+  rng = np.random.default_rng(7)
+  uneven = np.where(np.arange(n_row) % 10 == 3, long, short)
+  even = np.full(n_row, uneven.sum() // n_row)
+  times = []
+  for counts in (uneven, even):
+    nnz = int(counts.sum())
+    ptr = torch.from_numpy(np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)).cuda()
+    idx = torch.from_numpy(rng.integers(0, n_col, nnz).astype(np.int32)).cuda()
+    if events:
+      data, v = torch.full((1,), 0.5, device="cuda"), torch.from_numpy(rng.random(n_col) < 0.05).cuda()
+      call = lambda: bpl.event_csr_matvec(data, idx, ptr, v, shape=(n_row, n_col))
+    else:
+      data, v = torch.ones(nnz, device="cuda"), torch.ones(n_col, device="cuda")
+      call = lambda: bpl.csr_matvec(data, idx, ptr, v, shape=(n_row, n_col))
+      assert np.array_equal(call().cpu().numpy(), counts.astype(np.float32))
+    runs = []
+    for _ in range(6):
+      a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+      call()
+      a.record()
+      for _ in range(20):
+        call()
+      b.record()
+      b.synchronize()
+      runs.append(a.elapsed_time(b) / 20 * 1e3)
+    times.append(min(runs))
+  print("us", times)
+  assert times[0] < 1.6 * times[1], times
