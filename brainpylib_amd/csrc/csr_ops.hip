@@ -667,6 +667,16 @@ __device__ __forceinline__ void event_hits(const uint32_t *s_bits, const VT *__r
   }
 }
 
+// Element `col` of the dense vector.  BITS == 2: its first `lds_n` elements are staged in LDS (`s_x`), the rest is
+// gathered from global memory.
+template <typename VT, int BITS>
+__device__ __forceinline__ VT dense_element(const VT *__restrict__ x, const uint32_t *s_x, uint32_t lds_n, uint32_t col) {
+  if constexpr (BITS == 2) {
+    if (col < lds_n) return reinterpret_cast<const VT *>(s_x)[col];
+  }
+  return x[col];
+}
+
 typedef uint32_t row_u32x4 __attribute__((ext_vector_type(4), aligned(4)));  // (a row begins at any nonzero)
 typedef float row_f32x4 __attribute__((ext_vector_type(4), aligned(4)));
 template <typename F, typename VT, bool HETER, int MODE, int BITS, int G, int U>
@@ -775,7 +785,7 @@ __device__ __forceinline__ void gather_rows(const F *__restrict__ data, const ui
         if constexpr (kWeightRuns) d = wgt[u];
         else if constexpr (HETER) d = data[ok ? j : (end ? end - 1 : 0u)];
         // product formed in F, then widened (the reference multiplies two F values)
-        val[u] = static_cast<F>(static_cast<F>(x[col[u]]) * d);
+        val[u] = static_cast<F>(static_cast<F>(dense_element<VT, BITS>(x, s_bits, coarse_g, col[u])) * d);
       }
     }
     // indices of the next step, and the row bounds one row further ahead
@@ -863,7 +873,7 @@ __device__ __forceinline__ void gather_rows_wave(const F *__restrict__ data, con
         if (ok[u]) {
           const F d = HETER ? stream_load(dp + off) : w_homo;
           // product formed in F, then widened (the reference multiplies two F values)
-          val[u] = static_cast<F>(static_cast<F>(x[col[u]]) * d);
+          val[u] = static_cast<F>(static_cast<F>(dense_element<VT, BITS>(x, s_bits, coarse_g, col[u])) * d);
         }
       }
     }
@@ -954,7 +964,7 @@ __device__ __forceinline__ void gather_hub_rows(const F *__restrict__ data, cons
           }
         } else {
           const F d = HETER ? data[start + j] : w_homo;
-          acc += static_cast<double>(static_cast<F>(static_cast<F>(x[col[u]]) * d));
+          acc += static_cast<double>(static_cast<F>(static_cast<F>(dense_element<VT, BITS>(x, s_bits, coarse_g, col[u])) * d));
         }
       }
 #pragma unroll
@@ -1293,8 +1303,11 @@ __global__ __launch_bounds__(1024, (MODE == kEvent && BITS == 1) ? 8 : 4) void c
   if constexpr (MODE == kDense) {
     // BITS == 1: the dense vector itself is staged in LDS (the host checked that it fits), so the
     // per-nonzero gather is an LDS read instead of an L2 request and the kernel streams at HBM speed
-    if constexpr (BITS == 1) {
-      copy_to_lds(reinterpret_cast<VT *>(s_bits), x, n_col);
+    // BITS == 2: as much of it as fits; the kernel gathers the rest from L2 as without LDS
+    if constexpr (BITS == 1 || BITS == 2) {
+      constexpr uint32_t kFits = kLdsBitmapCap / sizeof(VT);
+      coarse_g = n_col < kFits ? n_col : kFits;  // (the walks take it as the number of staged elements)
+      copy_to_lds(reinterpret_cast<VT *>(s_bits), x, coarse_g);
       __syncthreads();
     }
   } else if constexpr (BITS == 3) {
@@ -1345,6 +1358,10 @@ __global__ __launch_bounds__(1024, (MODE == kEvent && BITS == 1) ? 8 : 4) void c
     else if (mean >= 24) { gpb = blockDim.x / 8; hub_len = hub_length(mean, 8 * 8); gather_rows<F, VT, HETER, MODE, BITS, 8, 8>(data, indices, indptr, xs, y, n_row, s_bits, coarse_g, hub_len); }
     else if (mean >= 12) { gpb = blockDim.x / 4; hub_len = hub_length(mean, 8 * 4); gather_rows<F, VT, HETER, MODE, BITS, 4, 8>(data, indices, indptr, xs, y, n_row, s_bits, coarse_g, hub_len); }
     else { gpb = blockDim.x / 4; hub_len = hub_length(mean, 4 * 4); gather_rows<F, VT, HETER, MODE, BITS, 4, 4>(data, indices, indptr, xs, y, n_row, s_bits, coarse_g, hub_len); }
+  } else if constexpr (MODE == kDense && BITS == 2) {  // (long rows only)
+    gpb = 1;
+    hub_len = hub_length(mean, kWaveStep, wave_least);
+    gather_rows_wave<F, VT, HETER, MODE, BITS, 8>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len);
   } else if constexpr (MODE == kEvent && (BITS == 2 || BITS == 3)) {
     // An event bitmap above 80 KB leaves room for one workgroup (16 waves) per CU only: every lane
     // then keeps 16 (rows under 48 nonzeros: 8) loads in flight instead of 2 to 8, in groups of
@@ -1868,6 +1885,20 @@ void launch_gather(const char *target, const ScratchSource &src, const F *data, 
       // columns: 9 us against 14; 50,000 uneven rows of 20: 16.6 against 17.1).
       constexpr uint32_t kFlatMinMean = 4, kFlatMinNnz = 1u << 20;
       const bool known = nnz != kUnknownNnz;
+      // Long rows and a vector a little longer than what fits: a wave per row with 159 KB of it staged, where the flat walk's
+      // windows leave 147 KB and its row bookkeeping is most of what a nonzero of one weight costs.  One weight, up to 4 / 3 of
+      // what fits: 17,000 x 46,000 with 500 / 1,500 per row 31 / 62 -> 20 / 34 us, x 54,000 33 / 63 -> 22 / 45, log-normal rows 0.8
+      // to 1.0 of the time; shorter rows (lanes share a wave) lose as much when they are uneven.  Weights per nonzero,
+      // float, up to 8 / 7: 17,000 x 46,000 with 600 / 1,500 36 / 65 -> 26 / 53 us, log-normal 0.97 to 1.13; under 576 per row most
+      // of a wave's second step is empty (50,000 x 41,000 with 500: 59 -> 70).  Double with weights: 0.87 even, 1.15 uneven: not.
+      constexpr uint32_t kStagedWaveMinMean = HETER ? 576 : 384;
+      const bool staged_wave = known && n_row >= 16384 && nnz / n_row >= kStagedWaveMinMean && !(HETER && sizeof(F) == 8) &&
+                               lds_bytes > kLdsBitmapCap && lds_bytes <= kLdsBitmapCap + kLdsBitmapCap / (HETER ? 7 : 3);
+      if (staged_wave) {
+        if (launch_gather_impl<F, VT, HETER, MODE, 2>(target, stream, data, indices, indptr, x, y, n_row, n_col, kLdsBitmapCap))
+          return;
+        bpl_clear_error();
+      }
       const bool flat = known ? nnz >= kFlatMinNnz && nnz <= kFlatMaxNnz && nnz / n_row >= kFlatMinMean &&
                                   (n_row >= 16384 || flat_stages<F>(n_col))
                               : n_row >= 16384;

@@ -1129,9 +1129,11 @@ def test_csr_matvec_flat_walk_over_the_nonzeros(cuda, oracle_mod, kind):
 
 
 # vectors one element longer than what a workgroup stages whole, up to the last partly staged size and one beyond (gathered
-# from L2 only); below and above 16,384 rows; just below and above a million nonzeros (a row-wise walk below)
+# from L2 only); below and above 16,384 rows; just below and above a million nonzeros (a row-wise walk below); long rows
+# and the last sizes that a wave per row takes with one weight and with weights per nonzero, and one more
 @pytest.mark.parametrize("n_row,n_col,mean", [(20_000, 35_329, 56), (3000, 35_329, 500), (300, 141_312, 4000),
                                               (300, 37_632, 4000), (300, 37_633, 4000), (300, 37_634, 4000),
+                                              (16_384, 46_518, 700), (16_384, 54_273, 700),
                                               (20_000, 141_312, 50), (20_000, 141_313, 60), (400_000, 40_705, 4)])
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 @pytest.mark.parametrize("homo", [False, True])
@@ -1297,3 +1299,29 @@ def test_many_long_rows_cost_what_their_nonzeros_cost(cuda, n_row, n_col, long, 
     times.append(min(runs))
   print("us", times)
   assert times[0] < 1.6 * times[1], times
+
+
+def test_a_vector_a_little_longer_than_lds_costs_little_more(cuda):
+  # 17,000 rows of 1,000 and one weight: over 46,000 columns (a part of the vector gathered from L2) no more than 1.6 times
+  # the time over 40,000, whose vector lies in LDS whole (measured 1.2; with the walk over the nonzeros 2.1)
+  n_row, per = 17_000, 1000
+  ptr = torch.arange(n_row + 1, dtype=torch.int32, device="cuda") * per
+  w = torch.full((1,), 0.5, device="cuda")
+  best = []
+  for n_col in (46_000, 40_000):
+    idx = torch.randint(n_col, (n_row * per,), dtype=torch.int32, device="cuda")
+    v = torch.ones(n_col, device="cuda")
+    call = lambda: bpl.csr_matvec(w, idx, ptr, v, shape=(n_row, n_col))
+    assert bool((call() == 500.0).all())
+    runs = []
+    for _ in range(6):
+      a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+      a.record()
+      for _ in range(20):
+        call()
+      b.record()
+      b.synchronize()
+      runs.append(a.elapsed_time(b) / 20 * 1e3)
+    best.append(min(runs))
+  print("us", best)
+  assert best[0] < 1.6 * best[1], best
