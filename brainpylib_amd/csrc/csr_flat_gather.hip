@@ -482,11 +482,15 @@ static bool launch_flat(const char *target, hipStream_t stream, const F *data, c
   if (STAGED) {
     constexpr uint32_t kMost = flat_staged_bytes<F, OUT>();
     lds = static_cast<size_t>(n_col) * sizeof(F) < kMost ? static_cast<size_t>(n_col) * sizeof(F) : kMost;
-    if (hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                            static_cast<int>(kMost)) != hipSuccess) {
-      (void)hipGetLastError();
-      set_error("%s: the device does not give a workgroup %u bytes of LDS", target, kMost);
-      return false;
+    static thread_local bool attr_set = false;  // (per instantiation)
+    if (!attr_set) {
+      if (hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                              static_cast<int>(kMost)) != hipSuccess) {
+        (void)hipGetLastError();
+        set_error("%s: the device does not give a workgroup %u bytes of LDS", target, kMost);
+        return false;
+      }
+      attr_set = true;
     }
   }
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(flat_threads(STAGED)), lds, stream, data, indices, indptr, x, y, n_row,
