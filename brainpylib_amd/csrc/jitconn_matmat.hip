@@ -84,10 +84,6 @@ __global__ __launch_bounds__(256) void jitconn_matmat_kernel(const T1 *__restric
   constexpr uint32_t row_bytes = MT * kWave * static_cast<uint32_t>(sizeof(T1));
   // (a wave-uniform base and a 32-bit offset per lane: one address add per synapse and the base in scalar registers)
   const char *xt_base = reinterpret_cast<const char *>(XT + static_cast<size_t>(pass) * k * (MT * kWave));
-  // lane l accumulates rows MT l .. MT l + MT - 1 of the pass: one load per synapse, MT entries wide
-  struct __attribute__((aligned(MT * sizeof(T1)))) Rows {
-    T1 x[MT];
-  };
   const uint32_t lane_bytes = static_cast<uint32_t>(lane) * static_cast<uint32_t>(sizeof(T1));
 
   // columns first .. first + count - 1 of M, their generators seeded ahead: states[c] for column first + c
@@ -100,7 +96,7 @@ __global__ __launch_bounds__(256) void jitconn_matmat_kernel(const T1 *__restric
     // Every valid lane leaves its synapses (the byte offset of their rows of XT, their weights) in the
     // wave's LDS slots, in lane order (which is stream order); every lane then reads the slots
     // one after the other (one address per read: a broadcast), so a synapse costs one LDS read,
-    // one address add, one load and MT multiply-adds, with U synapses' loads in flight.
+    // one address add, MT loads and MT multiply-adds, with U synapses' loads in flight.
     auto take = [&](uint32_t count) {
       constexpr int U = 8;
       uint32_t i = 0;

@@ -65,9 +65,6 @@ __device__ __forceinline__ uint32_t wave_shift_up1(uint32_t v) {
   return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(static_cast<int>(v), static_cast<int>(v), 0x138 /* wave_shr:1 */,
                                                            0xf, 0xf, false));
 }
-__device__ __forceinline__ float wave_shift_up1(float v) {
-  return __builtin_bit_cast(float, wave_shift_up1(__builtin_bit_cast(uint32_t, v)));
-}
 __device__ __forceinline__ double wave_shift_up1(double v) {
   const unsigned long long b = static_cast<unsigned long long>(__double_as_longlong(v));
   const uint32_t lo = wave_shift_up1(static_cast<uint32_t>(b)), hi = wave_shift_up1(static_cast<uint32_t>(b >> 32));
