@@ -33,11 +33,12 @@ namespace {
 // LDS the row walk gives to an event bitmap when it wants two 16-wave workgroups per CU (each wave
 // can issue one instruction every four cycles, so the number of resident waves bounds the VALU
 // utilisation: 32 waves per CU walk 290 G synapses/s, the 15 that fit beside a 125 KB bitmap 228).
-// What two workgroups leave of a CU's 160 KB beside their 16 waves' states and queues.
+// What two workgroups leave of a CU's 160 KB beside their 16 waves' states and queues (normal weights: 18,944 bytes).
+constexpr uint32_t kRowwalkCoarseMost = 38912;
 template <typename T1, int W>
 constexpr uint32_t rowwalk_coarse_bytes() {
   const uint32_t left = (80u * 1024u - 16u * 4u * StreamLds<T1, W>::words - 64u) / 256u * 256u;
-  return left < 38912u ? left : 38912u;
+  return left < kRowwalkCoarseMost ? left : kRowwalkCoarseMost;
 }
 
 // BITS: where the event probes go.  0: the event vector in global memory; 1: its bitmap in LDS;
@@ -658,7 +659,12 @@ void launch_rowwalk(hipStream_t stream, const VT *in, T1 *out, uint32_t n_out, u
     bitmap_ws = (words + 1) * sizeof(uint32_t);
   }
   const RowwalkScratch sc = rowwalk_scratch(stream, n_out, bitmap_ws);
-  if (sc.refused) return;  // (the error stands: a graph must not record a slower path)
+  if (sc.refused) {
+    // (the error stands: a graph must not record a slower path.  But for byte events whose bitmap is no longer than what
+    // homo and uniform weights keep in LDS: without rings such a walk is captured without scratch memory.)
+    if (!(kEvents && sizeof(VT) == 1 && n_out < kSeedAheadMin && words * 4 <= kRowwalkCoarseMost)) return;
+    bpl_clear_error();
+  }
   if constexpr (kEvents) {
     if (uint32_t *bits = sc.bitmap()) {
       pack_event_bitmap<VT>(stream, in, n_in, bits);

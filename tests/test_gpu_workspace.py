@@ -167,3 +167,22 @@ def test_scratch_memory_of_a_batch_of_a_small_network(cuda):
   s.synchronize()
   assert has and size < 60e6, size
   assert torch.equal(out.cpu(), torch.bincount(indices[0].cpu(), minlength=1000).to(torch.float32).expand(20, -1))
+
+
+@pytest.mark.parametrize("n_in", [151_552, 151_553, 311_296])
+def test_normal_row_walk_is_captured_on_a_cold_stream(cuda, n_in):
+  # few outputs, byte events: their bitmap lies in LDS and no scratch memory is needed, whatever the weights
+  ev = torch.from_numpy(np.random.default_rng(n_in).random(n_in) < 0.1).to(cuda)
+  kw = dict(w_mu=0.1, w_sigma=0.5, conn_prob=0.01, shape=(300, n_in), seed=5, outdim_parallel=True)
+  want = bpl.event_matvec_prob_conn_normal_weight(ev, **kw)
+  torch.cuda.synchronize()
+  s, g = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+  with torch.cuda.graph(g, stream=s):
+    out = bpl.event_matvec_prob_conn_normal_weight(ev, **kw)
+  assert not _query(s.cuda_stream)[0], "nothing was allocated"
+  for _ in range(3):
+    out.zero_()
+    g.replay()
+    torch.cuda.synchronize()
+    # (the same addends in float64, in another order, rounded once)
+    torch.testing.assert_close(out, want, rtol=3e-7, atol=1e-6)
