@@ -148,6 +148,36 @@ def test_gradients_of_weights_and_vector_from_one_walk(cuda, n_row, n_col, mean,
     assert torch.equal(torch.autograd.grad(y, d, ct.cuda())[0].cpu(), want)
 
 
+# infinities and NaN in the weights and in both vectors: they stay in the rows and products that they belong to, also where a
+# neighbour shares a load of four nonzeros, a wave's range or the masked lanes of a step with them
+@pytest.mark.parametrize("n_row,n_col,mean", [(40, 30, 3), (3000, 700, 2), (500, 40_000, 60), (6, 150_000, 9000)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_gradients_with_infinities_and_nan(cuda, n_row, n_col, mean, dtype):
+  rng = np.random.default_rng(n_col)
+  counts = np.minimum(rng.poisson(mean, n_row), n_col)
+  idx, ptr = synth.counted_csr(counts, n_col, seed=n_row)
+  row, col = np.repeat(np.arange(n_row), counts), idx.astype(np.int64)
+  w, v, ct = (rng.standard_normal(n) for n in (idx.shape[0], n_row, n_col))
+  for a in (w, v, ct):  # (column 0 and row 0 among them: masked lanes point there)
+    a[rng.choice(a.shape[0], max(1, a.shape[0] // 50), replace=False)] = np.inf
+    a[rng.choice(a.shape[0], max(1, a.shape[0] // 50), replace=False)] = np.nan
+  ct[0], v[0] = np.nan, -np.inf
+  w, v, ct = (torch.from_numpy(a).to(dtype) for a in (w, v, ct))
+  d, t = w.cuda().requires_grad_(), v.cuda().requires_grad_()
+  y = bpl.cusparse_csr_matvec(d, idx, ptr, t, shape=(n_row, n_col), transpose=True)
+  got, sums = (g.cpu() for g in torch.autograd.grad(y, (d, t), ct.cuda()))
+  assert torch.equal(torch.nan_to_num(got, 7.0), torch.nan_to_num(v[row] * ct[col], 7.0))
+  assert torch.equal(got.isnan(), (v[row] * ct[col]).isnan())
+  addend = (w * ct[col]).to(torch.float64)
+  want = torch.zeros(n_row, dtype=torch.float64).index_add_(0, torch.from_numpy(row), addend)
+  mag = torch.zeros(n_row, dtype=torch.float64).index_add_(0, torch.from_numpy(row), addend.abs())
+  finite = want.isfinite()
+  assert torch.equal(sums.isnan(), want.isnan()) and torch.equal(sums[want.isinf()].to(torch.float64), want[want.isinf()])
+  # (float64 sums in another order, rounded once)
+  bound = torch.finfo(dtype).eps * want.abs() + 4 * torch.finfo(torch.float64).eps * mag
+  assert bool(((sums.to(torch.float64) - want).abs() <= bound)[finite].all()) and (bool(finite.any()) or mean > 1000)
+
+
 # arrays longer than indptr says, by less than a quad and by more than the walk has threads; a matrix without nonzeros and
 # one without rows.  Nothing depends on what lies beyond: its gradient is zero, whatever its columns are.
 @pytest.mark.parametrize("n_row,mean,extra", [(50, 7, 3), (2000, 40, 300_000), (2000, 0, 1000), (0, 0, 5)])
