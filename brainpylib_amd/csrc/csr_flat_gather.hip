@@ -3,7 +3,7 @@
 // nonzero.  (A row-wise walk, groups of lanes taking whole rows in steps of 16-byte loads, pads each row to
 // whole steps of its group: with 100 nonzeros per row a fifth of the lanes of its gather instructions lie
 // beyond the row, and a gather instruction costs the address unit the same whether its lanes are masked or
-// not.  That walk took 633 us at 1e8 nonzeros in rows of 100, this one 570; rows of 30: 449 against 315.)
+// not.  That walk took 633 us at 1e8 nonzeros in rows of 100, this one 546; rows of 30: 449 against 315.)
 //
 // Measured on this device: a product that reads one 4-byte element of a 4 MB vector per nonzero is bound by
 // the rate at which a CU's vector cache takes misses (about one 128-byte line per 3.2 clocks and CU, whatever
@@ -30,8 +30,8 @@
 // OUT: what the walk leaves behind.  kFlatSums: y = A x.  kFlatProducts: products[j] = v[row of j] * x[column of j]
 // for every nonzero j (the gradient of the weights), stored with the quads' own 16-byte width; the rows of the
 // nonzeros are at hand in the window anyway, v's 64 elements of the window lie beside it.  Both at once read the
-// indices and gather x once.  Measured: 1e7 nonzeros, both, x of 30,011 floats in LDS: 32 us, 3.7 TB/s of the 120 MB it
-// must move; 3e7 nonzeros, products alone, x of 120,011 floats: 126 us, bound by the lines that the gathers move out
+// indices and gather x once.  Measured: 1e7 nonzeros, both, x of 30,011 floats in LDS: 33 us, 3.6 TB/s of the 120 MB it
+// must move; 3e7 nonzeros, products alone, x of 120,011 floats: 122 us, bound by the lines that the gathers move out
 // of the L2s (2.7 GB, 54 us without those gathers).  An expanded list of the rows, two gathers and a product as
 // passes of their own took 215 and 850 us.
 // STAGED: one workgroup of 1,024 threads per CU keeps the first elements of x (139 to 151 KB) in LDS and gathers only the
