@@ -106,15 +106,22 @@ __device__ __forceinline__ void flat_store_quad(double *__restrict__ p, const do
 // one wave, a window of 64 rows after the other (1,000,000 rows and 5e6 nonzeros, all in the first tenth of the rows: 21 ms,
 // now 70 us; 2,000 rows of 20,000 among as many of 0.1: 5.8 ms, now 0.61; the weights' gradient with 100 nonzeros: 26 ms,
 // now 80 us).  Even matrices: 0.91 to 1.02 of the time before, 1.05 with doubles of 30,000 columns and ten per row.
+// A row's end counts as four nonzeros: 64 empty rows are a window with its dependent load, 2.5 us, where a step of 1,024
+// nonzeros takes some 10 (346,000 rows of 870 in the first tenth, x 42,500: 300 us with one, 87 with four or eight; from eight
+// on a long row among many of one nonzero per step is the last to end: 988,000 x 116,000 57 -> 66 us, with sixteen 91).
 // row, pos: of the first `diag` entries of the list, how many are rows (= the row the next nonzero belongs to or the next
 // end is of) and how many nonzeros; two places side by side, 64 probes a round (four rounds for a million rows).
 // A place moves back to a multiple of 32 nonzeros (a line of indices) where the row that holds that one is among the
 // last round's probes: the loads of a wave then cover whole lines.  (A function of `diag` alone and monotone in it: the
 // last round's probes are a fixed division of the rows.)
+constexpr uint32_t kFlatRowWeight = 4;
+__device__ __forceinline__ uint64_t flat_list(uint32_t n_row, uint32_t nnz) {  // entries of the list
+  return static_cast<uint64_t>(kFlatRowWeight) * n_row + nnz;
+}
 __device__ __forceinline__ void flat_split(const uint32_t *__restrict__ indptr, uint32_t n_row, uint32_t nnz,
                                            const uint64_t (&diag)[2], uint32_t lane, uint32_t (&row)[2],
                                            uint32_t (&pos)[2]) {
-  const uint64_t total = static_cast<uint64_t>(n_row) + nnz;
+  const uint64_t total = flat_list(n_row, nnz);
   uint32_t lo[2] = {0, 0}, first[2], ptr[2];
   uint64_t hi[2] = {n_row, n_row};
   for (uint32_t stride = n_row / kWave + (n_row % kWave ? 1u : 0u);; stride = stride / kWave + (stride % kWave ? 1u : 0u)) {
@@ -126,7 +133,7 @@ __device__ __forceinline__ void flat_split(const uint32_t *__restrict__ indptr, 
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
       const uint64_t probe = static_cast<uint64_t>(lo[k]) + static_cast<uint64_t>(lane) * stride;
-      const bool below = lane == 0 || (probe < hi[k] && probe + ptr[k] <= diag[k]);  // (a prefix of the lanes)
+      const bool below = lane == 0 || (probe < hi[k] && kFlatRowWeight * probe + ptr[k] <= diag[k]);  // (a prefix of the lanes)
       first[k] = lo[k];
       lo[k] += (static_cast<uint32_t>(__popcll(__ballot(below))) - 1u) * stride;
       const uint64_t top = static_cast<uint64_t>(lo[k]) + stride;
@@ -140,10 +147,13 @@ __device__ __forceinline__ void flat_split(const uint32_t *__restrict__ indptr, 
       row[k] = n_row, pos[k] = nnz;
       continue;
     }
-    const uint64_t p = diag[k] - lo[k];
-    row[k] = lo[k], pos[k] = p < nnz ? static_cast<uint32_t>(p) : nnz;
+    const uint32_t at = lo[k] - first[k];
+    uint32_t row_end = at + 1u < kWave ? static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(ptr[k]), at + 1u)) : 0xffffffffu;
+    if (row_end == 0xffffffffu) row_end = indptr[lo[k] + 1u];  // (not among the probes)
+    const uint64_t p = diag[k] - static_cast<uint64_t>(kFlatRowWeight) * lo[k];
+    row[k] = lo[k], pos[k] = p < row_end ? static_cast<uint32_t>(p) : row_end;
     const uint32_t back = pos[k] & ~31u;
-    const uint32_t rows = static_cast<uint32_t>(__popcll(__ballot(lane <= lo[k] - first[k] && ptr[k] <= back)));
+    const uint32_t rows = static_cast<uint32_t>(__popcll(__ballot(lane <= at && ptr[k] <= back)));
     if (rows != 0u) row[k] = first[k] + rows - 1u, pos[k] = back;
   }
 }
@@ -185,11 +195,11 @@ __global__ __launch_bounds__(flat_threads(STAGED), 4) void csr_flat_gather_kerne
   }
   const uint32_t waves = gridDim.x * kFlatWaves, w = blockIdx.x * kFlatWaves + wv;
   // the wave owns the nonzeros [begin, end) and stores the rows [r, row_end), but for one that began before `begin`
-  uint32_t share = nnz / waves + n_row / waves + 2u;
+  uint32_t share = nnz / waves + kFlatRowWeight * (n_row / waves + 1u) + 1u;
   if (share < flat_min_share<F, OUT, STAGED>()) share = flat_min_share<F, OUT, STAGED>();
   const uint64_t diag[2] = {static_cast<uint64_t>(w) * share, (static_cast<uint64_t>(w) + 1u) * share};
   uint32_t split_row[2], split_pos[2];
-  if (diag[0] >= static_cast<uint64_t>(n_row) + nnz) {
+  if (diag[0] >= flat_list(n_row, nnz)) {
     if (kSums && lane == 0) head[w] = 0.0, tail[w] = 0.0, tail_row[w] = kNoRow, range[w] = nnz;
     return;
   }

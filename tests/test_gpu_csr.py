@@ -1325,3 +1325,38 @@ def test_a_vector_a_little_longer_than_lds_costs_little_more(cuda):
     best.append(min(runs))
   print("us", best)
   assert best[0] < 1.6 * best[1], best
+
+
+@pytest.mark.parametrize("n_row,n_col,long,events", [(346_000, 42_500, 867, False)])
+def test_a_block_of_rows_costs_what_its_nonzeros_cost(cuda, n_row, n_col, long, events):
+  # all nonzeros in the first tenth of the rows: no longer than twice the same rows in a random order (all of them taken by
+  # the few workgroups that the block is dealt to, or empty rows that count no more than a nonzero: 2.3 to 4 times)
+  rng = np.random.default_rng(3)
+  counts = np.zeros(n_row, np.int64)
+  counts[:n_row // 10] = long
+  times = []
+  for c in (counts, rng.permutation(counts)):
+    nnz = int(c.sum())
+    ptr = torch.from_numpy(np.concatenate([[0], np.cumsum(c)]).astype(np.int32)).cuda()
+    idx = torch.from_numpy(rng.integers(0, n_col, nnz).astype(np.int32)).cuda()
+    data = torch.ones(nnz, device="cuda", dtype=torch.float64 if events else torch.float32)
+    if events:
+      x = torch.from_numpy(rng.random(n_col) < 0.2).cuda()
+      call = lambda: bpl.event_csr_matvec(data, idx, ptr, x, shape=(n_row, n_col))
+    else:
+      x = torch.ones(n_col, device="cuda")
+      call = lambda: bpl.csr_matvec(data, idx, ptr, x, shape=(n_row, n_col))
+      assert np.array_equal(call().cpu().numpy(), c.astype(np.float32))
+    runs = []
+    for _ in range(6):
+      a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+      call()
+      a.record()
+      for _ in range(20):
+        call()
+      b.record()
+      b.synchronize()
+      runs.append(a.elapsed_time(b) / 20 * 1e3)
+    times.append(min(runs))
+  print("us", times)
+  assert times[0] < 2.0 * times[1], times
