@@ -696,10 +696,11 @@ __device__ __forceinline__ void gather_rows(const F *__restrict__ data, const ui
   constexpr int Q = ((U == 4 || U == 8) && !(MODE == kDense && BITS == 1)) ? 4 : 1;
   auto slot = [&](int u) { return static_cast<uint32_t>(Q * ((u / Q) * G) + u % Q) + static_cast<uint32_t>(Q) * gl; };
   const uint32_t nnz = Q > 1 ? indptr[n_row] : 0u;  // (a run of Q is loaded whole only where the arrays hold all of it)
-  // A row of more than hub_len nonzeros looks empty here: gather_hub_rows() gives it to a wave or the whole workgroup.
+  // A row of more than hub_len nonzeros ends before it begins here and is not stored: gather_hub_rows() takes it, mostly in
+  // another workgroup.
   auto bounds = [&](uint32_t r, uint32_t &s, uint32_t &e) {
     s = indptr[r], e = indptr[r + 1];
-    if (e - s > hub_len) e = s;
+    if (e - s > hub_len) s = 1, e = 0;
   };
 
   uint32_t row = blockIdx.x * groups_per_block + threadIdx.x / G;
@@ -757,6 +758,8 @@ __device__ __forceinline__ void gather_rows(const F *__restrict__ data, const ui
     const uint32_t next_base = last_of_row ? nrow_start : base + U * G;
     const uint32_t next_end = last_of_row ? nrow_end : end;
     const bool more = next_row < n_row;
+    // (kept as a lane mask: the comparison at the end would keep both bounds in registers, and some kernels have none left)
+    const uint64_t stored = __builtin_amdgcn_ballot_w64(gl == 0 && base <= end);
 
     // loads that depend on this step's indices
     F val[U];
@@ -803,11 +806,11 @@ __device__ __forceinline__ void gather_rows(const F *__restrict__ data, const ui
       if (MODE == kEvent && !HETER) {
         hits = group_sum<G>(hits);
         // n additions of the same fp32 value into a float64 accumulator are exact: n * w
-        if (gl == 0) y[row] = gathered_sum(w_homo, hits);
+        if (__builtin_amdgcn_inverse_ballot_w64(stored)) y[row] = gathered_sum(w_homo, hits);
         hits = 0;
       } else {
         acc = group_sum<G>(acc);
-        if (gl == 0) y[row] = static_cast<F>(acc);
+        if (__builtin_amdgcn_inverse_ballot_w64(stored)) y[row] = static_cast<F>(acc);
         acc = 0.0;
       }
     }
@@ -914,23 +917,32 @@ __device__ __forceinline__ void gather_rows_wave(const F *__restrict__ data, con
 // Hub rows.  The walks above give a row to G lanes (or one wave), so one row that holds a large share
 // of the nonzeros would be walked by a handful of lanes while the rest of the device is done (a row of
 // 1e6 nonzeros among 20,000 of 50: 19 ms).  They treat a row of more than hub_len nonzeros as
-// empty, and after its walk every workgroup looks through the bounds of the rows it was dealt again
-// (workgroup b: rows b * gpb + g + k * total_groups, g < gpb).  Its waves take the ones of up to kHubWave nonzeros
-// in turn, each by itself, and then all its threads the longer ones together: partial sums per lane, a wave sum,
-// one float64 (or integer) LDS atomic per wave.
-// The walk with a wave per row skips such rows without storing anything (they all go to the whole workgroup), and
-// they are dealt one by one (gpb = 1: workgroup b looks at rows b, b + gridDim.x, ...): in a matrix of a few thousand
-// rows that are all this long, sixteen consecutive rows per workgroup would leave most of the device idle (2,000 rows of
-// 50,000: an eighth of the workgroups had rows).
-constexpr uint32_t kHubWave = 4096;  // eight steps of a wave
+// ended before it begins and store nothing, and after its walk every workgroup looks through the bounds of the rows it is
+// dealt here (workgroup b: rows b * gpb + g + k * total_groups, g < gpb).  Eight consecutive rows at a time where the walk
+// dealt more: a block of long rows (72,000 rows, the first tenth of 1,800, double: 117 -> 29 us) else falls to the few
+// workgroups that walked it; in matrices of two and more rounds of the walk it does not, and the wider reads stay
+// (815,000 thin rows 16.4 us, eight at a time 19.1).  Rows of up to kHubWave nonzeros (1,024 where there are at most four
+// longer ones: a step of 256 of a wave takes 0.8 us) go to 64 lanes each, or to as few as 8 where the workgroup has that
+// many of them, the longer ones one after the other to all threads, sixteen between two barriers (4,745 rows, a tenth of
+// 20,000, one weight, double: 99 -> 65 us): partial sums per lane, a wave sum, one float64 (or integer) LDS atomic per wave.
+// The rows of the walk with a wave per row are dealt one by one (gpb = 1: workgroup b looks at rows b, b + gridDim.x, ...):
+// in a matrix of a few thousand rows that are all this long, sixteen consecutive rows per workgroup would leave most of the
+// device idle (2,000 rows of 50,000: an eighth of the workgroups had rows); where a workgroup has as many of them as
+// waves, a wave takes a row of up to 64 steps.
+constexpr uint32_t kHubWave = 4096;
+constexpr uint32_t kHubLanes = 8;  // the fewest lanes that take such a row
+constexpr uint32_t kHubDeal = 8;   // consecutive rows that go to one workgroup
 template <typename F, typename VT, bool HETER, int MODE, int BITS>
 __device__ __forceinline__ void gather_hub_rows(const F *__restrict__ data, const uint32_t *__restrict__ indices,
                                                 const uint32_t *__restrict__ indptr, const VT *__restrict__ x,
                                                 F *__restrict__ y, uint32_t n_row, const uint32_t *s_bits,
-                                                uint32_t coarse_g, uint32_t gpb, uint32_t hub_len) {
+                                                uint32_t coarse_g, uint32_t nnz, uint32_t gpb, uint32_t hub_len) {
+  // Rows of a whole workgroup between two barriers.  (One with a dense vector: with more than 80 scalar registers no two
+  // workgroups share a CU, and even rows of 900 with the vector in LDS take 13 -> 18 us.)
+  constexpr uint32_t kHubBatch = MODE == kDense ? 1 : 16;
   __shared__ unsigned long long s_mask[1024 / kWave];
-  __shared__ double s_acc;
-  __shared__ uint32_t s_hits;
+  __shared__ double s_acc[kHubBatch];
+  __shared__ uint32_t s_hits[kHubBatch], s_row[kHubBatch];
   const uint32_t tid = threadIdx.x, lane = tid % kWave, nwaves = blockDim.x / kWave;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const uint32_t total_groups = gridDim.x * gpb;
@@ -938,40 +950,69 @@ __device__ __forceinline__ void gather_hub_rows(const F *__restrict__ data, cons
   if (first >= n_row) return;
   const uint32_t count = ((n_row - first + total_groups - 1u) / total_groups) * gpb;  // rows dealt to this workgroup
   const F w_homo = HETER ? F(0) : data[0];
-  auto row_of = [&](uint32_t i) { return (i / gpb) * total_groups + first + (i % gpb); };
-  // thread t of `team` of them: its part of a row (the sum over the wave)
-  auto walk = [&](uint32_t start, uint32_t len, uint32_t t, uint32_t team, double &acc, uint32_t &hits) {
-    constexpr uint32_t U = 4;  // loads in flight per lane and step; the next step's are requested before this one's are used
-    uint32_t col[U], ncol[U];
-    auto load_cols = [&](uint32_t j0, uint32_t (&c)[U]) {  // (beyond the row: its last index again)
+  const uint32_t deal_bits = static_cast<uint32_t>(__builtin_ctz(gpb));  // (a power of two)
+  auto row_of = [&](uint32_t i) { return (i >> deal_bits) * total_groups + first + (i & (gpb - 1u)); };
+  // lane t of `team`: its part of the nonzeros [begin, end), one or more
+  auto walk = [&](uint32_t begin, uint32_t end, uint32_t t, uint32_t team, double &acc, uint32_t &hits) {
+    // Nonzeros of a lane and step, in runs of four with one load each; the next step's indices are requested before this
+    // one's are used.  (Eight where a CU has one workgroup in any case: with more than 64 registers no two share one.)
+    constexpr uint32_t U = (MODE == kEvent && BITS >= 2) ? 8 : 4;
+    const uint32_t step = U * team;
+    auto slot = [&](uint32_t u) { return 4u * ((u / 4u) * team + t) + u % 4u; };
+    auto whole = [&](uint32_t b) { return nnz - b >= step; };
+    auto load_cols = [&](uint32_t b, uint32_t (&c)[U]) {
+      if (whole(b)) {  // (beyond the row: the next rows' indices, left out by their number)
 #pragma unroll
-      for (uint32_t u = 0; u < U; ++u) {
-        const uint32_t j = j0 + u * team;
-        c[u] = indices[start + (j < len ? j : len - 1u)];
+        for (uint32_t u = 0; u < U; u += 4) {
+          const row_u32x4 v = *reinterpret_cast<const row_u32x4 *>(indices + b + slot(u));
+          c[u] = v.x, c[u + 1] = v.y, c[u + 2] = v.z, c[u + 3] = v.w;
+        }
+      } else {
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) c[u] = indices[slot(u) < end - b ? b + slot(u) : end - 1u];
       }
     };
-    load_cols(t, col);
-    for (uint32_t j0 = t; j0 < len; j0 += U * team) {
-      load_cols(j0 + U * team, ncol);
-#pragma unroll
-      for (uint32_t u = 0; u < U; ++u) {
-        const uint32_t j = j0 + u * team;
-        if (j >= len) continue;
-        if (MODE == kEvent) {
-          if (event_hit<BITS>(s_bits, x, col[u], coarse_g)) {
-            if (HETER) acc += static_cast<double>(data[start + j]);
-            else ++hits;
-          }
+    uint32_t col[U], ncol[U];
+    load_cols(begin, col);
+    for (uint32_t b = begin;; b += step) {
+      const uint32_t left = end - b;
+      bool use[U];
+      F val[U];
+      if constexpr (MODE == kDense && HETER) {
+        constexpr bool kQuads = BITS != 0 || sizeof(F) == 8;  // (float gathered from L2: 81 scalar registers, see above)
+        if (kQuads && whole(b)) {
+          typedef F quad __attribute__((ext_vector_type(4), aligned(sizeof(F))));
+          const quad v = *reinterpret_cast<const quad *>(data + b + slot(0));
+          val[0] = v.x, val[1] = v.y, val[2] = v.z, val[3] = v.w;
         } else {
-          const F d = HETER ? data[start + j] : w_homo;
-          acc += static_cast<double>(static_cast<F>(static_cast<F>(dense_element<VT, BITS>(x, s_bits, coarse_g, col[u])) * d));
+#pragma unroll
+          for (uint32_t u = 0; u < U; ++u) val[u] = data[slot(u) < left ? b + slot(u) : end - 1u];
+        }
+      }
+      if (left > step) load_cols(b + step, ncol);
+      if constexpr (MODE == kEvent) event_hits<BITS, static_cast<int>(U)>(s_bits, x, col, coarse_g, use);
+#pragma unroll
+      for (uint32_t u = 0; u < U; ++u) {  // (all loads first)
+        const bool ok = slot(u) < left;
+        if (MODE == kEvent) {
+          use[u] = use[u] && ok;
+          val[u] = F(0);
+          if (HETER && use[u]) val[u] = data[b + slot(u)];
+        } else {
+          use[u] = ok;
+          const F d = HETER ? val[u] : w_homo;
+          val[u] = static_cast<F>(static_cast<F>(dense_element<VT, BITS>(x, s_bits, coarse_g, col[u])) * d);
         }
       }
 #pragma unroll
+      for (uint32_t u = 0; u < U; ++u) {
+        if (MODE == kEvent && !HETER) hits += use[u] ? 1u : 0u;
+        else acc += use[u] ? static_cast<double>(val[u]) : 0.0;
+      }
+      if (left <= step) break;
+#pragma unroll
       for (uint32_t u = 0; u < U; ++u) col[u] = ncol[u];
     }
-    if (MODE == kEvent && !HETER) hits = wave_sum(hits);
-    else acc = wave_sum(acc);
   };
   for (uint32_t i0 = 0; i0 < count; i0 += blockDim.x) {
     uint32_t len = 0;
@@ -979,47 +1020,78 @@ __device__ __forceinline__ void gather_hub_rows(const F *__restrict__ data, cons
       const uint32_t r = row_of(i0 + tid);
       if (r < n_row) len = indptr[r + 1] - indptr[r];
     }
-    const bool hub = len > hub_len, alone = hub && (gpb == 1u || len > kHubWave);
-    const unsigned long long by_wave = __ballot(hub && !alone), by_all = __ballot(alone);
-    if (!__syncthreads_or(hub)) continue;  // (the usual case: none)
-    if (lane == 0) s_mask[wave] = by_wave;
+    const bool hub = len > hub_len;
+    const uint32_t n_hub = static_cast<uint32_t>(__syncthreads_count(hub));
+    if (n_hub == 0) continue;  // (the usual case)
+    uint32_t most = kHubWave;
+    if (gpb == 1u) most = n_hub >= nwaves ? kHubSteps * 8 * kWave : 0u;
+    else if (__syncthreads_count(len > kHubWave / 4u) <= 4) most = kHubWave / 4u;
+    const bool alone = len > most;
+    const unsigned long long by_team = __ballot(hub && !alone), by_all = __ballot(hub && alone);
+    if (lane == 0) s_mask[wave] = by_team;
     __syncthreads();
-    uint32_t turn = 0;
-    for (uint32_t w = 0; w < nwaves; ++w) {
-      unsigned long long m = s_mask[w];
-      for (; m != 0; m &= m - 1ull, ++turn) {
-        if (turn % nwaves != wave) continue;
-        const uint32_t r = row_of(i0 + w * kWave + static_cast<uint32_t>(__ffsll(m) - 1));
-        const uint32_t start = indptr[r];
+    uint32_t n_team = 0;
+    for (uint32_t w = 0; w < nwaves; ++w) n_team += static_cast<uint32_t>(__popcll(s_mask[w]));
+    if (n_team != 0) {
+      uint32_t team = kWave;
+      while (team > kHubLanes && team * n_team > blockDim.x) team /= 2;
+      for (uint32_t k = tid / team; k < n_team; k += blockDim.x / team) {
+        uint32_t nth = k, at = 0;  // the k-th bit of the masks
+        unsigned long long m = s_mask[0];
+        while (nth >= static_cast<uint32_t>(__popcll(m))) {
+          nth -= static_cast<uint32_t>(__popcll(m));
+          at += kWave;
+          m = s_mask[at / kWave];
+        }
+#pragma unroll
+        for (uint32_t s = kWave / 2; s != 0; s /= 2) {
+          const uint32_t below = static_cast<uint32_t>(__popcll(m & ((1ull << s) - 1ull)));
+          if (nth >= below) nth -= below, m >>= s, at += s;
+        }
+        const uint32_t r = row_of(i0 + at);
         double acc = 0.0;
         uint32_t hits = 0;
-        walk(start, indptr[r + 1] - start, lane, kWave, acc, hits);
-        if (lane == 0) y[r] = (MODE == kEvent && !HETER) ? gathered_sum(w_homo, hits) : static_cast<F>(acc);
+        walk(indptr[r], indptr[r + 1], tid % team, team, acc, hits);
+        for (uint32_t s = team / 2; s != 0; s /= 2) {
+          if (MODE == kEvent && !HETER) hits += static_cast<uint32_t>(__shfl_xor(static_cast<int>(hits), static_cast<int>(s)));
+          else acc += __shfl_xor(acc, static_cast<int>(s));
+        }
+        if (tid % team == 0) y[r] = (MODE == kEvent && !HETER) ? gathered_sum(w_homo, hits) : static_cast<F>(acc);
       }
     }
     __syncthreads();
     if (lane == 0) s_mask[wave] = by_all;
+    if (tid < kHubBatch) s_acc[tid] = 0.0, s_hits[tid] = 0u;
     __syncthreads();
+    uint32_t n_all = 0;  // rows whose sums are under way
+    auto store = [&]() {
+      __syncthreads();
+      if (tid < n_all) {
+        y[s_row[tid]] = (MODE == kEvent && !HETER) ? gathered_sum(w_homo, s_hits[tid]) : static_cast<F>(s_acc[tid]);
+        s_acc[tid] = 0.0, s_hits[tid] = 0u;
+      }
+      __syncthreads();
+      n_all = 0;
+    };
     for (uint32_t w = 0; w < nwaves; ++w) {
       unsigned long long m = s_mask[w];
       for (; m != 0; m &= m - 1ull) {
         const uint32_t r = row_of(i0 + w * kWave + static_cast<uint32_t>(__ffsll(m) - 1));
-        if (tid == 0) s_acc = 0.0, s_hits = 0u;
-        __syncthreads();
-        const uint32_t start = indptr[r];
         double acc = 0.0;
         uint32_t hits = 0;
-        walk(start, indptr[r + 1] - start, tid, blockDim.x, acc, hits);
+        walk(indptr[r], indptr[r + 1], tid, blockDim.x, acc, hits);
+        if (tid == 0) s_row[n_all] = r;
         if (MODE == kEvent && !HETER) {
-          if (lane == 0 && hits != 0u) atomicAdd(&s_hits, hits);
+          hits = wave_sum(hits);
+          if (lane == 0 && hits != 0u) atomicAdd(&s_hits[n_all], hits);
         } else {
-          if (lane == 0) atomicAdd(&s_acc, acc);
+          acc = wave_sum(acc);
+          if (lane == 0) atomicAdd(&s_acc[n_all], acc);
         }
-        __syncthreads();
-        if (tid == 0) y[r] = (MODE == kEvent && !HETER) ? gathered_sum(w_homo, s_hits) : static_cast<F>(s_acc);
-        __syncthreads();
+        if (++n_all == kHubBatch) store();
       }
     }
+    if (n_all != 0) store();
     __syncthreads();  // (the masks are written again)
   }
 }
@@ -1335,17 +1407,23 @@ __global__ __launch_bounds__(1024, (MODE == kEvent && BITS == 1) ? 8 : 4) void c
   // it: 60,000 rows of 700, log-normal, double: 88 us with 512 here; 50,000 rows of 200, a tenth of 2,600: 54 -> 29 us)
   constexpr uint32_t kWaveStep = 8 * kWave * (MODE == kEvent && !HETER ? 4 : 1);
   // A hub row costs its workgroup 2.4 us whatever its length (three barriers, a chain of loads), a step in the wave walk
-  // 0.4 to 0.7 us with a dense vector or one weight and up to 1.8 with weights per nonzero.  So a workgroup of 256 threads
-  // leaves rows of up to eight (dense), six or, above, sixteen steps to their waves (5,000 rows of 100, every fifth of 3,000, weights
-  // per nonzero 24 -> 21 us, 300 uneven rows of 500 12.5 -> 10.3), and with a dense vector a row of up to twice a wave's
-  // share of the nonzeros is none (20,000 x 30,000, a tenth of the rows of 4,000, the others of 100: 60 -> 34 us).
+  // 0.4 to 0.7 us with a dense vector or one weight and up to 1.8 with weights per nonzero.  So rows of up to sixteen (dense),
+  // six or, above, sixteen steps are left to their waves (5,000 rows of 100, every fifth of 3,000, weights
+  // per nonzero 24 -> 21 us, 300 uneven rows of 500 12.5 -> 10.3, 6,249 x 4,014 log-normal of 840, dense, double 37 -> 23), and
+  // a row of up to twice a wave's share of the nonzeros is none (20,000 x 30,000, a tenth of the rows of 4,000, the others
+  // of 100, dense: 60 -> 34 us; 28,000 log-normal rows of 1,000, events: 46 -> 38).
+  // (Groups of lanes: what every one of them walks anyway, twice its share of the nonzeros, does not make a row a hub:
+  // 1,028,000 rows, a tenth of 290, one weight 118 -> 60 us; nor do 8 to 16 short steps, which cost less than the pass.)
+  auto hub_of_group = [&](uint32_t step) {
+    const uint32_t share = nnz / (gridDim.x * gpb);
+    const uint32_t least = MODE == kEvent ? 256u : 128u;
+    return hub_length(mean, step, share >= 0x10000000u ? 0xffffffffu : 2u * share > least ? 2u * share : least);
+  };
   uint32_t wave_least = 0;
-  if constexpr (MODE == kDense) {
+  if (MODE == kDense || HETER) {
     const uint32_t share = nnz / (gridDim.x * (blockDim.x / kWave));
-    wave_least = blockDim.x < 1024u ? 8u * kWaveStep : 0u;
+    wave_least = (MODE == kDense ? 16u : 6u) * kWaveStep;
     if (share < 0x10000000u && 2u * share > wave_least) wave_least = 2u * share;
-  } else if (HETER) {
-    wave_least = blockDim.x < 1024u ? 6u * kWaveStep : 0u;
   }
   if constexpr (MODE == kDense && BITS == 0) {
     // (rows of `skip_mean` nonzeros or more on average: the launcher's other kernel has taken this matrix)
@@ -1355,9 +1433,9 @@ __global__ __launch_bounds__(1024, (MODE == kEvent && BITS == 1) ? 8 : 4) void c
     // (nothing left to hide but the index and weight streams: the walks of the event gather)
     const VT *xs = reinterpret_cast<const VT *>(s_bits);
     if (mean >= 384) { gpb = 1; hub_len = hub_length(mean, kWaveStep, wave_least); gather_rows_wave<F, VT, HETER, MODE, BITS, 8>(data, indices, indptr, xs, y, n_row, s_bits, coarse_g, hub_len); }
-    else if (mean >= 24) { gpb = blockDim.x / 8; hub_len = hub_length(mean, 8 * 8); gather_rows<F, VT, HETER, MODE, BITS, 8, 8>(data, indices, indptr, xs, y, n_row, s_bits, coarse_g, hub_len); }
-    else if (mean >= 12) { gpb = blockDim.x / 4; hub_len = hub_length(mean, 8 * 4); gather_rows<F, VT, HETER, MODE, BITS, 4, 8>(data, indices, indptr, xs, y, n_row, s_bits, coarse_g, hub_len); }
-    else { gpb = blockDim.x / 4; hub_len = hub_length(mean, 4 * 4); gather_rows<F, VT, HETER, MODE, BITS, 4, 4>(data, indices, indptr, xs, y, n_row, s_bits, coarse_g, hub_len); }
+    else if (mean >= 24) { gpb = blockDim.x / 8; hub_len = hub_of_group(8 * 8); gather_rows<F, VT, HETER, MODE, BITS, 8, 8>(data, indices, indptr, xs, y, n_row, s_bits, coarse_g, hub_len); }
+    else if (mean >= 12) { gpb = blockDim.x / 4; hub_len = hub_of_group(8 * 4); gather_rows<F, VT, HETER, MODE, BITS, 4, 8>(data, indices, indptr, xs, y, n_row, s_bits, coarse_g, hub_len); }
+    else { gpb = blockDim.x / 4; hub_len = hub_of_group(4 * 4); gather_rows<F, VT, HETER, MODE, BITS, 4, 4>(data, indices, indptr, xs, y, n_row, s_bits, coarse_g, hub_len); }
   } else if constexpr (MODE == kDense && BITS == 2) {  // (long rows only)
     gpb = 1;
     hub_len = hub_length(mean, kWaveStep, wave_least);
@@ -1376,8 +1454,8 @@ __global__ __launch_bounds__(1024, (MODE == kEvent && BITS == 1) ? 8 : 4) void c
       }
     }
     if (mean >= 384) { gpb = 1; hub_len = hub_length(mean, kWaveStep, wave_least); gather_rows_wave<F, VT, HETER, MODE, BITS, 8>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
-    else if (mean >= 48) { gpb = blockDim.x / 8; hub_len = hub_length(mean, 16 * 8); gather_rows<F, VT, HETER, MODE, BITS, 8, 16>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
-    else { gpb = blockDim.x / 4; hub_len = hub_length(mean, 8 * 4); gather_rows<F, VT, HETER, MODE, BITS, 4, 8>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
+    else if (mean >= 48) { gpb = blockDim.x / 8; hub_len = hub_of_group(16 * 8); gather_rows<F, VT, HETER, MODE, BITS, 8, 16>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
+    else { gpb = blockDim.x / 4; hub_len = hub_of_group(8 * 4); gather_rows<F, VT, HETER, MODE, BITS, 4, 8>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
   } else {
     if constexpr (MODE == kEvent && BITS == 1 && HETER) {
       // The same walk within 64 registers, where the launcher left room for it behind the bitmap.  A wave's steps
@@ -1396,22 +1474,23 @@ __global__ __launch_bounds__(1024, (MODE == kEvent && BITS == 1) ? 8 : 4) void c
     if (mean >= 384) { gpb = 1; hub_len = hub_length(mean, kWaveStep, wave_least); gather_rows_wave<F, VT, HETER, MODE, BITS, 8>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
     // (a dense vector is gathered from L2: for rows of 48 .. 191 nonzeros the pipelined 32-lane walk keeps more
     // of those gathers in flight than a wave per row does)
-    else if (MODE == kEvent && mean >= 48u) { gpb = blockDim.x / 8; hub_len = hub_length(mean, 8 * 8); gather_rows<F, VT, HETER, MODE, BITS, 8, 8>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
+    else if (MODE == kEvent && mean >= 48u) { gpb = blockDim.x / 8; hub_len = hub_of_group(8 * 8); gather_rows<F, VT, HETER, MODE, BITS, 8, 8>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
     else if (MODE == kDense && mean >= 192u) { gpb = 1; hub_len = hub_length(mean, 2 * kWave); gather_rows_wave<F, VT, HETER, MODE, BITS, 2>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
-    else if (mean >= 48) { gpb = blockDim.x / 32; hub_len = hub_length(mean, 4 * 32); gather_rows<F, VT, HETER, MODE, BITS, 32, 4>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
-    else if (MODE == kEvent && mean >= 24) { gpb = blockDim.x / 8; hub_len = hub_length(mean, 8 * 8); gather_rows<F, VT, HETER, MODE, BITS, 8, 8>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
-    else if (MODE == kEvent && mean >= 12) { gpb = blockDim.x / 4; hub_len = hub_length(mean, 8 * 4); gather_rows<F, VT, HETER, MODE, BITS, 4, 8>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
-    else if (MODE == kEvent) { gpb = blockDim.x / 4; hub_len = hub_length(mean, 4 * 4); gather_rows<F, VT, HETER, MODE, BITS, 4, 4>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
-    else if (mean >= 24) { gpb = blockDim.x / 32; hub_len = hub_length(mean, 2 * 32); gather_rows<F, VT, HETER, MODE, BITS, 32, 2>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
-    else if (mean >= 12) { gpb = blockDim.x / 16; hub_len = hub_length(mean, 2 * 16); gather_rows<F, VT, HETER, MODE, BITS, 16, 2>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
-    else { gpb = blockDim.x / 8; hub_len = hub_length(mean, 2 * 8); gather_rows<F, VT, HETER, MODE, BITS, 8, 2>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
+    else if (mean >= 48) { gpb = blockDim.x / 32; hub_len = hub_of_group(4 * 32); gather_rows<F, VT, HETER, MODE, BITS, 32, 4>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
+    else if (MODE == kEvent && mean >= 24) { gpb = blockDim.x / 8; hub_len = hub_of_group(8 * 8); gather_rows<F, VT, HETER, MODE, BITS, 8, 8>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
+    else if (MODE == kEvent && mean >= 12) { gpb = blockDim.x / 4; hub_len = hub_of_group(8 * 4); gather_rows<F, VT, HETER, MODE, BITS, 4, 8>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
+    else if (MODE == kEvent) { gpb = blockDim.x / 4; hub_len = hub_of_group(4 * 4); gather_rows<F, VT, HETER, MODE, BITS, 4, 4>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
+    else if (mean >= 24) { gpb = blockDim.x / 32; hub_len = hub_of_group(2 * 32); gather_rows<F, VT, HETER, MODE, BITS, 32, 2>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
+    else if (mean >= 12) { gpb = blockDim.x / 16; hub_len = hub_of_group(2 * 16); gather_rows<F, VT, HETER, MODE, BITS, 16, 2>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
+    else { gpb = blockDim.x / 8; hub_len = hub_of_group(2 * 8); gather_rows<F, VT, HETER, MODE, BITS, 8, 2>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
   }
   // the rows the walk left to the whole workgroup
+  const uint32_t hub_deal = gpb < kHubDeal || n_row / 2u > gridDim.x * gpb ? gpb : kHubDeal;
   if constexpr (MODE == kDense && BITS == 1)
     gather_hub_rows<F, VT, HETER, MODE, BITS>(data, indices, indptr, reinterpret_cast<const VT *>(s_bits), y, n_row, s_bits,
-                                              coarse_g, gpb, hub_len);
+                                              coarse_g, nnz, hub_deal, hub_len);
   else
-    gather_hub_rows<F, VT, HETER, MODE, BITS>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, gpb, hub_len);
+    gather_hub_rows<F, VT, HETER, MODE, BITS>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, nnz, hub_deal, hub_len);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1876,13 +1955,15 @@ void launch_gather(const char *target, const ScratchSource &src, const F *data, 
       // A longer vector is gathered from L2 (up to four times what fits in LDS: less the part that does).
       // Rows of 4 nonzeros or more on average: the flat walk over the nonzeros with 16-byte loads of the index and
       // weight streams (csr_flat_gather.hip; 4,000,000 rows of 8: 224 against 304 us, 2,000,000 rows of 20: 255
-      // against 348 us); shorter ones: the walks below.  Where the number of nonzeros is known on the device only,
+      // against 348 us); shorter ones: the walks below, the vector gathered from L2 (1,000,000 x 60,000 with 3 per
+      // row, a weight each, 26 us; with 159 KB of it staged 46).  Where the number of nonzeros is known on the device only,
       // both are enqueued and one returns at once (4.5 us).
       // Under 16,384 rows only with a part of the vector staged (300 rows of 10,000 and 140,000 columns: 116 -> 21 us,
       // 10,000 rows of 1,300 and 43,818 columns: 58 -> 43 us): with 2,000 rows of 40,000 and a vector of 12 MB the
       // walk that keeps a row's gathers together takes 507 us, the flat one 835.
       // Under a million nonzeros the row-wise walk, one launch and nothing to stage (20,000 rows of 10 to 30 and 60,000
-      // columns: 9 us against 14; 50,000 uneven rows of 20: 16.6 against 17.1).
+      // columns: 9 us against 14; 50,000 uneven rows of 20: 16.6 against 17.1; 28,000 log-normal rows with sigma 1.8, double:
+      // 24 against 17).
       constexpr uint32_t kFlatMinMean = 4, kFlatMinNnz = 1u << 20;
       const bool known = nnz != kUnknownNnz;
       // Long rows and a vector a little longer than what fits: a wave per row with 159 KB of it staged, where the flat walk's

@@ -1327,7 +1327,47 @@ def test_a_vector_a_little_longer_than_lds_costs_little_more(cuda):
   assert best[0] < 1.6 * best[1], best
 
 
-@pytest.mark.parametrize("n_row,n_col,long,events", [(346_000, 42_500, 867, False)])
+# Rows that are left to a pass after the walk: a few of a workgroup's or all of them (8 to 64 lanes each), long ones next to
+# short ones, a wave's rows of which most are long (dealt one by one); lengths around the lines between those ways and
+# around whole steps of each; the matrix's last nonzeros in such a row.
+@pytest.mark.parametrize("n_row,n_col,base,kind", [
+  (3000, 2000, 3, "block"), (3000, 2000, 3, "block end"), (1200, 9000, 20, "special"), (9000, 9000, 2, "special"),
+  (20_000, 9000, 30, "special"), (20_000, 30_000, 1, "every third"), (600, 9000, 700, "every third"), (150_000, 3000, 2, "block"),
+  (4000, 20_000, 400, "special"), (300_000, 5000, 1, "special"), (17_000, 700_000, 3, "special"), (900, 20_000, 450, "all")])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_gather_long_rows_by_themselves_and_in_blocks(cuda, oracle_mod, n_row, n_col, base, kind, dtype):
+  rng = np.random.default_rng(n_row)
+  counts = rng.poisson(base, n_row)
+  special = [b + d for b in (64, 128, 256, 512, 1024, 2048, 4096, 8192) for d in (-1, 0, 1)]
+  if kind == "block":
+    counts[5:5 + n_row // 20] = 700
+  elif kind == "block end":
+    counts[-(n_row // 20):] = 1301
+  elif kind == "every third":
+    counts[::3] = rng.integers(120, 1500, counts[::3].shape[0])
+  elif kind == "all":
+    counts[:] = rng.integers(2000, 9000, n_row)
+  else:
+    counts[rng.permutation(n_row)[:len(special)]] = special
+    counts[-1] = special[-1]
+  counts = np.minimum(counts, n_col)
+  indices, indptr = synth.counted_csr(counts, n_col, seed=n_col)
+  print("case", n_row, n_col, kind, dtype.__name__, indices.shape[0], flush=True)
+  shape = (n_row, n_col)
+  ev = rng.random(n_col) < 0.4
+  v = rng.integers(-3, 4, size=n_col).astype(dtype)
+  data = rng.integers(-2, 3, size=indices.shape[0]).astype(dtype)
+  for d in (data, np.array([0.6], dtype=dtype)):  # (integers, and counts of one weight: every sum is exact)
+    for e in (ev, ev.astype(dtype)):
+      got = bpl.event_csr_matvec(d, indices, indptr, e, shape=shape).cpu().numpy()
+      assert np.array_equal(got, oracle_mod.event_csr_matvec(d, indices, indptr, ev, shape=shape))
+    if d is data:
+      got = bpl.csr_matvec(d, indices, indptr, v, shape=shape).cpu().numpy()
+      assert np.array_equal(got, oracle_mod.csr_matvec(d, indices, indptr, v, shape=shape))
+
+
+@pytest.mark.parametrize("n_row,n_col,long,events", [(72_000, 100_000, 1800, True), (888, 14_838, 1560, True),
+                                                      (346_000, 42_500, 867, False)])
 def test_a_block_of_rows_costs_what_its_nonzeros_cost(cuda, n_row, n_col, long, events):
   # all nonzeros in the first tenth of the rows: no longer than twice the same rows in a random order (all of them taken by
   # the few workgroups that the block is dealt to, or empty rows that count no more than a nonzero: 2.3 to 4 times)
