@@ -1963,7 +1963,9 @@ void launch_gather(const char *target, const ScratchSource &src, const F *data, 
       // walk that keeps a row's gathers together takes 507 us, the flat one 835.
       // Under a million nonzeros the row-wise walk, one launch and nothing to stage (20,000 rows of 10 to 30 and 60,000
       // columns: 9 us against 14; 50,000 uneven rows of 20: 16.6 against 17.1; 28,000 log-normal rows with sigma 1.8, double:
-      // 24 against 17).
+      // 24 against 17).  Under 16,384 rows three million (10,000 x 60,000 and 1.1 / 2 / 4 / 8 million 9 / 13 / 21 / 37 us against 16 /
+      // 17 / 21 / 28) and more than 8,192 columns (1,000 x 5,000 and four million: 13 against 16); but for under 2,048 rows and
+      // more than 32,768 columns, which leave most waves without a row (300 x 60,000 and 1.1 million: 36 against 16).
       constexpr uint32_t kFlatMinMean = 4, kFlatMinNnz = 1u << 20;
       const bool known = nnz != kUnknownNnz;
       // Long rows and a vector a little longer than what fits: a wave per row with 159 KB of it staged, where the flat walk's
@@ -1980,8 +1982,10 @@ void launch_gather(const char *target, const ScratchSource &src, const F *data, 
           return;
         bpl_clear_error();
       }
-      const bool flat = known ? nnz >= kFlatMinNnz && nnz <= kFlatMaxNnz && nnz / n_row >= kFlatMinMean &&
-                                  (n_row >= 16384 || flat_stages<F>(n_col))
+      const bool few = n_row < 2048 && n_col > 32768;
+      const uint32_t min_nnz = n_row >= 16384 || few ? kFlatMinNnz : 3u * kFlatMinNnz;
+      const bool flat = known ? nnz >= min_nnz && nnz <= kFlatMaxNnz && nnz / n_row >= kFlatMinMean &&
+                                  (n_row >= 16384 || (n_col > 8192 && flat_stages<F>(n_col)))
                               : n_row >= 16384;
       if (flat && n_col > 0) {
         if (csr_flat_gather<F>(target, stream, data, HETER, indices, indptr, x, y, n_row, n_col, known ? 0u : kFlatMinMean)) {

@@ -1131,7 +1131,7 @@ def test_csr_matvec_flat_walk_over_the_nonzeros(cuda, oracle_mod, kind):
 # vectors one element longer than what a workgroup stages whole, up to the last partly staged size and one beyond (gathered
 # from L2 only); below and above 16,384 rows; just below and above a million nonzeros (a row-wise walk below); long rows
 # and the last sizes that a wave per row takes with one weight and with weights per nonzero, and one more
-@pytest.mark.parametrize("n_row,n_col,mean", [(20_000, 35_329, 56), (3000, 35_329, 500), (300, 141_312, 4000),
+@pytest.mark.parametrize("n_row,n_col,mean", [(20_000, 35_329, 56), (3000, 35_329, 500), (3000, 35_329, 1000), (300, 141_312, 4000),
                                               (300, 37_632, 4000), (300, 37_633, 4000), (300, 37_634, 4000),
                                               (16_384, 46_518, 700), (16_384, 54_273, 700),
                                               (20_000, 141_312, 50), (20_000, 141_313, 60), (400_000, 40_705, 4)])
