@@ -1410,8 +1410,8 @@ __global__ __launch_bounds__(1024, (MODE == kEvent && BITS == 1) ? 8 : 4) void c
   // 0.4 to 0.7 us with a dense vector or one weight and up to 1.8 with weights per nonzero.  So rows of up to sixteen (dense),
   // six or, above, sixteen steps are left to their waves (5,000 rows of 100, every fifth of 3,000, weights
   // per nonzero 24 -> 21 us, 300 uneven rows of 500 12.5 -> 10.3, 6,249 x 4,014 log-normal of 840, dense, double 37 -> 23), and
-  // a row of up to twice a wave's share of the nonzeros is none (20,000 x 30,000, a tenth of the rows of 4,000, the others
-  // of 100, dense: 60 -> 34 us; 28,000 log-normal rows of 1,000, events: 46 -> 38).
+  // with a dense vector a row of up to twice a wave's share of the nonzeros is none (20,000 x 30,000, a tenth of the rows of
+  // 4,000, the others of 100: 60 -> 34 us; events: 28,000 log-normal rows of 1,000 the same, 60,000 of 700, double, 90 -> 119).
   // (Groups of lanes: what every one of them walks anyway, twice its share of the nonzeros, does not make a row a hub:
   // 1,028,000 rows, a tenth of 290, one weight 118 -> 60 us; nor do 8 to 16 short steps, which cost less than the pass.)
   auto hub_of_group = [&](uint32_t step) {
@@ -1423,7 +1423,7 @@ __global__ __launch_bounds__(1024, (MODE == kEvent && BITS == 1) ? 8 : 4) void c
   if (MODE == kDense || HETER) {
     const uint32_t share = nnz / (gridDim.x * (blockDim.x / kWave));
     wave_least = (MODE == kDense ? 16u : 6u) * kWaveStep;
-    if (share < 0x10000000u && 2u * share > wave_least) wave_least = 2u * share;
+    if (MODE == kDense && share < 0x10000000u && 2u * share > wave_least) wave_least = 2u * share;
   }
   if constexpr (MODE == kDense && BITS == 0) {
     // (rows of `skip_mean` nonzeros or more on average: the launcher's other kernel has taken this matrix)

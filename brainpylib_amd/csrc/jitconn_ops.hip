@@ -33,7 +33,8 @@ namespace {
 // LDS the row walk gives to an event bitmap when it wants two 16-wave workgroups per CU (each wave
 // can issue one instruction every four cycles, so the number of resident waves bounds the VALU
 // utilisation: 32 waves per CU walk 290 G synapses/s, the 15 that fit beside a 125 KB bitmap 228).
-// What two workgroups leave of a CU's 160 KB beside their 16 waves' states and queues (normal weights: 18,944 bytes).
+// What two workgroups leave of a CU's 160 KB beside their 16 waves' states and queues (normal weights: 18,944 bytes; 1e5
+// streams of 1,000 synapses over 1e6 inputs 625 / 628 / 628 us at 1 / 10 / 100 % events: the second probe hides behind the weights).
 constexpr uint32_t kRowwalkCoarseMost = 38912;
 template <typename T1, int W>
 constexpr uint32_t rowwalk_coarse_bytes() {

@@ -155,7 +155,8 @@ def event_csr_matvec_batching(values, indices, indptr, events, *, batch_size: in
 
   The reference has this operator on the CPU only.  Here one matrix shared by the whole batch
   (B_v = B_i = B_p = 1) with ``transpose=False`` streams the column indices once per eight event
-  vectors; every other combination runs the single operator once per batch entry."""
+  vectors and with ``transpose=True`` goes through one sorted scatter per group of entries; every other
+  combination runs the single operator once per batch entry."""
   values = as_tensor(values)
   indices = as_tensor(indices)
   indptr = as_tensor(indptr)
