@@ -55,10 +55,12 @@ const DeviceInfo &device_info();
 void *stream_workspace(hipStream_t stream, size_t bytes);
 
 // A few zero-initialised 32-bit counters per (device, stream).  The first one (the scatter's
-// active-row count) is left at zero again by every user; the others carry nothing from call to
+// active-row count) and the two from kWalkCounters on (work that workgroups take as they come) are left at zero again
+// by every user; the others carry nothing from call to
 // call.  nullptr if the allocation fails (or would be needed during a capture).
 uint32_t *stream_counters(hipStream_t stream);
 constexpr size_t kStreamCounterBytes = 256;
+constexpr uint32_t kWalkCounters = 60;
 
 // True if the calling thread's most recent stream_workspace() / stream_counters() call failed
 // because the stream was being captured.  A launcher that would otherwise fall back to a path
@@ -324,10 +326,13 @@ __device__ __forceinline__ bool probe_event<PackedBits>(const PackedBits *__rest
   return (ev[i >> 5].w >> (i & 31u)) & 1u;
 }
 
-// bits[w] bit b = ev[32 w + b] != 0 (zero beyond n): coalesced loads, one ballot per 64 elements.
+// bits[lead + w] bit b = ev[32 w + b] != 0 (zero beyond n), behind `lead` empty words: coalesced loads, one ballot per 64
+// elements.
 template <typename VT>
 __global__ __launch_bounds__(256) void pack_event_bitmap_kernel(const VT *__restrict__ ev, uint32_t n,
-                                                                uint32_t *__restrict__ bits) {
+                                                                uint32_t *__restrict__ bits, uint32_t lead) {
+  if (blockIdx.x == 0 && threadIdx.x < lead) bits[threadIdx.x] = 0u;
+  bits += lead;
   const uint32_t lane = threadIdx.x & (kWave - 1);
   const uint32_t waves = gridDim.x * (256 / kWave);
   const uint32_t groups = (n + kWave - 1) / kWave;
@@ -377,11 +382,11 @@ static __global__ __launch_bounds__(256) void coarsen_bitmap_kernel(const uint32
 }
 
 template <typename VT>
-inline void pack_event_bitmap(hipStream_t stream, const VT *ev, uint32_t n, uint32_t *bits) {
+inline void pack_event_bitmap(hipStream_t stream, const VT *ev, uint32_t n, uint32_t *bits, uint32_t lead = 0) {
   if (n == 0) return;
   const unsigned groups = div_up(n, kWave);
   const unsigned grid = div_up(groups, 256 / kWave);
-  hipLaunchKernelGGL(pack_event_bitmap_kernel<VT>, dim3(grid < 2048 ? grid : 2048), dim3(256), 0, stream, ev, n, bits);
+  hipLaunchKernelGGL(pack_event_bitmap_kernel<VT>, dim3(grid < 2048 ? grid : 2048), dim3(256), 0, stream, ev, n, bits, lead);
 }
 
 // Copies n elements of x to LDS with all threads of the workgroup: 16-byte loads, eight of a lane in flight (a loop of

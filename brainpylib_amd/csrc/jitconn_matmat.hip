@@ -66,7 +66,7 @@ struct __attribute__((aligned(2 * sizeof(T1)))) Synapse {
 template <typename T1, int W, int MT>
 __global__ __launch_bounds__(256) void jitconn_matmat_kernel(const T1 *__restrict__ XT, T1 *__restrict__ Y,
                                                              uint32_t m, uint32_t k, uint32_t n, uint32_t m_pad,
-                                                             uint32_t seed, double log_p, T1 wa, T1 wb,
+                                                             uint32_t seed, SkipParams skips, T1 wa, T1 wb,
                                                              uint32_t first, uint32_t count,
                                                              const uint32_t *__restrict__ states, uint32_t pass) {
   constexpr int kWaves = 4;
@@ -129,7 +129,7 @@ __global__ __launch_bounds__(256) void jitconn_matmat_kernel(const T1 *__restric
       syn[slot].w = w;
     };
     if constexpr (W == kNormal) {
-      walk_stream<T1, W>(st, lane, seed + j, pre, k, log_p, wa, wb,
+      walk_stream<T1, W>(st, lane, seed + j, pre, k, skips, wa, wb,
                          [&](uint32_t idx0, T1 w0, bool valid0, uint32_t idx1, T1 w1, bool valid1) {
         __builtin_amdgcn_wave_barrier();  // the reads of the batch before are done
         if (valid0) {
@@ -140,7 +140,7 @@ __global__ __launch_bounds__(256) void jitconn_matmat_kernel(const T1 *__restric
         take(static_cast<uint32_t>(__popcll(__ballot(valid0)) + __popcll(__ballot(valid1))));
       });
     } else {
-      walk_stream<T1, W>(st, lane, seed + j, pre, k, log_p, wa, wb, [&](uint32_t idx, T1 w, bool valid) {
+      walk_stream<T1, W>(st, lane, seed + j, pre, k, skips, wa, wb, [&](uint32_t idx, T1 w, bool valid, bool) {
         __builtin_amdgcn_wave_barrier();
         if (valid) put(static_cast<uint32_t>(lane), idx, w);
         __builtin_amdgcn_wave_barrier();
@@ -210,10 +210,10 @@ void matmat_entry(const char *target, hipStream_t stream, void **buffers, const 
     for (uint32_t pass = 0; pass < passes; ++pass) {
       if (tiles == 1) {
         hipLaunchKernelGGL((jitconn_matmat_kernel<T1, W, 1>), dim3(grid_x), dim3(256), 0, stream, XT, Y, m, k, n, m_pad,
-                           d.seed, d.log_p, wa, wb, first, count, pre, pass);
+                           d.seed, make_skip_params(d.log_p), wa, wb, first, count, pre, pass);
       } else {
         hipLaunchKernelGGL((jitconn_matmat_kernel<T1, W, 2>), dim3(grid_x), dim3(256), 0, stream, XT, Y, m, k, n, m_pad,
-                           d.seed, d.log_p, wa, wb, first, count, pre, pass);
+                           d.seed, make_skip_params(d.log_p), wa, wb, first, count, pre, pass);
       }
     }
   }

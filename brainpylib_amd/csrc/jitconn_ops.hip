@@ -43,44 +43,53 @@ constexpr uint32_t rowwalk_coarse_bytes() {
 }
 
 // BITS: where the event probes go.  0: the event vector in global memory; 1: its bitmap in LDS;
-// 2: a coarse bitmap in LDS (one bit per 2^g inputs, at most rowwalk_coarse_bytes<T1, W>()) and, where its
-// bit is set, the exact packed bitmap in global memory (`in`, the coarse one behind it).
+// 2: a coarse bitmap in LDS (one bit per 2^g positions, at most rowwalk_coarse_bytes<T1, W>()) and, where its
+// bit is set, the exact packed bitmap in global memory (`in`, the coarse one behind it).  Positions count from
+// kRowwalkLead: the first word of the exact bitmap is empty, and a lane that has nothing to look up reads it.
+constexpr uint32_t kRowwalkLead = 32;
 // (With the coarse bitmap two 16-wave workgroups are meant to share a CU: 8 waves per SIMD, which
 // the register allocation has to leave room for; the normal-weight walk needs 66 otherwise.)
 // Register budget: eight waves per SIMD need at most 64 vector AND at most 80 scalar registers per
 // wave here (with 81..96 scalar registers only seven fit, so a second 16-wave workgroup does not).
 constexpr uint32_t kFuseBatch = 64;   // streams seeded together, one per lane
 constexpr uint32_t kFuseSlots = 3;    // batches of seeded states in a workgroup's ring
+constexpr uint32_t kFuseNumbers = 8;  // batch numbers a row-walk workgroup remembers (more than a wave can fall behind)
+constexpr uint32_t kFuseLdsWords = 16;  // the row walk's counters and numbers, in front of the states
+static_assert(1 + 2 * kFuseSlots + kFuseNumbers <= kFuseLdsWords, "room for them");
 constexpr uint32_t kFuseSpin = 1u << 22;           // polls of a flag in LDS before a wave stops waiting
 constexpr uint32_t kFuseNotSeeded = 0x80000000u;   // flag bit: the batch's rows seed their own generators
 constexpr size_t kFuseRingBytes = static_cast<size_t>(kFuseSlots) * kFuseBatch * kMtN * sizeof(uint32_t);  // per workgroup
-static_assert(kMtSeedTileWords <= kMtStateWords, "the seeding wave transposes through its own state buffer");
+static_assert(kMtSeedTileWords <= kMtN, "the seeding wave transposes through its own state buffer");
 
 template <typename T1, typename VT, int IN, int W, int BITS, bool FUSED>
 __global__ __launch_bounds__(1024, (BITS == 2 || (W == kNormal && sizeof(T1) == 4)) ? 8 : 4)
     __attribute__((amdgpu_num_sgpr(80))) void jitconn_rowwalk_kernel(const VT *__restrict__ in, T1 *__restrict__ out,
                                                                uint32_t n_out, uint32_t n_in, uint32_t seed,
-                                                               double log_p, T1 wa, T1 wb, uint32_t first,
+                                                               SkipParams skips, T1 wa, T1 wb, uint32_t *next,
                                                                uint32_t *states) {
-  // Handles the n_out outputs first .. first + n_out - 1; `states` (optional) holds their
-  // generators' seeded states.  FUSED: all outputs from 0, `states` is the workgroups' rings
-  // (kFuseRingBytes each).
-  extern __shared__ __attribute__((aligned(8))) uint32_t smem[];
+  // `states` (optional) holds the outputs' generators' seeded states.  FUSED: `states` is the workgroups' rings
+  // (kFuseRingBytes each), `next` (optional) two counters that are zero.
+  extern __shared__ __attribute__((aligned(8))) uint32_t smem_raw[];
+  uint32_t *smem = smem_raw + (FUSED ? kFuseLdsWords : 0u);
   const int lane = lane_id();
   const uint32_t wave = threadIdx.x / kWave;
   const uint32_t nwaves = blockDim.x / kWave;
   constexpr int kWords = StreamLds<T1, W>::words;
   uint32_t *st = smem + wave * kWords;
   const uint32_t *bits = smem + nwaves * kWords;
-  uint32_t coarse_g = 0, coarse_g5 = 5;
+  constexpr uint32_t kLead = BITS == 2 ? kRowwalkLead : 0u;  // positions in front of the first input
+  const uint8_t *coarse_bytes = reinterpret_cast<const uint8_t *>(smem + 16 * kWords);  // (BITS == 2: sixteen waves)
+  uint32_t coarse_g = 0, coarse_g3 = 3;
   if constexpr (BITS == 2) {
-    uint32_t *wbits = smem + nwaves * kWords;
-    coarse_g = coarse_shift(n_in, rowwalk_coarse_bytes<T1, W>());
-    coarse_g5 = coarse_g + 5u;
-    const uint32_t words = (coarse_bits(n_in, coarse_g) + 31u) >> 5;
-    const uint32_t *coarse = reinterpret_cast<const uint32_t *>(in) + coarse_offset_words(n_in);
+    uint32_t *wbits = smem + 16 * kWords;
+    coarse_g = coarse_shift(n_in + kLead, rowwalk_coarse_bytes<T1, W>());
+    coarse_g3 = coarse_g + 3u;
+    const uint32_t words = (coarse_bits(n_in + kLead, coarse_g) + 31u) >> 5;
+    const uint32_t *coarse = reinterpret_cast<const uint32_t *>(in) + coarse_offset_words(n_in + kLead);
     for (uint32_t i = threadIdx.x; i < words; i += blockDim.x) wbits[i] = coarse[i];
     __syncthreads();
+    // (a shift by a scalar register takes twice the cycles; the other weights have no vector registers to spare)
+    if constexpr (W == kHomo) asm volatile("" : "+v"(coarse_g), "+v"(coarse_g3));
   } else if constexpr (BITS == 1) {
     uint32_t *wbits = smem + nwaves * kWords;
     const uint32_t words = (n_in + 31u) >> 5;
@@ -94,49 +103,46 @@ __global__ __launch_bounds__(1024, (BITS == 2 || (W == kNormal && sizeof(T1) == 
     // two-level bitmap: the exact word of a batch is requested when the batch is drawn and looked
     // at when the next one is, so that no wave waits for it
     uint32_t late_word = 0, late_idx = 0;
-    uint64_t late_coarse = 0;  // lanes whose coarse bit was set (wave uniform, so the scalar unit combines the masks)
-    bool late_lane = false;    // this lane's bit of it
     T1 late_w = T1(0);
-    auto settle = [&]() {
-      const bool bit = __builtin_amdgcn_ubfe(late_word, late_idx, 1u) != 0u;
-      if (W == kHomo) cnt += static_cast<uint32_t>(__popcll(late_coarse & __builtin_amdgcn_ballot_w64(bit)));
-      else if (bit && late_lane) acc += static_cast<double>(late_w);
+    auto count_event = [&](uint32_t bit, T1 w) {  // bit: 0 or 1
+      if (W == kHomo) cnt += bit;
+      else if (bit) acc += static_cast<double>(w);
     };
-    walk_stream<T1, W, W != kNormal>(st, lane, seed + o, pre, n_in, log_p, wa, wb, [&](uint32_t idx, T1 w, bool valid) {
+    auto settle = [&]() { count_event(__builtin_amdgcn_ubfe(late_word, late_idx, 1u), late_w); };
+    walk_stream<T1, W, W != kNormal>(st, lane, seed + o, pre, n_in + kLead, skips, wa, wb,
+                                     [&](uint32_t idx, T1 w, bool valid, bool partial) {
       if constexpr (IN == kInEvent && BITS == 2) {
         settle();
-        // bit c = idx >> g of the coarse bitmap: word c >> 5, bit c & 31 (the bit-field extract takes the
-        // low five bits).  Lanes past the end of the row extract a field of width 0, which is 0 whatever
-        // the word holds: the word they read may lie past the bitmap, even past the workgroup's LDS
-        // (such a read returns 0 and cannot fault), and its value is never looked at.
-        const uint32_t c = idx >> coarse_g;
-        const bool coarse = __builtin_amdgcn_ubfe(bits[idx >> coarse_g5], c, valid ? 1u : 0u) != 0u;
-        // (lanes without a coarse hit read word 0 and ignore it: a plain load for the whole wave)
-        late_word = reinterpret_cast<const uint32_t *>(in)[coarse ? idx >> 5 : 0u];
+        // position idx: bit (idx >> g) of the coarse bitmap, bit idx of the exact one, whose word 0 holds no input: it is
+        // what lanes beyond the row (position 0) and lanes without a coarse hit read
+        const uint32_t byte = coarse_bytes[idx >> coarse_g3];
+        const uint32_t hit = static_cast<uint32_t>(__builtin_amdgcn_sbfe(static_cast<int>(byte), (idx >> coarse_g) & 7u, 1u));
+        const uint32_t off = __builtin_amdgcn_bitop3_b32(idx >> 3, ~3u, hit, 0x80);  // a & b & c
+        late_word = *reinterpret_cast<const uint32_t *>(reinterpret_cast<const char *>(in) + off);
         late_idx = idx;
-        late_coarse = __builtin_amdgcn_ballot_w64(coarse);
-        late_lane = coarse;
         late_w = w;
-        return;
-      }
-      if (IN == kInDense) {
-        if (valid) {
+      } else if constexpr (IN == kInEvent && BITS == 1) {
+        uint32_t bit = __builtin_amdgcn_ubfe(reinterpret_cast<const uint8_t *>(bits)[idx >> 3], idx & 7u, 1u);
+        if (partial) {
+          bit = valid ? bit : 0u;
+          asm volatile("" : "+v"(bit));  // (a branch, not a select in every batch)
+        }
+        count_event(bit, w);
+      } else if constexpr (IN == kInEvent) {
+        if (valid) count_event(probe_event(in, idx) ? 1u : 0u, w);
+      } else {
+        auto add = [&]() {
           const T1 v = static_cast<T1>(in[idx]);
           acc += static_cast<double>(W == kHomo ? v : static_cast<T1>(w * v));
-        }
-      } else {
-        bool hit = false;
-        if (valid) {
-          if (BITS == 1) hit = (bits[idx >> 5] >> (idx & 31u)) & 1u;
-          else hit = probe_event(in, idx);
-        }
-        if (W == kHomo) cnt += static_cast<uint32_t>(__popcll(__ballot(hit)));
-        else if (hit) acc += static_cast<double>(w);
+        };
+        if (!partial) add();
+        else if (valid) add();
       }
-    }, loaded);
+    }, loaded, kLead);
     if constexpr (IN == kInEvent && BITS == 2) settle();
     if (IN == kInEvent && W == kHomo) {
-      if (lane == 0) out[o] = static_cast<T1>(cnt);
+      cnt = wave_inclusive_scan_u32(cnt);
+      if (lane == kWave - 1) out[o] = static_cast<T1>(cnt);
     } else {
       acc = wave_sum(acc);
       if (lane == 0) out[o] = static_cast<T1>(acc);
@@ -145,34 +151,51 @@ __global__ __launch_bounds__(1024, (BITS == 2 || (W == kNormal && sizeof(T1) == 
 
   if constexpr (!FUSED) {
     for (uint32_t i = blockIdx.x * nwaves + wave; i < n_out; i += gridDim.x * nwaves)
-      walk_row(first + i, states ? states + static_cast<size_t>(i) * kMtN : nullptr, NoLoadHook());
+      walk_row(i, states ? states + static_cast<size_t>(i) * kMtN : nullptr, NoLoadHook());
   } else {
     // The generators are seeded inside the kernel, 64 streams at a time on the vector unit (the scalar
     // unit, one per CU, cannot seed a stream per wave fast enough), while the other waves walk: the
-    // workgroup takes batches of 64 consecutive outputs (batch blockIdx.x + j * gridDim.x is its j-th),
-    // its waves take (batch, row) tasks from a counter in LDS, and the wave that takes the first row of
-    // batch j first seeds batch j + 1 into slot (j + 1) % 3 of the workgroup's ring of seeded states in
+    // workgroup takes batches of 64 consecutive outputs, its waves take (batch, row) tasks from a counter in LDS, and the
+    // wave that takes the first row of the workgroup's batch j first takes batch j + 1 and seeds it into slot (j + 1) % 3 of
+    // the workgroup's ring of seeded states in
     // device memory (`states`), which stays in the L2.  A slot is written again only after all 64 rows
     // of its previous batch have copied their state to LDS, and read only after its flag says which
     // batch it holds; every wait is bounded, and a wave that gives up seeds its own generator instead.
-    __shared__ uint32_t s_task, s_ready[kFuseSlots], s_loaded[kFuseSlots];
+    //
+    // Which batch is next comes from a counter of the device (`next`: batches taken, workgroups at their end): of two
+    // workgroups on a CU the older one gets more of the issue slots, and with equal shares the younger one worked
+    // alone, four waves to a SIMD, for the last fifth (1,000,000 streams of 1,000 synapses: KBAL).  Without one
+    // (`next` null), batch blockIdx.x + j * gridDim.x.
+    uint32_t &s_task = smem_raw[0], *const s_ready = smem_raw + 1, *const s_loaded = s_ready + kFuseSlots,
+             *const s_batch = s_loaded + kFuseSlots;
     const uint32_t n_batches = (n_out + kFuseBatch - 1u) / kFuseBatch;
-    const uint32_t mine = n_batches > blockIdx.x ? (n_batches - blockIdx.x + gridDim.x - 1u) / gridDim.x : 0u;
     // (`states` is neither const nor restrict: other waves write what this one reads behind a flag)
     uint32_t *ring = states + static_cast<size_t>(blockIdx.x) * kFuseSlots * kFuseBatch * kMtN;
     if (threadIdx.x == 0) {
       s_task = 0;
       for (uint32_t k = 0; k < kFuseSlots; ++k) s_ready[k] = 0, s_loaded[k] = 0;
+      for (uint32_t k = 0; k < kFuseNumbers; ++k) s_batch[k] = n_batches;
     }
     __syncthreads();
-    if (mine == 0) return;
-    auto seed_batch = [&](uint32_t j) {
+    auto take_batch = [&](uint32_t j) {
+      uint32_t b = blockIdx.x + j * gridDim.x;
+      if (next != nullptr) {
+        if (lane == 0) b = atomicAdd(&next[0], 1u);
+        b = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(b)));
+      }
+      s_batch[j % kFuseNumbers] = b;
+      return b;
+    };
+    auto seed_batch = [&](uint32_t j, uint32_t b) {
       const uint32_t slot = j % kFuseSlots;
-      mt_seed_batch(st, lane, seed + (blockIdx.x + j * gridDim.x) * kFuseBatch + static_cast<uint32_t>(lane),
-                    ring + static_cast<size_t>(slot) * kFuseBatch * kMtN);
+      mt_seed_batch(st, lane, seed + b * kFuseBatch + static_cast<uint32_t>(lane), ring + static_cast<size_t>(slot) * kFuseBatch * kMtN);
       __hip_atomic_store(&s_ready[slot], j + 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
     };
-    if (wave == 0) seed_batch(0);
+    if (wave == 0) {
+      const uint32_t b = take_batch(0);
+      if (b < n_batches) seed_batch(0, b);
+      else __hip_atomic_store(&s_ready[0], 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
     for (;;) {
       // Every lane adds one, so the counter advances by 64 per task and any lane's old value / 64 is the
       // task.  (With the add under `if (lane == 0)` the compiler split the loop by lane: lane 0 went back
@@ -180,33 +203,40 @@ __global__ __launch_bounds__(1024, (BITS == 2 || (W == kNormal && sizeof(T1) == 
       const uint32_t t = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(
                              static_cast<int>(atomicAdd(&s_task, 1u)))) / kWave;
       const uint32_t j = t / kFuseBatch, r = t % kFuseBatch;
-      if (j >= mine) break;
-      if (r == 0 && j + 1 < mine) {
-        // slot (j + 1) % 3 last held batch j - 2: (j + 1) / 3 batches have used it, 64 loads each
-        const uint32_t slot = (j + 1u) % kFuseSlots, need = ((j + 1u) / kFuseSlots) * kFuseBatch;
-        bool free_ = false;
-        for (uint32_t spin = 0; spin < kFuseSpin && !free_; ++spin) {
-          free_ = __hip_atomic_load(&s_loaded[slot], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) >= need;
-          if (!free_) __builtin_amdgcn_s_sleep(2);
-        }
-        if (free_) seed_batch(j + 1u);
-        else __hip_atomic_store(&s_ready[slot], kFuseNotSeeded | (j + 2u), __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
-      }
       const uint32_t slot = j % kFuseSlots;
       uint32_t flag = 0;
-      for (uint32_t spin = 0; spin < kFuseSpin; ++spin) {
+      // (twice as many polls as the seeding wave waits for the slot: the flag tells which batch it is)
+      for (uint32_t spin = 0; spin < 2u * kFuseSpin; ++spin) {
         flag = __hip_atomic_load(&s_ready[slot], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
         if ((flag & ~kFuseNotSeeded) >= j + 1u) break;
-        flag = kFuseNotSeeded;
         __builtin_amdgcn_s_sleep(2);
+      }
+      const uint32_t batch = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(s_batch[j % kFuseNumbers])));
+      if (batch >= n_batches || (flag & ~kFuseNotSeeded) < j + 1u) break;  // (every wave's first task of the batch behind the last one)
+      if (r == 0) {
+        const uint32_t b = take_batch(j + 1u);
+        // slot (j + 1) % 3 last held batch j - 2: (j + 1) / 3 batches have used it, 64 loads each
+        const uint32_t slot1 = (j + 1u) % kFuseSlots, need = ((j + 1u) / kFuseSlots) * kFuseBatch;
+        bool free_ = b >= n_batches;  // (nothing to seed)
+        for (uint32_t spin = 0; spin < kFuseSpin && !free_; ++spin) {
+          free_ = __hip_atomic_load(&s_loaded[slot1], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) >= need;
+          if (!free_) __builtin_amdgcn_s_sleep(2);
+        }
+        if (free_ && b < n_batches) seed_batch(j + 1u, b);
+        else __hip_atomic_store(&s_ready[slot1], (free_ ? 0u : kFuseNotSeeded) | (j + 2u), __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
       }
       const uint32_t *pre = (flag & kFuseNotSeeded) ? nullptr : ring + (static_cast<size_t>(slot) * kFuseBatch + r) * kMtN;
       auto loaded = [&]() {
         if (lane == 0) __hip_atomic_fetch_add(&s_loaded[slot], 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
       };
-      const uint32_t o = (blockIdx.x + j * gridDim.x) * kFuseBatch + r;
+      const uint32_t o = batch * kFuseBatch + r;
       if (o < n_out) walk_row(o, pre, loaded);
       else loaded();
+    }
+    // (the last workgroup to take a batch behind the last one leaves the counter as it was found)
+    if (next != nullptr) {
+      __syncthreads();
+      if (threadIdx.x == 0 && atomicAdd(&next[1], 1u) == gridDim.x - 1u) next[0] = 0u, next[1] = 0u;
     }
   }
 }
@@ -217,7 +247,7 @@ constexpr int kColThreads = 256;
 template <typename T1, typename VT, int IN, int W>
 __global__ __launch_bounds__(kColThreads) void jitconn_colwalk_kernel(const VT *__restrict__ in,
                                                                       T1 *__restrict__ out, uint32_t n_out,
-                                                                      uint32_t n_in, uint32_t seed, double log_p,
+                                                                      uint32_t n_in, uint32_t seed, SkipParams skips,
                                                                       T1 wa, T1 wb) {
   constexpr int kWaves = kColThreads / kWave;
   constexpr int kWords = StreamLds<T1, W>::words;
@@ -256,7 +286,7 @@ __global__ __launch_bounds__(kColThreads) void jitconn_colwalk_kernel(const VT *
   for (uint32_t k = wave; k < count; k += kWaves) {
     const uint32_t col = s_col[k];
     const T1 val = s_val[k];
-    walk_stream<T1, W>(st, lane, seed + col, nullptr, n_out, log_p, wa, wb, [&](uint32_t idx, T1 w, bool valid) {
+    walk_stream<T1, W>(st, lane, seed + col, nullptr, n_out, skips, wa, wb, [&](uint32_t idx, T1 w, bool valid, bool) {
       if (valid) {
         T1 add;
         if (IN == kInDense) add = (W == kHomo) ? val : static_cast<T1>(w * val);
@@ -346,13 +376,14 @@ constexpr size_t kColBinBytesMax = static_cast<size_t>(3) << 30;  // bins of the
 // first batch of a workgroup is waited for; n_seeded is not used.
 template <typename T1, typename VT, int IN, int W, bool FUSED>
 __global__ __launch_bounds__(kColBinThreads, sizeof(T1) == 4 ? 8 : 4) void jitconn_colwalk_bins_kernel(
-    const VT *__restrict__ in, T1 *__restrict__ out, uint32_t n_out, uint32_t seed, double log_p, T1 wa, T1 wb,
+    const VT *__restrict__ in, T1 *__restrict__ out, uint32_t n_out, uint32_t seed, SkipParams skips, T1 wa, T1 wb,
     uint32_t first, uint32_t n_list_host, const uint32_t *__restrict__ n_list_dev,
     const uint32_t *__restrict__ list_col, const T1 *__restrict__ list_val, uint32_t *states,
     uint32_t n_seeded, uint32_t n_win, uint32_t shift, uint32_t cap, void *__restrict__ pairs, uint64_t n_pairs,
     uint32_t packed, uint32_t *__restrict__ counts) {
   constexpr int kWaves = kColBinThreads / kWave;
-  constexpr int kWords = StreamLds<T1, W>::words;
+  constexpr bool kShort = W == kNormal;  // (sixteen waves' states and queues within 64 KB of static LDS)
+  constexpr int kWords = StreamLds<T1, W, kShort>::words;
   __shared__ __attribute__((aligned(8))) uint32_t s_state[kWaves * kWords];
   __shared__ uint32_t s_cnt[kBinMaxWindows];
   __shared__ uint32_t s_task, s_ready[kFuseSlots], s_loaded[kFuseSlots];
@@ -387,7 +418,7 @@ __global__ __launch_bounds__(kColBinThreads, sizeof(T1) == 4 ? 8 : 4) void jitco
         return;
       }
     }
-    walk_stream<T1, W>(st, lane, seed + col, pre, n_out, log_p, wa, wb, [&](uint32_t idx, T1 w, bool valid) {
+    walk_stream<T1, W, false, kShort>(st, lane, seed + col, pre, n_out, skips, wa, wb, [&](uint32_t idx, T1 w, bool valid, bool) {
       const uint32_t b = idx >> shift;
       // The positions rise from lane to lane and the lanes that hold a synapse are the first ones of the
       // wave, so the lanes of a batch that meet in one window are neighbours (sixteen of them with
@@ -501,7 +532,7 @@ __global__ __launch_bounds__(kSeedThreads) void mt_seed_streams_kernel(uint32_t 
                                                                       uint32_t *__restrict__ states,
                                                                       const uint32_t *__restrict__ ids,
                                                                       const uint32_t *__restrict__ count_dev) {
-  __shared__ uint32_t s_tile[kSeedThreads / kWave][kMtSeedTileWords];
+  __shared__ __attribute__((aligned(8))) uint32_t s_tile[kSeedThreads / kWave][kMtSeedTileWords];
   const int lane = lane_id();
   const uint32_t wave = threadIdx.x / kWave;
   const uint32_t base = (blockIdx.x * (kSeedThreads / kWave) + wave) * kWave;  // first stream of this wave
@@ -585,6 +616,7 @@ void launch_rowwalk_impl(hipStream_t stream, const VT *in, T1 *out, uint32_t n_o
     int per_cu;
   };
   static thread_local Cached cached_for[2] = {{~size_t(0), 0, 0}, {~size_t(0), 0, 0}};
+  if (fused) lds_bytes += kFuseLdsWords * sizeof(uint32_t);
   Cached &cached = cached_for[fused];
   if (cached.lds_bytes != lds_bytes || cached.block != block) {
     if (lds_bytes > 64 * 1024)
@@ -604,8 +636,15 @@ void launch_rowwalk_impl(hipStream_t stream, const VT *in, T1 *out, uint32_t n_o
   unsigned needed = fused ? div_up(n_out, kFuseBatch) : div_up(n_out, nwaves);
   if (fused && needed > sc.ring_groups) needed = sc.ring_groups;
   const unsigned grid = needed < resident ? needed : resident;
-  hipLaunchKernelGGL(kernel, dim3(grid), dim3(block), lds_bytes, stream, in, out, n_out, n_in, seed, log_p, wa, wb, 0u,
-                     sc.rings());
+  // (more batches than workgroups: taken as they come; a capture that finds no counters shares them out evenly)
+  uint32_t *next = nullptr;
+  if (fused && grid < div_up(n_out, kFuseBatch)) {
+    next = stream_counters(stream);
+    if (next != nullptr) next += kWalkCounters;
+    else bpl_clear_error();
+  }
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(block), lds_bytes, stream, in, out, n_out, n_in, seed,
+                     make_skip_params(log_p), wa, wb, next, sc.rings());
 }
 
 // Event probes from an LDS bitmap when it fits beside the generator states, else from global memory.
@@ -647,14 +686,14 @@ void launch_rowwalk(hipStream_t stream, const VT *in, T1 *out, uint32_t n_out, u
   // An event bitmap that would leave room for fewer than two 16-wave workgroups per CU: two levels
   // instead, the exact bitmap packed into global memory and a coarse one made for LDS.  Wide event
   // types: the vector is packed to one bit per element once, instead of once per workgroup.
-  const bool two_level = kEvents && words * 4 > rowwalk_coarse_bytes<T1, W>();
+  const bool two_level = kEvents && words * 4 > rowwalk_coarse_bytes<T1, W>() && n_in <= 0xffffffffu - kRowwalkLead;
   const bool packed = kEvents && (two_level || sizeof(VT) > 1);
   uint32_t g = 0, off = 0, c_words = 0;
   size_t bitmap_ws = 0;
   if (two_level) {
-    g = coarse_shift(n_in, rowwalk_coarse_bytes<T1, W>());
-    off = coarse_offset_words(n_in);
-    c_words = (coarse_bits(n_in, g) + 31u) / 32u;
+    g = coarse_shift(n_in + kRowwalkLead, rowwalk_coarse_bytes<T1, W>());
+    off = coarse_offset_words(n_in + kRowwalkLead);
+    c_words = (coarse_bits(n_in + kRowwalkLead, g) + 31u) / 32u;
     bitmap_ws = (static_cast<size_t>(off) + c_words + 1) * sizeof(uint32_t);
   } else if (packed) {
     bitmap_ws = (words + 1) * sizeof(uint32_t);
@@ -668,11 +707,11 @@ void launch_rowwalk(hipStream_t stream, const VT *in, T1 *out, uint32_t n_out, u
   }
   if constexpr (kEvents) {
     if (uint32_t *bits = sc.bitmap()) {
-      pack_event_bitmap<VT>(stream, in, n_in, bits);
+      pack_event_bitmap<VT>(stream, in, n_in, bits, two_level ? kRowwalkLead / 32u : 0u);
       const PackedBits *pin = reinterpret_cast<const PackedBits *>(bits);
       if (two_level) {
         hipLaunchKernelGGL(coarsen_bitmap_kernel, dim3(div_up(c_words, 256)), dim3(256), 0, stream, bits,
-                           static_cast<uint32_t>(words), g, bits + off, c_words);
+                           static_cast<uint32_t>(words + kRowwalkLead / 32u), g, bits + off, c_words);
         const size_t state_bytes = StreamLds<T1, W>::words * 4;
         launch_rowwalk_impl<T1, PackedBits, IN, W, 2>(stream, pin, out, n_out, n_in, seed, log_p, wa, wb, 16,
                                                       static_cast<size_t>(c_words) * 4 + 16 * state_bytes, sc);
@@ -761,7 +800,8 @@ void launch_colwalk(hipStream_t stream, const VT *in, T1 *out, uint32_t n_out, u
           // the active columns, then one walk that seeds their generators as it goes
           hipLaunchKernelGGL((collect_active_columns_kernel<T1, VT>), dim3(div_up(n_in, kCollectCols)), dim3(1024), 0, stream,
                              in, n_in, list_count, list_col, list_val, counts, n_win * producers, out, n_out);
-          hipLaunchKernelGGL(walk, dim3(producers), dim3(kColBinThreads), 0, stream, in, out, n_out, seed, log_p, wa, wb,
+          hipLaunchKernelGGL(walk, dim3(producers), dim3(kColBinThreads), 0, stream, in, out, n_out, seed,
+                             make_skip_params(log_p), wa, wb,
                              0u, 0u, static_cast<const uint32_t *>(list_count), static_cast<const uint32_t *>(list_col),
                              static_cast<const T1 *>(list_val), states, 0u, n_win, shift, cap, pairs, n_pairs, packed ? 1u : 0u, counts);
         } else {
@@ -771,7 +811,8 @@ void launch_colwalk(hipStream_t stream, const VT *in, T1 *out, uint32_t n_out, u
           uint32_t in_bins = 0;
           for (uint32_t first = 0; first < n_in; first += kSeedChunk) {
             const uint32_t count = (n_in - first < kSeedChunk) ? n_in - first : kSeedChunk;
-            hipLaunchKernelGGL(walk, dim3(producers), dim3(kColBinThreads), 0, stream, in, out, n_out, seed, log_p, wa,
+            hipLaunchKernelGGL(walk, dim3(producers), dim3(kColBinThreads), 0, stream, in, out, n_out, seed,
+                               make_skip_params(log_p), wa,
                                wb, first, count, static_cast<const uint32_t *>(nullptr),
                                static_cast<const uint32_t *>(nullptr), static_cast<const T1 *>(nullptr), states, 0u,
                                n_win, shift, cap, pairs, n_pairs, packed ? 1u : 0u, counts);
@@ -801,7 +842,7 @@ void launch_colwalk(hipStream_t stream, const VT *in, T1 *out, uint32_t n_out, u
   }
   if (!out_cleared) fill_zero(stream, out, n_out);
   hipLaunchKernelGGL((jitconn_colwalk_kernel<T1, VT, IN, W>), dim3(div_up(n_in, kColThreads)), dim3(kColThreads), 0,
-                     stream, in, out, n_out, n_in, seed, log_p, wa, wb);
+                     stream, in, out, n_out, n_in, seed, make_skip_params(log_p), wa, wb);
 }
 
 // buffers = [input, out].  RAW_PROB: the descriptor's probability field holds conn_prob itself, as the
@@ -851,9 +892,8 @@ __device__ __forceinline__ uint64_t mix64(uint64_t z) {
   return z ^ (z >> 31);
 }
 
-__global__ __launch_bounds__(256) void check_skips_kernel(uint32_t seed, uint64_t n, int mode, double log_p,
+__global__ __launch_bounds__(256) void check_skips_kernel(uint32_t seed, uint64_t n, int mode, SkipParams sp,
                                                           unsigned long long *__restrict__ counts) {
-  const SkipParams sp = make_skip_params(log_p);
   unsigned long long differ = 0, untrusted = 0;
   for (uint64_t t = static_cast<uint64_t>(blockIdx.x) * 256u + threadIdx.x; t < n;
        t += static_cast<uint64_t>(gridDim.x) * 256u) {
@@ -861,18 +901,21 @@ __global__ __launch_bounds__(256) void check_skips_kernel(uint32_t seed, uint64_
     if (mode == 0) {
       bits = mix64(t + (static_cast<uint64_t>(seed) << 32));
     } else {
-      const double edge = exp(static_cast<double>(t / 64u + 1u) * log_p) * 0x1p64;
+      const double edge = exp(static_cast<double>(t / 64u + 1u) * sp.log_p) * 0x1p64;
       bits = (edge < 0x1p64 ? static_cast<uint64_t>(edge) : ~0ull) +
              static_cast<uint64_t>((static_cast<int64_t>(t % 64u) - 32) * 2048);
     }
     const uint32_t lo = static_cast<uint32_t>(bits), hi = static_cast<uint32_t>(bits >> 32);
-    bool safe;
-    const uint32_t fast = skip_fast(lo, hi, sp, safe);
+    uint64_t unsafe;
+    const uint64_t me = 1ull << lane_id();
+    const uint32_t fast = skip_fast(lo, hi, sp, unsafe);
     const uint32_t exact = skip_exact(lo, hi, sp);
-    if (!safe) ++untrusted;
+    if (unsafe & me) ++untrusted;
     else if (fast != exact) ++differ;
-    const uint32_t quick = skip_quick(hi, sp, safe);
-    if (sp.quick && safe && quick != exact) ++differ;
+    const uint32_t close = skip_close(lo, hi, sp, unsafe);
+    if (!(unsafe & me) && close != exact) ++differ;
+    const uint32_t quick = skip_quick(hi, sp, unsafe);
+    if (sp.quick && !(unsafe & me) && quick != exact) ++differ;
   }
   if (differ) atomicAdd(&counts[0], differ);
   if (untrusted) atomicAdd(&counts[1], untrusted);
@@ -914,7 +957,7 @@ extern "C" int bpl_selfcheck_jitconn_skips(bpl_stream_t stream, uint32_t seed, u
   }
   hipStream_t s = static_cast<hipStream_t>(stream);
   unsigned long long *c = reinterpret_cast<unsigned long long *>(counts);
-  hipLaunchKernelGGL(check_skips_kernel, dim3(2048), dim3(256), 0, s, seed, n_draws, near_boundaries ? 1 : 0, log_p, c);
+  hipLaunchKernelGGL(check_skips_kernel, dim3(2048), dim3(256), 0, s, seed, n_draws, near_boundaries ? 1 : 0, make_skip_params(log_p), c);
   hipLaunchKernelGGL(check_log2_kernel, dim3((1u << 23) / 256u), dim3(256), 0, s, c + 2, c);
   return check_launch("bpl_selfcheck_jitconn_skips") ? 0 : 1;
 }

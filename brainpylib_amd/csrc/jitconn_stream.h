@@ -45,10 +45,20 @@ struct NormalQueue {
   static_assert(spill <= kWave && 2 * drain <= 2 * kWave, "one lane per attempt and per position moved");
 };
 
-// LDS words one wave needs: the generator state and, for normal weights, the queue behind it.
+// Words a lane takes from the generator per batch, and how many lanes take some.
 template <typename T1, int W>
+struct StreamBatch {
+  static constexpr int K = W == kUniform ? WeightWords<T1>::value + 2 : 2;
+  static constexpr int NL = K <= 3 ? kWave : 56;  // K * NL <= 227
+};
+
+// LDS words one wave needs: the generator state and, for normal weights, the queue behind it.  kShort: the state with the
+// least mirror (mt_wave.h).
+template <typename T1, int W, bool kShort = false>
 struct StreamLds {
-  static constexpr int words = kMtStateWords + (W == kNormal ? NormalQueue<T1>::words : 0);
+  static constexpr int mirror = kShort ? kMtLeastMirror : StreamBatch<T1, W>::K * StreamBatch<T1, W>::NL;
+  static constexpr int state_words = kMtN + mirror;
+  static constexpr int words = state_words + (W == kNormal ? NormalQueue<T1>::words : 0);
   static_assert(words % 2 == 0, "the queue of the next wave stays aligned");
 };
 
@@ -146,9 +156,10 @@ __device__ __forceinline__ uint32_t lanes_below(uint64_t mask, uint32_t base) {
                                    __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(mask), base));
 }
 
-// Walks stream std::mt19937{stream_seed} over [0, n): calls f(index, weight, valid) once per
+// Walks stream std::mt19937{stream_seed} over [0, n): calls f(index, weight, valid, partial) once per
 // batch with the whole wave converged; `valid` marks the lanes that hold a synapse of the row: the first
-// lanes of the wave, their indices rising from lane to lane.  Normal weights come two at a time: synapses
+// lanes of the wave, their indices rising from lane to lane; all of them unless `partial` (wave uniform); the others
+// get index 0.  Normal weights come two at a time: synapses
 // 2 l and 2 l + 1 of a group are lane l's.  f is called for the first and then for the second ones, or, if
 // it can be called so, f(index, weight, valid, index, weight, valid) for both.
 //
@@ -158,58 +169,81 @@ __device__ __forceinline__ uint32_t lanes_below(uint64_t mask, uint32_t base) {
 // kQuick: skips are first tried on the upper words alone (skip_quick).
 //
 // `loaded()` is called once, when the generator state is in LDS and `pre` is no longer read.
+//
+// `start`: what the indices are counted from (the walk ends at `n`, counted alike).
 struct NoLoadHook {
   __device__ __forceinline__ void operator()() const {}
 };
-template <typename T1, int W, bool kQuick = false, typename F, typename L = NoLoadHook>
+template <typename T1, int W, bool kQuick = false, bool kShort = false, typename F, typename L = NoLoadHook>
 __device__ __forceinline__ void walk_stream(uint32_t *st, int lane, uint32_t stream_seed, const uint32_t *pre,
-                                            uint32_t n, double log_p_, T1 wa, T1 wb, F &&f, L &&loaded = L()) {
-  const SkipParams log_p = make_skip_params(log_p_);
-  if (pre != nullptr) mt_load(st, pre, lane);
-  else mt_seed(st, stream_seed, lane);
+                                            uint32_t n, const SkipParams &sp, T1 wa, T1 wb, F &&f, L &&loaded = L(),
+                                            uint32_t start = 0u) {
+  constexpr int K = StreamBatch<T1, W>::K, NL = StreamBatch<T1, W>::NL, kMirror = StreamLds<T1, W, kShort>::mirror;
+  if (pre != nullptr) mt_load<kMirror>(st, pre, lane);
+  else mt_seed<kMirror>(st, stream_seed, lane);
   loaded();
   uint32_t pos = 0;
-  // With every skip >= 1 a row ends within n/64 + 1 batches; the cap only guards against a
-  // generator state that yields zero skips forever (log_p is validated on the host).
-  const uint32_t max_batches = n / 16u + 1024u;
+  LdsWord *const base = mt_base<K, NL, kMirror>(st, lane);
+  // (Every skip is at least 1 (log_p is validated on the host), but for U = 0; a walk that does not get on all the same ends.)
+  // A batch's last position says on the scalar unit whether the row goes on behind it, unless 64 skips of up to 64 *
+  // |inv_log2| could lead around 2^32: then every batch is looked at lane by lane.
+  uint32_t whole_below = !sp.narrow || n > 0xf0000000u ? 0u : n;
+  asm volatile("" : "+s"(whole_below));  // (one comparison per batch instead of three)
   if constexpr (W == kHomo) {
     // stream: K K K ...   synapse s sits at K_0 + ... + K_s
-    uint32_t carry = 0;
-    for (uint32_t b = 0; b < max_batches; ++b) {
-      uint32_t w[2] = {1u, 1u};
-      mt_generate<2, kQuick ? 0 : -1>(st, pos, lane, kWave, w);
-      const uint32_t skip = skip_from_words<kQuick, !kQuick>(w[0], w[1], log_p);
-      const uint32_t idx = carry + wave_inclusive_scan_u32(skip);
-      // (the positions rise from lane to lane: the lanes of the row are exactly those below n)
-      const bool over = idx >= n;
-      const uint64_t done = __ballot(over);
-      f(idx, T1(1), !over);
-      if (done) break;
+    uint32_t carry = start;
+    for (;;) {
+      uint32_t w[K];
+      mt_generate<K, NL, kMirror, kQuick ? 0 : -1>(base, pos, lane, w);
+      uint32_t incl = wave_inclusive_scan_u32(skip_from_words<kQuick, !kQuick>(w[0], w[1], sp));
+      asm volatile("" : "+v"(incl));  // (else the last step of the scan and this addition become three instructions)
+      uint32_t idx = carry + incl;
+      const uint32_t before = carry;
       carry = __builtin_amdgcn_readlane(idx, kWave - 1);
+      const bool partial = carry >= whole_below;
+      bool valid = true;
+      uint64_t done = 0;
+      if (partial) {
+        // (the positions rise from lane to lane: the lanes of the row are those below the first one at or past n)
+        done = __builtin_amdgcn_ballot_w64(idx >= n);
+        valid = done == 0 || lane < static_cast<int>(__builtin_ctzll(done));
+        idx = valid ? idx : 0u;
+        asm volatile("" : "+v"(idx));  // (a branch, not a select in every batch)
+      }
+      f(idx, T1(1), valid, partial);
+      if (done || carry == before) break;
     }
   } else if constexpr (W == kUniform) {
     // stream: K  (w K) (w K) ...   synapse s sits at K_0 + ... + K_s, its weight precedes K_{s+1}
     constexpr int WW = WeightWords<T1>::value;
-    constexpr int K = WW + 2;
-    constexpr int NL = (K == 3) ? 64 : 56;  // K * NL <= 227
     uint32_t w0[2] = {1u, 1u};
-    mt_generate<2>(st, pos, lane, 1, w0);
-    uint32_t carry = __builtin_amdgcn_readfirstlane(skip_from_words<false, true>(w0[0], w0[1], log_p, 1ull));
-    for (uint32_t b = 0; b < max_batches; ++b) {
+    mt_generate<2, 1, kMirror>(mt_base<2, 1, kMirror>(st, lane), pos, lane, w0);
+    uint32_t carry = start + __builtin_amdgcn_readfirstlane(skip_from_words<false, true>(w0[0], w0[1], sp, 1ull));
+    for (;;) {
       uint32_t w[K];
 #pragma unroll
       for (int i = 0; i < K; ++i) w[i] = 1u;
-      mt_generate<K, kQuick ? WW : -1>(st, pos, lane, NL, w);
+      mt_generate<K, NL, kMirror, kQuick ? WW : -1>(base, pos, lane, w);
       const T1 weight = uniform_weight(w, wa, wb);
-      uint32_t skip = skip_from_words<kQuick, !kQuick>(w[WW], w[WW + 1], log_p, ~0ull >> (kWave - NL));
-      if (lane >= NL) skip = 0;
-      const uint32_t incl = wave_inclusive_scan_u32(skip);
-      const uint32_t idx = carry + incl - skip;
-      const uint64_t done = __ballot(lane < NL && idx >= n);
-      const int nvalid = done ? (__ffsll(static_cast<unsigned long long>(done)) - 1) : NL;
-      f(idx, weight, lane < nvalid);
-      if (done) break;
-      carry += __builtin_amdgcn_readlane(incl, kWave - 1);
+      uint32_t skip = skip_from_words<kQuick, !kQuick>(w[WW], w[WW + 1], sp, ~0ull >> (kWave - NL));
+      if (NL < kWave && lane >= NL) skip = 0;
+      uint32_t incl = wave_inclusive_scan_u32(skip);
+      asm volatile("" : "+v"(incl));
+      const uint32_t behind = carry + incl;
+      uint32_t idx = behind - skip;
+      const uint32_t before = carry;
+      carry = __builtin_amdgcn_readlane(behind, kWave - 1);
+      const bool partial = NL < kWave || carry >= whole_below;
+      bool valid = true;
+      uint64_t done = 0;
+      if (partial) {
+        done = __builtin_amdgcn_ballot_w64(idx >= n) & (~0ull >> (kWave - NL));
+        valid = lane < (done ? static_cast<int>(__builtin_ctzll(done)) : NL);
+        idx = valid ? idx : 0u;
+        asm volatile("" : "+v"(idx));
+      }
+      f(idx, weight, valid, partial);
+      if (done || carry == before) break;
     }
   } else {
     // float: the stream in 2-word units is  K  (A..A K) (K) (A..A K) (K) ...   A = polar attempt (x word, y
@@ -220,17 +254,19 @@ __device__ __forceinline__ void walk_stream(uint32_t *st, int lane, uint32_t str
     // and 2 a + 1 of the stream so belong to its accepted attempt a.
     using Q = NormalQueue<T1>;
     constexpr bool kWide = sizeof(T1) == 8;
-    T1 *const q_attempt = reinterpret_cast<T1 *>(st + kMtStateWords);           // x, y of the attempts queued
-    uint32_t *const q_pos = st + kMtStateWords + Q::attempts * (2 * sizeof(T1) / 4);  // their synapses' positions
+    uint32_t *const queue = st + StreamLds<T1, W, kShort>::state_words;
+    T1 *const q_attempt = reinterpret_cast<T1 *>(queue);              // x, y of the attempts queued
+    uint32_t *const q_pos = queue + Q::attempts * (2 * sizeof(T1) / 4);  // their synapses' positions
     uint32_t n_attempt = 0, n_pos = 0;
     uint32_t w0[2] = {1u, 1u};
-    mt_generate<2>(st, pos, lane, 1, w0);
-    uint32_t carry = __builtin_amdgcn_readfirstlane(skip_from_words<false, true>(w0[0], w0[1], log_p, 1ull));
+    mt_generate<2, 1, kMirror>(mt_base<2, 1, kMirror>(st, lane), pos, lane, w0);
+    uint32_t carry = start + __builtin_amdgcn_readfirstlane(skip_from_words<false, true>(w0[0], w0[1], sp, 1ull));
     uint32_t entered = 0;
     double prev_v63 = 0.0;
+    const uint32_t max_batches = n / 16u + 1024u;
     for (uint32_t b = 0; b < max_batches; ++b) {
       uint32_t w[2] = {1u, 1u};
-      mt_generate<2>(st, pos, lane, kWave, w);
+      mt_generate<2, kWave, kMirror>(base, pos, lane, w);
       T1 x, y;
       bool ok;
       if constexpr (!kWide) {
@@ -255,7 +291,7 @@ __device__ __forceinline__ void walk_stream(uint32_t *st, int lane, uint32_t str
         skips = __ballot(state >= 2u);
       }
       const bool is_k = __builtin_amdgcn_inverse_ballot_w64(skips);
-      const uint32_t skip_any = skip_from_words<false, true>(w[0], w[1], log_p, skips);  // wave-converged call
+      const uint32_t skip_any = skip_from_words<false, true>(w[0], w[1], sp, skips);  // wave-converged call
       const uint32_t skip = is_k ? skip_any : 0u;
       const uint32_t incl = wave_inclusive_scan_u32(skip);
       const uint32_t idx = carry + incl - skip;
@@ -286,7 +322,7 @@ __device__ __forceinline__ void walk_stream(uint32_t *st, int lane, uint32_t str
           f(idx0, first, valid0, idx1, second, valid1);
         } else {
 #pragma unroll kWide ? 1 : 2
-          for (int h = 0; h < 2; ++h) f(h ? idx1 : idx0, h ? second : first, h ? valid1 : valid0);
+          for (int h = 0; h < 2; ++h) f(h ? idx1 : idx0, h ? second : first, h ? valid1 : valid0, true);
         }
         if (n_pos <= 2u * Q::drain && done) break;
         // what the group left goes to the front
