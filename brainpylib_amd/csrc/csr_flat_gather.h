@@ -14,11 +14,13 @@ constexpr uint32_t kFlatMaxNnz = 0xffffffffu - 8192u;
 // y = A x, walked flat: every wave owns a contiguous range of the nonzeros and tells the rows apart through
 // windows of indptr in LDS.  For matrices with min_mean <= nnz / n_row and nnz <= kFlatMaxNnz; for others the kernels
 // return at once and write nothing (the mean is known on the device only, so the caller enqueues its kernel
-// for short rows behind this one).  x must have at least one element.  Takes 24 bytes of the stream's scratch
+// for short rows behind this one).  x must have at least one element.
+// nnz: the number of nonzeros as far as the caller knows it (0: not), for the choice of a kernel alone.  Takes 24 bytes of the stream's scratch
 // memory per wave of its launch.  false: no scratch memory, or the launch failed (error recorded).
 template <typename F>
 bool csr_flat_gather(const char *target, hipStream_t stream, const F *data, bool heter, const uint32_t *indices,
-                     const uint32_t *indptr, const F *x, F *y, uint32_t n_row, uint32_t n_col, uint32_t min_mean);
+                     const uint32_t *indptr, const F *x, F *y, uint32_t n_row, uint32_t n_col, uint32_t nnz,
+                     uint32_t min_mean);
 
 // Whether the walk keeps a part of x in LDS (one of up to four times what fits).
 template <typename F>

@@ -34,9 +34,14 @@
 // must move; 3e7 nonzeros, products alone, x of 120,011 floats: 122 us, bound by the lines that the gathers move out
 // of the L2s (2.7 GB, 54 us without those gathers).  An expanded list of the rows, two gathers and a product as
 // passes of their own took 215 and 850 us.
-// STAGED: one workgroup of 1,024 threads per CU keeps the first elements of x (139 to 151 KB) in LDS and gathers only the
+// kStaged: one workgroup of 1,024 threads per CU keeps the first elements of x (139 to 151 KB) in LDS and gathers only the
 // rest from L2 (flat_stages()).  Every gather it spares counts: with 147 instead of 138 KB 1,000,000 x 50,000 with 100 per row
 // takes 221 instead of 234 us, 200,000 x 50,000 56 instead of 58.
+// kSwept: x passes through the LDS of every CU in windows of 147 KB, once per round; a round is what the CU's 16 waves hold
+// in registers, 24 to 48 nonzeros a lane.  A CU then requests x in whole lines, 3,750 of them for 120,000 floats and 24,576
+// nonzeros, instead of a line per nonzero.  The rounds' other traffic is under way meanwhile: a step's registers are
+// filled with the next round's indices as soon as its rows are done.  Bound by what of a round does not overlap: staging
+// (1.5 us a window), the test of every place against every window (three instructions), the rows (flat_vector() has the times).
 #include <type_traits>
 
 #include "common.h"
@@ -52,9 +57,10 @@ typedef float f32x4 __attribute__((ext_vector_type(4), aligned(4)));
 typedef double f64x2 __attribute__((ext_vector_type(2), aligned(8)));
 
 enum : int { kFlatSums = 1, kFlatProducts = 2 };
-// 16 waves per CU either way: two workgroups, or one that has the LDS to itself (STAGED)
-constexpr int flat_threads(bool staged) { return staged ? 1024 : 512; }
-constexpr unsigned flat_per_cu(bool staged) { return staged ? 1u : 2u; }
+enum class FlatVector { kL2, kStaged, kSwept };
+// 16 waves per CU either way: two workgroups, or one that has the LDS to itself
+constexpr int flat_threads(FlatVector from) { return from == FlatVector::kL2 ? 512 : 1024; }
+constexpr unsigned flat_per_cu(FlatVector from) { return from == FlatVector::kL2 ? 2u : 1u; }
 constexpr uint32_t kFlatRows = 64;  // rows of an indptr window (one per lane)
 // bytes of x in LDS: what the windows, accumulators and v's elements of the 16 waves leave (147 KB beside the sums, 139 to
 // 143 beside both)
@@ -65,19 +71,85 @@ constexpr uint32_t flat_staged_bytes() {
   return (160u * 1024u - 16u * (kFlatRows + 2u) * 4u - sums - v - 64u) / 1024u * 1024u;
 }
 constexpr uint32_t kNoRow = 0xffffffffu;
+enum : int { kStepIndices = 1, kStepWeights = 2 };  // what is loaded of a step
 
 // quads per lane and step, as many as 128 registers hold (with sums and products of floats at once two as well: the
 // elements of x and the weights both live until the rows are known)
-template <typename F, int OUT>
+template <typename F, int OUT, FlatVector FROM>
 struct FlatQuads {
-  static constexpr int value = sizeof(F) == 4 && OUT != (kFlatSums | kFlatProducts) ? 4 : 2;
+  static constexpr int value = sizeof(F) == 4 && OUT != (kFlatSums | kFlatProducts) && FROM != FlatVector::kSwept ? 4 : 2;
 };
 
 // The least a wave takes, in nonzeros and rows: a wavefront of quads.  (The plain sums of x in L2 whole steps: a gather
 // costs the address unit the same however many of its lanes hold a nonzero.)
-template <typename F, int OUT, bool STAGED>
+template <typename F, int OUT, FlatVector FROM>
 constexpr uint32_t flat_min_share() {
-  return 4u * kWave * ((OUT == kFlatSums && !STAGED) ? FlatQuads<F, OUT>::value : 1);
+  return 4u * kWave * ((OUT == kFlatSums && FROM == FlatVector::kL2) ? FlatQuads<F, OUT, FROM>::value : 1);
+}
+
+// kSwept: steps whose nonzeros a wave keeps in registers while the windows of x pass by, as many as 128 registers hold.
+template <typename F, bool HETER, int OUT>
+struct FlatHeld {
+  static constexpr int value = (OUT == kFlatProducts ? 6 : HETER && sizeof(F) == 4 ? 3 : 4) /
+                               static_cast<int>(sizeof(F) / 4);
+};
+
+// (Sums and products of doubles at once: the registers hold one step, and no size pays for the windows.)
+template <typename F, int OUT>
+constexpr bool flat_sweeps() { return !(sizeof(F) == 8 && OUT == (kFlatSums | kFlatProducts)); }
+
+// kSwept: a nonzero's register holds where its element of x lies until a window brings the element itself.  The place is
+// written as a NaN with its sign set, one that no element has in LDS: those are stored as the NaN without a payload.
+__device__ __forceinline__ float flat_place(float, uint32_t c) { return __uint_as_float(0xff800004u + 4u * c); }
+__device__ __forceinline__ double flat_place(double, uint32_t c) {
+  return __hiloint2double(static_cast<int>(0xfff00001u + c), 0);
+}
+__device__ __forceinline__ float flat_no_place(float v) {
+  return __float_as_uint(v) > 0xff800000u ? __uint_as_float(0x7fc00000u) : v;
+}
+__device__ __forceinline__ double flat_no_place(double v) {
+  return static_cast<uint32_t>(__double2hiint(v)) > 0xfff00000u ? __hiloint2double(0x7ff80000, 0) : v;
+}
+// v = the element whose place it holds, if that lies among the n in LDS, which begin with element `first`.  (origin: kept
+// in one scalar register, so that a nonzero costs a subtraction, a comparison and a read of the lanes concerned.)
+typedef __attribute__((address_space(3))) const unsigned char *flat_lds;
+__device__ __forceinline__ uint32_t flat_origin(float, uint32_t first) { return 0xff800004u + 4u * first; }
+__device__ __forceinline__ uint32_t flat_origin(double, uint32_t first) { return 0xfff00001u + first; }
+__device__ __forceinline__ void flat_take(float &v, flat_lds window, uint32_t origin, uint32_t bytes) {
+  const uint32_t at = __float_as_uint(v) - origin;
+  if (at < bytes) v = *reinterpret_cast<__attribute__((address_space(3))) const float *>(window + at);
+}
+__device__ __forceinline__ void flat_take(double &v, flat_lds window, uint32_t origin, uint32_t bytes) {
+  const uint32_t at = static_cast<uint32_t>(__double2hiint(v)) - origin;
+  if (at < bytes / 8u) v = *reinterpret_cast<__attribute__((address_space(3))) const double *>(window + 8u * at);
+}
+constexpr uint32_t kFlatMostPlaces = 1u << 20;  // (of both types' NaNs fewer than that are taken)
+
+// The n elements of x from `first` on to LDS, eight 16-byte loads of every thread in flight.
+template <typename F>
+__device__ __forceinline__ void flat_stage_window(F *to, const F *__restrict__ x, uint32_t n) {
+  constexpr uint32_t kPer = 16 / sizeof(F), kUnroll = 3;
+  typedef F piece __attribute__((ext_vector_type(kPer), aligned(sizeof(F))));
+  typedef F lds_piece __attribute__((ext_vector_type(kPer)));
+  const uint32_t pieces = n / kPer;
+  for (uint32_t i0 = threadIdx.x; i0 < pieces; i0 += kUnroll * blockDim.x) {
+    piece v[kUnroll];
+#pragma unroll
+    for (uint32_t k = 0; k < kUnroll; ++k) {
+      const uint32_t i = i0 + k * blockDim.x;
+      v[k] = reinterpret_cast<const piece *>(x)[i < pieces ? i : pieces - 1u];
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < kUnroll; ++k) {
+      const uint32_t i = i0 + k * blockDim.x;
+      lds_piece t;
+#pragma unroll
+      for (uint32_t j = 0; j < kPer; ++j) t[j] = flat_no_place(v[k][j]);
+      if (i < pieces) reinterpret_cast<lds_piece *>(to)[i] = t;
+    }
+  }
+  const uint32_t rest = pieces * kPer + threadIdx.x;
+  if (rest < n) to[rest] = flat_no_place(x[rest]);
 }
 
 // Four consecutive indices / weights, whole quad q of the array.
@@ -158,15 +230,16 @@ __device__ __forceinline__ void flat_split(const uint32_t *__restrict__ indptr, 
   }
 }
 
-template <typename F, bool HETER, int OUT, bool STAGED>
-__global__ __launch_bounds__(flat_threads(STAGED), 4) void csr_flat_gather_kernel(
+template <typename F, bool HETER, int OUT, FlatVector FROM>
+__global__ __launch_bounds__(flat_threads(FROM), 4) void csr_flat_gather_kernel(
     const F *__restrict__ data, const uint32_t *__restrict__ indices, const uint32_t *__restrict__ indptr,
     const F *__restrict__ x, F *__restrict__ y, uint32_t n_row, uint32_t n_col, uint32_t min_mean,
     double *__restrict__ head, double *__restrict__ tail, uint32_t *__restrict__ tail_row, uint32_t *__restrict__ range,
     const F *__restrict__ v, F *__restrict__ products, uint32_t n_products) {
-  constexpr int U = FlatQuads<F, OUT>::value;
+  constexpr int U = FlatQuads<F, OUT, FROM>::value;
   constexpr uint32_t kStepQuads = U * kWave;
-  constexpr int kFlatWaves = flat_threads(STAGED) / kWave;
+  constexpr int kFlatWaves = flat_threads(FROM) / kWave;
+  constexpr bool kStaged = FROM == FlatVector::kStaged, kSwept = FROM == FlatVector::kSwept;
   constexpr bool kSums = (OUT & kFlatSums) != 0, kProducts = (OUT & kFlatProducts) != 0;
   constexpr bool kWeights = kSums && HETER;  // (the products of v and x alone do not need them)
   extern __shared__ __attribute__((aligned(16))) unsigned char s_staged[];
@@ -186,26 +259,28 @@ __global__ __launch_bounds__(flat_threads(STAGED), 4) void csr_flat_gather_kerne
   double *s_sum = s_sum_all[kSums ? wv : 0];
   F *s_v = s_v_all[kProducts ? wv : 0];
   F *s_x = reinterpret_cast<F *>(s_staged);
-  uint32_t staged = 0;
-  if constexpr (STAGED) {
-    constexpr uint32_t kFits = flat_staged_bytes<F, OUT>() / sizeof(F);
-    staged = n_col < kFits ? n_col : kFits;
+  constexpr uint32_t kFits = flat_staged_bytes<F, OUT>() / sizeof(F);  // elements of x in LDS
+  const uint32_t staged = n_col < kFits ? n_col : kFits;       // (kStaged)
+  if constexpr (kStaged) {
     copy_to_lds(s_x, x, staged);
     __syncthreads();
   }
   const uint32_t waves = gridDim.x * kFlatWaves, w = blockIdx.x * kFlatWaves + wv;
   // the wave owns the nonzeros [begin, end) and stores the rows [r, row_end), but for one that began before `begin`
   uint32_t share = nnz / waves + kFlatRowWeight * (n_row / waves + 1u) + 1u;
-  if (share < flat_min_share<F, OUT, STAGED>()) share = flat_min_share<F, OUT, STAGED>();
+  if (share < flat_min_share<F, OUT, FROM>()) share = flat_min_share<F, OUT, FROM>();
   const uint64_t diag[2] = {static_cast<uint64_t>(w) * share, (static_cast<uint64_t>(w) + 1u) * share};
   uint32_t split_row[2], split_pos[2];
-  if (diag[0] >= flat_list(n_row, nnz)) {
+  const bool idle = diag[0] >= flat_list(n_row, nnz);
+  if (idle) {
     if (kSums && lane == 0) head[w] = 0.0, tail[w] = 0.0, tail_row[w] = kNoRow, range[w] = nnz;
-    return;
+    if constexpr (!kSwept) return;
+    split_row[0] = split_row[1] = n_row, split_pos[0] = split_pos[1] = nnz;  // (it helps to bring the windows)
+  } else {
+    flat_split(indptr, n_row, nnz, diag, lane, split_row, split_pos);
   }
-  flat_split(indptr, n_row, nnz, diag, lane, split_row, split_pos);
   const uint32_t begin = split_pos[0], end = split_pos[1], row_end = split_row[1];
-  if (kSums && lane == 0) head[w] = 0.0, tail[w] = 0.0, tail_row[w] = kNoRow, range[w] = begin;
+  if (kSums && !idle && lane == 0) head[w] = 0.0, tail[w] = 0.0, tail_row[w] = kNoRow, range[w] = begin;
   const F w_homo = (HETER || !kSums) ? F(0) : data[0];
 
   // Invariant at the start of a step [s0, s1): r is the first row whose end is not behind the wave; s_sum[0] holds what
@@ -224,14 +299,22 @@ __global__ __launch_bounds__(flat_threads(STAGED), 4) void csr_flat_gather_kerne
   // three nonzeros behind it are read where they are used.
   constexpr uint32_t kStep = 4u * kStepQuads;
   const uint32_t whole = nnz / 4u;
-  auto load_streams = [&](uint32_t s0, u32x4 (&ci)[U], F (&cd)[U][4]) {  // lane l: quads s0 / 4 + l, + 64, ...
-    if (s0 >= end || whole == 0) return;
+  auto load_step = [&](uint32_t s0, auto which, u32x4 (&ci)[U], F (&cd)[U][4]) {  // lane l: quads s0 / 4 + l, + 64, ...
+    constexpr int kWhich = decltype(which)::value;
+    if (s0 >= end || whole == 0) {
+      // (what is not loaded is not kept either: its registers are free)
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const uint32_t q = s0 / 4u + static_cast<uint32_t>(u) * kWave + lane;
-      ci[u] = flat_index_quad(indices, q < whole ? q : whole - 1u);
+      for (int u = 0; kSwept && (kWhich & kStepIndices) && u < U; ++u) ci[u] = u32x4{};
+      return;
     }
-    if constexpr (kWeights) {
+    if constexpr ((kWhich & kStepIndices) != 0) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const uint32_t q = s0 / 4u + static_cast<uint32_t>(u) * kWave + lane;
+        ci[u] = flat_index_quad(indices, q < whole ? q : whole - 1u);
+      }
+    }
+    if constexpr (kWeights && (kWhich & kStepWeights) != 0) {
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const uint32_t q = s0 / 4u + static_cast<uint32_t>(u) * kWave + lane;
@@ -239,92 +322,49 @@ __global__ __launch_bounds__(flat_threads(STAGED), 4) void csr_flat_gather_kerne
       }
     }
   };
-  u32x4 ci[U] = {};
-  F cd[U][4] = {};
-  load_streams(begin & ~3u, ci, cd);
-  // (a range without nonzeros has one step, for its rows)
-  for (uint32_t s0 = begin & ~3u;; s0 += kStep) {
-    const uint32_t s1 = (end - s0 > kStep) ? s0 + kStep : end;
-    uint32_t ptr_lane, ptr_last;
-    F v_lane = F(0);
-    auto load_window = [&]() {
-      const uint64_t k = static_cast<uint64_t>(r) + lane;
-      if constexpr (kProducts) v_lane = k < n_row ? v[k] : F(0);
-      ptr_lane = k <= n_row ? indptr[k] : 0xffffffffu;
-      // (a load of the vector unit: one of the scalar unit would be waited for together with every LDS read)
-      uint32_t last = r + kFlatRows;
-      asm volatile("" : "+v"(last));
-      ptr_last = static_cast<uint64_t>(r) + kFlatRows <= n_row ? indptr[last] : 0xffffffffu;
-    };
-    load_window();
-    if (s1 > 4u * whole) {  // (the array's last one to three nonzeros)
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        if (s0 / 4u + static_cast<uint32_t>(u) * kWave + lane != whole) continue;
-        const uint32_t p0 = 4u * whole;
-        ci[u] = u32x4{indices[p0], p0 + 1u < nnz ? indices[p0 + 1u] : 0u, p0 + 2u < nnz ? indices[p0 + 2u] : 0u, 0u};
-        if constexpr (kWeights) {
-          cd[u][0] = data[p0];
-          if (p0 + 1u < nnz) cd[u][1] = data[p0 + 1u];
-          if (p0 + 2u < nnz) cd[u][2] = data[p0 + 2u];
-        }
-      }
-    }
-    F prod[U][4];  // (the vector's elements first, then the products: in F, as the reference forms them)
-    auto column = [&](int u, int t) {  // (beyond the step: element 0, unused)
-      const uint32_t p = 4u * (s0 / 4u + static_cast<uint32_t>(u) * kWave + lane) + static_cast<uint32_t>(t);
-      return p < s1 ? ci[u][t] : 0u;
-    };
-    if constexpr (STAGED) {
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          const uint32_t c = column(u, t);
-          prod[u][t] = s_x[c < staged ? c : 0u];
-        }
-      }
-      if (staged < n_col) {  // (uniform)
-        // (all LDS reads first: without the empty statements each would be moved into the branch around the load)
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-#pragma unroll
-          for (int t = 0; t < 4; ++t) asm volatile("" : "+v"(prod[u][t]));
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-#pragma unroll
-          for (int t = 0; t < 4; ++t) {
-            const uint32_t c = column(u, t);
-            if (c >= staged) prod[u][t] = x[c];
-          }
-        }
-      }
-    } else {
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-#pragma unroll
-        for (int t = 0; t < 4; ++t) prod[u][t] = x[column(u, t)];
-      }
-    }
-    F cw[U][4];
+  uint32_t ptr_lane, ptr_last;
+  F v_lane = F(0);
+  auto load_window = [&]() {
+    const uint64_t k = static_cast<uint64_t>(r) + lane;
+    if constexpr (kProducts) v_lane = k < n_row ? v[k] : F(0);
+    ptr_lane = k <= n_row ? indptr[k] : 0xffffffffu;
+    // (a load of the vector unit: one of the scalar unit would be waited for together with every LDS read)
+    uint32_t last = r + kFlatRows;
+    asm volatile("" : "+v"(last));
+    ptr_last = static_cast<uint64_t>(r) + kFlatRows <= n_row ? indptr[last] : 0xffffffffu;
+  };
+  // The window's loads are waited for here, where the number of loads behind them is known: at the head of the loop over the
+  // windows the compiler waits for every load that either way in may have left.
+  auto await_window = [&]() {
+    if constexpr (FROM == FlatVector::kL2) return;
+    asm volatile("" : "+v"(ptr_lane), "+v"(ptr_last));
+    if constexpr (kProducts) asm volatile("" : "+v"(v_lane));
+  };
+  // The array's last one to three nonzeros, where the step holds them.
+  auto load_last = [&](uint32_t s0, auto which, u32x4 (&ci)[U], F (&cd)[U][4]) {
+    constexpr int kWhich = decltype(which)::value;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-#pragma unroll
-      for (int t = 0; t < 4; ++t) cw[u][t] = kWeights ? cd[u][t] : w_homo;
-    }
-    load_streams(s1, ci, cd);  // (a step at or beyond the end of the range loads nothing)
-    if constexpr (!kProducts) {
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-#pragma unroll
-        for (int t = 0; t < 4; ++t) prod[u][t] = static_cast<F>(prod[u][t] * cw[u][t]);
+      if (s0 / 4u + static_cast<uint32_t>(u) * kWave + lane != whole) continue;
+      const uint32_t p0 = 4u * whole;
+      if constexpr ((kWhich & kStepIndices) != 0)
+        ci[u] = u32x4{indices[p0], p0 + 1u < nnz ? indices[p0 + 1u] : 0u, p0 + 2u < nnz ? indices[p0 + 2u] : 0u, 0u};
+      if constexpr (kWeights && (kWhich & kStepWeights) != 0) {
+        cd[u][0] = data[p0];
+        if (p0 + 1u < nnz) cd[u][1] = data[p0 + 1u];
+        if (p0 + 2u < nnz) cd[u][2] = data[p0 + 2u];
       }
     }
-    // (with products the elements of x are kept: this is the addend of the row's sum)
+  };
+  using Indices = std::integral_constant<int, kStepIndices>;
+  using Weights = std::integral_constant<int, kStepWeights>;
+  using Both = std::integral_constant<int, kStepIndices | kStepWeights>;
+  // The rows of the step [s0, s1).  prod: its products, with products to store (kProducts) the elements of x; cw: its weights.
+  auto walk_rows = [&](uint32_t s0, uint32_t s1, const F (&prod)[U][4], const F (&cw)[U][4]) {
     auto addend = [&](int u, int t) {
       return static_cast<double>(kProducts ? static_cast<F>(prod[u][t] * cw[u][t]) : prod[u][t]);
     };
+    await_window();
     // windows of 64 rows from r on, until one reaches beyond the step
     for (;;) {
       s_ptr[lane] = ptr_lane;
@@ -425,9 +465,163 @@ __global__ __launch_bounds__(flat_threads(STAGED), 4) void csr_flat_gather_kerne
         break;
       }
       load_window();
+      await_window();
     }
     __builtin_amdgcn_wave_barrier();
-    if (s1 == end) break;
+  };
+  auto multiply = [&](F (&prod)[U][4], const F (&cw)[U][4]) {
+    if constexpr (!kProducts) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) prod[u][t] = static_cast<F>(prod[u][t] * (kWeights ? cw[u][t] : w_homo));
+      }
+    }
+  };
+  if constexpr (!kSwept) {
+    u32x4 ci[U] = {};
+    F cd[U][4] = {};
+    load_step(begin & ~3u, Both(), ci, cd);
+    // (a range without nonzeros has one step, for its rows)
+    for (uint32_t s0 = begin & ~3u;; s0 += kStep) {
+      const uint32_t s1 = (end - s0 > kStep) ? s0 + kStep : end;
+      load_window();
+      if (s1 > 4u * whole) load_last(s0, Both(), ci, cd);
+      F prod[U][4];  // (the vector's elements first, then the products: in F, as the reference forms them)
+      auto column = [&](int u, int t) {  // (beyond the step: element 0, unused)
+        const uint32_t p = 4u * (s0 / 4u + static_cast<uint32_t>(u) * kWave + lane) + static_cast<uint32_t>(t);
+        return p < s1 ? ci[u][t] : 0u;
+      };
+      if constexpr (kStaged) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+#pragma unroll
+          for (int t = 0; t < 4; ++t) {
+            const uint32_t c = column(u, t);
+            prod[u][t] = s_x[c < staged ? c : 0u];
+          }
+        }
+        if (staged < n_col) {  // (uniform)
+          // (all LDS reads first: without the empty statements each would be moved into the branch around the load)
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t) asm volatile("" : "+v"(prod[u][t]));
+          }
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+              const uint32_t c = column(u, t);
+              if (c >= staged) prod[u][t] = x[c];
+            }
+          }
+        }
+      } else {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+#pragma unroll
+          for (int t = 0; t < 4; ++t) prod[u][t] = x[column(u, t)];
+        }
+      }
+      F cw[U][4];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) cw[u][t] = cd[u][t];
+      }
+      load_step(s1, Both(), ci, cd);  // (a step at or beyond the end of the range loads nothing)
+      multiply(prod, cw);
+      walk_rows(s0, s1, prod, cw);
+      if (s1 == end) break;
+    }
+  } else {
+    constexpr int H = FlatHeld<F, HETER, OUT>::value;
+    u32x4 ci[H][U] = {};
+    F cd[2][U][4] = {};  // weights, a step ahead
+    //static_assert(H % 2 == 0 || !kWeights);
+    uint32_t s0 = begin & ~3u;  // the round takes [s0, s0 + H * kStep)
+    const uint32_t own = idle ? 0u : s0 < end ? (end - s0 - 1u) / (H * kStep) + 1u : 1u;
+    __shared__ uint32_t s_rounds;
+    if (threadIdx.x == 0) s_rounds = 0;
+    __syncthreads();
+    if (lane == 0) atomicMax(&s_rounds, own);
+#pragma unroll
+    for (int h = 0; h < H; ++h) load_step(s0 + static_cast<uint32_t>(h) * kStep, Indices(), ci[h], cd[0]);
+    load_step(s0, Weights(), ci[0], cd[0]);
+    __syncthreads();
+    const uint32_t rounds = __builtin_amdgcn_readfirstlane(s_rounds);
+    const uint32_t windows = (n_col - 1u) / kFits + 1u;
+    const uint32_t width = ((n_col - 1u) / windows + 4u) & ~3u;  // (at most kFits, a multiple of 4)
+    uint32_t here = kNoRow;                                      // the window in LDS
+    for (uint32_t round = 0; round < rounds; ++round) {
+      const bool work = round < own;  // (uniform over the wave; without work it brings its part of the windows)
+      F prod[H][U][4];
+      if (work) {
+#pragma unroll
+        for (int h = 0; h < H; ++h) {
+          const uint32_t sh = s0 + static_cast<uint32_t>(h) * kStep;
+          if (sh < end && end - sh <= kStep && end > 4u * whole) load_last(sh, Indices(), ci[h], cd[0]);
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+              const uint32_t p = 4u * (sh / 4u + static_cast<uint32_t>(u) * kWave + lane) + static_cast<uint32_t>(t);
+              prod[h][u][t] = p < end ? flat_place(F(0), ci[h][u][t]) : F(0);
+            }
+          }
+        }
+      }
+      // (there and back: a round begins with the window that the one before ended with)
+      for (uint32_t i = 0; i < windows; ++i) {
+        const uint32_t window = (round & 1u) ? windows - 1u - i : i;
+        const uint32_t first = window * width, n = n_col - first < width ? n_col - first : width;
+        if (window != here) {
+          if (here != kNoRow) __syncthreads();
+          flat_stage_window(s_x, x + first, n);
+          here = window;
+          __syncthreads();
+        }
+        if (work) {
+          uint32_t origin = flat_origin(F(0), first), bytes = n * static_cast<uint32_t>(sizeof(F));
+          asm volatile("" : "+s"(origin), "+s"(bytes));
+#pragma unroll
+          for (int h = 0; h < H; ++h) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+#pragma unroll
+              for (int t = 0; t < 4; ++t) flat_take(prod[h][u][t], (flat_lds)s_staged, origin, bytes);
+            }
+          }
+        }
+      }
+      if (work) {
+#pragma unroll
+        for (int h = 0; h < H; ++h) {
+          const uint32_t sh = s0 + static_cast<uint32_t>(h) * kStep;
+          const bool step = h == 0 || sh < end;
+          if (step) load_window();
+          load_step(sh + kStep, Weights(), ci[0], cd[(h + 1) % 2]);
+          // (the steps behind are done with their registers: the next round's indices are requested)
+          if (h != 0) load_step(sh + (H - 1u) * kStep, Indices(), ci[h - 1], cd[0]);
+          if (step) {
+            const uint32_t s1 = end - sh > kStep ? sh + kStep : end;
+            if (s1 > 4u * whole) load_last(sh, Weights(), ci[0], cd[h % 2]);
+            multiply(prod[h], cd[h % 2]);
+            walk_rows(sh, s1, prod[h], cd[h % 2]);
+          }
+        }
+        load_step(s0 + (2u * H - 1u) * kStep, Indices(), ci[H - 1], cd[0]);
+        s0 += H * kStep;
+        if constexpr (H % 2 != 0) {
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t) cd[0][u][t] = cd[1][u][t];
+          }
+        }
+      }
+    }
   }
   // the row that is still open at the end of the range (if it has nonzeros in it)
   if (kSums && lane == 0 && r < n_row) {
@@ -471,13 +665,38 @@ bool flat_stages(uint32_t n_col) {
   return static_cast<uint64_t>(n_col) * sizeof(F) <= 552ull * 1024u;
 }
 
-template <typename F, bool HETER, int OUT, bool STAGED>
+// Where the walk takes x from.  A visit of a window (147 KB staged and a test of every place held, 3 us with nothing beside
+// it) has to spare 1.15 million gathers (double 0.7; with one weight 1.5: no weights to request meanwhile), and a call a
+// million.  Measured, before and now (300,000 rows of 100 where not said; the weights' gradient with them):
+// 60,000 / 120,000 / 180,000 floats 95 / 133 / 154 -> 89 / 111 / 128 us, one weight and 120,000 107 -> 102, 30,000 / 60,000
+// doubles 124 / 159 -> 105 / 140; 30,000 rows of 1,000 and 150,000 146 -> 118.  On the other side of the line: 240,000 floats 156
+// and 157 (149 with 32 places a lane, which spill), 480,000 158 and 261, 100,000 rows of 80 and 75,000 36.2 and 37.1, of 30 and
+// 120,000 23 and 28, one weight and 60,000 doubles 112 and 123.
+template <typename F, bool HETER, int OUT>
+static FlatVector flat_vector(uint32_t n_col, uint32_t nnz) {
+  constexpr uint32_t kFits = flat_staged_bytes<F, OUT>() / sizeof(F);
+  constexpr FlatVector kSwept = FlatVector::kSwept;
+  if (n_col <= kFits) return FlatVector::kStaged;
+  if constexpr (flat_sweeps<F, OUT>()) {
+    const uint64_t waves = static_cast<uint64_t>(device_info().num_cu) * (flat_threads(kSwept) / kWave);
+    const uint64_t round = waves * kWave * 4u * FlatQuads<F, OUT, kSwept>::value * FlatHeld<F, HETER, OUT>::value;
+    const uint64_t visits = 1u + static_cast<uint64_t>((n_col - 1u) / kFits) * (nnz / round + 1u);
+    const uint64_t gathers = flat_stages<F>(n_col) ? nnz - static_cast<uint64_t>(nnz) * kFits / n_col : nnz;
+    constexpr bool kOneWeight = !HETER && (OUT & kFlatSums);
+    constexpr uint32_t kPerVisit = kOneWeight ? 1500000u : sizeof(F) == 4 ? 1150000u : 700000u;
+    constexpr uint32_t kPerCall = sizeof(F) == 4 ? 1000000u : 500000u;
+    if (n_col <= kFlatMostPlaces && gathers >= visits * kPerVisit + kPerCall) return kSwept;
+  }
+  return flat_stages<F>(n_col) ? FlatVector::kStaged : FlatVector::kL2;
+}
+
+template <typename F, bool HETER, int OUT, FlatVector FROM>
 static bool launch_flat(const char *target, hipStream_t stream, const F *data, const uint32_t *indices,
                         const uint32_t *indptr, const F *x, F *y, uint32_t n_row, uint32_t n_col, uint32_t min_mean,
                         const F *v, F *products, uint32_t n_products) {
   constexpr bool kSums = (OUT & kFlatSums) != 0;
-  const unsigned grid = static_cast<unsigned>(device_info().num_cu) * flat_per_cu(STAGED);
-  const uint32_t waves = grid * (flat_threads(STAGED) / kWave);
+  const unsigned grid = static_cast<unsigned>(device_info().num_cu) * flat_per_cu(FROM);
+  const uint32_t waves = grid * (flat_threads(FROM) / kWave);
   double *head = nullptr, *tail = nullptr;
   uint32_t *tail_row = nullptr, *range = nullptr;
   if (kSums) {
@@ -487,9 +706,9 @@ static bool launch_flat(const char *target, hipStream_t stream, const F *data, c
     head = reinterpret_cast<double *>(ws), tail = head + waves;
     tail_row = reinterpret_cast<uint32_t *>(tail + waves), range = tail_row + waves;
   }
-  auto kernel = csr_flat_gather_kernel<F, HETER, OUT, STAGED>;
+  auto kernel = csr_flat_gather_kernel<F, HETER, OUT, FROM>;
   size_t lds = 0;
-  if (STAGED) {
+  if (FROM != FlatVector::kL2) {
     constexpr uint32_t kMost = flat_staged_bytes<F, OUT>();
     lds = static_cast<size_t>(n_col) * sizeof(F) < kMost ? static_cast<size_t>(n_col) * sizeof(F) : kMost;
     static thread_local bool attr_set = false;  // (per instantiation)
@@ -503,7 +722,7 @@ static bool launch_flat(const char *target, hipStream_t stream, const F *data, c
       attr_set = true;
     }
   }
-  hipLaunchKernelGGL(kernel, dim3(grid), dim3(flat_threads(STAGED)), lds, stream, data, indices, indptr, x, y, n_row,
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(flat_threads(FROM)), lds, stream, data, indices, indptr, x, y, n_row,
                      n_col, min_mean, head, tail, tail_row, range, v, products, n_products);
   if (kSums)
     hipLaunchKernelGGL(csr_flat_finish_kernel<F>, dim3(waves), dim3(kWave), 0, stream, indptr, y, n_row, min_mean,
@@ -512,16 +731,29 @@ static bool launch_flat(const char *target, hipStream_t stream, const F *data, c
   return check_launch(target);
 }
 
+template <typename F, bool HETER, int OUT>
+static bool flat_walk(const char *target, hipStream_t stream, const F *data, const uint32_t *indices, const uint32_t *indptr,
+                      const F *x, F *y, uint32_t n_row, uint32_t n_col, uint32_t nnz, uint32_t min_mean, const F *v,
+                      F *products) {
+  auto launch = [&](auto from) {
+    return launch_flat<F, HETER, OUT, decltype(from)::value>(target, stream, data, indices, indptr, x, y, n_row, n_col,
+                                                             min_mean, v, products, (OUT & kFlatProducts) ? nnz : 0u);
+  };
+  switch (flat_vector<F, HETER, OUT>(n_col, nnz)) {
+    case FlatVector::kStaged: return launch(std::integral_constant<FlatVector, FlatVector::kStaged>());
+    case FlatVector::kSwept:
+      if constexpr (flat_sweeps<F, OUT>()) return launch(std::integral_constant<FlatVector, FlatVector::kSwept>());
+    default: return launch(std::integral_constant<FlatVector, FlatVector::kL2>());
+  }
+}
+
 template <typename F>
 bool csr_flat_gather(const char *target, hipStream_t stream, const F *data, bool heter, const uint32_t *indices,
-                     const uint32_t *indptr, const F *x, F *y, uint32_t n_row, uint32_t n_col, uint32_t min_mean) {
+                     const uint32_t *indptr, const F *x, F *y, uint32_t n_row, uint32_t n_col, uint32_t nnz,
+                     uint32_t min_mean) {
   if (n_row == 0) return true;
-  auto launch = [&](auto h, auto staged) {
-    return launch_flat<F, decltype(h)::value, kFlatSums, decltype(staged)::value>(
-      target, stream, data, indices, indptr, x, y, n_row, n_col, min_mean, nullptr, nullptr, 0u);
-  };
-  if (flat_stages<F>(n_col)) return heter ? launch(std::true_type(), std::true_type()) : launch(std::false_type(), std::true_type());
-  return heter ? launch(std::true_type(), std::false_type()) : launch(std::false_type(), std::false_type());
+  auto walk = heter ? flat_walk<F, true, kFlatSums> : flat_walk<F, false, kFlatSums>;
+  return walk(target, stream, data, indices, indptr, x, y, n_row, n_col, nnz, min_mean, nullptr, nullptr);
 }
 
 template <typename F>
@@ -535,14 +767,8 @@ bool csr_gradient(const char *target, hipStream_t stream, const F *data, const u
     set_error("%s: %u nonzeros are more than the walk's positions can number", target, nnz);
     return false;
   }
-  auto launch = [&](auto out, auto staged) {
-    return launch_flat<F, true, decltype(out)::value, decltype(staged)::value>(target, stream, data, indices, indptr, x, sums,
-                                                                               n_row, n_col, 0u, v, products, nnz);
-  };
-  using Products = std::integral_constant<int, kFlatProducts>;
-  using Both = std::integral_constant<int, kFlatSums | kFlatProducts>;
-  if (flat_stages<F>(n_col)) return sums != nullptr ? launch(Both(), std::true_type()) : launch(Products(), std::true_type());
-  return sums != nullptr ? launch(Both(), std::false_type()) : launch(Products(), std::false_type());
+  auto walk = sums != nullptr ? flat_walk<F, true, kFlatSums | kFlatProducts> : flat_walk<F, true, kFlatProducts>;
+  return walk(target, stream, data, indices, indptr, x, sums, n_row, n_col, nnz, 0u, v, products);
 }
 
 // csr_matvec_gradient: buffers = [data, indices, indptr, row vector, column vector, products, sums (or null)]
@@ -564,9 +790,9 @@ static void csr_matvec_gradient_entry(const char *target, hipStream_t stream, vo
 template bool flat_stages<float>(uint32_t);
 template bool flat_stages<double>(uint32_t);
 template bool csr_flat_gather<float>(const char *, hipStream_t, const float *, bool, const uint32_t *, const uint32_t *,
-                                     const float *, float *, uint32_t, uint32_t, uint32_t);
+                                     const float *, float *, uint32_t, uint32_t, uint32_t, uint32_t);
 template bool csr_flat_gather<double>(const char *, hipStream_t, const double *, bool, const uint32_t *, const uint32_t *,
-                                      const double *, double *, uint32_t, uint32_t, uint32_t);
+                                      const double *, double *, uint32_t, uint32_t, uint32_t, uint32_t);
 
 }  // namespace bpl
 

@@ -1988,7 +1988,8 @@ void launch_gather(const char *target, const ScratchSource &src, const F *data, 
                                   (n_row >= 16384 || (n_col > 8192 && flat_stages<F>(n_col)))
                               : n_row >= 16384;
       if (flat && n_col > 0) {
-        if (csr_flat_gather<F>(target, stream, data, HETER, indices, indptr, x, y, n_row, n_col, known ? 0u : kFlatMinMean)) {
+        if (csr_flat_gather<F>(target, stream, data, HETER, indices, indptr, x, y, n_row, n_col, known ? nnz : 0u,
+                               known ? 0u : kFlatMinMean)) {
           if (!known)
             launch_gather_impl<F, VT, HETER, MODE, 0>(target, stream, data, indices, indptr, x, y, n_row, n_col, 0,
                                                       kFlatMinMean);

@@ -1400,3 +1400,54 @@ def test_a_block_of_rows_costs_what_its_nonzeros_cost(cuda, n_row, n_col, long, 
     times.append(min(runs))
   print("us", times)
   assert times[0] < 2.0 * times[1], times
+
+
+# Vectors longer than LDS whose windows pass by while the waves hold the places of their nonzeros: two windows that are
+# just full, a third one of few elements, several rounds with a last one of few nonzeros, one to three nonzeros behind
+# the last whole quad.  Integers: every order of the sums gives the same bits.
+@pytest.mark.parametrize("dtype,n_col,nnz,homo", [
+  (np.float32, 75_264, 9_400_003, False), (np.float32, 75_265, 18_800_001, False), (np.float32, 150_001, 25_000_002, False),
+  (np.float32, 75_000, 12_000_001, True), (np.float64, 37_632, 8_000_001, False), (np.float64, 60_001, 24_000_003, False)])
+def test_csr_matvec_windows_of_the_vector_pass_by(dtype, n_col, nnz, homo):
+  rng = np.random.default_rng(n_col + nnz)
+  n_row = 50_021
+  # a tenth of the rows empty in one block, one row of 300,000, the rest uneven
+  lengths = np.concatenate([np.zeros(5_000, np.int64), [300_000],
+                            rng.multinomial(nnz - 300_000, rng.dirichlet(np.full(n_row - 5_001, 0.5)))])
+  indptr = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+  row = np.repeat(np.arange(n_row), lengths)
+  indices = rng.integers(0, n_col, nnz).astype(np.int32)
+  x = rng.integers(-8, 9, n_col).astype(dtype)
+  data = np.array([3.0], dtype) if homo else rng.integers(-4, 5, nnz).astype(dtype)
+  dev = [torch.from_numpy(a).cuda() for a in (data, indices, indptr)]
+
+  def product(vector):
+    return np.bincount(row, weights=(data * vector[indices]).astype(np.float64), minlength=n_row)
+  got = bpl.csr_matvec(*dev, torch.from_numpy(x).cuda(), shape=(n_row, n_col)).cpu().numpy()
+  np.testing.assert_array_equal(got, product(x).astype(dtype))
+  # infinities, and NaNs of any sign and payload, are the vector's values like others
+  word = np.uint32 if dtype == np.float32 else np.uint64
+  odd = x.copy()
+  bits = odd.view(word)
+  place = (lambda c: 0xff800004 + 4 * c) if dtype == np.float32 else (lambda c: (0xfff00001 + c) << 32)
+  for c, b in ((3, place(n_col - 1)), (n_col // 2, place(0)), (n_col - 2, place(n_col // 2 + 1)),
+               (n_col - 1, 0xffc00000 if dtype == np.float32 else 0xfff8000000000000)):
+    bits[c] = word(b)
+  odd[5] = -np.inf
+  got = bpl.csr_matvec(*dev, torch.from_numpy(odd).cuda(), shape=(n_row, n_col)).cpu().numpy()
+  with np.errstate(invalid="ignore"):
+    want = product(odd)
+  assert np.isnan(want).any() and np.isinf(want).any()
+  np.testing.assert_array_equal(got, want.astype(dtype))
+  if homo:
+    return
+  # the gradients: the weights' alone, and with the vector's in the same walk
+  v = rng.integers(-8, 9, n_row).astype(dtype)
+  for transpose in (False, True):
+    w = dev[0].clone().requires_grad_()
+    vec = torch.from_numpy(v if transpose else x).cuda().requires_grad_()
+    out = bpl.cusparse_csr_matvec(w, *dev[1:], vec, shape=(n_row, n_col), transpose=transpose)
+    g_w, g_v = torch.autograd.grad(out, (w, vec), torch.from_numpy(x if transpose else v).cuda())
+    np.testing.assert_array_equal(g_w.cpu().numpy(), v[row] * x[indices])
+    if transpose:
+      np.testing.assert_array_equal(g_v.cpu().numpy(), product(x).astype(dtype))
