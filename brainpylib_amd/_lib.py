@@ -18,6 +18,8 @@ _lib = None
 _TARGET_FN = ctypes.CFUNCTYPE(None, ctypes.c_void_p, ctypes.POINTER(ctypes.c_void_p), ctypes.c_char_p,
                               ctypes.c_size_t)
 _targets = {}
+_addresses = {}
+_enqueue = None
 
 
 class GPUOperatorNotFound(Exception):
@@ -77,30 +79,55 @@ def last_error():
 _PTR_ARRAYS = {}
 
 
-def custom_call(name, buffers, opaque, stream=None):
-  """Enqueue custom-call target ``name`` on ``stream`` (default: torch's current stream).
-
-  ``buffers``: torch CUDA tensors (operands, then results), contiguous.  Asynchronous."""
-  import torch
-  fn = target(name)
-  if stream is None:
-    # (the raw handle; torch.cuda.current_stream() builds a Stream object first, which costs
-    # several microseconds per call)
-    try:
-      stream = torch._C._cuda_getCurrentRawStream(buffers[0].device.index)
-    except (AttributeError, TypeError):
-      stream = torch.cuda.current_stream(buffers[0].device).cuda_stream
+def _enqueue_ctypes(address, stream, opaque, *buffers):
   n = len(buffers)
   array_type = _PTR_ARRAYS.get(n)
   if array_type is None:
     array_type = _PTR_ARRAYS[n] = ctypes.c_void_p * n
-  ptrs = array_type(*[b.data_ptr() for b in buffers])
-  fn(stream, ptrs, opaque, len(opaque))
+  _TARGET_FN(address)(stream, array_type(*[b.data_ptr() for b in buffers]), opaque, len(opaque))
   # the error string is per thread and empty unless a target has just failed
   err = lib().bpl_last_error()
   if err:
     lib().bpl_clear_error()
     raise RuntimeError(err.decode())
+
+
+def _native_enqueue():
+  """The extension module's call into a target; ctypes where the module was not built (it needs pybind11)."""
+  global _enqueue
+  lib()
+  try:
+    from .gpu_ops import enqueue
+  except ImportError:
+    enqueue = _enqueue_ctypes
+  _enqueue = enqueue
+  return enqueue
+
+
+def custom_call(name, buffers, opaque, stream=None):
+  """Enqueue custom-call target ``name`` on ``stream`` (default: torch's current stream).
+
+  ``buffers``: torch CUDA tensors (operands, then results), contiguous.  Asynchronous."""
+  address = _addresses.get(name)
+  if address is None:
+    address = _addresses[name] = ctypes.cast(target(name), ctypes.c_void_p).value
+  if stream is None:
+    # (the raw handle; torch.cuda.current_stream() builds a Stream object first, which costs
+    # several microseconds per call)
+    try:
+      stream = _current_raw_stream(buffers[0].device.index)
+    except (AttributeError, TypeError):
+      import torch
+      stream = torch.cuda.current_stream(buffers[0].device).cuda_stream
+  (_enqueue or _native_enqueue())(address, stream, opaque, *buffers)
+
+
+def _current_raw_stream(index):
+  """torch's current stream on a device, replaced by torch's own function at its first call."""
+  global _current_raw_stream
+  import torch
+  _current_raw_stream = torch._C._cuda_getCurrentRawStream
+  return _current_raw_stream(index)
 
 
 # ---- descriptor builders (same names and argument order as the reference's gpu_ops module,

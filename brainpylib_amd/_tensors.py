@@ -38,6 +38,37 @@ def as_tensor(a):
   return torch.from_numpy(np.ascontiguousarray(arr))
 
 
+class _NumberTensor:
+  """A Python number as a host tensor of shape (1,), with that tensor's copies on devices."""
+  __slots__ = ("host", "copies")
+
+  def __init__(self, value):
+    self.host = as_tensor(value).reshape(1)
+    self.copies = {}
+
+
+_PY_NUMBERS = {}
+
+
+def number_operand(value):
+  """The _NumberTensor of a Python int or float (a homogeneous weight), made once per value."""
+  # keyed by the value's bits, as in as_tensor
+  key = struct.pack("<d", value) if type(value) is float else value
+  number = _PY_NUMBERS.get(key)
+  if number is None:
+    if len(_PY_NUMBERS) >= 256:
+      _PY_NUMBERS.clear()
+    number = _PY_NUMBERS[key] = _NumberTensor(value)
+  return number
+
+
+def number_to_device(number, device):
+  copy = number.copies.get(device)
+  if copy is None:
+    copy = number.copies[device] = to_device(number.host, device)
+  return copy
+
+
 def device_of(*args):
   """The device the call runs on: that of the first CUDA tensor argument, else the current one."""
   for a in args:
@@ -78,9 +109,30 @@ def is_index_dtype(dt):
   return dt in _INDEX_DTYPES
 
 
+class _PositionalSignature(inspect.Signature):
+  """The signature of a ``forward`` that is only called with all its arguments by position: there is nothing to match."""
+  __slots__ = ()
+
+  def bind(self, *args, **kwargs):
+    if kwargs or len(args) != len(self.parameters):
+      return super().bind(*args, **kwargs)
+    return _PositionalArguments(args)
+
+
+class _PositionalArguments:
+  __slots__ = ("args",)
+
+  def __init__(self, args):
+    self.args = args
+
+  def apply_defaults(self):
+    pass
+
+
 def keep_signature(function):
   """Class decorator for autograd functions: torch binds the arguments of one with a ``setup_context`` through
-  ``inspect.signature(forward)`` on every call and builds it anew each time; kept on ``forward`` it is only
-  looked up."""
-  function.forward.__signature__ = inspect.signature(function.forward)
+  ``inspect.signature(forward).bind`` on every call, which costs more host time than the call it prepares; the
+  signature kept on ``forward`` passes arguments given by position through."""
+  function.forward.__signature__ = _PositionalSignature(
+    list(inspect.signature(function.forward).parameters.values()))
   return function

@@ -9,7 +9,8 @@ from typing import Tuple
 import torch
 
 from . import _lib, sparse_ops
-from ._tensors import FLOAT_DTYPES, as_tensor, device_of, is_index_dtype, keep_signature, to_device
+from ._tensors import (FLOAT_DTYPES, as_tensor, device_of, is_index_dtype, keep_signature, number_operand,
+                       number_to_device, to_device)
 
 __all__ = ["event_csr_matvec", "event_csr_matvec_batching", "event_info"]
 
@@ -26,7 +27,8 @@ def event_csr_matvec(data, indices, indptr, events, *, shape: Tuple[int, int], t
   events   (shape[0] if transpose else shape[1],) bool, or the float dtype of ``data``
   returns  (shape[1] if transpose else shape[0],) tensor of ``data``'s dtype on the GPU.
   """
-  data = as_tensor(data)
+  number = number_operand(data) if type(data) in (float, int) else None
+  data = as_tensor(data) if number is None else number.host
   indices = as_tensor(indices)
   indptr = as_tensor(indptr)
   events = as_tensor(events)
@@ -68,7 +70,8 @@ def event_csr_matvec(data, indices, indptr, events, *, shape: Tuple[int, int], t
     raise ValueError('events should be bool or have the dtype of data, '
                      f'but we got {events.dtype} != {data.dtype}.')
   device = device_of(data, indices, indptr, events)
-  data, indices, indptr, events = (to_device(t, device) for t in (data, indices, indptr, events))
+  data = to_device(data, device) if number is None else number_to_device(number, device)
+  indices, indptr, events = to_device(indices, device), to_device(indptr, device), to_device(events, device)
   if sparse_ops._wants_grad(data, events):
     return _EventCSRMatvec.apply(data, indices, indptr, events, tuple(shape), bool(transpose))
   return _launch(data, indices, indptr, events, shape, transpose)
@@ -100,7 +103,7 @@ class _EventCSRMatvec(torch.autograd.Function):
 
   @staticmethod
   def forward(data, indices, indptr, events, shape, transpose):
-    return _launch(data.detach(), indices, indptr, events.detach(), shape, transpose)
+    return _launch(data, indices, indptr, events, shape, transpose)
 
   @staticmethod
   def setup_context(ctx, inputs, output):

@@ -16,6 +16,7 @@ import torch
 
 from . import _lib
 from ._tensors import FLOAT_DTYPES, as_tensor, device_of, keep_signature, to_device
+from .sparse_ops import _wants_grad
 
 __all__ = [
   'event_matvec_prob_conn_homo_weight', 'event_matvec_prob_conn_uniform_weight',
@@ -132,8 +133,7 @@ class _JitconnMatvec(torch.autograd.Function):
 
 
 def _run(fn_prefix, w_kind, inp, out_dtype, suffix, **kw):
-  if inp.is_floating_point() and (inp.requires_grad or
-                                  torch.autograd.forward_ad.unpack_dual(inp).tangent is not None):
+  if inp.is_floating_point() and _wants_grad(inp):
     # move first (differentiably), so that the gradient comes back on the caller's device
     return _JitconnMatvec.apply(to_device(inp, device_of(inp)), fn_prefix, w_kind, out_dtype, suffix, kw)
   return _launch(fn_prefix, w_kind, inp, out_dtype, suffix, **kw)

@@ -9,18 +9,25 @@ reference hands to cuSPARSE and this package computes with its own scatter kerne
 from typing import Tuple
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _lib
-from ._tensors import FLOAT_DTYPES, as_tensor, device_of, is_index_dtype, keep_signature, to_device
+from ._tensors import (FLOAT_DTYPES, as_tensor, device_of, is_index_dtype, keep_signature, number_operand,
+                       number_to_device, to_device)
 
 __all__ = ["csr_matvec", "cusparse_csr_matvec", "csr_to_coo", "coo_to_csr", "csr_to_dense", "check_csr"]
 
 
 def _prepare(data, indices, indptr, vector):
-  data = as_tensor(data)
-  if data.ndim == 0:
-    data = data.reshape(1)
-  return data, as_tensor(indices), as_tensor(indptr), as_tensor(vector)
+  indices = as_tensor(indices)
+  if type(data) in (float, int):
+    number = number_operand(data)
+    data = number_to_device(number, indices.device) if indices.is_cuda else number.host
+  else:
+    data = as_tensor(data)
+    if data.ndim == 0:
+      data = data.reshape(1)
+  return data, indices, as_tensor(indptr), as_tensor(vector)
 
 
 def _move(*tensors):
@@ -139,19 +146,21 @@ def _launch(data, indices, indptr, vector, shape, transpose, method='vector'):
 def _wants_grad(*tensors):
   """True if a floating-point argument takes part in reverse- or forward-mode differentiation."""
   for t in tensors:
-    if t.requires_grad:
-      return True
-    # (outside a dual level unpack_dual returns at once with no tangent)
-    if t.is_floating_point() and torch.autograd.forward_ad.unpack_dual(t).tangent is not None:
+    if t.requires_grad or (t.is_floating_point() and _has_tangent(t)):
       return True
   return False
+
+
+def _has_tangent(t):
+  # (outside a dual level, where unpack_dual finds no tangent either, its named tuple is most of the cost)
+  return forward_ad._current_level >= 0 and forward_ad.unpack_dual(t).tangent is not None
 
 
 def _transformed(t):
   """True for a tensor whose products must stay visible to a differentiation or batching transform."""
   if torch.is_grad_enabled() and t.requires_grad:
     return True
-  if torch.autograd.forward_ad.unpack_dual(t).tangent is not None:
+  if _has_tangent(t):
     return True
   try:
     t.data_ptr()
@@ -185,7 +194,7 @@ def _gradients(data, indices, indptr, row_vector, col_vector, shape, want_sums):
   sums = torch.empty(shape[0] if want_sums else 0, dtype=data.dtype, device=data.device)
   name = 'csr_matvec_gradient_' + ('float' if data.dtype == torch.float32 else 'double')
   opaque = _lib.build_csr_transpose_descriptor(shape[0], shape[1], nnz)
-  buffers = [data.detach(), indices, indptr, row_vector.detach(), col_vector.detach(), products, sums]
+  buffers = [data, indices, indptr, row_vector, col_vector, products, sums]
   try:
     _lib.custom_call(name, buffers, opaque)
   except RuntimeError:
@@ -207,7 +216,7 @@ class _CSRMatvec(torch.autograd.Function):
 
   @staticmethod
   def forward(data, indices, indptr, vector, shape, transpose, method):
-    return _launch(data.detach(), indices, indptr, vector.detach(), shape, transpose, method)
+    return _launch(data, indices, indptr, vector, shape, transpose, method)
 
   @staticmethod
   def setup_context(ctx, inputs, output):

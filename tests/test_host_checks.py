@@ -1,5 +1,8 @@
 """Argument checking of the host-side operator wrappers (same conditions as the reference's
 wrappers; no GPU needed: the checks run before a device is touched)."""
+import ctypes
+import inspect
+
 import numpy as np
 import pytest
 import torch
@@ -90,3 +93,51 @@ def test_python_scalars_are_kept_by_bit_pattern():
   n1, n2 = _tensors.as_tensor(float("nan")), _tensors.as_tensor(float("nan"))
   assert n1 is n2 and math.isnan(n1.item())
   assert _tensors.as_tensor(True).dtype == torch.bool and _tensors.as_tensor(1).dtype == torch.float32
+
+
+def test_numbers_as_weights_are_told_apart_by_their_bits():
+  from brainpylib_amd._tensors import number_operand
+  for a, b in ((0.0, -0.0), (1, 2), (0.5, 0.25), (3, 3.5)):
+    assert number_operand(a).host is not number_operand(b).host
+    for v in (a, b):
+      host = number_operand(v).host
+      assert host is number_operand(v).host
+      assert host.shape == (1,) and host.dtype == torch.float32
+      assert host.item() == v and np.signbit(host.item()) == np.signbit(v)
+  nan = number_operand(float("nan"))
+  assert np.isnan(nan.host.item()) and nan is number_operand(float("nan"))
+
+
+def test_native_enqueue_refuses_what_is_no_call():
+  gpu_ops = pytest.importorskip("brainpylib_amd.gpu_ops")
+  from brainpylib_amd import _lib
+  address = ctypes.cast(_lib.target("event_csr_matvec_homo_float_bool"), ctypes.c_void_p).value
+  for args in ((), (address, 0), (address, 0, "text"), (address, 0, b"") + (torch.zeros(1),) * 17):
+    with pytest.raises(TypeError):
+      gpu_ops.enqueue(*args)
+  with pytest.raises(ValueError):
+    gpu_ops.enqueue(0, 0, b"")
+  with pytest.raises(AttributeError):
+    gpu_ops.enqueue(address, 0, b"", 1)
+  # a target's own error comes back as the exception and leaves nothing behind
+  for _ in range(2):
+    with pytest.raises(RuntimeError, match="event_csr_matvec_homo_float_bool"):
+      gpu_ops.enqueue(address, 0, b"short", torch.zeros(1))
+  assert not _lib.last_error()
+
+
+def test_signature_of_an_autograd_function_binds_other_calls_as_inspect_does():
+  from brainpylib_amd._tensors import keep_signature
+
+  @keep_signature
+  class F:
+    @staticmethod
+    def forward(a, b, c=3):
+      return a
+  sig = inspect.signature(F.forward)
+  assert sig.bind(1, 2, 4).args == (1, 2, 4)
+  bound = sig.bind(1, b=2)
+  bound.apply_defaults()
+  assert bound.args == (1, 2, 3)
+  with pytest.raises(TypeError):
+    sig.bind(1)
