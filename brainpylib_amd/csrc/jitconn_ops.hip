@@ -164,7 +164,7 @@ __global__ __launch_bounds__(1024, (BITS == 2 || (W == kNormal && sizeof(T1) == 
     //
     // Which batch is next comes from a counter of the device (`next`: batches taken, workgroups at their end): of two
     // workgroups on a CU the older one gets more of the issue slots, and with equal shares the younger one worked
-    // alone, four waves to a SIMD, for the last fifth (1,000,000 streams of 1,000 synapses: KBAL).  Without one
+    // alone, four waves to a SIMD, for the last fifth (1,000,000 streams of 1,000 synapses: 1,665 us, with the counter 1,552).  Without one
     // (`next` null), batch blockIdx.x + j * gridDim.x.
     uint32_t &s_task = smem_raw[0], *const s_ready = smem_raw + 1, *const s_loaded = s_ready + kFuseSlots,
              *const s_batch = s_loaded + kFuseSlots;
