@@ -129,7 +129,7 @@ __global__ __launch_bounds__(256) void jitconn_matmat_kernel(const T1 *__restric
       syn[slot].w = w;
     };
     if constexpr (W == kNormal) {
-      walk_stream<T1, W>(st, lane, seed + j, pre, k, skips, wa, wb,
+      walk_stream<T1, W, true>(st, lane, seed + j, pre, k, skips, wa, wb,
                          [&](uint32_t idx0, T1 w0, bool valid0, uint32_t idx1, T1 w1, bool valid1) {
         __builtin_amdgcn_wave_barrier();  // the reads of the batch before are done
         if (valid0) {

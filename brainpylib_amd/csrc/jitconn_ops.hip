@@ -33,12 +33,19 @@ namespace {
 // LDS the row walk gives to an event bitmap when it wants two 16-wave workgroups per CU (each wave
 // can issue one instruction every four cycles, so the number of resident waves bounds the VALU
 // utilisation: 32 waves per CU walk 290 G synapses/s, the 15 that fit beside a 125 KB bitmap 228).
-// What two workgroups leave of a CU's 160 KB beside their 16 waves' states and queues (normal weights: 18,944 bytes; 1e5
-// streams of 1,000 synapses over 1e6 inputs 625 / 628 / 628 us at 1 / 10 / 100 % events: the second probe hides behind the weights).
+// What two workgroups leave of a CU's 160 KB beside their 16 waves' states and queues (float normal
+// weights: 18,944 bytes; the share of events hardly matters there, the second probe hides behind the weights).
 constexpr uint32_t kRowwalkCoarseMost = 38912;
+// Float normal weights with events keep the state with the least mirror: wrapping a batch's addresses lane by lane costs
+// eight instructions, and the LDS that it saves holds twice the events' bitmap (1e5 streams of 1,000 to 1,500 synapses over
+// 40,000 / 130,000 / 150,000 / 900,000 inputs: 590 / 637 / 726 / 693 us, with the long mirror 600 / 675 / 835 / 705).  Not double, whose
+// batches cost more than the probes (818 / 868 / 987 / 910 with the long mirror, else 837 / 902 / 1,033 / 928), nor a dense vector
+// (matvec and its gradient 1,769 us, else 1,780).
+template <typename T1, int IN, int W>
+constexpr bool rowwalk_short() { return IN == kInEvent && W == kNormal && sizeof(T1) == 4; }
 template <typename T1, int W>
 constexpr uint32_t rowwalk_coarse_bytes() {
-  const uint32_t left = (80u * 1024u - 16u * 4u * StreamLds<T1, W>::words - 64u) / 256u * 256u;
+  const uint32_t left = (80u * 1024u - 16u * 4u * StreamLds<T1, W, rowwalk_short<T1, kInEvent, W>()>::words - 64u) / 256u * 256u;
   return left < kRowwalkCoarseMost ? left : kRowwalkCoarseMost;
 }
 
@@ -74,7 +81,8 @@ __global__ __launch_bounds__(1024, (BITS == 2 || (W == kNormal && sizeof(T1) == 
   const int lane = lane_id();
   const uint32_t wave = threadIdx.x / kWave;
   const uint32_t nwaves = blockDim.x / kWave;
-  constexpr int kWords = StreamLds<T1, W>::words;
+  constexpr bool kShort = rowwalk_short<T1, IN, W>();
+  constexpr int kWords = StreamLds<T1, W, kShort>::words;
   uint32_t *st = smem + wave * kWords;
   const uint32_t *bits = smem + nwaves * kWords;
   constexpr uint32_t kLead = BITS == 2 ? kRowwalkLead : 0u;  // positions in front of the first input
@@ -109,7 +117,7 @@ __global__ __launch_bounds__(1024, (BITS == 2 || (W == kNormal && sizeof(T1) == 
       else if (bit) acc += static_cast<double>(w);
     };
     auto settle = [&]() { count_event(__builtin_amdgcn_ubfe(late_word, late_idx, 1u), late_w); };
-    walk_stream<T1, W, W != kNormal>(st, lane, seed + o, pre, n_in + kLead, skips, wa, wb,
+    walk_stream<T1, W, true, kShort>(st, lane, seed + o, pre, n_in + kLead, skips, wa, wb,
                                      [&](uint32_t idx, T1 w, bool valid, bool partial) {
       if constexpr (IN == kInEvent && BITS == 2) {
         settle();
@@ -418,7 +426,7 @@ __global__ __launch_bounds__(kColBinThreads, sizeof(T1) == 4 ? 8 : 4) void jitco
         return;
       }
     }
-    walk_stream<T1, W, false, kShort>(st, lane, seed + col, pre, n_out, skips, wa, wb, [&](uint32_t idx, T1 w, bool valid, bool) {
+    walk_stream<T1, W, W == kNormal, kShort>(st, lane, seed + col, pre, n_out, skips, wa, wb, [&](uint32_t idx, T1 w, bool valid, bool) {
       const uint32_t b = idx >> shift;
       // The positions rise from lane to lane and the lanes that hold a synapse are the first ones of the
       // wave, so the lanes of a batch that meet in one window are neighbours (sixteen of them with
@@ -651,7 +659,7 @@ void launch_rowwalk_impl(hipStream_t stream, const VT *in, T1 *out, uint32_t n_o
 template <typename T1, typename VT, int IN, int W>
 void launch_rowwalk_plain(hipStream_t stream, const VT *in, T1 *out, uint32_t n_out, uint32_t n_in, uint32_t seed,
                           double log_p, T1 wa, T1 wb, const RowwalkScratch &sc) {
-  const size_t state_bytes = StreamLds<T1, W>::words * 4;
+  const size_t state_bytes = StreamLds<T1, W, rowwalk_short<T1, IN, W>()>::words * 4;
   const size_t cap = static_cast<size_t>(160) * 1024 - 512;
   // With the generators seeded inside the kernel every workgroup has a ring of seeded states in device
   // memory: 16-wave workgroups, so that the rings in use together are half as many and stay in the L2
@@ -712,7 +720,7 @@ void launch_rowwalk(hipStream_t stream, const VT *in, T1 *out, uint32_t n_out, u
       if (two_level) {
         hipLaunchKernelGGL(coarsen_bitmap_kernel, dim3(div_up(c_words, 256)), dim3(256), 0, stream, bits,
                            static_cast<uint32_t>(words + kRowwalkLead / 32u), g, bits + off, c_words);
-        const size_t state_bytes = StreamLds<T1, W>::words * 4;
+        const size_t state_bytes = StreamLds<T1, W, rowwalk_short<T1, IN, W>()>::words * 4;
         launch_rowwalk_impl<T1, PackedBits, IN, W, 2>(stream, pin, out, n_out, n_in, seed, log_p, wa, wb, 16,
                                                       static_cast<size_t>(c_words) * 4 + 16 * state_bytes, sc);
       } else {
@@ -914,8 +922,11 @@ __global__ __launch_bounds__(256) void check_skips_kernel(uint32_t seed, uint64_
     else if (fast != exact) ++differ;
     const uint32_t close = skip_close(lo, hi, sp, unsafe);
     if (!(unsafe & me) && close != exact) ++differ;
-    const uint32_t quick = skip_quick(hi, sp, unsafe);
-    if (sp.quick && !(unsafe & me) && quick != exact) ++differ;
+    const float uppers[] = {static_cast<float>(hi), canonical_f32_scaled(hi)};
+    for (const float upper : uppers) {
+      const uint32_t quick = skip_quick(hi, upper, sp, unsafe);
+      if (sp.quick && !(unsafe & me) && quick != exact) ++differ;
+    }
   }
   if (differ) atomicAdd(&counts[0], differ);
   if (untrusted) atomicAdd(&counts[1], untrusted);

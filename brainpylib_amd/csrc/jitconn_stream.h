@@ -32,8 +32,8 @@ struct WeightWords {
 // Normal weights: a wave queues the accepted polar attempts and the positions of their synapses in LDS and
 // works the attempts off `drain` at a time, a lane each (the logarithm, division and square root of a weight
 // are two thirds of the instructions of a unit, and three units of ten are accepted attempts: evaluated in
-// place they ran for all 64 lanes of every batch: matvec and its gradient over 1.5e8 synapses 2.35 ms, now
-// 1.87; matmat of 128 rows with 1e7 synapses 234 -> 214 us).  A batch of 64 units accepts at most 22 attempts (an
+// place they ran for all 64 lanes of every batch: matvec and its gradient over 1.5e8 synapses 2.35 -> 1.87
+// ms; matmat of 128 rows with 1e7 synapses 234 -> 214 us).  A batch of 64 units accepts at most 22 attempts (an
 // attempt and its two skips are three units; of double coordinates four, 17), and the positions lag behind the
 // attempts by two at most.  `drain` in double is what leaves 16 waves their 64 KB of static LDS.
 template <typename T1>
@@ -83,15 +83,16 @@ __device__ __forceinline__ double wave_shift_up1(double v) {
 
 // std::normal_distribution<float> (libstdc++, Marsaglia polar): candidate pair from two words
 struct PolarF32 {
-  float x, y, r2;
+  float x, y, r2, u1;  // u1: the second word (capped) as a float
   bool ok;
 };
 __device__ __forceinline__ PolarF32 polar_attempt(uint32_t w0, uint32_t w1) {
   PolarF32 a;
   // 2 * canonical - 1: the scalings by powers of two are exact, so one fused multiply-add rounds where
   // the subtraction of the CPU code rounds
+  a.u1 = canonical_f32_scaled(w1);
   a.x = fmaf(canonical_f32_scaled(w0), 0x1p-31f, -1.0f);
-  a.y = fmaf(canonical_f32_scaled(w1), 0x1p-31f, -1.0f);
+  a.y = fmaf(a.u1, 0x1p-31f, -1.0f);
   a.r2 = __fadd_rn(__fmul_rn(a.x, a.x), __fmul_rn(a.y, a.y));
   a.ok = !(a.r2 > 1.0f || a.r2 == 0.0f);
   return a;
@@ -116,21 +117,31 @@ struct UnitMaps {
   static constexpr uint32_t rejects = kWide ? state_map(1, 0, 3, 0) : state_map(0, 2, 3, 0);
 };
 template <int kDpp, int kRows>
-__device__ __forceinline__ uint32_t compose_behind(uint32_t map) {
-  const uint32_t before = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(
-    static_cast<int>(state_map(0, 1, 2, 3)), static_cast<int>(map), kDpp, kRows, 0xf, false));
+__device__ __forceinline__ uint32_t compose_behind(uint32_t map, uint32_t &before) {
+  before = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(static_cast<int>(before), static_cast<int>(map), kDpp, kRows, 0xf, false));
   return __builtin_amdgcn_perm(map, map, before);
 }
+// What a lane composes its map with in each step.  A step's move leaves the lanes without a lane so far below as they
+// were: they hold the identity for the whole walk (else a register is set to it in front of each of the six moves).
+struct ScanBefore {
+  uint32_t at[6] = {state_map(0, 1, 2, 3), state_map(0, 1, 2, 3), state_map(0, 1, 2, 3),
+                    state_map(0, 1, 2, 3), state_map(0, 1, 2, 3), state_map(0, 1, 2, 3)};
+  // (each in a register of its own from the start)
+  __device__ __forceinline__ ScanBefore() {
+#pragma unroll
+    for (int i = 0; i < 6; ++i) asm volatile("" : "+v"(at[i]));
+  }
+};
 // the state behind this lane's unit; `entered` is the state in front of lane 0's and becomes the one behind lane 63's
 template <bool kWide>
-__device__ __forceinline__ uint32_t state_behind(bool ok, uint32_t &entered) {
+__device__ __forceinline__ uint32_t state_behind(bool ok, uint32_t &entered, ScanBefore &before) {
   uint32_t map = ok ? UnitMaps<kWide>::accepts : UnitMaps<kWide>::rejects;
-  map = compose_behind<0x111, 0xf>(map);  // row_shr:1, 2, 4, 8, then the rows' totals (wave_inclusive_scan_u32)
-  map = compose_behind<0x112, 0xf>(map);
-  map = compose_behind<0x114, 0xf>(map);
-  map = compose_behind<0x118, 0xf>(map);
-  map = compose_behind<0x142, 0xa>(map);
-  map = compose_behind<0x143, 0xc>(map);
+  map = compose_behind<0x111, 0xf>(map, before.at[0]);  // row_shr:1, 2, 4, 8, then the rows' totals (wave_inclusive_scan_u32)
+  map = compose_behind<0x112, 0xf>(map, before.at[1]);
+  map = compose_behind<0x114, 0xf>(map, before.at[2]);
+  map = compose_behind<0x118, 0xf>(map, before.at[3]);
+  map = compose_behind<0x142, 0xa>(map, before.at[4]);
+  map = compose_behind<0x143, 0xc>(map, before.at[5]);
   const uint32_t state = __builtin_amdgcn_ubfe(map, 8u * entered, 8u);
   entered = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(state), kWave - 1));
   return state;
@@ -252,6 +263,10 @@ __device__ __forceinline__ void walk_stream(uint32_t *st, int lane, uint32_t str
     // accepted attempt belongs to the synapse that receives y*mult, the second K to the one that receives the
     // saved x*mult.  Every lane evaluates its unit both ways; state_behind() assigns the roles.  Synapses 2 a
     // and 2 a + 1 of the stream so belong to its accepted attempt a.
+    //
+    // Bound by the issue of vector instructions: 107 per batch of 64 units (39 synapses), a fifth of them the attempts
+    // worked off; 130 before a skip was tried on its upper word, the scan of the roles kept its identities and one count of
+    // lanes gave the queue slots of attempts and positions (row walk of 1.5e8 synapses 841 -> 771 us, double with events 1,847 -> 1,593).
     using Q = NormalQueue<T1>;
     constexpr bool kWide = sizeof(T1) == 8;
     uint32_t *const queue = st + StreamLds<T1, W, kShort>::state_words;
@@ -262,16 +277,18 @@ __device__ __forceinline__ void walk_stream(uint32_t *st, int lane, uint32_t str
     mt_generate<2, 1, kMirror>(mt_base<2, 1, kMirror>(st, lane), pos, lane, w0);
     uint32_t carry = start + __builtin_amdgcn_readfirstlane(skip_from_words<false, true>(w0[0], w0[1], sp, 1ull));
     uint32_t entered = 0;
+    ScanBefore scan_before;
     double prev_v63 = 0.0;
     const uint32_t max_batches = n / 16u + 1024u;
     for (uint32_t b = 0; b < max_batches; ++b) {
       uint32_t w[2] = {1u, 1u};
       mt_generate<2, kWave, kMirror>(base, pos, lane, w);
       T1 x, y;
+      float upper = 0.0f;  // the upper word of a unit that is a skip
       bool ok;
       if constexpr (!kWide) {
         const PolarF32 a = polar_attempt(w[0], w[1]);
-        x = a.x, y = a.y, ok = a.ok;
+        x = a.x, y = a.y, upper = a.u1, ok = a.ok;
       } else {
         y = __dsub_rn(__dmul_rn(2.0, canonical_f64(w[0], w[1])), 1.0);
         x = wave_shift_up1(y);
@@ -281,7 +298,7 @@ __device__ __forceinline__ void walk_stream(uint32_t *st, int lane, uint32_t str
         ok = !(r2 > 1.0 || r2 == 0.0);  // an attempt (lane - 1, lane) would be accepted
       }
       const uint32_t before = entered;
-      const uint32_t state = state_behind<kWide>(ok, entered);
+      const uint32_t state = state_behind<kWide>(ok, entered, scan_before);
       const bool accepted = state == (kWide ? 2u : 1u);
       uint64_t skips;
       if constexpr (kWide) {
@@ -291,21 +308,34 @@ __device__ __forceinline__ void walk_stream(uint32_t *st, int lane, uint32_t str
         skips = __ballot(state >= 2u);
       }
       const bool is_k = __builtin_amdgcn_inverse_ballot_w64(skips);
-      const uint32_t skip_any = skip_from_words<false, true>(w[0], w[1], sp, skips);  // wave-converged call
+      if constexpr (kWide) upper = static_cast<float>(w[1]);
+      const uint32_t skip_any = skip_from_words<kQuick, true>(w[0], w[1], upper, sp, skips);  // wave-converged call
       const uint32_t skip = is_k ? skip_any : 0u;
-      const uint32_t incl = wave_inclusive_scan_u32(skip);
-      const uint32_t idx = carry + incl - skip;
+      uint32_t incl = wave_inclusive_scan_u32(skip);
+      asm volatile("" : "+v"(incl));  // (else the last step of the scan and the addition behind it become three instructions)
+      const uint32_t idx = incl + (carry - skip);
       const uint64_t acc = __ballot(accepted);
+      // Attempt a is in slot a of the queue and its two synapses' positions in slots 2 a and 2 a + 1: the attempts
+      // accepted below a lane give its slot, whichever of the two it holds.
+      const uint32_t attempt = lanes_below(acc, n_attempt);
       if (accepted) {
-        T1 *const q = q_attempt + 2u * lanes_below(acc, n_attempt);
+        T1 *const q = q_attempt + 2u * attempt;
         q[0] = x;
         q[1] = y;
       }
-      if (is_k) q_pos[lanes_below(skips, n_pos)] = idx;
-      const uint64_t done = __ballot(idx >= n) & skips;
-      // (the positions rise: the synapses of the row are the skips below the first one at or past n)
+      if (is_k) {  // (of the attempt before: attempt - 1)
+        if constexpr (kWide) q_pos[2u * attempt - (state == 3u ? 2u : 1u)] = idx;
+        else q_pos[2u * attempt + state - 4u] = idx;
+      }
+      carry += __builtin_amdgcn_readlane(incl, kWave - 1);
+      uint64_t done = 0;
+      if (carry >= whole_below) {
+        done = __ballot(idx >= n) & skips;
+        // (the positions rise: the synapses of the row are the skips below the first one at or past n)
+        if (done) skips &= (done ^ (done - 1u)) & ~done;
+      }
       n_attempt += static_cast<uint32_t>(__popcll(acc));
-      n_pos += static_cast<uint32_t>(__popcll(done ? skips & (done ^ (done - 1u)) & ~done : skips));
+      n_pos += static_cast<uint32_t>(__popcll(skips));
       while (n_pos >= 2u * Q::drain || (done && n_pos != 0u)) {
         __builtin_amdgcn_wave_barrier();
         const uint32_t at = static_cast<uint32_t>(lane);
@@ -339,7 +369,6 @@ __device__ __forceinline__ void walk_stream(uint32_t *st, int lane, uint32_t str
         n_pos -= 2u * Q::drain;
       }
       if (done) break;
-      carry += __builtin_amdgcn_readlane(incl, kWave - 1);
     }
   }
 }

@@ -292,8 +292,9 @@ constexpr double kSkipLog2Error = 3e-7;
 // (measured over all of them by bpl_selfcheck_jitconn_skips); together 1.212e-6, the rest is margin.  It saves
 // 13 of 22 instructions, the tempering of the lower word among them, wherever all of a batch's draws can be trusted: at
 // conn_prob 0.001 in 80 % of the batches (row walk of 1e6 streams of 1,000 synapses: 2,060 -> 1,998 us; 1e5 streams of
-// 1,000 with conn_prob 0.03: 236 -> 215 us, uniform weights 303 -> 279).  Not for normal weights, which need both words
-// of a unit anyway, nor in the column walk into bins, whose 64 registers are full (1e6 short streams: 1,010 -> 1,140 us).
+// 1,000 with conn_prob 0.03: 236 -> 215 us, uniform weights 303 -> 279).  Normal weights have tempered both words of a unit
+// and the upper one as a float for the polar attempt: 6 instructions instead of 14.  Not in the column walk of homogeneous and
+// uniform weights into bins, whose 64 registers are full (1e6 short streams: 1,010 -> 1,140 us).
 constexpr double kQuickLog2Error = 1.4e-6, kQuickLog2Short = 1.72e-7;
 constexpr uint32_t kQuickMin = 1u << 22;
 // Above this guard (conn_prob below about 3e-4) more than half of the batches would take the fast path after it.
@@ -390,8 +391,9 @@ __device__ __forceinline__ uint32_t skip_close(uint32_t lo, uint32_t hi, const S
   return skip;
 }
 
-__device__ __forceinline__ uint32_t skip_quick(uint32_t hi, const SkipParams &sp, uint64_t &unsafe) {
-  const float l2 = __builtin_amdgcn_logf(static_cast<float>(hi) * 0x1p-32f);
+// `upper`: `hi` as a float, or that of `hi` capped at 0xffffff7f (canonical_f32_scaled), which is 2^-24 too little at most.
+__device__ __forceinline__ uint32_t skip_quick(uint32_t hi, float upper, const SkipParams &sp, uint64_t &unsafe) {
+  const float l2 = __builtin_amdgcn_logf(upper * 0x1p-32f);
   const double z = fma(static_cast<double>(l2), sp.inv_log2, sp.quick_offset);
   const uint32_t skip = fixed_skip(z, true, sp.quick_band, unsafe);
   unsafe |= __builtin_amdgcn_ballot_w64(hi < kQuickMin);
@@ -401,12 +403,13 @@ __device__ __forceinline__ uint32_t skip_quick(uint32_t hi, const SkipParams &sp
 // If any lane of the wave is inside the band, the whole wave takes the next path (wave-uniform
 // branches): the fast, the close and the exact one.  Only the lanes in `needed` have to be right.  kQuick: the quick path is
 // tried first.  kTempered: `lo` is a word of the stream; else it is still to be tempered.
+// `upper`: see skip_quick.
 template <bool kQuick, bool kTempered>
-__device__ __forceinline__ uint32_t skip_from_words(uint32_t lo, uint32_t hi, const SkipParams &sp,
+__device__ __forceinline__ uint32_t skip_from_words(uint32_t lo, uint32_t hi, float upper, const SkipParams &sp,
                                                     uint64_t needed = ~0ull) {
   uint64_t unsafe;
   if (kQuick && sp.quick) {
-    const uint32_t quick = skip_quick(hi, sp, unsafe);
+    const uint32_t quick = skip_quick(hi, upper, sp, unsafe);
     if ((unsafe & needed) == 0) return quick;
   }
   if (!kTempered) lo = mt_temper(lo);
@@ -415,6 +418,10 @@ __device__ __forceinline__ uint32_t skip_from_words(uint32_t lo, uint32_t hi, co
   const uint32_t close = skip_close(lo, hi, sp, unsafe);
   if ((unsafe & needed) == 0) return close;
   return skip_exact(lo, hi, sp);
+}
+template <bool kQuick, bool kTempered>
+__device__ __forceinline__ uint32_t skip_from_words(uint32_t lo, uint32_t hi, const SkipParams &sp, uint64_t needed = ~0ull) {
+  return skip_from_words<kQuick, kTempered>(lo, hi, static_cast<float>(hi), sp, needed);
 }
 
 }  // namespace bpl
