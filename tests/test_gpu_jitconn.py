@@ -637,6 +637,21 @@ def test_normal_weights_worked_off_in_groups(cuda, oracle_mod, n_syn, dtype):
   assert_close_reordered(got, want, mag, dtype, what="normal weights, matmat")
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n_in", [90_112, 90_113, 151_552, 151_553])
+@pytest.mark.parametrize("p", [0.003, 0.0002, 0.00005])
+def test_normal_weights_on_both_sides_of_the_bitmaps_and_skip_paths(cuda, oracle_mod, p, n_in, dtype):
+  # the last bitmaps that are exact in LDS and the first two-level ones (float 151,552 inputs, double 90,112), and
+  # conn_probs whose skips are tried on the upper word alone, on both words, and in 13 bits of fraction less
+  rng = np.random.default_rng(n_in)
+  ev = rng.random(n_in) < 0.2
+  kw = dict(w_kind="normal", w_a=0.5, w_b=2.0, log_p=oracle_mod.log_p_of(p), seed=5, n_row=301, n_col=n_in)
+  print("case", p, n_in, dtype.__name__, flush=True)
+  want, mag = oracle_mod.jitconn_matvec(ev, dense=False, return_abs=True, out_dtype=dtype, **kw)
+  assert_close_reordered(kernel_call(ev, col_walk=False, dense=False, out_dtype=dtype, **kw), want, mag, dtype,
+                         what="normal weights, events")
+
+
 @pytest.mark.parametrize("n_out,n_in", [(8192, 3000), (10_007, 200_000), (20_000, 400_000), (70_001, 5000)])
 def test_row_walk_with_generators_seeded_inside_the_kernel(cuda, oracle_mod, n_out, n_in):
   # from 8,192 outputs the row walk seeds its generators itself, 64 streams at a time, into rings of
