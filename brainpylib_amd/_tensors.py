@@ -1,7 +1,9 @@
 """Argument plumbing shared by the operator wrappers: everything becomes a contiguous torch
 CUDA tensor (device memory is PyTorch-ROCm's; nothing is computed with torch)."""
+import ctypes
 import inspect
 import struct
+import threading
 
 import numpy as np
 import torch
@@ -11,6 +13,41 @@ _INDEX_DTYPES = (torch.int32, torch.uint32)
 
 
 _PY_SCALARS = {}  # host tensors of Python numbers seen as operands (read-only)
+
+
+def _is_plain(t):
+  if type(t) is not torch.Tensor or t.is_inference():
+    return False
+  try:
+    t.data_ptr()
+  except RuntimeError:  # a wrapper of a function transform
+    return False
+  return True
+
+
+def _plain(make):
+  """``make()``, a tensor that later calls are given too: one that belongs to no inference mode, function transform or
+  dispatch mode that happens to be active at the first of them.  All of these are a thread's own, so where leaving inference
+  mode is not enough the tensor is made by another thread (on the caller's stream)."""
+  with torch.inference_mode(False):
+    t = make()
+  if _is_plain(t):
+    return t
+  made = []
+  stream = torch.cuda.current_stream() if torch.cuda.is_available() else None
+
+  def work():
+    try:
+      with torch.cuda.stream(stream):
+        made.append(make())
+    except Exception as e:  # (raised below, in the caller's thread)
+      made.append(e)
+  thread = threading.Thread(target=work)
+  thread.start()
+  thread.join()
+  if isinstance(made[0], Exception):
+    raise made[0]
+  return made[0]
 
 
 def as_tensor(a):
@@ -28,7 +65,8 @@ def as_tensor(a):
     if t is None:
       if len(_PY_SCALARS) >= 256:
         _PY_SCALARS.clear()
-      t = _PY_SCALARS[key] = torch.tensor(a, dtype=torch.bool if isinstance(a, bool) else torch.float32)
+      dtype = torch.bool if isinstance(a, bool) else torch.float32
+      t = _PY_SCALARS[key] = _plain(lambda: torch.tensor(a, dtype=dtype, device="cpu"))
     return t
   arr = np.asarray(a)
   if arr.dtype == np.uint32:
@@ -43,7 +81,8 @@ class _NumberTensor:
   __slots__ = ("host", "copies")
 
   def __init__(self, value):
-    self.host = as_tensor(value).reshape(1)
+    scalar = as_tensor(value)
+    self.host = _plain(lambda: scalar.reshape(1))
     self.copies = {}
 
 
@@ -82,18 +121,28 @@ def device_of(*args):
 _HOST_SCALARS = {}
 
 
+def _bits(t):
+  """The bytes of a host tensor of one element."""
+  try:
+    return t.numpy().tobytes()
+  except RuntimeError:
+    if not _is_plain(t):
+      raise
+    return ctypes.string_at(t.data_ptr(), t.element_size())  # (inside a function transform, where numpy() is not to be had)
+
+
 def to_device(t, device):
   if t.device != device:
     if t.numel() == 1 and t.device.type == 'cpu' and not t.requires_grad:
       # A one-element host operand (a homogeneous weight given as a Python number): its device copy
       # is made once per value.  A pageable host-to-device copy per call would cost more than the
       # kernels of a small network.  The operators only read their operands.
-      key = (t.numpy().tobytes(), t.dtype, tuple(t.shape), device)  # (the bits: -0.0 is not 0.0, NaN equals itself)
+      key = (_bits(t), t.dtype, tuple(t.shape), device)  # (the bits: -0.0 is not 0.0, NaN equals itself)
       hit = _HOST_SCALARS.get(key)
       if hit is None:
         if len(_HOST_SCALARS) >= 256:
           _HOST_SCALARS.clear()
-        hit = _HOST_SCALARS[key] = t.to(device).contiguous()
+        hit = _HOST_SCALARS[key] = _plain(lambda: t.to(device).contiguous())
       return hit
     t = t.to(device)
   return t.contiguous()

@@ -141,3 +141,38 @@ def test_signature_of_an_autograd_function_binds_other_calls_as_inspect_does():
   assert bound.args == (1, 2, 3)
   with pytest.raises(TypeError):
     sig.bind(1)
+
+
+@pytest.mark.parametrize("context", ["inference_mode", "grad", "jvp", "vmap"])
+def test_numbers_first_seen_inside_a_mode_or_transform_are_kept_as_plain_tensors(context, monkeypatch):
+  # (the meta device stands for a GPU)
+  from brainpylib_amd import _tensors
+  for table in ("_PY_SCALARS", "_PY_NUMBERS", "_HOST_SCALARS"):
+    monkeypatch.setattr(_tensors, table, {})
+  device = torch.device("meta")
+  own = torch.tensor([0.75])
+
+  def first_call(x):
+    _tensors.number_to_device(_tensors.number_operand(0.6), device)
+    _tensors.as_tensor(0.7)
+    _tensors.to_device(own, device)
+    return (x * x).sum()
+  x = torch.ones(3)
+  if context == "inference_mode":
+    with torch.inference_mode():
+      first_call(x)
+  elif context == "grad":
+    torch.func.grad(first_call)(x)
+  elif context == "jvp":
+    torch.func.jvp(first_call, (x,), (x,))
+  else:
+    torch.func.vmap(first_call)(torch.ones(2, 3))
+  number = _tensors.number_operand(0.6)
+  kept = [number.host, number.copies[device], _tensors.as_tensor(0.6), _tensors.as_tensor(0.7), _tensors.to_device(own, device)]
+  assert kept[1] is _tensors.number_to_device(number, device)
+  for t in kept:
+    t.data_ptr()  # (raises for a transform's wrapper)
+    assert not t.is_inference()
+    y = torch.ones(1, device=t.device, requires_grad=True)
+    (y * t).sum().backward()  # (saves t)
+  assert torch.equal(number.host, torch.tensor([0.6])) and _tensors.as_tensor(0.7).item() == np.float32(0.7)
