@@ -7,6 +7,7 @@ import threading
 
 import numpy as np
 import torch
+from torch.autograd import forward_ad
 
 FLOAT_DTYPES = (torch.float32, torch.float64)
 _INDEX_DTYPES = (torch.int32, torch.uint32)
@@ -118,6 +119,11 @@ def device_of(*args):
   return torch.device("cuda", torch.cuda.current_device())
 
 
+def has_tangent(t):
+  # (outside a dual level, where unpack_dual finds no tangent either, its named tuple is most of the cost)
+  return forward_ad._current_level >= 0 and t.is_floating_point() and forward_ad.unpack_dual(t).tangent is not None
+
+
 _HOST_SCALARS = {}
 
 
@@ -133,7 +139,7 @@ def _bits(t):
 
 def to_device(t, device):
   if t.device != device:
-    if t.numel() == 1 and t.device.type == 'cpu' and not t.requires_grad:
+    if t.numel() == 1 and t.device.type == 'cpu' and not t.requires_grad and not has_tangent(t):
       # A one-element host operand (a homogeneous weight given as a Python number): its device copy
       # is made once per value.  A pageable host-to-device copy per call would cost more than the
       # kernels of a small network.  The operators only read their operands.

@@ -9,10 +9,9 @@ reference hands to cuSPARSE and this package computes with its own scatter kerne
 from typing import Tuple
 
 import torch
-from torch.autograd import forward_ad
 
 from . import _lib
-from ._tensors import (FLOAT_DTYPES, as_tensor, device_of, is_index_dtype, keep_signature, number_operand,
+from ._tensors import (FLOAT_DTYPES, as_tensor, device_of, has_tangent, is_index_dtype, keep_signature, number_operand,
                        number_to_device, to_device)
 
 __all__ = ["csr_matvec", "cusparse_csr_matvec", "csr_to_coo", "coo_to_csr", "csr_to_dense", "check_csr"]
@@ -146,21 +145,16 @@ def _launch(data, indices, indptr, vector, shape, transpose, method='vector'):
 def _wants_grad(*tensors):
   """True if a floating-point argument takes part in reverse- or forward-mode differentiation."""
   for t in tensors:
-    if t.requires_grad or (t.is_floating_point() and _has_tangent(t)):
+    if t.requires_grad or has_tangent(t):
       return True
   return False
-
-
-def _has_tangent(t):
-  # (outside a dual level, where unpack_dual finds no tangent either, its named tuple is most of the cost)
-  return forward_ad._current_level >= 0 and forward_ad.unpack_dual(t).tangent is not None
 
 
 def _transformed(t):
   """True for a tensor whose products must stay visible to a differentiation or batching transform."""
   if torch.is_grad_enabled() and t.requires_grad:
     return True
-  if _has_tangent(t):
+  if has_tangent(t):
     return True
   try:
     t.data_ptr()

@@ -176,3 +176,18 @@ def test_numbers_first_seen_inside_a_mode_or_transform_are_kept_as_plain_tensors
     y = torch.ones(1, device=t.device, requires_grad=True)
     (y * t).sum().backward()  # (saves t)
   assert torch.equal(number.host, torch.tensor([0.6])) and _tensors.as_tensor(0.7).item() == np.float32(0.7)
+
+
+def test_a_host_number_with_a_tangent_keeps_it_on_its_way_to_the_device(monkeypatch):
+  # (the meta device stands for a GPU)
+  import torch.autograd.forward_ad as fwAD
+  from brainpylib_amd import _tensors
+  monkeypatch.setattr(_tensors, "_HOST_SCALARS", {})
+  device = torch.device("meta")
+  t = torch.tensor([0.5])
+  plain = _tensors.to_device(t, device)
+  with fwAD.dual_level():
+    assert _tensors.to_device(t, device) is plain
+    moved = _tensors.to_device(fwAD.make_dual(t, torch.tensor([2.0])), device)
+    assert fwAD.unpack_dual(moved).tangent is not None
+  assert _tensors.to_device(t, device) is plain
