@@ -105,7 +105,9 @@ def number_operand(value):
 def number_to_device(number, device):
   copy = number.copies.get(device)
   if copy is None:
-    copy = number.copies[device] = to_device(number.host, device)
+    copy, kept = _scalar_copy(number.host, device)
+    if kept:
+      number.copies[device] = copy
   return copy
 
 
@@ -124,7 +126,10 @@ def has_tangent(t):
   return forward_ad._current_level >= 0 and t.is_floating_point() and forward_ad.unpack_dual(t).tangent is not None
 
 
+# Device copies of one-element host operands.  One that is here stays: queued calls on other streams and captured graphs
+# may still read it.  What comes when the table is full (512 bytes of device memory an entry) is copied for its call alone.
 _HOST_SCALARS = {}
+_MOST_HOST_SCALARS = 4096
 
 
 def _bits(t):
@@ -137,19 +142,25 @@ def _bits(t):
     return ctypes.string_at(t.data_ptr(), t.element_size())  # (inside a function transform, where numpy() is not to be had)
 
 
+def _scalar_copy(t, device):
+  """A one-element host tensor on a device, and whether the table of copies holds it."""
+  key = (_bits(t), t.dtype, tuple(t.shape), device)  # (the bits: -0.0 is not 0.0, NaN equals itself)
+  hit = _HOST_SCALARS.get(key)
+  if hit is not None:
+    return hit, True
+  copy = _plain(lambda: t.to(device).contiguous())
+  if len(_HOST_SCALARS) >= _MOST_HOST_SCALARS:
+    return copy, False
+  return _HOST_SCALARS.setdefault(key, copy), True  # (another thread may have been first)
+
+
 def to_device(t, device):
   if t.device != device:
     if t.numel() == 1 and t.device.type == 'cpu' and not t.requires_grad and not has_tangent(t):
       # A one-element host operand (a homogeneous weight given as a Python number): its device copy
       # is made once per value.  A pageable host-to-device copy per call would cost more than the
       # kernels of a small network.  The operators only read their operands.
-      key = (_bits(t), t.dtype, tuple(t.shape), device)  # (the bits: -0.0 is not 0.0, NaN equals itself)
-      hit = _HOST_SCALARS.get(key)
-      if hit is None:
-        if len(_HOST_SCALARS) >= 256:
-          _HOST_SCALARS.clear()
-        hit = _HOST_SCALARS[key] = _plain(lambda: t.to(device).contiguous())
-      return hit
+      return _scalar_copy(t, device)[0]
     t = t.to(device)
   return t.contiguous()
 

@@ -191,3 +191,19 @@ def test_a_host_number_with_a_tangent_keeps_it_on_its_way_to_the_device(monkeypa
     moved = _tensors.to_device(fwAD.make_dual(t, torch.tensor([2.0])), device)
     assert fwAD.unpack_dual(moved).tangent is not None
   assert _tensors.to_device(t, device) is plain
+
+
+def test_device_copies_of_numbers_stay_where_graphs_and_streams_may_read_them(monkeypatch):
+  # (the meta device stands for a GPU)
+  from brainpylib_amd import _tensors
+  for table in ("_PY_SCALARS", "_PY_NUMBERS", "_HOST_SCALARS"):
+    monkeypatch.setattr(_tensors, table, {})
+  device = torch.device("meta")
+  copy = lambda v: _tensors.number_to_device(_tensors.number_operand(v), device)
+  most = _tensors._MOST_HOST_SCALARS
+  kept = [copy(i + 0.5) for i in range(most)]
+  late = copy(-1.0)
+  assert _tensors._MOST_HOST_SCALARS <= 4096 and len(_tensors._HOST_SCALARS) == most
+  assert all(any(t is k for k in _tensors._HOST_SCALARS.values()) for t in (kept[0], kept[-1]))
+  assert copy(0.5) is kept[0] and copy(most - 0.5) is kept[-1]
+  assert copy(-1.0) is not late and torch.device("meta") not in _tensors.number_operand(-1.0).copies
