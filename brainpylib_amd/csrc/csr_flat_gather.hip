@@ -42,6 +42,12 @@
 // nonzeros, instead of a line per nonzero.  The rounds' other traffic is under way meanwhile: a step's registers are
 // filled with the next round's indices as soon as its rows are done.  Bound by what of a round does not overlap: staging
 // (1.5 us a window), the test of every place against every window (three instructions), the rows (flat_vector() has the times).
+// A workgroup whose columns lie together has no use for that: it looks at sixteen columns of every wave's first step, and
+// where one window of x holds them or nearly so (the threshold below), it walks step by step with that window in LDS and
+// gathers what it misses.  Which of the two a matrix wants is known on the device only: 300,000 rows of 100 and 120,000 floats,
+// columns within 300 / 3,000 of the row's place 70 / 71 us, with all windows passing by 109 / 109, with the first 147 KB staged
+// 69 / 99; a tenth of them anywhere 78, 109 and 72.  What the look costs where the windows pass by: 0 to 2 us of 85 to 140 (from loads
+// of its own, spread over the workgroup's nonzeros, 2 to 5).
 #include <type_traits>
 
 #include "common.h"
@@ -80,6 +86,13 @@ struct FlatQuads {
   static constexpr int value = sizeof(F) == 4 && OUT != (kFlatSums | kFlatProducts) && FROM != FlatVector::kSwept ? 4 : 2;
 };
 
+// A lane's index quads of a step.
+template <int N>
+struct FlatIndices {
+  static constexpr int count = N;
+  u32x4 q[N];
+};
+
 // The least a wave takes, in nonzeros and rows: a wavefront of quads.  (The plain sums of x in L2 whole steps: a gather
 // costs the address unit the same however many of its lanes hold a nonzero.)
 template <typename F, int OUT, FlatVector FROM>
@@ -94,9 +107,10 @@ struct FlatHeld {
                                static_cast<int>(sizeof(F) / 4);
 };
 
-// (Sums and products of doubles at once: the registers hold one step, and no size pays for the windows.)
-template <typename F, int OUT>
-constexpr bool flat_sweeps() { return !(sizeof(F) == 8 && OUT == (kFlatSums | kFlatProducts)); }
+// (Sums and products of doubles at once: the registers hold one step, and no size pays for the windows.  Doubles with one
+// weight: 150,000 to 500,000 rows of 100 with 37,500 columns take as long either way, more columns longer.)
+template <typename F, bool HETER, int OUT>
+constexpr bool flat_sweeps() { return sizeof(F) == 4 || (HETER && OUT != (kFlatSums | kFlatProducts)); }
 
 // kSwept: a nonzero's register holds where its element of x lies until a window brings the element itself.  The place is
 // written as a NaN with its sign set, one that no element has in LDS: those are stored as the NaN without a payload.
@@ -124,6 +138,12 @@ __device__ __forceinline__ void flat_take(double &v, flat_lds window, uint32_t o
   if (at < bytes / 8u) v = *reinterpret_cast<__attribute__((address_space(3))) const double *>(window + 8u * at);
 }
 constexpr uint32_t kFlatMostPlaces = 1u << 20;  // (of both types' NaNs fewer than that are taken)
+
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {  // (of all 64 lanes, to all of them)
+#pragma unroll
+  for (int d = 1; d < kWave; d *= 2) v = max(v, static_cast<uint32_t>(__shfl_xor(static_cast<int>(v), d, kWave)));
+  return __builtin_amdgcn_readfirstlane(v);
+}
 
 // The n elements of x from `first` on to LDS, eight 16-byte loads of every thread in flight.
 template <typename F>
@@ -235,9 +255,7 @@ __global__ __launch_bounds__(flat_threads(FROM), 4) void csr_flat_gather_kernel(
     const F *__restrict__ data, const uint32_t *__restrict__ indices, const uint32_t *__restrict__ indptr,
     const F *__restrict__ x, F *__restrict__ y, uint32_t n_row, uint32_t n_col, uint32_t min_mean,
     double *__restrict__ head, double *__restrict__ tail, uint32_t *__restrict__ tail_row, uint32_t *__restrict__ range,
-    const F *__restrict__ v, F *__restrict__ products, uint32_t n_products) {
-  constexpr int U = FlatQuads<F, OUT, FROM>::value;
-  constexpr uint32_t kStepQuads = U * kWave;
+    const F *__restrict__ v, F *__restrict__ products, uint32_t n_products, uint32_t least) {
   constexpr int kFlatWaves = flat_threads(FROM) / kWave;
   constexpr bool kStaged = FROM == FlatVector::kStaged, kSwept = FROM == FlatVector::kSwept;
   constexpr bool kSums = (OUT & kFlatSums) != 0, kProducts = (OUT & kFlatProducts) != 0;
@@ -266,6 +284,16 @@ __global__ __launch_bounds__(flat_threads(FROM), 4) void csr_flat_gather_kernel(
     __syncthreads();
   }
   const uint32_t waves = gridDim.x * kFlatWaves, w = blockIdx.x * kFlatWaves + wv;
+  static_assert(sizeof(s_ptr_all) + (kSums ? sizeof(s_sum_all) : 0u) + (kProducts ? sizeof(s_v_all) : 0u) +
+                  (kWave + 4u) * sizeof(uint32_t) + flat_staged_bytes<F, OUT>() <= 160u * 1024u, "LDS of a CU");
+  // (kSwept: how many of the columns looked at lie in each half of a window, the first and the last of them, their number)
+  constexpr uint32_t kHalf = kFits / 2u;
+  __shared__ uint32_t s_half[kSwept ? kWave : 1], s_lowest, s_highest, s_sampled, s_rounds;
+  if constexpr (kSwept) {
+    if (threadIdx.x < kWave) s_half[threadIdx.x] = 0;
+    if (threadIdx.x == 0) s_lowest = kNoRow, s_highest = 0, s_sampled = 0, s_rounds = 0;
+    __syncthreads();
+  }
   // the wave owns the nonzeros [begin, end) and stores the rows [r, row_end), but for one that began before `begin`
   uint32_t share = nnz / waves + kFlatRowWeight * (n_row / waves + 1u) + 1u;
   if (share < flat_min_share<F, OUT, FROM>()) share = flat_min_share<F, OUT, FROM>();
@@ -297,21 +325,20 @@ __global__ __launch_bounds__(flat_threads(FROM), 4) void csr_flat_gather_kernel(
   // The loads carry no condition (a branch per load keeps the compiler from leaving them in flight): a lane beyond
   // the array's last whole quad reads that one again and its elements are masked by their position, and the one to
   // three nonzeros behind it are read where they are used.
-  constexpr uint32_t kStep = 4u * kStepQuads;
   const uint32_t whole = nnz / 4u;
-  auto load_step = [&](uint32_t s0, auto which, u32x4 (&ci)[U], F (&cd)[U][4]) {  // lane l: quads s0 / 4 + l, + 64, ...
-    constexpr int kWhich = decltype(which)::value;
+  auto load_step = [&](uint32_t s0, auto which, auto &ci, auto &cd) {  // lane l: quads s0 / 4 + l, + 64, ...
+    constexpr int kWhich = decltype(which)::value, U = std::remove_reference_t<decltype(ci)>::count;
     if (s0 >= end || whole == 0) {
       // (what is not loaded is not kept either: its registers are free)
 #pragma unroll
-      for (int u = 0; kSwept && (kWhich & kStepIndices) && u < U; ++u) ci[u] = u32x4{};
+      for (int u = 0; kSwept && (kWhich & kStepIndices) && u < U; ++u) ci.q[u] = u32x4{};
       return;
     }
     if constexpr ((kWhich & kStepIndices) != 0) {
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const uint32_t q = s0 / 4u + static_cast<uint32_t>(u) * kWave + lane;
-        ci[u] = flat_index_quad(indices, q < whole ? q : whole - 1u);
+        ci.q[u] = flat_index_quad(indices, q < whole ? q : whole - 1u);
       }
     }
     if constexpr (kWeights && (kWhich & kStepWeights) != 0) {
@@ -341,14 +368,14 @@ __global__ __launch_bounds__(flat_threads(FROM), 4) void csr_flat_gather_kernel(
     if constexpr (kProducts) asm volatile("" : "+v"(v_lane));
   };
   // The array's last one to three nonzeros, where the step holds them.
-  auto load_last = [&](uint32_t s0, auto which, u32x4 (&ci)[U], F (&cd)[U][4]) {
-    constexpr int kWhich = decltype(which)::value;
+  auto load_last = [&](uint32_t s0, auto which, auto &ci, auto &cd) {
+    constexpr int kWhich = decltype(which)::value, U = std::remove_reference_t<decltype(ci)>::count;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       if (s0 / 4u + static_cast<uint32_t>(u) * kWave + lane != whole) continue;
       const uint32_t p0 = 4u * whole;
       if constexpr ((kWhich & kStepIndices) != 0)
-        ci[u] = u32x4{indices[p0], p0 + 1u < nnz ? indices[p0 + 1u] : 0u, p0 + 2u < nnz ? indices[p0 + 2u] : 0u, 0u};
+        ci.q[u] = u32x4{indices[p0], p0 + 1u < nnz ? indices[p0 + 1u] : 0u, p0 + 2u < nnz ? indices[p0 + 2u] : 0u, 0u};
       if constexpr (kWeights && (kWhich & kStepWeights) != 0) {
         cd[u][0] = data[p0];
         if (p0 + 1u < nnz) cd[u][1] = data[p0 + 1u];
@@ -360,7 +387,8 @@ __global__ __launch_bounds__(flat_threads(FROM), 4) void csr_flat_gather_kernel(
   using Weights = std::integral_constant<int, kStepWeights>;
   using Both = std::integral_constant<int, kStepIndices | kStepWeights>;
   // The rows of the step [s0, s1).  prod: its products, with products to store (kProducts) the elements of x; cw: its weights.
-  auto walk_rows = [&](uint32_t s0, uint32_t s1, const F (&prod)[U][4], const F (&cw)[U][4]) {
+  auto walk_rows = [&](uint32_t s0, uint32_t s1, const auto &prod, const auto &cw) {
+    constexpr int U = static_cast<int>(std::extent_v<std::remove_reference_t<decltype(prod)>>);
     auto addend = [&](int u, int t) {
       return static_cast<double>(kProducts ? static_cast<F>(prod[u][t] * cw[u][t]) : prod[u][t]);
     };
@@ -469,7 +497,8 @@ __global__ __launch_bounds__(flat_threads(FROM), 4) void csr_flat_gather_kernel(
     }
     __builtin_amdgcn_wave_barrier();
   };
-  auto multiply = [&](F (&prod)[U][4], const F (&cw)[U][4]) {
+  auto multiply = [&](auto &prod, const auto &cw) {
+    constexpr int U = static_cast<int>(std::extent_v<std::remove_reference_t<decltype(prod)>>);
     if constexpr (!kProducts) {
 #pragma unroll
       for (int u = 0; u < U; ++u) {
@@ -478,30 +507,42 @@ __global__ __launch_bounds__(flat_threads(FROM), 4) void csr_flat_gather_kernel(
       }
     }
   };
-  if constexpr (!kSwept) {
-    u32x4 ci[U] = {};
+  // Step by step, with the n_lds elements of x from `origin` on in LDS (kInLds).
+  auto walk_steps = [&](auto in_lds, auto origin, uint32_t n_lds, auto &&stage) {
+    constexpr bool kInLds = decltype(in_lds)::value;
+    constexpr int U = FlatQuads<F, OUT, kInLds ? FlatVector::kStaged : FlatVector::kL2>::value;
+    constexpr uint32_t kStep = 4u * U * kWave;
+    FlatIndices<U> ci = {};
     F cd[U][4] = {};
     load_step(begin & ~3u, Both(), ci, cd);
+    stage();
     // (a range without nonzeros has one step, for its rows)
     for (uint32_t s0 = begin & ~3u;; s0 += kStep) {
       const uint32_t s1 = (end - s0 > kStep) ? s0 + kStep : end;
       load_window();
       if (s1 > 4u * whole) load_last(s0, Both(), ci, cd);
       F prod[U][4];  // (the vector's elements first, then the products: in F, as the reference forms them)
-      auto column = [&](int u, int t) {  // (beyond the step: element 0, unused)
+      auto column = [&](int u, int t) {  // (beyond the step: one that costs nothing, unused)
         const uint32_t p = 4u * (s0 / 4u + static_cast<uint32_t>(u) * kWave + lane) + static_cast<uint32_t>(t);
-        return p < s1 ? ci[u][t] : 0u;
+        return p < s1 ? ci.q[u][t] : static_cast<uint32_t>(origin);
       };
-      if constexpr (kStaged) {
+      auto place = [&](uint32_t c) {  // (in a window that may run on at element 0)
+        if constexpr (std::is_same_v<decltype(origin), uint32_t>) return min(c - origin, c - origin + n_col);
+        else return c;
+      };
+      if constexpr (kInLds) {
+        const uint32_t last = n_lds - 1u;
+        uint32_t furthest = 0;
 #pragma unroll
         for (int u = 0; u < U; ++u) {
 #pragma unroll
           for (int t = 0; t < 4; ++t) {
-            const uint32_t c = column(u, t);
-            prod[u][t] = s_x[c < staged ? c : 0u];
+            const uint32_t at = place(column(u, t));
+            prod[u][t] = s_x[min(at, last)];
+            furthest = max(furthest, at);
           }
         }
-        if (staged < n_col) {  // (uniform)
+        if (__builtin_amdgcn_ballot_w64(furthest > last) != 0) {
           // (all LDS reads first: without the empty statements each would be moved into the branch around the load)
 #pragma unroll
           for (int u = 0; u < U; ++u) {
@@ -513,7 +554,7 @@ __global__ __launch_bounds__(flat_threads(FROM), 4) void csr_flat_gather_kernel(
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
               const uint32_t c = column(u, t);
-              if (c >= staged) prod[u][t] = x[c];
+              if (place(c) > last) prod[u][t] = x[c];
             }
           }
         }
@@ -535,21 +576,67 @@ __global__ __launch_bounds__(flat_threads(FROM), 4) void csr_flat_gather_kernel(
       walk_rows(s0, s1, prod, cw);
       if (s1 == end) break;
     }
-  } else {
-    constexpr int H = FlatHeld<F, HETER, OUT>::value;
-    u32x4 ci[H][U] = {};
-    F cd[2][U][4] = {};  // weights, a step ahead
-    //static_assert(H % 2 == 0 || !kWeights);
-    uint32_t s0 = begin & ~3u;  // the round takes [s0, s0 + H * kStep)
-    const uint32_t own = idle ? 0u : s0 < end ? (end - s0 - 1u) / (H * kStep) + 1u : 1u;
-    __shared__ uint32_t s_rounds;
-    if (threadIdx.x == 0) s_rounds = 0;
-    __syncthreads();
+  };
+  constexpr int kHeldSteps = FlatHeld<F, HETER, OUT>::value, kHeldQuads = FlatQuads<F, OUT, FROM>::value;
+  constexpr uint32_t kHeld = 4u * kHeldQuads * kWave * kHeldSteps;  // nonzeros of a wave's round
+  const uint32_t own = idle ? 0u : (begin & ~3u) < end ? (end - (begin & ~3u) - 1u) / kHeld + 1u : 1u;  // its rounds
+  uint32_t origin = kNoRow, n_lds = kFits;
+  FlatIndices<kHeldQuads> first_step = {};
+  if constexpr (kSwept) {
+    F unused[kHeldQuads][4];
+    load_step(begin & ~3u, Indices(), first_step, unused);  // (under way meanwhile)
+    if ((begin & ~3u) < end && whole != 0) {  // sixteen columns of every wave
+      const uint32_t column = first_step.q[0][0];
+      const bool sampled = lane % 4u == 0;
+      if (sampled) atomicAdd(&s_half[column / kHalf < kWave ? column / kHalf : kWave - 1u], 1u);
+      const uint32_t lowest = ~wave_max_u32(sampled ? ~column : 0u), highest = wave_max_u32(sampled ? column : 0u);
+      if (lane == 0) atomicMin(&s_lowest, lowest), atomicMax(&s_highest, highest), atomicAdd(&s_sampled, kWave / 4u);
+    }
     if (lane == 0) atomicMax(&s_rounds, own);
-#pragma unroll
-    for (int h = 0; h < H; ++h) load_step(s0 + static_cast<uint32_t>(h) * kStep, Indices(), ci[h], cd[0]);
-    load_step(s0, Weights(), ci[0], cd[0]);
     __syncthreads();
+    // One window for all columns looked at, with room for those between and beyond them; else the two neighbouring halves
+    // that hold most (the last and the first element are neighbours: a ring's first and last rows), if what they miss is at
+    // most half of what the launcher takes to be worth the windows (where every column is as likely, 256 columns tell a
+    // share of 0.3 to 0.03, and one workgroup that gathers a third of its elements is the last of all: a threshold of
+    // three quarters took 60,000,000 nonzeros over 200,000 floats from 250 to 259 us).
+    const uint32_t lowest = s_lowest, highest = s_highest;
+    if (lowest <= highest && highest < n_col) {
+      const uint32_t pad = (highest - lowest) / 16u + 64u;
+      const uint32_t from = (lowest > pad ? lowest - pad : 0u) & ~3u, to = n_col - highest > pad ? highest + pad : n_col;
+      if (to - from <= kFits) {
+        origin = from, n_lds = to - from;
+      } else {
+        const uint32_t halves = (n_col - 1u) / kHalf + 1u;
+        const uint32_t both = lane < halves ? s_half[lane] + s_half[lane + 1u < halves ? lane + 1u : 0u] : 0u;
+        const uint32_t most = wave_max_u32(both), sampled = s_sampled;
+        const uint32_t first = kHalf * static_cast<uint32_t>(__builtin_ctzll(__builtin_amdgcn_ballot_w64(both == most)));
+        if (2u * (sampled - most) * static_cast<uint64_t>(nnz) < sampled * static_cast<uint64_t>(least))
+          origin = first + (n_col - first) % 4u;  // (what lies behind the last element is a multiple of 16 bytes from the first)
+      }
+      origin = __builtin_amdgcn_readfirstlane(origin), n_lds = __builtin_amdgcn_readfirstlane(n_lds);
+    }
+  }
+  if constexpr (!kSwept) {
+    walk_steps(std::integral_constant<bool, kStaged>(), std::integral_constant<uint32_t, 0u>(), staged, []() {});
+  } else if (origin != kNoRow) {
+    auto stage = [&]() {
+      const uint32_t to_end = n_col - origin;
+      copy_to_lds(s_x, x + origin, n_lds < to_end ? n_lds : to_end);
+      if (n_lds > to_end) copy_to_lds(s_x + to_end, x, n_lds - to_end);
+      __syncthreads();
+    };
+    if (idle) stage();
+    else walk_steps(std::true_type(), origin, n_lds, stage);
+  } else {
+    constexpr int H = kHeldSteps, U = kHeldQuads;
+    constexpr uint32_t kStep = 4u * U * kWave;
+    FlatIndices<U> ci[H] = {};
+    F cd[2][U][4] = {};  // weights, a step ahead
+    uint32_t s0 = begin & ~3u;  // the round takes [s0, s0 + H * kStep)
+    ci[0] = first_step;
+#pragma unroll
+    for (int h = 1; h < H; ++h) load_step(s0 + static_cast<uint32_t>(h) * kStep, Indices(), ci[h], cd[0]);
+    load_step(s0, Weights(), ci[0], cd[0]);
     const uint32_t rounds = __builtin_amdgcn_readfirstlane(s_rounds);
     const uint32_t windows = (n_col - 1u) / kFits + 1u;
     const uint32_t width = ((n_col - 1u) / windows + 4u) & ~3u;  // (at most kFits, a multiple of 4)
@@ -567,7 +654,7 @@ __global__ __launch_bounds__(flat_threads(FROM), 4) void csr_flat_gather_kernel(
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
               const uint32_t p = 4u * (sh / 4u + static_cast<uint32_t>(u) * kWave + lane) + static_cast<uint32_t>(t);
-              prod[h][u][t] = p < end ? flat_place(F(0), ci[h][u][t]) : F(0);
+              prod[h][u][t] = p < end ? flat_place(F(0), ci[h].q[u][t]) : F(0);
             }
           }
         }
@@ -665,27 +752,33 @@ bool flat_stages(uint32_t n_col) {
   return static_cast<uint64_t>(n_col) * sizeof(F) <= 552ull * 1024u;
 }
 
-// Where the walk takes x from.  A visit of a window (147 KB staged and a test of every place held, 3 us with nothing beside
-// it) has to spare 1.15 million gathers (double 0.7; with one weight 1.5: no weights to request meanwhile), and a call a
-// million.  Measured, before and now (300,000 rows of 100 where not said; the weights' gradient with them):
-// 60,000 / 120,000 / 180,000 floats 95 / 133 / 154 -> 89 / 111 / 128 us, one weight and 120,000 107 -> 102, 30,000 / 60,000
-// doubles 124 / 159 -> 105 / 140; 30,000 rows of 1,000 and 150,000 146 -> 118.  On the other side of the line: 240,000 floats 156
-// and 157 (149 with 32 places a lane, which spill), 480,000 158 and 261, 100,000 rows of 80 and 75,000 36.2 and 37.1, of 30 and
-// 120,000 23 and 28, one weight and 60,000 doubles 112 and 123.
+// Where the walk takes x from, if its columns lie anywhere (the kernel itself looks whether they do).  A visit of a window (147 KB staged
+// and a test of every place held, 3 us with nothing beside it) has to spare 1.15 million gathers (double 0.7; with one weight
+// 1.4: no weights to request meanwhile), a call a million (one weight 2.0), and x has to be longer than what fits by as much as makes a gather cost a
+// line of its own (weights 1.5 times, one weight twice: 50,000 floats and 1e8 nonzeros in rows of 100 220 us, by windows 242, one weight and 75,000
+// 241 and 241).  Measured without windows and now (300,000 rows of 100 where not said): 60,000 / 120,000 / 180,000 floats 92 / 130 / 152
+// -> 86 / 107 / 122 us, the weights' gradient 91 / 118 / 144 -> 71 / 85 / 97, both gradients 123 / 159 / 172 -> 102 / 123 / 139, one weight
+// 120,000 / 180,000 106 / 139 -> 100 / 113, doubles 30,000 / 60,000 / 90,000 123 / 158 / 183 -> 104 / 137 / 160, their gradient 140 / 166 / 183 ->
+// 106 / 127 / 142; 30,000 rows of 1,000 and 150,000 floats 150 -> 114.  On the other side of the line, with and without:
+// 260,000 floats 148 and 154, 200,000 with 1e7 nonzeros 58 and 59, 5e6 37 and 36; one weight and 60,000 84 and 73, 260,000 135 and 141.
 template <typename F, bool HETER, int OUT>
-static FlatVector flat_vector(uint32_t n_col, uint32_t nnz) {
+static FlatVector flat_vector(uint32_t n_col, uint32_t nnz, uint32_t *least) {
   constexpr uint32_t kFits = flat_staged_bytes<F, OUT>() / sizeof(F);
   constexpr FlatVector kSwept = FlatVector::kSwept;
   if (n_col <= kFits) return FlatVector::kStaged;
-  if constexpr (flat_sweeps<F, OUT>()) {
+  if constexpr (flat_sweeps<F, HETER, OUT>()) {
     const uint64_t waves = static_cast<uint64_t>(device_info().num_cu) * (flat_threads(kSwept) / kWave);
     const uint64_t round = waves * kWave * 4u * FlatQuads<F, OUT, kSwept>::value * FlatHeld<F, HETER, OUT>::value;
     const uint64_t visits = 1u + static_cast<uint64_t>((n_col - 1u) / kFits) * (nnz / round + 1u);
     const uint64_t gathers = flat_stages<F>(n_col) ? nnz - static_cast<uint64_t>(nnz) * kFits / n_col : nnz;
-    constexpr bool kOneWeight = !HETER && (OUT & kFlatSums);
-    constexpr uint32_t kPerVisit = kOneWeight ? 1500000u : sizeof(F) == 4 ? 1150000u : 700000u;
-    constexpr uint32_t kPerCall = sizeof(F) == 4 ? 1000000u : 500000u;
-    if (n_col <= kFlatMostPlaces && gathers >= visits * kPerVisit + kPerCall) return kSwept;
+    constexpr uint32_t kPerVisit = !HETER ? 1400000u : sizeof(F) == 4 ? 1150000u : 700000u;
+    constexpr uint32_t kPerCall = !HETER ? 2000000u : 1000000u;
+    constexpr uint32_t kLeast = !HETER ? 2u * kFits : OUT == kFlatSums && sizeof(F) == 4 ? kFits + kFits / 2u : kFits;
+    const uint64_t worth = visits * kPerVisit + kPerCall;
+    *least = static_cast<uint32_t>(worth);  // (gathers is below 2^32)
+    constexpr uint32_t kHalves = kFits / 2u * kWave;  // (the kernel's histogram of the columns)
+    constexpr uint32_t kMost = kHalves < kFlatMostPlaces ? kHalves : kFlatMostPlaces;
+    if (n_col > kLeast && n_col <= kMost && gathers >= worth) return kSwept;
   }
   return flat_stages<F>(n_col) ? FlatVector::kStaged : FlatVector::kL2;
 }
@@ -693,7 +786,7 @@ static FlatVector flat_vector(uint32_t n_col, uint32_t nnz) {
 template <typename F, bool HETER, int OUT, FlatVector FROM>
 static bool launch_flat(const char *target, hipStream_t stream, const F *data, const uint32_t *indices,
                         const uint32_t *indptr, const F *x, F *y, uint32_t n_row, uint32_t n_col, uint32_t min_mean,
-                        const F *v, F *products, uint32_t n_products) {
+                        const F *v, F *products, uint32_t n_products, uint32_t least) {
   constexpr bool kSums = (OUT & kFlatSums) != 0;
   const unsigned grid = static_cast<unsigned>(device_info().num_cu) * flat_per_cu(FROM);
   const uint32_t waves = grid * (flat_threads(FROM) / kWave);
@@ -723,7 +816,7 @@ static bool launch_flat(const char *target, hipStream_t stream, const F *data, c
     }
   }
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(flat_threads(FROM)), lds, stream, data, indices, indptr, x, y, n_row,
-                     n_col, min_mean, head, tail, tail_row, range, v, products, n_products);
+                     n_col, min_mean, head, tail, tail_row, range, v, products, n_products, least);
   if (kSums)
     hipLaunchKernelGGL(csr_flat_finish_kernel<F>, dim3(waves), dim3(kWave), 0, stream, indptr, y, n_row, min_mean,
                        waves, static_cast<const double *>(head), static_cast<const double *>(tail),
@@ -735,14 +828,16 @@ template <typename F, bool HETER, int OUT>
 static bool flat_walk(const char *target, hipStream_t stream, const F *data, const uint32_t *indices, const uint32_t *indptr,
                       const F *x, F *y, uint32_t n_row, uint32_t n_col, uint32_t nnz, uint32_t min_mean, const F *v,
                       F *products) {
+  uint32_t least = 0;
+  const FlatVector from = flat_vector<F, HETER, OUT>(n_col, nnz, &least);
   auto launch = [&](auto from) {
     return launch_flat<F, HETER, OUT, decltype(from)::value>(target, stream, data, indices, indptr, x, y, n_row, n_col,
-                                                             min_mean, v, products, (OUT & kFlatProducts) ? nnz : 0u);
+                                                             min_mean, v, products, (OUT & kFlatProducts) ? nnz : 0u, least);
   };
-  switch (flat_vector<F, HETER, OUT>(n_col, nnz)) {
+  switch (from) {
     case FlatVector::kStaged: return launch(std::integral_constant<FlatVector, FlatVector::kStaged>());
     case FlatVector::kSwept:
-      if constexpr (flat_sweeps<F, OUT>()) return launch(std::integral_constant<FlatVector, FlatVector::kSwept>());
+      if constexpr (flat_sweeps<F, HETER, OUT>()) return launch(std::integral_constant<FlatVector, FlatVector::kSwept>());
     default: return launch(std::integral_constant<FlatVector, FlatVector::kL2>());
   }
 }

@@ -1407,7 +1407,7 @@ def test_a_block_of_rows_costs_what_its_nonzeros_cost(cuda, n_row, n_col, long, 
 # the last whole quad.  Integers: every order of the sums gives the same bits.
 @pytest.mark.parametrize("dtype,n_col,nnz,homo", [
   (np.float32, 75_264, 9_400_003, False), (np.float32, 75_265, 18_800_001, False), (np.float32, 150_001, 25_000_002, False),
-  (np.float32, 75_000, 12_000_001, True), (np.float64, 37_632, 8_000_001, False), (np.float64, 60_001, 24_000_003, False)])
+  (np.float32, 75_000, 12_000_001, True), (np.float32, 110_000, 30_000_002, True), (np.float64, 37_632, 8_000_001, False), (np.float64, 60_001, 24_000_003, False)])
 def test_csr_matvec_windows_of_the_vector_pass_by(dtype, n_col, nnz, homo):
   rng = np.random.default_rng(n_col + nnz)
   n_row = 50_021
@@ -1451,3 +1451,51 @@ def test_csr_matvec_windows_of_the_vector_pass_by(dtype, n_col, nnz, homo):
     np.testing.assert_array_equal(g_w.cpu().numpy(), v[row] * x[indices])
     if transpose:
       np.testing.assert_array_equal(g_v.cpu().numpy(), product(x).astype(dtype))
+
+
+# The same sizes where the columns of a workgroup's rows lie together: one window in LDS instead of all that pass by, chosen by
+# each workgroup (a window around all columns looked at, two halves that hold most of them, the last and the first
+# elements of a ring), and matrices whose workgroups choose differently.
+@pytest.mark.parametrize("dtype,n_col,nnz,homo", [
+  (np.float32, 150_001, 25_000_002, False), (np.float32, 120_002, 40_000_003, True), (np.float64, 60_001, 24_000_003, False)])
+@pytest.mark.parametrize("columns", ["band", "wide band", "ring", "few anywhere", "half the rows anywhere", "last elements"])
+def test_csr_matvec_columns_that_lie_together(dtype, n_col, nnz, homo, columns):
+  rng = np.random.default_rng(n_col + nnz)
+  n_row = 40_009
+  lengths = np.concatenate([np.zeros(300, np.int64), [100_000],
+                            rng.multinomial(nnz - 100_000, rng.dirichlet(np.full(n_row - 301, 0.5)))])
+  indptr = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+  row = np.repeat(np.arange(n_row), lengths)
+  near = row * (n_col / n_row)
+  width = {"wide band": 14_000, "last elements": 200}.get(columns, 300)
+  if columns == "last elements":
+    near[:] = n_col - 1 - width
+  indices = near.astype(np.int64) + rng.integers(-width, width + 1, nnz)
+  if columns in ("ring", "few anywhere"):
+    indices %= n_col
+  indices = np.clip(indices, 0, n_col - 1)
+  if columns == "few anywhere":
+    indices = np.where(rng.random(nnz) < 0.08, rng.integers(0, n_col, nnz), indices)
+  elif columns == "half the rows anywhere":
+    indices = np.where(row % 10_000 < 5_000, rng.integers(0, n_col, nnz), indices)
+  indices = indices.astype(np.int32)
+  x = rng.integers(-8, 9, n_col).astype(dtype)
+  x[[0, n_col // 3, n_col - 1]] = np.inf, np.nan, -np.inf
+  data = np.array([3.0], dtype) if homo else rng.integers(1, 5, nnz).astype(dtype)
+  dev = [torch.from_numpy(a).cuda() for a in (data, indices, indptr)]
+  print("case", dtype.__name__, n_col, nnz, homo, columns, flush=True)
+  got = bpl.csr_matvec(*dev, torch.from_numpy(x).cuda(), shape=(n_row, n_col)).cpu().numpy()
+  with np.errstate(invalid="ignore"):
+    want = np.bincount(row, weights=(data * x[indices]).astype(np.float64), minlength=n_row)
+  np.testing.assert_array_equal(got, want.astype(dtype))
+  if homo:
+    return
+  v = rng.integers(1, 9, n_row).astype(dtype)
+  for transpose in (False, True):  # the weights' gradient alone, and with the vector's in the same walk
+    weights = dev[0].clone().requires_grad_()
+    vec = torch.from_numpy(v if transpose else x).cuda().requires_grad_()
+    out = bpl.cusparse_csr_matvec(weights, *dev[1:], vec, shape=(n_row, n_col), transpose=transpose)
+    g_w, g_v = torch.autograd.grad(out, (weights, vec), torch.from_numpy(x if transpose else v).cuda())
+    np.testing.assert_array_equal(g_w.cpu().numpy(), v[row] * x[indices])
+    if transpose:
+      np.testing.assert_array_equal(g_v.cpu().numpy(), want.astype(dtype))
