@@ -181,7 +181,8 @@ __device__ __forceinline__ uint32_t lanes_below(uint64_t mask, uint32_t base) {
 //
 // `loaded()` is called once, when the generator state is in LDS and `pre` is no longer read.
 //
-// `start`: what the indices are counted from (the walk ends at `n`, counted alike).
+// `start`: what the indices are counted from (the walk ends at `n`, counted alike).  The ends are found in positions without
+// it: a skip may lead to a position just under 2^32, which is beyond every row, and `start` more would lead around.
 struct NoLoadHook {
   __device__ __forceinline__ void operator()() const {}
 };
@@ -216,7 +217,7 @@ __device__ __forceinline__ void walk_stream(uint32_t *st, int lane, uint32_t str
       uint64_t done = 0;
       if (partial) {
         // (the positions rise from lane to lane: the lanes of the row are those below the first one at or past n)
-        done = __builtin_amdgcn_ballot_w64(idx >= n);
+        done = __builtin_amdgcn_ballot_w64(idx - start >= n - start);
         valid = done == 0 || lane < static_cast<int>(__builtin_ctzll(done));
         idx = valid ? idx : 0u;
         asm volatile("" : "+v"(idx));  // (a branch, not a select in every batch)
@@ -248,7 +249,7 @@ __device__ __forceinline__ void walk_stream(uint32_t *st, int lane, uint32_t str
       bool valid = true;
       uint64_t done = 0;
       if (partial) {
-        done = __builtin_amdgcn_ballot_w64(idx >= n) & (~0ull >> (kWave - NL));
+        done = __builtin_amdgcn_ballot_w64(idx - start >= n - start) & (~0ull >> (kWave - NL));
         valid = lane < (done ? static_cast<int>(__builtin_ctzll(done)) : NL);
         idx = valid ? idx : 0u;
         asm volatile("" : "+v"(idx));
@@ -330,7 +331,7 @@ __device__ __forceinline__ void walk_stream(uint32_t *st, int lane, uint32_t str
       carry += __builtin_amdgcn_readlane(incl, kWave - 1);
       uint64_t done = 0;
       if (carry >= whole_below) {
-        done = __ballot(idx >= n) & skips;
+        done = __ballot(idx - start >= n - start) & skips;
         // (the positions rise: the synapses of the row are the skips below the first one at or past n)
         if (done) skips &= (done ^ (done - 1u)) & ~done;
       }

@@ -652,6 +652,36 @@ def test_normal_weights_on_both_sides_of_the_bitmaps_and_skip_paths(cuda, oracle
                          what="normal weights, events")
 
 
+def _stream_that_skips_to_the_end_of_the_integers(w_kind, n_in):
+  """(seed, log_p, the index that the second skip would lead to from 2^32 - 16 on, counted around): the first skip of the
+  stream is 2^32 - 16, the second one so short that a walk that went on would find an input."""
+  for seed in range(200_000):
+    words = np.random.RandomState(seed).randint(0, 1 << 32, 64, dtype=np.uint64).astype(np.float64)
+    log_u = lambda i: np.log((words[i] + words[i + 1] * 2.0 ** 32) * 2.0 ** -64)
+    at = {"homo": 2, "uniform": 3, "normal": 2}[w_kind]
+    if w_kind == "normal":
+      while (2 * words[at] * 2.0 ** -32 - 1) ** 2 + (2 * words[at + 1] * 2.0 ** -32 - 1) ** 2 > 1:
+        at += 2
+      at += 2
+    log_p = log_u(0) / (2.0 ** 32 - 16.5)
+    second = np.ceil(log_u(at) / log_p)
+    if np.ceil(log_u(0) / log_p) == 2.0 ** 32 - 16 and 100 < second < n_in - 100:
+      return seed, log_p, int(second) - 16
+  raise AssertionError("no such stream")
+
+
+@pytest.mark.parametrize("w_kind", KINDS_BUILT)
+@pytest.mark.parametrize("dtype", [np.bool_, np.float32])
+def test_a_skip_to_just_below_two_to_the_32_ends_the_row(cuda, oracle_mod, w_kind, dtype):
+  n_in = 400_000  # (a two-level bitmap, whose positions begin at 32)
+  seed, log_p, index = _stream_that_skips_to_the_end_of_the_integers(w_kind, n_in)
+  ev = np.zeros(n_in, dtype)
+  ev[index] = 1
+  kw = dict(w_kind=w_kind, w_a=0.5, w_b=2.0, log_p=log_p, seed=seed, n_row=1, n_col=n_in)
+  assert oracle_mod.jitconn_matvec(ev, dense=False, **kw)[0] == 0
+  assert kernel_call(ev, col_walk=False, dense=False, **kw)[0] == 0
+
+
 @pytest.mark.parametrize("n_out,n_in", [(8192, 3000), (10_007, 200_000), (20_000, 400_000), (70_001, 5000)])
 def test_row_walk_with_generators_seeded_inside_the_kernel(cuda, oracle_mod, n_out, n_in):
   # from 8,192 outputs the row walk seeds its generators itself, 64 streams at a time, into rings of
