@@ -62,18 +62,23 @@ constexpr uint32_t kFuseBatch = 64;   // streams seeded together, one per lane
 constexpr uint32_t kFuseSlots = 3;    // batches of seeded states in a workgroup's ring
 constexpr uint32_t kFuseNumbers = 8;  // batch numbers a row-walk workgroup remembers (more than a wave can fall behind)
 constexpr uint32_t kFuseLdsWords = 16;  // the row walk's counters and numbers, in front of the states
+constexpr uint32_t kFuseRoundBits = 5;  // a number's place in the eight is told from its last use by this many bits below it
 static_assert(1 + 2 * kFuseSlots + kFuseNumbers <= kFuseLdsWords, "room for them");
 constexpr uint32_t kFuseSpin = 1u << 22;           // polls of a flag in LDS before a wave stops waiting
 constexpr uint32_t kFuseNotSeeded = 0x80000000u;   // flag bit: the batch's rows seed their own generators
 constexpr size_t kFuseRingBytes = static_cast<size_t>(kFuseSlots) * kFuseBatch * kMtN * sizeof(uint32_t);  // per workgroup
 static_assert(kMtSeedTileWords <= kMtN, "the seeding wave transposes through its own state buffer");
 
-template <typename T1, typename VT, int IN, int W, int BITS, bool FUSED>
-__global__ __launch_bounds__(1024, (BITS == 2 || (W == kNormal && sizeof(T1) == 4)) ? 8 : 4)
+// (The self-check's waves give up waiting for a seeded state after no poll or after three: kNoPolls, kThreePolls added to BITS.)
+constexpr int kNoPolls = 4, kThreePolls = 8;
+template <typename T1, typename VT, int IN, int W, int FORM, bool FUSED>
+__global__ __launch_bounds__(1024, (FORM == 2 || (W == kNormal && sizeof(T1) == 4)) ? 8 : 4)
     __attribute__((amdgpu_num_sgpr(80))) void jitconn_rowwalk_kernel(const VT *__restrict__ in, T1 *__restrict__ out,
                                                                uint32_t n_out, uint32_t n_in, uint32_t seed,
                                                                SkipParams skips, T1 wa, T1 wb, uint32_t *next,
                                                                uint32_t *states) {
+  constexpr int BITS = FORM & 3;
+  constexpr uint32_t SPIN = (FORM & kNoPolls) ? 0u : (FORM & kThreePolls) ? 3u : kFuseSpin;
   // `states` (optional) holds the outputs' generators' seeded states.  FUSED: `states` is the workgroups' rings
   // (kFuseRingBytes each), `next` (optional) two counters that are zero.
   extern __shared__ __attribute__((aligned(8))) uint32_t smem_raw[];
@@ -168,12 +173,14 @@ __global__ __launch_bounds__(1024, (BITS == 2 || (W == kNormal && sizeof(T1) == 
     // the workgroup's ring of seeded states in
     // device memory (`states`), which stays in the L2.  A slot is written again only after all 64 rows
     // of its previous batch have copied their state to LDS, and read only after its flag says which
-    // batch it holds; every wait is bounded, and a wave that gives up seeds its own generator instead.
+    // batch it holds; these waits are bounded, and a wave that gives up seeds its own generator instead.
     //
     // Which batch is next comes from a counter of the device (`next`: batches taken, workgroups at their end): of two
     // workgroups on a CU the older one gets more of the issue slots, and with equal shares the younger one worked
     // alone, four waves to a SIMD, for the last fifth (1,000,000 streams of 1,000 synapses: 1,665 us, with the counter 1,552).  Without one
-    // (`next` null), batch blockIdx.x + j * gridDim.x.
+    // (`next` null), batch blockIdx.x + j * gridDim.x.  A wave knows its rows by these numbers, whatever became of the
+    // seeding.  Number j + 1 is taken by the wave that seeds, as soon as batch j is ready or the wave has given up on it (taken
+    // before that wait, 100,000 streams of 500 synapses go from 116 to 121 us), so that it comes before twice as many polls are over.
     uint32_t &s_task = smem_raw[0], *const s_ready = smem_raw + 1, *const s_loaded = s_ready + kFuseSlots,
              *const s_batch = s_loaded + kFuseSlots;
     const uint32_t n_batches = (n_out + kFuseBatch - 1u) / kFuseBatch;
@@ -182,16 +189,18 @@ __global__ __launch_bounds__(1024, (BITS == 2 || (W == kNormal && sizeof(T1) == 
     if (threadIdx.x == 0) {
       s_task = 0;
       for (uint32_t k = 0; k < kFuseSlots; ++k) s_ready[k] = 0, s_loaded[k] = 0;
-      for (uint32_t k = 0; k < kFuseNumbers; ++k) s_batch[k] = n_batches;
+      for (uint32_t k = 0; k < kFuseNumbers; ++k) s_batch[k] = 0;
     }
     __syncthreads();
+    auto round_of = [&](uint32_t j) { return (j / kFuseNumbers + 1u) & ((1u << kFuseRoundBits) - 1u); };
     auto take_batch = [&](uint32_t j) {
       uint32_t b = blockIdx.x + j * gridDim.x;
       if (next != nullptr) {
         if (lane == 0) b = atomicAdd(&next[0], 1u);
         b = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(b)));
       }
-      s_batch[j % kFuseNumbers] = b;
+      b = min(b, n_batches);  // (at most 2^26)
+      __hip_atomic_store(&s_batch[j % kFuseNumbers], b << kFuseRoundBits | round_of(j), __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
       return b;
     };
     auto seed_batch = [&](uint32_t j, uint32_t b) {
@@ -202,7 +211,6 @@ __global__ __launch_bounds__(1024, (BITS == 2 || (W == kNormal && sizeof(T1) == 
     if (wave == 0) {
       const uint32_t b = take_batch(0);
       if (b < n_batches) seed_batch(0, b);
-      else __hip_atomic_store(&s_ready[0], 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
     for (;;) {
       // Every lane adds one, so the counter advances by 64 per task and any lane's old value / 64 is the
@@ -212,26 +220,35 @@ __global__ __launch_bounds__(1024, (BITS == 2 || (W == kNormal && sizeof(T1) == 
                              static_cast<int>(atomicAdd(&s_task, 1u)))) / kWave;
       const uint32_t j = t / kFuseBatch, r = t % kFuseBatch;
       const uint32_t slot = j % kFuseSlots;
-      uint32_t flag = 0;
-      // (twice as many polls as the seeding wave waits for the slot: the flag tells which batch it is)
+      uint32_t number = 0, flag = 0;  // (read together: a wave that waits for neither spends one turn of the LDS on them)
       for (uint32_t spin = 0; spin < 2u * kFuseSpin; ++spin) {
+        number = __hip_atomic_load(&s_batch[j % kFuseNumbers], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         flag = __hip_atomic_load(&s_ready[slot], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
-        if ((flag & ~kFuseNotSeeded) >= j + 1u) break;
+        if ((number & ((1u << kFuseRoundBits) - 1u)) == round_of(j)) break;
         __builtin_amdgcn_s_sleep(2);
       }
-      const uint32_t batch = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(s_batch[j % kFuseNumbers])));
-      if (batch >= n_batches || (flag & ~kFuseNotSeeded) < j + 1u) break;  // (every wave's first task of the batch behind the last one)
-      if (r == 0) {
-        const uint32_t b = take_batch(j + 1u);
-        // slot (j + 1) % 3 last held batch j - 2: (j + 1) / 3 batches have used it, 64 loads each
+      number = __builtin_amdgcn_readfirstlane(number);
+      const uint32_t batch = number >> kFuseRoundBits;
+      // (every wave's first task of the batch behind the last one)
+      if (batch >= n_batches || (number & ((1u << kFuseRoundBits) - 1u)) != round_of(j)) break;
+      for (uint32_t spin = 0; spin < SPIN && (flag & ~kFuseNotSeeded) < j + 1u; ++spin) {
+        __builtin_amdgcn_s_sleep(2);
+        flag = __hip_atomic_load(&s_ready[slot], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
+      }
+      if ((flag & ~kFuseNotSeeded) < j + 1u) flag = kFuseNotSeeded;
+      const uint32_t behind = r == 0 ? take_batch(j + 1u) : n_batches;  // (the batch that this wave is to seed)
+      if (behind < n_batches) {
+        // slot (j + 1) % 3 last held batch j - 2: (j + 1) / 3 batches have used it, 64 loads each, and its flag is j - 1
+        // (a wave that gave up on batch j - 2 counts as one that has loaded, also while the states are still being written)
         const uint32_t slot1 = (j + 1u) % kFuseSlots, need = ((j + 1u) / kFuseSlots) * kFuseBatch;
-        bool free_ = b >= n_batches;  // (nothing to seed)
-        for (uint32_t spin = 0; spin < kFuseSpin && !free_; ++spin) {
-          free_ = __hip_atomic_load(&s_loaded[slot1], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) >= need;
+        bool free_ = false;
+        for (uint32_t spin = 0; spin < SPIN && !free_; ++spin) {
+          free_ = __hip_atomic_load(&s_loaded[slot1], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) >= need &&
+                  (__hip_atomic_load(&s_ready[slot1], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) & ~kFuseNotSeeded) + 3u >= j + 2u;
           if (!free_) __builtin_amdgcn_s_sleep(2);
         }
-        if (free_ && b < n_batches) seed_batch(j + 1u, b);
-        else __hip_atomic_store(&s_ready[slot1], (free_ ? 0u : kFuseNotSeeded) | (j + 2u), __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (free_) seed_batch(j + 1u, behind);
+        else __hip_atomic_store(&s_ready[slot1], kFuseNotSeeded | (j + 2u), __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
       }
       const uint32_t *pre = (flag & kFuseNotSeeded) ? nullptr : ring + (static_cast<size_t>(slot) * kFuseBatch + r) * kMtN;
       auto loaded = [&]() {
@@ -971,6 +988,34 @@ extern "C" int bpl_selfcheck_jitconn_skips(bpl_stream_t stream, uint32_t seed, u
   hipLaunchKernelGGL(check_skips_kernel, dim3(2048), dim3(256), 0, s, seed, n_draws, near_boundaries ? 1 : 0, make_skip_params(log_p), c);
   hipLaunchKernelGGL(check_log2_kernel, dim3((1u << 23) / 256u), dim3(256), 0, s, c + 2, c);
   return check_launch("bpl_selfcheck_jitconn_skips") ? 0 : 1;
+}
+
+extern "C" int bpl_selfcheck_jitconn_rowwalk(bpl_stream_t stream, const uint8_t *events, float *out, uint32_t n_out,
+                                             uint32_t n_in, uint32_t seed, double log_p, uint32_t polls, uint32_t groups,
+                                             int counter) {
+  const char *const name = "bpl_selfcheck_jitconn_rowwalk";
+  const uint32_t batches = div_up(n_out, kFuseBatch);
+  if (events == nullptr || out == nullptr || !(log_p < 0.0) || n_in == 0 || n_in > 131072u || groups == 0 ||
+      groups > batches || groups > rowwalk_max_groups() || (polls != 0 && polls != 3)) {
+    set_error("%s: up to 131,072 inputs, no more workgroups than batches of %u outputs, 0 or 3 polls", name, kFuseBatch);
+    return 1;
+  }
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  void *const rings = stream_workspace(s, static_cast<size_t>(groups) * kFuseRingBytes);
+  uint32_t *const counters = counter ? stream_counters(s) : nullptr;
+  if (rings == nullptr || (counter && counters == nullptr)) return 1;
+  auto kernel = polls == 0 ? jitconn_rowwalk_kernel<float, uint8_t, kInEvent, kHomo, 1 + kNoPolls, true>
+                           : jitconn_rowwalk_kernel<float, uint8_t, kInEvent, kHomo, 1 + kThreePolls, true>;
+  const size_t lds = (kFuseLdsWords + 16 * StreamLds<float, kHomo>::words + div_up(n_in, 32)) * sizeof(uint32_t);
+  if (hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                          static_cast<int>(lds)) != hipSuccess) {
+    (void)hipGetLastError();
+    set_error("%s: %zu bytes of LDS are not to be had", name, lds);
+    return 1;
+  }
+  hipLaunchKernelGGL(kernel, dim3(groups), dim3(1024), lds, s, events, out, n_out, n_in, seed, make_skip_params(log_p),
+                     0.0f, 0.0f, counters ? counters + kWalkCounters : nullptr, static_cast<uint32_t *>(rings));
+  return check_launch(name) ? 0 : 1;
 }
 
 #define BPL_DEFINE(name, ...)                                                                      \

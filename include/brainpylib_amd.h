@@ -224,6 +224,15 @@ void bpl_batched_scatter_plan(uint32_t n_row, uint32_t n_col, uint32_t nnz, uint
 int bpl_selfcheck_jitconn_skips(bpl_stream_t stream, uint32_t seed, uint64_t n_draws, int near_boundaries,
                                 double log_p, uint64_t *counts);
 
+/* Self-check of what the row walk does where a generator's seeded state is not there in time (no counterpart in the
+ * reference, whose kernels seed in place): out = counts of the events (n_in bytes, at most 131,072) that the n_out
+ * homogeneous streams meet, by `groups` workgroups (at most one per 64 outputs) whose waves poll for a seeded state `polls` (0 or
+ * 3) times and then seed their own generator; with `counter` the workgroups take batches of 64 streams from the stream's
+ * counter, else they share them out.  The result is that of gpu_event_matvec_prob_homo_v2_float_bool.  Returns 0 when the
+ * kernel was enqueued on `stream`. */
+int bpl_selfcheck_jitconn_rowwalk(bpl_stream_t stream, const uint8_t *events, float *out, uint32_t n_out, uint32_t n_in,
+                                  uint32_t seed, double log_p, uint32_t polls, uint32_t groups, int counter);
+
 /* ------------------------------------------------------------------------------------------
  * event_csr_matvec  (lib/gpu_event_csr_matvec.cu:222-260; launchers :148-217)
  *   buffers = [data, indices, indptr, events, out]

@@ -682,6 +682,27 @@ def test_a_skip_to_just_below_two_to_the_32_ends_the_row(cuda, oracle_mod, w_kin
   assert kernel_call(ev, col_walk=False, dense=False, **kw)[0] == 0
 
 
+@pytest.mark.parametrize("counter", [0, 1])
+@pytest.mark.parametrize("polls", [0, 3])
+@pytest.mark.parametrize("n_out,groups", [(64, 1), (1_000, 1), (8_200, 3), (9_001, 40)])
+def test_waves_that_do_not_wait_for_their_generators_write_their_rows_all_the_same(cuda, n_out, groups, polls, counter):
+  # one to many batches per workgroup; the counters are found as they were left, so each form runs twice
+  import ctypes
+  n_in, seed, log_p = 5_000, 11, float(np.log(1 - 0.02))
+  ev = np.random.default_rng(n_out).random(n_in) < 0.3
+  want = kernel_call(ev, w_kind="homo", log_p=log_p, seed=seed, n_row=n_out, n_col=n_in, col_walk=False, dense=False)
+  events = torch.from_numpy(ev).cuda()
+  check = _lib.lib().bpl_selfcheck_jitconn_rowwalk
+  check.argtypes = [ctypes.c_void_p] * 3 + [ctypes.c_uint32] * 3 + [ctypes.c_double] + [ctypes.c_uint32] * 2 + [ctypes.c_int]
+  print("case", n_out, groups, polls, counter, flush=True)
+  for _ in range(2):
+    out = torch.full((n_out,), -1.0, device="cuda")
+    rc = check(torch.cuda.current_stream().cuda_stream, events.data_ptr(), out.data_ptr(), n_out, n_in, seed, log_p, polls,
+               groups, counter)
+    assert rc == 0, _lib.last_error()
+    np.testing.assert_array_equal(out.cpu().numpy(), want)
+
+
 @pytest.mark.parametrize("n_out,n_in", [(8192, 3000), (10_007, 200_000), (20_000, 400_000), (70_001, 5000)])
 def test_row_walk_with_generators_seeded_inside_the_kernel(cuda, oracle_mod, n_out, n_in):
   # from 8,192 outputs the row walk seeds its generators itself, 64 streams at a time, into rings of
