@@ -32,9 +32,10 @@ namespace {
 // ---- row walk -------------------------------------------------------------------------------------
 // LDS the row walk gives to an event bitmap when it wants two 16-wave workgroups per CU (each wave
 // can issue one instruction every four cycles, so the number of resident waves bounds the VALU
-// utilisation: 32 waves per CU walk 290 G synapses/s, the 15 that fit beside a 125 KB bitmap 228).
-// What two workgroups leave of a CU's 160 KB beside their 16 waves' states and queues (float normal
-// weights: 18,944 bytes; the share of events hardly matters there, the second probe hides behind the weights).
+// utilisation: 1,000,000 streams of 1,000 synapses, 32 waves per CU, 650 G synapses/s).
+// What two workgroups leave of a CU's 160 KB beside their 16 waves' states and queues (homogeneous weights 33,536 bytes,
+// uniform ones 29,440, double 27,392, normal ones 18,944, double 11,264: the share of events hardly matters to those, the
+// second probe hides behind the weights), this at most.
 constexpr uint32_t kRowwalkCoarseMost = 38912;
 // Float normal weights with events keep the state with the least mirror: wrapping a batch's addresses lane by lane costs
 // eight instructions, and the LDS that it saves holds twice the events' bitmap (1e5 streams of 1,000 to 1,500 synapses over
@@ -43,11 +44,13 @@ constexpr uint32_t kRowwalkCoarseMost = 38912;
 // (matvec and its gradient 1,769 us, else 1,780).
 template <typename T1, int IN, int W>
 constexpr bool rowwalk_short() { return IN == kInEvent && W == kNormal && sizeof(T1) == 4; }
-template <typename T1, int W>
-constexpr uint32_t rowwalk_coarse_bytes() {
-  const uint32_t left = (80u * 1024u - 16u * 4u * StreamLds<T1, W, rowwalk_short<T1, kInEvent, W>()>::words - 64u) / 256u * 256u;
+template <typename T1, int W, bool kShort>
+constexpr uint32_t rowwalk_bytes_for_two() {
+  const uint32_t left = (80u * 1024u - 16u * 4u * StreamLds<T1, W, kShort>::words - 64u) / 256u * 256u;
   return left < kRowwalkCoarseMost ? left : kRowwalkCoarseMost;
 }
+template <typename T1, int W>
+constexpr uint32_t rowwalk_coarse_bytes() { return rowwalk_bytes_for_two<T1, W, rowwalk_short<T1, kInEvent, W>()>(); }
 
 // BITS: where the event probes go.  0: the event vector in global memory; 1: its bitmap in LDS;
 // 2: a coarse bitmap in LDS (one bit per 2^g positions, at most rowwalk_coarse_bytes<T1, W>()) and, where its
@@ -692,6 +695,12 @@ void launch_rowwalk_plain(hipStream_t stream, const VT *in, T1 *out, uint32_t n_
       if (bitmap > 16 * 1024) {
         nw = static_cast<int>((cap - bitmap) / state_bytes);
         if (nw > 16) nw = 16;
+        // Rows that seed in place and are more than one workgroup a CU works on: two workgroups of fewer waves, if they
+        // hold them all (300,000 inputs, 6,000 rows of 300: 59.5 -> 58.1 us, uniform weights 61.6 -> 57.9, double 64.2 -> 59.7;
+        // 8,000 rows in two turns 80).
+        const size_t half = cap / 2 > bitmap ? (cap / 2 - bitmap) / state_bytes : 0, cus = static_cast<size_t>(device_info().num_cu);
+        if (sc.rings() == nullptr && half < 16 && n_out > 16 * cus && n_out <= 2 * half * cus)
+          nw = static_cast<int>(half);
       }
       launch_rowwalk_impl<T1, VT, IN, W, 1>(stream, in, out, n_out, n_in, seed, log_p, wa, wb, nw,
                                             bitmap + nw * state_bytes, sc);
@@ -702,16 +711,31 @@ void launch_rowwalk_plain(hipStream_t stream, const VT *in, T1 *out, uint32_t n_
                                         fused_waves * state_bytes, sc);
 }
 
+// The longest event bitmap that is kept whole in LDS.  Rows that one workgroup a CU works on: kRowwalkCoarseMost, for the two
+// levels take two launches more and save nothing (4,000 rows of 20 and of 300, 300,000 inputs: 32 / 34 us, in two levels 36 / 38,
+// uniform weights 32 / 35 and 36 / 39, normal ones 33 / 39 and 37 / 44, double 34 / 47 and 38 / 51; 16,000 rows, seeded in the
+// kernel, 29 / 35 and 33 / 39, normal ones 33 / 55 and 37 / 60).  More rows: what leaves room for two workgroups
+// (20,000 / 100,000 rows of 1,000, 300,000 inputs: 76 / 195 us, 85 / 222 with one workgroup), which for rows that seed in
+// place is counted with the least mirror, as the scalar unit bounds those (8,000 rows of 20 and of 300, 300,000 inputs:
+// 55 / 60 us, in two levels 58 / 61).
+template <typename T1, int W>
+uint32_t rowwalk_exact_bytes(uint32_t n_out) {
+  const uint32_t cus = static_cast<uint32_t>(device_info().num_cu);
+  const bool fused = n_out >= kSeedAheadMin;
+  if (n_out <= (fused ? kFuseBatch : 16u) * cus) return kRowwalkCoarseMost;
+  return fused ? rowwalk_coarse_bytes<T1, W>() : rowwalk_bytes_for_two<T1, W, true>();
+}
+
 template <typename T1, typename VT, int IN, int W>
 void launch_rowwalk(hipStream_t stream, const VT *in, T1 *out, uint32_t n_out, uint32_t n_in, uint32_t seed,
                     double log_p, T1 wa, T1 wb) {
   if (n_out == 0) return;
   constexpr bool kEvents = IN == kInEvent;
   const size_t words = (static_cast<size_t>(n_in) + 31) / 32;
-  // An event bitmap that would leave room for fewer than two 16-wave workgroups per CU: two levels
-  // instead, the exact bitmap packed into global memory and a coarse one made for LDS.  Wide event
-  // types: the vector is packed to one bit per element once, instead of once per workgroup.
-  const bool two_level = kEvents && words * 4 > rowwalk_coarse_bytes<T1, W>() && n_in <= 0xffffffffu - kRowwalkLead;
+  // A longer event bitmap (rowwalk_exact_bytes): two levels, the exact bitmap packed into global memory and a
+  // coarse one made for LDS.  Wide event types: the vector is packed to one bit per element once, instead of once per workgroup.
+  const uint32_t exact_most = rowwalk_exact_bytes<T1, W>(n_out);
+  const bool two_level = kEvents && words * 4 > exact_most && n_in <= 0xffffffffu - kRowwalkLead;
   const bool packed = kEvents && (two_level || sizeof(VT) > 1);
   uint32_t g = 0, off = 0, c_words = 0;
   size_t bitmap_ws = 0;

@@ -136,7 +136,7 @@ def test_event_column_walk_in_every_regime(cuda, oracle_mod, n_out, n_in, p):
 
 @pytest.mark.parametrize("n_in", [320_000, 1_500_000, 5_000_000])
 def test_row_walk_with_a_two_level_event_bitmap(cuda, oracle_mod, n_in):
-  # more inputs than the 38 KB of LDS the row walk gives to a bitmap cover (311,296): a coarse
+  # more inputs than the row walk ever keeps an exact bitmap of in LDS (311,296): a coarse
   # bitmap in LDS (one bit per 2, 8 and 32 inputs here) and the exact one in global memory, whose
   # word is looked at one batch late.  Bool and float events, all weight kinds; counts exact.
   n_out = 300
@@ -158,9 +158,8 @@ def test_row_walk_with_a_two_level_event_bitmap(cuda, oracle_mod, n_in):
 
 def test_row_walk_lanes_past_the_end_of_a_row_count_nothing(cuda, oracle_mod):
   # two-level bitmap with EVERY event set (all coarse and exact bits are ones): the lanes of a row's last
-  # batch that lie past the end of the row index words beyond the coarse bitmap, or any word of it if their
-  # position wrapped; they extract a bit field of width 0 from it, so a row's count is its stream's
-  # synapse count exactly.  Rows of about 3 synapses: nearly every lane of every row's only batch is past the end.
+  # batch that lie past the end of the row look up position 0, whose word of the exact bitmap holds no input, so a
+  # row's count is its stream's synapse count exactly.  Rows of about 3 synapses: nearly every lane of every row's only batch is past the end.
   # (8,200 outputs: the walk that seeds its generators itself)
   for n_out, n_in in ((400, 311_297), (400, 320_000), (400, 1_310_720), (8_200, 320_000)):
     ev = np.ones(n_in, dtype=np.bool_)
@@ -650,6 +649,27 @@ def test_normal_weights_on_both_sides_of_the_bitmaps_and_skip_paths(cuda, oracle
   want, mag = oracle_mod.jitconn_matvec(ev, dense=False, return_abs=True, out_dtype=dtype, **kw)
   assert_close_reordered(kernel_call(ev, col_walk=False, dense=False, out_dtype=dtype, **kw), want, mag, dtype,
                          what="normal weights, events")
+
+
+@pytest.mark.parametrize("w_kind,dtype,last", [("homo", np.float32, 268_288), ("uniform", np.float32, 235_520),
+                                               ("uniform", np.float64, 219_136), ("normal", np.float32, 151_552),
+                                               ("normal", np.float64, 90_112)])
+def test_row_walk_on_both_sides_of_the_exact_bitmaps(cuda, oracle_mod, w_kind, dtype, last):
+  # (outputs, inputs): exact bitmaps of up to 311,296 inputs where one workgroup a CU has all rows; two workgroups of
+  # fewer waves; two turns of one; two 16-wave workgroups, up to `last` inputs (16,384 outputs: one)
+  place = {"homo": 311_296, "uniform": 311_296, "normal": 151_552 if dtype == np.float32 else 153_600}[w_kind]
+  rng = np.random.default_rng(last)
+  for n_out, n_in in ((301, 311_296), (301, 311_297), (4_101, place), (4_101, place + 1), (6_000, place), (8_191, place),
+                      (16_384, 311_296), (16_385, last), (16_385, last + 1)):
+    ev = rng.random(n_in) < 0.2
+    kw = dict(w_kind=w_kind, w_a=0.5, w_b=2.0, log_p=oracle_mod.log_p_of(70.0 / n_in), seed=9, n_row=n_out, n_col=n_in)
+    print("case", n_out, n_in, flush=True)
+    want, mag = oracle_mod.jitconn_matvec(ev, dense=False, return_abs=True, out_dtype=dtype, **kw)
+    got = kernel_call(ev, col_walk=False, dense=False, out_dtype=dtype, **kw)
+    if w_kind == "homo":
+      assert np.array_equal(got, want)
+    else:
+      assert_close_reordered(got, want, mag, dtype, what="row walk, %s weights" % w_kind)
 
 
 def _stream_that_skips_to_the_end_of_the_integers(w_kind, n_in):
