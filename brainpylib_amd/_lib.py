@@ -107,7 +107,8 @@ def _native_enqueue():
 def custom_call(name, buffers, opaque, stream=None):
   """Enqueue custom-call target ``name`` on ``stream`` (default: torch's current stream).
 
-  ``buffers``: torch CUDA tensors (operands, then results), contiguous.  Asynchronous."""
+  ``buffers``: torch CUDA tensors (operands, then results), contiguous.  ``stream``: a raw handle, or what ctypes takes
+  for a pointer (a ``c_void_p``, a torch stream).  Asynchronous."""
   address = _addresses.get(name)
   if address is None:
     address = _addresses[name] = ctypes.cast(target(name), ctypes.c_void_p).value
@@ -119,7 +120,10 @@ def custom_call(name, buffers, opaque, stream=None):
     except (AttributeError, TypeError):
       import torch
       stream = torch.cuda.current_stream(buffers[0].device).cuda_stream
-  (_enqueue or _native_enqueue())(address, stream, opaque, *buffers)
+  if type(stream) is int and type(opaque) is bytes and len(buffers) <= 16:
+    (_enqueue or _native_enqueue())(address, stream, opaque, *buffers)
+  else:  # (what the native call does not take)
+    _enqueue_ctypes(address, stream, opaque, *buffers)
 
 
 def _current_raw_stream(index):

@@ -126,6 +126,20 @@ def test_native_enqueue_refuses_what_is_no_call():
   assert not _lib.last_error()
 
 
+def test_custom_call_takes_what_ctypes_takes():
+  from brainpylib_amd import _lib
+
+  class Stream:  # (as torch's streams are)
+    _as_parameter_ = ctypes.c_void_p(0)
+  one = torch.zeros(1)
+  opaque = ctypes.create_string_buffer(b"short")
+  for stream, descriptor, buffers in ((0, b"short", [one]), (ctypes.c_void_p(0), b"short", [one]), (Stream(), b"short", [one]),
+                                      (0, opaque, [one]), (0, b"short", [one] * 17)):
+    with pytest.raises(RuntimeError, match="event_csr_matvec_homo_float_bool"):  # (the target's own error)
+      _lib.custom_call("event_csr_matvec_homo_float_bool", buffers, descriptor, stream=stream)
+  assert not _lib.last_error()
+
+
 def test_signature_of_an_autograd_function_binds_other_calls_as_inspect_does():
   from brainpylib_amd._tensors import keep_signature
 
