@@ -122,8 +122,9 @@ def device_of(*args):
 
 
 def has_tangent(t):
-  # (outside a dual level, where unpack_dual finds no tangent either, its named tuple is most of the cost)
-  return forward_ad._current_level >= 0 and t.is_floating_point() and forward_ad.unpack_dual(t).tangent is not None
+  # (outside a dual level, where unpack_dual finds no tangent either, its named tuple is most of the cost; the level is
+  # torch's own name, and without it every tensor is looked at)
+  return getattr(forward_ad, "_current_level", 0) >= 0 and t.is_floating_point() and forward_ad.unpack_dual(t).tangent is not None
 
 
 # Device copies of one-element host operands.  One that is here stays: queued calls on other streams and captured graphs
@@ -182,14 +183,24 @@ class _PositionalSignature(inspect.Signature):
   def bind(self, *args, **kwargs):
     if kwargs or len(args) != len(self.parameters):
       return super().bind(*args, **kwargs)
-    return _PositionalArguments(args)
+    return _PositionalArguments(self, args)
 
 
-class _PositionalArguments:
+class _PositionalArguments(inspect.BoundArguments):
+  """Arguments that were all given by position; by name only if somebody asks."""
   __slots__ = ("args",)
 
-  def __init__(self, args):
+  def __init__(self, signature, args):
+    self._signature = signature
     self.args = args
+
+  @property
+  def arguments(self):
+    return dict(zip(self._signature.parameters, self.args))
+
+  @property
+  def kwargs(self):
+    return {}
 
   def apply_defaults(self):
     pass

@@ -150,11 +150,27 @@ def test_signature_of_an_autograd_function_binds_other_calls_as_inspect_does():
       return a
   sig = inspect.signature(F.forward)
   assert sig.bind(1, 2, 4).args == (1, 2, 4)
+  usual = inspect.Signature(list(sig.parameters.values()))
+  bound = sig.bind(1, 2, 4)
+  bound.apply_defaults()
+  assert bound == usual.bind(1, 2, 4)
+  assert bound.kwargs == {} and bound.arguments == {"a": 1, "b": 2, "c": 4}
   bound = sig.bind(1, b=2)
   bound.apply_defaults()
   assert bound.args == (1, 2, 3)
   with pytest.raises(TypeError):
     sig.bind(1)
+
+
+def test_tangents_are_found_where_torch_does_not_tell_its_level(monkeypatch):
+  import types
+  import torch.autograd.forward_ad as fwAD
+  from brainpylib_amd import _tensors
+  monkeypatch.setattr(_tensors, "forward_ad", types.SimpleNamespace(unpack_dual=fwAD.unpack_dual))
+  t = torch.ones(2)
+  assert not _tensors.has_tangent(t)
+  with fwAD.dual_level():
+    assert _tensors.has_tangent(fwAD.make_dual(t, t)) and not _tensors.has_tangent(t)
 
 
 @pytest.mark.parametrize("context", ["inference_mode", "grad", "jvp", "vmap"])
