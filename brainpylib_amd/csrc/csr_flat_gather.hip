@@ -137,7 +137,10 @@ __device__ __forceinline__ void flat_take(double &v, flat_lds window, uint32_t o
   const uint32_t at = static_cast<uint32_t>(__double2hiint(v)) - origin;
   if (at < bytes / 8u) v = *reinterpret_cast<__attribute__((address_space(3))) const double *>(window + 8u * at);
 }
-constexpr uint32_t kFlatMostPlaces = 1u << 20;  // (of both types' NaNs fewer than that are taken)
+// Columns that have a place: the places of both types end in front of 2^32, behind which the words of zeros and denormals begin.
+constexpr uint32_t kFlatMostPlaces = (1u << 20) - 1u;
+static_assert(0xfff00001ull + kFlatMostPlaces - 1u <= 0xffffffffull && 0xff800004ull + 4ull * (kFlatMostPlaces - 1u) <= 0xffffffffull,
+              "no place is taken for a number");
 
 __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {  // (of all 64 lanes, to all of them)
 #pragma unroll
@@ -145,7 +148,7 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {  // (of all 64 la
   return __builtin_amdgcn_readfirstlane(v);
 }
 
-// The n elements of x from `first` on to LDS, eight 16-byte loads of every thread in flight.
+// The n elements of x to LDS, three 16-byte loads of every thread in flight.
 template <typename F>
 __device__ __forceinline__ void flat_stage_window(F *to, const F *__restrict__ x, uint32_t n) {
   constexpr uint32_t kPer = 16 / sizeof(F), kUnroll = 3;
