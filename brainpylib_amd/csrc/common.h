@@ -52,13 +52,14 @@ const DeviceInfo &device_info();
 // needs hipMalloc, which cannot run while the stream is being captured into a graph: then the
 // call fails (nullptr, error recorded, nothing enqueued), so every size must have been used once
 // on the stream before it is captured.  nullptr (error recorded) also if the allocation fails.
-void *stream_workspace(hipStream_t stream, size_t bytes);
+// `optional`: the caller can do without during a capture, which then records no error.
+void *stream_workspace(hipStream_t stream, size_t bytes, bool optional = false);
 
 // A few zero-initialised 32-bit counters per (device, stream).  The first one (the scatter's
 // active-row count) and the two from kWalkCounters on (work that workgroups take as they come) are left at zero again
 // by every user; the others carry nothing from call to
 // call.  nullptr if the allocation fails (or would be needed during a capture).
-uint32_t *stream_counters(hipStream_t stream);
+uint32_t *stream_counters(hipStream_t stream, bool optional = false);
 constexpr size_t kStreamCounterBytes = 256;
 constexpr uint32_t kWalkCounters = 60;
 

@@ -608,7 +608,8 @@ struct RowwalkScratch {
 // At most four row-walk workgroups share a CU (eight waves each; sixteen-wave ones two).
 inline uint32_t rowwalk_max_groups() { return 4u * static_cast<uint32_t>(device_info().num_cu); }
 
-inline RowwalkScratch rowwalk_scratch(hipStream_t stream, uint32_t n_out, size_t bitmap_bytes) {
+// `optional`: a capture that finds none goes on without.
+inline RowwalkScratch rowwalk_scratch(hipStream_t stream, uint32_t n_out, size_t bitmap_bytes, bool optional) {
   RowwalkScratch sc;
   sc.bitmap_bytes = (bitmap_bytes + 255) / 256 * 256;
   if (n_out >= kSeedAheadMin) {
@@ -617,7 +618,7 @@ inline RowwalkScratch rowwalk_scratch(hipStream_t stream, uint32_t n_out, size_t
   }
   const size_t want = sc.bitmap_bytes + sc.ring_groups * kFuseRingBytes;
   if (want == 0) return sc;
-  sc.base = static_cast<unsigned char *>(stream_workspace(stream, want));
+  sc.base = static_cast<unsigned char *>(stream_workspace(stream, want, optional));
   if (sc.base == nullptr && !scratch_refused_by_capture() && sc.ring_groups != 0 && sc.bitmap_bytes != 0) {
     // no room for the rings: the bitmap alone (the waves then seed their own generators)
     bpl_clear_error();
@@ -667,9 +668,8 @@ void launch_rowwalk_impl(hipStream_t stream, const VT *in, T1 *out, uint32_t n_o
   // (more batches than workgroups: taken as they come; a capture that finds no counters shares them out evenly)
   uint32_t *next = nullptr;
   if (fused && grid < div_up(n_out, kFuseBatch)) {
-    next = stream_counters(stream);
+    next = stream_counters(stream, true);
     if (next != nullptr) next += kWalkCounters;
-    else bpl_clear_error();
   }
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(block), lds_bytes, stream, in, out, n_out, n_in, seed,
                      make_skip_params(log_p), wa, wb, next, sc.rings());
@@ -747,13 +747,11 @@ void launch_rowwalk(hipStream_t stream, const VT *in, T1 *out, uint32_t n_out, u
   } else if (packed) {
     bitmap_ws = (words + 1) * sizeof(uint32_t);
   }
-  const RowwalkScratch sc = rowwalk_scratch(stream, n_out, bitmap_ws);
-  if (sc.refused) {
-    // (the error stands: a graph must not record a slower path.  But for byte events whose bitmap is no longer than what
-    // homo and uniform weights keep in LDS: without rings such a walk is captured without scratch memory.)
-    if (!(kEvents && sizeof(VT) == 1 && n_out < kSeedAheadMin && words * 4 <= kRowwalkCoarseMost)) return;
-    bpl_clear_error();
-  }
+  // (Refused in a capture, the call ends with the error: a graph must not record a slower path.  But for byte events whose
+  // bitmap is no longer than what LDS may keep of one: without rings such a walk is captured without scratch memory.)
+  const bool optional = kEvents && sizeof(VT) == 1 && n_out < kSeedAheadMin && words * 4 <= kRowwalkCoarseMost;
+  const RowwalkScratch sc = rowwalk_scratch(stream, n_out, bitmap_ws, optional);
+  if (sc.refused && !optional) return;
   if constexpr (kEvents) {
     if (uint32_t *bits = sc.bitmap()) {
       pack_event_bitmap<VT>(stream, in, n_in, bits, two_level ? kRowwalkLead / 32u : 0u);

@@ -96,7 +96,7 @@ void ensure_error(const char *target, const char *why) {
   if (t_error.empty()) set_error("%s: %s", target, why);
 }
 
-void *stream_workspace(hipStream_t stream, size_t bytes) {
+void *stream_workspace(hipStream_t stream, size_t bytes, bool optional) {
   t_refused_by_capture = false;
   int dev = 0;
   (void)hipGetDevice(&dev);
@@ -106,8 +106,9 @@ void *stream_workspace(hipStream_t stream, size_t bytes) {
     if (x.dev == dev && x.stream == stream) e = &x;
   if (e != nullptr && e->bytes >= bytes) return e->ptr;
   if (capturing(stream)) {
-    set_error("scratch memory of %zu bytes is needed while the stream is being captured (it holds %zu): run the "
-              "call once on this stream before capturing it", bytes, e ? e->bytes : size_t(0));
+    if (!optional)
+      set_error("scratch memory of %zu bytes is needed while the stream is being captured (it holds %zu): run the "
+                "call once on this stream before capturing it", bytes, e ? e->bytes : size_t(0));
     t_refused_by_capture = true;
     return nullptr;
   }
@@ -136,7 +137,7 @@ void *stream_workspace(hipStream_t stream, size_t bytes) {
   return e->ptr;
 }
 
-uint32_t *stream_counters(hipStream_t stream) {
+uint32_t *stream_counters(hipStream_t stream, bool optional) {
   struct Entry {
     int dev;
     hipStream_t stream;
@@ -157,8 +158,9 @@ uint32_t *stream_counters(hipStream_t stream) {
   for (auto &x : entries)
     if (x.dev == dev && x.stream == stream) return x.ptr;
   if (capturing(stream)) {
-    set_error("the stream's counters would be allocated while it is being captured: run the call once on this "
-              "stream before capturing it");
+    if (!optional)
+      set_error("the stream's counters would be allocated while it is being captured: run the call once on this "
+                "stream before capturing it");
     t_refused_by_capture = true;
     return nullptr;
   }

@@ -170,15 +170,17 @@ def test_scratch_memory_of_a_batch_of_a_small_network(cuda):
 
 
 @pytest.mark.parametrize("n_in", [151_552, 151_553, 311_296])
-def test_normal_row_walk_is_captured_on_a_cold_stream(cuda, n_in):
+def test_normal_row_walk_is_captured_on_a_cold_stream(cuda, n_in, capfd):
   # few outputs, byte events: their bitmap lies in LDS and no scratch memory is needed, whatever the weights
   ev = torch.from_numpy(np.random.default_rng(n_in).random(n_in) < 0.1).to(cuda)
   kw = dict(w_mu=0.1, w_sigma=0.5, conn_prob=0.01, shape=(300, n_in), seed=5, outdim_parallel=True)
   want = bpl.event_matvec_prob_conn_normal_weight(ev, **kw)
   torch.cuda.synchronize()
   s, g = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+  capfd.readouterr()
   with torch.cuda.graph(g, stream=s):
     out = bpl.event_matvec_prob_conn_normal_weight(ev, **kw)
+  assert "brainpylib_amd" not in capfd.readouterr().err
   assert not _query(s.cuda_stream)[0], "nothing was allocated"
   for _ in range(3):
     out.zero_()
@@ -186,3 +188,36 @@ def test_normal_row_walk_is_captured_on_a_cold_stream(cuda, n_in):
     torch.cuda.synchronize()
     # (the same addends in float64, in another order, rounded once)
     torch.testing.assert_close(out, want, rtol=3e-7, atol=1e-6)
+
+
+def test_row_walk_is_captured_where_the_stream_has_rings_but_no_counters(cuda, capfd):
+  # more batches of streams than workgroups, and no counter to take them from: they are shared out evenly, and the
+  # call, which succeeds, prints nothing
+  rng = np.random.default_rng(3)
+  handle = ctypes.c_void_p()  # (a stream of its own: torch's come from a pool and may have counters from elsewhere)
+  assert ctypes.CDLL("libamdhip64.so").hipStreamCreate(ctypes.byref(handle)) == 0
+  s, g = torch.cuda.ExternalStream(handle.value), torch.cuda.CUDAGraph()
+  x = torch.from_numpy(rng.random(100_000, dtype=np.float32)).to(cuda)
+  torch.cuda.synchronize()
+  with torch.cuda.stream(s):  # (bins of 0.75 GB: scratch memory, no counters)
+    bpl.matvec_prob_conn_homo_weight(x, 0.5, conn_prob=0.01, shape=(100_000, 100_000), seed=1, outdim_parallel=False)
+  s.synchronize()
+  before = _query(s.cuda_stream)
+  n_in = 20_000
+  ev = torch.zeros(n_in, dtype=torch.bool, device=cuda)
+  kw = dict(weight=1.0, conn_prob=0.005, shape=(70_001, n_in), seed=5, outdim_parallel=True)
+  bpl.event_matvec_prob_conn_homo_weight(ev, **kw)
+  torch.cuda.synchronize()
+  capfd.readouterr()
+  with torch.cuda.graph(g, stream=s):
+    out = bpl.event_matvec_prob_conn_homo_weight(ev, **kw)
+  assert "brainpylib_amd" not in capfd.readouterr().err
+  assert _query(s.cuda_stream) == before, "nothing was allocated"
+  for i in range(3):
+    ev.copy_(torch.from_numpy(rng.random(n_in) < 0.1))
+    out.zero_()
+    torch.cuda.synchronize()
+    g.replay()
+    torch.cuda.synchronize()
+    want = bpl.event_matvec_prob_conn_homo_weight(ev, **kw)
+    assert want.sum() > 0 and torch.equal(out, want), i
