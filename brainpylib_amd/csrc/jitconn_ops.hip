@@ -940,8 +940,9 @@ __device__ __forceinline__ uint64_t mix64(uint64_t z) {
 }
 
 __global__ __launch_bounds__(256) void check_skips_kernel(uint32_t seed, uint64_t n, int mode, SkipParams sp,
-                                                          unsigned long long *__restrict__ counts) {
-  unsigned long long differ = 0, untrusted = 0;
+                                                          unsigned long long *__restrict__ counts,
+                                                          unsigned long long *__restrict__ levels) {
+  unsigned long long differ = 0, untrusted = 0, untrusted_close = 0, untrusted_quick = 0;
   for (uint64_t t = static_cast<uint64_t>(blockIdx.x) * 256u + threadIdx.x; t < n;
        t += static_cast<uint64_t>(gridDim.x) * 256u) {
     uint64_t bits;
@@ -960,15 +961,23 @@ __global__ __launch_bounds__(256) void check_skips_kernel(uint32_t seed, uint64_
     if (unsafe & me) ++untrusted;
     else if (fast != exact) ++differ;
     const uint32_t close = skip_close(lo, hi, sp, unsafe);
-    if (!(unsafe & me) && close != exact) ++differ;
+    if (unsafe & me) ++untrusted_close;
+    else if (close != exact) ++differ;
     const float uppers[] = {static_cast<float>(hi), canonical_f32_scaled(hi)};
     for (const float upper : uppers) {
       const uint32_t quick = skip_quick(hi, upper, sp, unsafe);
-      if (sp.quick && !(unsafe & me) && quick != exact) ++differ;
+      if (unsafe & me) ++untrusted_quick;
+      else if (sp.quick && quick != exact) ++differ;
     }
   }
-  if (differ) atomicAdd(&counts[0], differ);
-  if (untrusted) atomicAdd(&counts[1], untrusted);
+  if (counts != nullptr && differ) atomicAdd(&counts[0], differ);
+  if (counts != nullptr && untrusted) atomicAdd(&counts[1], untrusted);
+  if (levels != nullptr) {
+    if (untrusted_quick) atomicAdd(&levels[0], untrusted_quick);
+    if (untrusted) atomicAdd(&levels[1], untrusted);
+    if (untrusted_close) atomicAdd(&levels[2], untrusted_close);
+    if (blockIdx.x == 0 && threadIdx.x == 0) levels[3] = sp.quick ? 1u : 0u;
+  }
 }
 
 // |hardware log2 - log2| over every fp32 in [0.5, 1): the largest, as the bits of a double; and over those in
@@ -1007,9 +1016,21 @@ extern "C" int bpl_selfcheck_jitconn_skips(bpl_stream_t stream, uint32_t seed, u
   }
   hipStream_t s = static_cast<hipStream_t>(stream);
   unsigned long long *c = reinterpret_cast<unsigned long long *>(counts);
-  hipLaunchKernelGGL(check_skips_kernel, dim3(2048), dim3(256), 0, s, seed, n_draws, near_boundaries ? 1 : 0, make_skip_params(log_p), c);
+  hipLaunchKernelGGL(check_skips_kernel, dim3(2048), dim3(256), 0, s, seed, n_draws, near_boundaries ? 1 : 0, make_skip_params(log_p), c,
+                     static_cast<unsigned long long *>(nullptr));
   hipLaunchKernelGGL(check_log2_kernel, dim3((1u << 23) / 256u), dim3(256), 0, s, c + 2, c);
   return check_launch("bpl_selfcheck_jitconn_skips") ? 0 : 1;
+}
+
+extern "C" int bpl_selfcheck_jitconn_trust(bpl_stream_t stream, uint32_t seed, uint64_t n_draws, double log_p, uint64_t *counts) {
+  if (counts == nullptr || !(log_p < 0.0)) {
+    set_error("bpl_selfcheck_jitconn_trust: counts must be device memory for four words and log_p negative");
+    return 1;
+  }
+  hipLaunchKernelGGL(check_skips_kernel, dim3(2048), dim3(256), 0, static_cast<hipStream_t>(stream), seed, n_draws, 0,
+                     make_skip_params(log_p), static_cast<unsigned long long *>(nullptr),
+                     reinterpret_cast<unsigned long long *>(counts));
+  return check_launch("bpl_selfcheck_jitconn_trust") ? 0 : 1;
 }
 
 extern "C" int bpl_selfcheck_jitconn_rowwalk(bpl_stream_t stream, const uint8_t *events, float *out, uint32_t n_out,

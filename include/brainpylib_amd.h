@@ -224,6 +224,13 @@ void bpl_batched_scatter_plan(uint32_t n_row, uint32_t n_col, uint32_t nnz, uint
 int bpl_selfcheck_jitconn_skips(bpl_stream_t stream, uint32_t seed, uint64_t n_draws, int near_boundaries,
                                 double log_p, uint64_t *counts);
 
+/* How much of the skips each of their levels decides (no counterpart in the reference either): of n_draws hashed values of
+ * U, `counts`, device memory for four 64-bit words which the caller has zeroed, [0] += those that the upper word alone
+ * leaves undecided (each is tried twice, with the word as it is and capped as the polar attempt caps it), [1] += the fast path,
+ * [2] += the 64-bit series; [3] = whether the kernels try the upper word at this log_p.  Returns 0 when the kernel was
+ * enqueued on `stream`. */
+int bpl_selfcheck_jitconn_trust(bpl_stream_t stream, uint32_t seed, uint64_t n_draws, double log_p, uint64_t *counts);
+
 /* Self-check of what the row walk does where a generator's seeded state is not there in time (no counterpart in the
  * reference, whose kernels seed in place): out = counts of the events (n_in bytes, at most 131,072) that the n_out
  * homogeneous streams meet, by `groups` workgroups (at most one per 64 outputs) whose waves poll for a seeded state `polls` (0 or

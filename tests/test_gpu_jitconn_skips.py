@@ -70,3 +70,37 @@ def test_hardware_log2_of_a_mantissa_is_within_the_error_the_guard_band_assumes(
   print("largest |hardware log2(m) - log2(m)| over the fp32 m in [0.5, 1): %.3e; allowed for log2(U): %.3e" % (worst, allowed))
   assert 1e-7 < allowed < 1e-6
   assert 0.0 < worst <= allowed - WORDS_TO_FP32 - 2e-8
+
+
+@pytest.mark.parametrize("conn_prob", [0.9, 0.1, 0.01, 1e-3, 3e-4, 1e-4, 5e-5, 1e-6, 1e-8])
+def test_each_level_of_the_skips_decides_all_but_its_band(conn_prob):
+  # a level that trusted nothing would pass every comparison above: the level behind it would decide.  Bands as wide
+  # as the errors allowed for log2(U) (1.4e-6, 3e-7, 1e-12) and the rounding of the fixed point; the quick level also
+  # leaves upper words under 2^22 to the next
+  import oracle
+  from brainpylib_amd import _lib
+  lib = _lib.lib()
+  lib.bpl_selfcheck_jitconn_trust.restype = ctypes.c_int
+  lib.bpl_selfcheck_jitconn_trust.argtypes = [ctypes.c_void_p, ctypes.c_uint32, ctypes.c_uint64, ctypes.c_double, ctypes.c_void_p]
+  log_p, n = oracle.log_p_of(conn_prob), 1 << 27
+  counts = torch.zeros(4, dtype=torch.int64, device="cuda:0")
+  rc = lib.bpl_selfcheck_jitconn_trust(ctypes.c_void_p(torch.cuda.current_stream().cuda_stream), 17, n, float(log_p),
+                                       ctypes.c_void_p(counts.data_ptr()))
+  assert rc == 0, _lib.last_error()
+  quick, fast, close, tries_quick = (int(v) for v in counts.cpu().numpy())
+  size = math.log(2.0) / abs(log_p)
+  narrow = size * 64 + 2 < 2 ** 19
+  rounding = 1e-9 if narrow else 2.0 ** -18
+  share = lambda error: min(1.0, 2 * (error * size + rounding)) if size * 64 + 2 < 4e9 else 1.0
+
+  def check(found, expect, draws, name):
+    # (the number found is binomial: six standard deviations; the band is a little wider than twice the guard, by a unit of its
+    # fixed point at most)
+    slack = 6 * math.sqrt(draws * expect) + 12 + draws * (2.0 ** -32 if narrow else 2.0 ** -18)
+    assert abs(found - draws * expect) <= slack + 0.01 * draws * expect, (name, found / draws, expect)
+  check(fast, share(3e-7), n, "fast")
+  check(close, share(1e-12), n, "close")
+  assert tries_quick == int(narrow and 1.4e-6 * size + 1e-9 < 0.004)
+  if tries_quick:
+    band = 2 * (1.4e-6 * size + 1e-9)
+    check(quick, 2.0 ** -10 + (1 - 2.0 ** -10) * band, 2 * n, "quick")  # (tried with the upper word and with the capped one)
