@@ -182,8 +182,12 @@ __global__ __launch_bounds__(1024, (FORM == 2 || (W == kNormal && sizeof(T1) == 
     // workgroups on a CU the older one gets more of the issue slots, and with equal shares the younger one worked
     // alone, four waves to a SIMD, for the last fifth (1,000,000 streams of 1,000 synapses: 1,665 us, with the counter 1,552).  Without one
     // (`next` null), batch blockIdx.x + j * gridDim.x.  A wave knows its rows by these numbers, whatever became of the
-    // seeding.  Number j + 1 is taken by the wave that seeds, as soon as batch j is ready or the wave has given up on it (taken
-    // before that wait, 100,000 streams of 500 synapses go from 116 to 121 us), so that it comes before twice that wait is over.
+    // seeding.  Number j + 1 is taken by the wave that seeds: from the counter as soon as batch j is ready or the wave has given up
+    // on it, so that it comes before twice that wait is over (taken before, a workgroup that is behind has one more batch to
+    // do).  Without one at once where rows are so short that the walk waits for the seeding alone, so that a workgroup's first
+    // two batches are seeded side by side (homogeneous weights, rows of 30, 33,000 / 38,000 / 45,000 / 60,000 of them 42 / 42 / 42.6 / 52.3 us,
+    // now 37 / 37 / 40.6 / 53; rows of 400 would lose, 45,000 of them 51 -> 55, and so would other weights, 60,000 rows of 30 with
+    // uniform ones 55 -> 59).
     uint32_t &s_task = smem_raw[0], *const s_ready = smem_raw + 1, *const s_loaded = s_ready + kFuseSlots,
              *const s_batch = s_loaded + kFuseSlots;
     const uint32_t n_batches = (n_out + kFuseBatch - 1u) / kFuseBatch;
@@ -195,6 +199,7 @@ __global__ __launch_bounds__(1024, (FORM == 2 || (W == kNormal && sizeof(T1) == 
       for (uint32_t k = 0; k < kFuseNumbers; ++k) s_batch[k] = 0;
     }
     __syncthreads();
+    const bool early = W == kHomo && next == nullptr && static_cast<double>(n_in) * skips.log_p > -64.0;
     auto round_of = [&](uint32_t j) { return (j / kFuseNumbers + 1u) & ((1u << kFuseRoundBits) - 1u); };
     auto take_batch = [&](uint32_t j) {
       uint32_t b = blockIdx.x + j * gridDim.x;
@@ -206,15 +211,10 @@ __global__ __launch_bounds__(1024, (FORM == 2 || (W == kNormal && sizeof(T1) == 
       __hip_atomic_store(&s_batch[j % kFuseNumbers], b << kFuseRoundBits | round_of(j), __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
       return b;
     };
-    // In front of the waves that walk and those that poll for it: short rows wait for nothing else (100,000 streams of 20 synapses
-    // 88.6 -> 85.1 us, uniform weights 94.6 -> 86.5, normal ones 98.8 -> 88.2), and the poll is as short as it can be for their sake
-    // (8,200 streams 22.9 -> 22.2 us, normal weights 27.0 -> 25.2).
     auto seed_batch = [&](uint32_t j, uint32_t b) {
       const uint32_t slot = j % kFuseSlots;
-      __builtin_amdgcn_s_setprio(3);
       mt_seed_batch(st, lane, seed + b * kFuseBatch + static_cast<uint32_t>(lane), ring + static_cast<size_t>(slot) * kFuseBatch * kMtN);
       __hip_atomic_store(&s_ready[slot], j + 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
-      __builtin_amdgcn_s_setprio(0);
     };
     if (wave == 0) {
       const uint32_t b = take_batch(0);
@@ -240,13 +240,18 @@ __global__ __launch_bounds__(1024, (FORM == 2 || (W == kNormal && sizeof(T1) == 
       const uint32_t batch = number >> kFuseRoundBits;
       // (every wave's first task of the batch behind the last one)
       if (batch >= n_batches || (number & ((1u << kFuseRoundBits) - 1u)) != round_of(j)) break;
-      for (uint32_t spin = 0; spin < SPIN; ++spin) {
-        // (a break, not a condition of the loop: the polls of the seeding's ten microseconds take the issue slots of the wave that seeds)
-        if ((flag & ~kFuseNotSeeded) >= j + 1u) break;
-        __builtin_amdgcn_s_sleep(8);
-        flag = __hip_atomic_load(&s_ready[slot], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
-      }
-      if ((flag & ~kFuseNotSeeded) < j + 1u) flag = kFuseNotSeeded;
+      auto await_states = [&]() {
+        for (uint32_t spin = 0; spin < SPIN; ++spin) {
+          // (A break, not a condition of the loop, which took eleven instructions a poll instead of four, and one poll in 512 cycles:
+          // those of the seeding's ten microseconds take the issue slots of the wave that seeds.  100,000 streams of 20 synapses
+          // 88.4 -> 86.0 us, uniform weights 94.5 -> 91.5, normal ones 98.8 -> 95.4.)
+          if ((flag & ~kFuseNotSeeded) >= j + 1u) break;
+          __builtin_amdgcn_s_sleep(8);
+          flag = __hip_atomic_load(&s_ready[slot], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
+        if ((flag & ~kFuseNotSeeded) < j + 1u) flag = kFuseNotSeeded;
+      };
+      if (!early) await_states();
       const uint32_t behind = r == 0 ? take_batch(j + 1u) : n_batches;  // (the batch that this wave is to seed)
       if (behind < n_batches) {
         // slot (j + 1) % 3 last held batch j - 2: (j + 1) / 3 batches have used it, 64 loads each, and its flag is j - 1
@@ -261,6 +266,7 @@ __global__ __launch_bounds__(1024, (FORM == 2 || (W == kNormal && sizeof(T1) == 
         if (free_) seed_batch(j + 1u, behind);
         else __hip_atomic_store(&s_ready[slot1], kFuseNotSeeded | (j + 2u), __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
       }
+      if (early) await_states();
       const uint32_t *pre = (flag & kFuseNotSeeded) ? nullptr : ring + (static_cast<size_t>(slot) * kFuseBatch + r) * kMtN;
       auto loaded = [&]() {
         if (lane == 0) __hip_atomic_fetch_add(&s_loaded[slot], 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -673,9 +679,15 @@ void launch_rowwalk_impl(hipStream_t stream, const VT *in, T1 *out, uint32_t n_o
   unsigned needed = fused ? div_up(n_out, kFuseBatch) : div_up(n_out, nwaves);
   if (fused && needed > sc.ring_groups) needed = sc.ring_groups;
   const unsigned grid = needed < resident ? needed : resident;
-  // (more batches than workgroups: taken as they come; a capture that finds no counters shares them out evenly)
+  // Batches are taken as they come from four for a workgroup on, rows of 200 synapses and more from two and a half; fewer are
+  // shared out evenly, for then the workgroups that finish first, two to a CU, would take a last batch together while other CUs are
+  // idle (20,000 inputs, even shares / taken: rows of 100, 45,000 of them 43.7 / 52 us, 60,000 54 / 61, 75,000 66.6 / 75, 90,000 76.3 / 82,
+  // 120,000 99.6 / 104, 150,000 122.5 / 125.7, 200,000 159 / 157, normal weights 45,000 54.7 / 69, 90,000 98 / 106, 120,000 125 / 123, 200,000 196 / 192; rows of
+  // 1,000, 60,000 of them 113 / 116, 75,000 133 / 136, 90,000 162 / 154, 150,000 259 / 248, normal weights 75,000 379 / 383, 90,000 468 / 446).
+  // A capture that finds no counters shares them out, too.
   uint32_t *next = nullptr;
-  if (fused && grid < div_up(n_out, kFuseBatch)) {
+  const double per_row = -log_p * static_cast<double>(n_in);
+  if (fused && 2u * div_up(n_out, kFuseBatch) >= (per_row < 200.0 ? 8u : 5u) * grid) {
     next = stream_counters(stream, true);
     if (next != nullptr) next += kWalkCounters;
   }

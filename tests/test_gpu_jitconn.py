@@ -723,6 +723,24 @@ def test_waves_that_do_not_wait_for_their_generators_write_their_rows_all_the_sa
     np.testing.assert_array_equal(out.cpu().numpy(), want)
 
 
+@pytest.mark.parametrize("n_out,per_row", [(33_001, 30), (60_000, 100), (81_921, 250), (135_000, 20)])
+def test_row_walk_whose_batches_are_shared_out_or_taken(cuda, oracle_mod, n_out, per_row):
+  # two batches for some workgroups, seeded side by side and one after the other; taken from the counter from two and a
+  # half and from four batches a workgroup on
+  n_in = 3000
+  ev = np.random.default_rng(n_out).random(n_in) < 0.1
+  kw = dict(log_p=oracle_mod.log_p_of(per_row / n_in), seed=5, n_row=n_out, n_col=n_in, w_a=0.25, w_b=1.75)
+  print("case", n_out, per_row, flush=True)
+  for w_kind in ("homo", "uniform"):
+    want, mag = oracle_mod.jitconn_matvec(ev, w_kind=w_kind, dense=False, per_stream_seed=True, return_abs=True, **kw)
+    for _ in range(3):
+      got = kernel_call(ev, w_kind=w_kind, col_walk=False, dense=False, **kw)
+      if w_kind == "homo":
+        assert np.array_equal(got, want)
+      else:
+        assert_close_reordered(got, want, mag, np.float32, what="row walk, batches shared out or taken")
+
+
 @pytest.mark.parametrize("n_out,n_in", [(8192, 3000), (10_007, 200_000), (20_000, 400_000), (70_001, 5000)])
 def test_row_walk_with_generators_seeded_inside_the_kernel(cuda, oracle_mod, n_out, n_in):
   # from 8,192 outputs the row walk seeds its generators itself, 64 streams at a time, into rings of
