@@ -46,7 +46,9 @@
 // where one window of x holds them or nearly so (the threshold below), it walks step by step with that window in LDS and
 // gathers what it misses.  Which of the two a matrix wants is known on the device only: 300,000 rows of 100 and 120,000 floats,
 // columns within 300 / 3,000 of the row's place 70 / 71 us, with all windows passing by 109 / 109, with the first 147 KB staged
-// 69 / 99; a tenth of them anywhere 78, 109 and 72.  What the look costs where the windows pass by: 0 to 2 us of 85 to 140 (from loads
+// 69 / 99; a tenth of them anywhere 78, 109 and 72.  Slower than gathers from L2 that hit: one weight and
+// 180,000 floats, columns within 300, 65 us (59), 30,000 rows of 1,000 and 150,000 floats 74 (64), and gathered so by this kernel,
+// too (65 and 70, but 73 instead of 70 with 120,000).  What the look costs where the windows pass by: 0 to 2 us of 85 to 140 (from loads
 // of its own, spread over the workgroup's nonzeros, 2 to 5).
 #include <type_traits>
 
