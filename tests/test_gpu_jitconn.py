@@ -637,10 +637,11 @@ def test_normal_weights_worked_off_in_groups(cuda, oracle_mod, n_syn, dtype):
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
-@pytest.mark.parametrize("n_in", [90_112, 90_113, 151_552, 151_553])
+@pytest.mark.parametrize("n_in", [90_112, 90_113, 151_552, 151_553, 311_296, 311_297])
 @pytest.mark.parametrize("p", [0.003, 0.0002, 0.00005])
 def test_normal_weights_on_both_sides_of_the_bitmaps_and_skip_paths(cuda, oracle_mod, p, n_in, dtype):
-  # the last bitmaps that are exact in LDS and the first two-level ones (float 151,552 inputs, double 90,112), and
+  # bitmaps exact in LDS, up to the last one and the first in two levels (for more rows than here they begin at 151,552 inputs,
+  # double 90,112: test_row_walk_on_both_sides_of_the_exact_bitmaps), and
   # conn_probs whose skips are tried on the upper word alone, on both words, and in 13 bits of fraction less
   rng = np.random.default_rng(n_in)
   ev = rng.random(n_in) < 0.2

@@ -191,7 +191,7 @@ def test_normal_row_walk_is_captured_on_a_cold_stream(cuda, n_in, capfd):
 
 
 def test_row_walk_is_captured_where_the_stream_has_rings_but_no_counters(cuda, capfd):
-  # more batches of streams than workgroups, and no counter to take them from: they are shared out evenly, and the
+  # more than four batches of streams for each of 512 workgroups, and no counter to take them from: they are shared out evenly, and the
   # call, which succeeds, prints nothing
   rng = np.random.default_rng(3)
   handle = ctypes.c_void_p()  # (a stream of its own: torch's come from a pool and may have counters from elsewhere)
@@ -205,7 +205,7 @@ def test_row_walk_is_captured_where_the_stream_has_rings_but_no_counters(cuda, c
   before = _query(s.cuda_stream)
   n_in = 20_000
   ev = torch.zeros(n_in, dtype=torch.bool, device=cuda)
-  kw = dict(weight=1.0, conn_prob=0.005, shape=(70_001, n_in), seed=5, outdim_parallel=True)
+  kw = dict(weight=1.0, conn_prob=0.005, shape=(140_001, n_in), seed=5, outdim_parallel=True)
   bpl.event_matvec_prob_conn_homo_weight(ev, **kw)
   torch.cuda.synchronize()
   capfd.readouterr()
