@@ -120,9 +120,9 @@ def custom_call(name, buffers, opaque, stream=None):
     except (AttributeError, TypeError):
       import torch
       stream = torch.cuda.current_stream(buffers[0].device).cuda_stream
-  if type(stream) is int and type(opaque) is bytes and len(buffers) <= 16:
+  try:
     (_enqueue or _native_enqueue())(address, stream, opaque, *buffers)
-  else:  # (what the native call does not take)
+  except TypeError:  # (a stream, descriptor or number of buffers that the native call does not take: it has enqueued nothing)
     _enqueue_ctypes(address, stream, opaque, *buffers)
 
 
