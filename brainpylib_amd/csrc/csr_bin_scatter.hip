@@ -680,12 +680,13 @@ __device__ __forceinline__ uint64_t synapse_count(double v) { return static_cast
 // descriptor of the event operators does not carry the nonzero count.  So the bins are not private
 // to a producer here: window b owns 8 runs of `cap` pairs each, shared by the producers p with the
 // same p % 8, and a producer reserves room for the pairs a round holds for a window with one
-// global atomic on the run's fill counter (at most one per window and round of 4,096 nonzeros;
+// global atomic on the run's fill counter (at most one per window and round of 5,120 nonzeros, doubles 3,072;
 // the event operators move far fewer pairs than the dense product, for which that many
 // same-address atomics would cost more than private regions).  Whatever the distribution of the
 // activity over rows and of the columns over windows, a run only overflows (into direct atomics
 // on y) when it receives more than `cap` pairs.
-constexpr uint32_t kPairsPerProducer = 4096;  // a producer takes part per that many active nonzeros (estimated): one round
+constexpr uint32_t kPairsPerProducer = 2048;  // a producer takes part per that many active nonzeros (31,337 x 47,011
+                                              // doubles, 282,000 pairs: 11.0 us, per 4,096 13.8)
 constexpr uint32_t kSubRuns = 8;              // a window's run is split: producer p appends to sub-run p % 8, so that
                                               // the atomics on one counter (about 15 ns each) stay few
 constexpr uint32_t kFillStride = 32;          // words between fill counters: one 128-byte line each
@@ -698,52 +699,96 @@ constexpr uint32_t kPairsPerPart = 8192;      // a consumer workgroup takes part
 // fill area (zeroed with it before every call) and the consumer's waves add the rows to y directly.
 constexpr uint32_t kDirectPairs = 131072;
 constexpr uint32_t kDirectWord = 1;           // (fill counters sit at multiples of kFillStride)
+// Up to this many listed rows are shared out by their nonzeros, whatever their lengths: every producer adds up the whole
+// list, 1 to 2 us for 4 rows a thread, 6 for 8; of more rows every one of 512 producers has eight and more to even them out.
+// (940 listed rows of 300 on average, log-normal, doubles: 21 -> 11 us.)
+constexpr uint32_t kExactRows = 4 * kBinThreads;
 
+// Bound by latency: of 22 us for 5e6 float pairs (100,000 x 100,000, 1e8 nonzeros, 5 % events; 25 before) 3 are the start,
+// 7 the rows' nonzeros, 4 the copy-out, the rest ranks, scan, reservation and sort between the three barriers of a round.
+// The nonzeros of a row mostly come in the order of their columns: runs of a wave's lanes meet in one window.  Their first
+// lane takes the ranks of the run; lane by lane their atomics on one counter took turns (4.8e6 pairs of rows of
+// 400 over five windows 33 -> 20 us).
+//
 // (At most 80 scalar registers: measured on this device, a 1,024-thread workgroup whose waves hold
 // 81..96 of them is alone on its CU, as it would be with more than 64 vector registers; the
 // float producer crossed that line by one register and took 37 instead of 27 us.)
 template <typename F, bool HETER, typename I>
-__global__ __launch_bounds__(kBinThreads) __attribute__((amdgpu_num_sgpr(80))) void bin_active_rows_kernel(
+__global__ __launch_bounds__(kBinThreads, 8) __attribute__((amdgpu_num_sgpr(80))) void bin_active_rows_kernel(
     const F *__restrict__ data, const I *__restrict__ indices, const I *__restrict__ indptr,
     uint32_t n_row, const uint32_t *__restrict__ active_count, const uint2 *__restrict__ active_list,
-    uint32_t list_cap, const uint32_t *__restrict__ active_colbase, F *__restrict__ y, uint32_t shift, uint32_t cap,
-    BinPair<F> *__restrict__ pairs, uint32_t *__restrict__ fill) {
+    uint32_t list_cap, const uint32_t *__restrict__ active_colbase, uint32_t entries, F *__restrict__ y, uint32_t shift,
+    uint32_t cap, BinPair<F> *__restrict__ pairs, uint32_t *__restrict__ fill) {
   __shared__ uint32_t s_ptr[kTileRows + 1];     // nonzeros of the tile's rows before row k
   __shared__ uint32_t s_start[kTileRows];       // first nonzero of row k in the matrix
   __shared__ uint32_t s_colbase[kTileRows];     // added to row k's columns (batched calls: batch entry * n_col)
   __shared__ uint32_t s_hint[kBinThreads + 1];
-  __shared__ uint32_t s_cnt[kMaxWindows];
-  __shared__ uint32_t s_off[kMaxWindows + 1];
-  __shared__ uint32_t s_base[kMaxWindows];      // where the round's pairs of a window go in its run
+  __shared__ uint32_t s_cnt[kMaxWindows];       // pairs of the current round, per window
+  __shared__ uint32_t s_off[kMaxWindows + 1];   // their offsets in the sorted round
+  __shared__ uint32_t s_base[kMaxWindows];      // place in the window's run of the pair at position i of the round: s_base + i
   __shared__ uint32_t s_wave[kBinThreads / kWave];
-  constexpr int U = (sizeof(F) == 4) ? 4 : 2;
+  __shared__ uint32_t s_share[4];               // this producer's first and last row, the nonzeros it leaves out of them
+  constexpr int U = (sizeof(F) == 4) ? 5 : 3;
   constexpr uint32_t kRound = U * kBinThreads;
-  __shared__ BinPair<F> s_sorted[kRound];
-  __shared__ uint8_t s_window[kRound];
+  __shared__ F s_val[kRound];
+  __shared__ uint32_t s_rel[kRound];            // (the window's number above the position, from bit kWindowIdShift)
   const uint32_t tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
   const uint32_t total = active_count[0] < list_cap ? active_count[0] : list_cap;  // (never beyond the list)
   const uint32_t nnz = static_cast<uint32_t>(indptr[n_row]);  // (64-bit offsets: listed only below 2^32 nonzeros)
+  // the listed rows' nonzeros: exact where every producer can look at the whole list, else from the mean row length
+  uint64_t work = static_cast<uint64_t>(total) * (nnz / n_row + 1u);
+  const bool exact = total <= kExactRows && static_cast<uint64_t>(nnz) * entries <= 0xffffffffu;
+  const uint32_t each = (total + kBinThreads - 1u) / kBinThreads;  // (of these, listed rows a thread)
+  uint32_t before_mine = 0;
+  if (exact) {
+    uint32_t mine = 0;
+    for (uint32_t e = 0; e < each; ++e) {
+      const uint32_t k = tid * each + e;
+      mine += k < total ? active_list[k].y : 0u;
+    }
+    const uint32_t incl = wave_inclusive_scan_u32(mine);
+    if (lane == kWave - 1) s_wave[wave] = incl;
+    __syncthreads();
+    uint32_t all = 0;
+    for (uint32_t w = 0; w < kBinThreads / kWave; ++w) {
+      if (w == wave) before_mine = all;
+      all += s_wave[w];
+    }
+    before_mine += incl - mine;
+    work = all;
+  }
   // with little activity a few producers finish sooner than a chip full of them
-  const uint64_t want = (static_cast<uint64_t>(total) * (nnz / n_row + 1u) + kPairsPerProducer - 1u) / kPairsPerProducer;
+  const uint64_t want = (work + kPairsPerProducer - 1u) / kPairsPerProducer;
   const uint32_t producers = want < 1u ? 1u : want > gridDim.x ? gridDim.x : static_cast<uint32_t>(want);
-  if (static_cast<uint64_t>(total) * (nnz / n_row + 1u) <= kDirectPairs) {
+  if (work <= kDirectPairs) {
     if (blockIdx.x == 0 && tid == 0) fill[kDirectWord] = total;
     return;
   }
   const uint32_t p = blockIdx.x;
   if (p >= producers) return;
   const uint32_t sub = p % kSubRuns;
-  // Producer p takes an equal share of the listed rows; where there are fewer rows than producers (a few
-  // long rows are active), `parts` producers take a row, each an equal part of its nonzeros.
-  uint32_t lo, hi, part = 0, parts = 1;
-  if (total < producers) {
-    parts = producers / total;
-    lo = p / parts, hi = lo + 1u, part = p % parts;
-    if (lo >= total) return;
+  // Producer p takes the rows [lo, hi) of the list, but for the first `skip` nonzeros of row lo and what lies behind the
+  // first `end` of row hi - 1: an equal share of the nonzeros, or, of a long list, of the rows.
+  uint32_t lo, hi, skip = 0, end = 0xffffffffu;
+  if (exact) {
+    const uint32_t all = static_cast<uint32_t>(work);
+    const uint32_t a = static_cast<uint32_t>(static_cast<uint64_t>(p) * all / producers);
+    const uint32_t b = static_cast<uint32_t>(static_cast<uint64_t>(p + 1u) * all / producers);
+    for (uint32_t e = 0; e < each; ++e) {  // (listed rows are never empty: one row holds nonzero a, one nonzero b - 1)
+      const uint32_t k = tid * each + e, len = k < total ? active_list[k].y : 0u;
+      if (a - before_mine < len) s_share[0] = k, s_share[2] = a - before_mine;
+      if (b - 1u - before_mine < len) s_share[1] = k + 1u, s_share[3] = b - before_mine;
+      before_mine += len;
+    }
+    __syncthreads();
+    lo = s_share[0], hi = s_share[1], skip = s_share[2], end = s_share[3];
   } else {
     lo = static_cast<uint32_t>(static_cast<uint64_t>(p) * total / producers);
     hi = static_cast<uint32_t>(static_cast<uint64_t>(p + 1) * total / producers);
   }
+  // (in scalar registers: the rounds take what vector registers there are)
+  auto uniform = [](uint32_t v) { return static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(v))); };
+  lo = uniform(lo), hi = uniform(hi), skip = uniform(skip), end = uniform(end);
   if (tid < kMaxWindows) s_cnt[tid] = 0;
   const F w_homo = HETER ? F(0) : data[0];
   // homogeneous weight: a run holds the pairs' columns only, `cap` of them
@@ -762,11 +807,10 @@ __global__ __launch_bounds__(kBinThreads) __attribute__((amdgpu_num_sgpr(80))) v
     const uint32_t rows = (hi - t0 < kTileRows) ? hi - t0 : kTileRows;
     __syncthreads();  // the previous tile is done with s_ptr / s_start (and s_cnt is cleared)
     uint2 e = make_uint2(0u, 0u);
-    if (tid < rows) e = active_list[t0 + tid];
-    if (parts > 1u) {  // (one row: this producer's part of it, which may be empty)
-      const uint32_t a = static_cast<uint32_t>(static_cast<uint64_t>(e.y) * part / parts);
-      const uint32_t b = static_cast<uint32_t>(static_cast<uint64_t>(e.y) * (part + 1u) / parts);
-      e.x += a, e.y = b - a;
+    if (tid < rows) {
+      e = active_list[t0 + tid];
+      if (t0 + tid == hi - 1u && end < e.y) e.y = end;
+      if (t0 + tid == lo) e.x += skip, e.y -= skip;
     }
     const uint32_t incl = wave_inclusive_scan_u32(e.y);
     if (lane == kWave - 1) s_wave[wave] = incl;
@@ -779,7 +823,7 @@ __global__ __launch_bounds__(kBinThreads) __attribute__((amdgpu_num_sgpr(80))) v
     }
     if (tid == rows - 1u) s_ptr[rows] = before + incl;
     __syncthreads();
-    const uint32_t j1 = s_ptr[rows];  // the tile's nonzeros, numbered from 0 (listed rows are never empty)
+    const uint32_t j1 = s_ptr[rows];  // the tile's nonzeros, numbered from 0 (no row is empty)
     for (uint32_t seg = 0; seg < j1; seg += kSegment) {
       const uint32_t seg_end = (j1 - seg < kSegment) ? j1 : seg + kSegment;
       __syncthreads();  // the previous segment is done with s_hint
@@ -789,16 +833,20 @@ __global__ __launch_bounds__(kBinThreads) __attribute__((amdgpu_num_sgpr(80))) v
         if (tid == 0) s_hint[kBinThreads] = rows - 1u;
       }
       __syncthreads();
+      // rounds of equal size, at most kRound nonzeros each
+      const uint32_t n_rounds = (seg_end - seg + kRound - 1u) / kRound;
+      const uint32_t step = (seg_end - seg + n_rounds - 1u) / n_rounds;
       // One round's column indices and weights are requested a round ahead, so that their latency
       // overlaps the sort, the reservation and the stores of the round before.
-      auto fetch = [&](uint32_t jb, uint32_t (&col)[U], F (&val)[U]) {
+      auto fetch = [&](uint32_t base, uint32_t (&col)[U], F (&val)[U]) {
         // first where every nonzero of the lane lies (LDS only), then all the loads together, without a
-        // branch around them (beyond the segment: its last nonzero again)
+        // branch around them (beyond the round: its last nonzero again)
+        const uint32_t round_end = base + step < seg_end ? base + step : seg_end;
         uint32_t at[U], cb[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-          const uint32_t j = jb + u * kBinThreads;
-          const uint32_t jc = j < seg_end ? j : seg_end - 1u;
+          const uint32_t j = base + tid + u * kBinThreads;
+          const uint32_t jc = j < round_end ? j : round_end - 1u;
           const uint32_t q = (jc - seg) >> kHintShift;
           const uint32_t k = row_of(jc, s_hint[q], s_hint[q + 1]);
           at[u] = s_start[k] + (jc - s_ptr[k]);
@@ -811,73 +859,84 @@ __global__ __launch_bounds__(kBinThreads) __attribute__((amdgpu_num_sgpr(80))) v
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-          const uint32_t j = jb + u * kBinThreads;
-          col[u] = j < seg_end ? col[u] + cb[u] : 0xffffffffu;  // (0xffffffff: no pair)
+          const uint32_t j = base + tid + u * kBinThreads;
+          col[u] = j < round_end ? col[u] + cb[u] : 0xffffffffu;  // (0xffffffff: no pair)
         }
       };
       uint32_t col[U];
       F val[U];
-      fetch(seg + tid, col, val);
-      for (uint32_t jb = seg + tid; jb - tid < seg_end; jb += kRound) {
+      fetch(seg, col, val);
+      // (Three barriers a round: what a round's stores read is written again only behind the next one's first two.)
+      for (uint32_t base = seg; base < seg_end; base += step) {
         uint32_t ncol[U];
         F nval[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) ncol[u] = 0xffffffffu, nval[u] = F(0);
-        if (jb - tid + kRound < seg_end) fetch(jb + kRound, ncol, nval);
-        uint32_t rank[U], win[U], rel[U];
+        if (base + step < seg_end) fetch(base + step, ncol, nval);
+        uint32_t rank[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-          rank[u] = 0;
-          win[u] = 0xffffffffu;
-          rel[u] = 0;
-          if (col[u] != 0xffffffffu) {
-            win[u] = col[u] >> shift;
-            rel[u] = col[u] & ((1u << shift) - 1u);
-          }
+          const uint32_t w = col[u] != 0xffffffffu ? col[u] >> shift : kMaxWindows;
+          const uint32_t prev = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(
+              static_cast<int>(~w), static_cast<int>(w), 0x138 /* wave_shr:1 */, 0xf, 0xf, false));
+          const uint64_t heads = __builtin_amdgcn_ballot_w64(w != prev);
+          const uint32_t off = static_cast<uint32_t>(__builtin_clzll(heads << (kWave - 1u - lane)));  // (lane 0 is a head)
+          const uint64_t behind = (heads >> lane) >> 1;
+          uint32_t taken = 0;
+          if (off == 0u && w != kMaxWindows)
+            taken = atomicAdd(&s_cnt[w], behind ? static_cast<uint32_t>(__builtin_ctzll(behind)) + 1u : kWave - lane);
+          rank[u] = static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(static_cast<int>(4u * (lane - off)), static_cast<int>(taken))) + off;
         }
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-          if (win[u] != 0xffffffffu) rank[u] = atomicAdd(&s_cnt[win[u]], 1u);
         __syncthreads();
         if (tid < kWave) {  // two windows per lane: offsets within the round, room in the windows' runs
           const uint32_t c0 = s_cnt[2 * tid], c1 = s_cnt[2 * tid + 1];
-          const uint32_t sum = wave_inclusive_scan_u32(c0 + c1);
-          s_off[2 * tid] = sum - (c0 + c1);
-          s_off[2 * tid + 1] = sum - c1;
-          if (tid == kWave - 1) s_off[kMaxWindows] = sum;
           // (both reservations under way together; a window without pairs adds nothing to its counter)
           const uint32_t b0 = atomicAdd(&fill[(2 * tid * kSubRuns + sub) * kFillStride], c0);
           const uint32_t b1 = atomicAdd(&fill[((2 * tid + 1) * kSubRuns + sub) * kFillStride], c1);
-          s_base[2 * tid] = b0;
-          s_base[2 * tid + 1] = b1;
+          const uint32_t sum = wave_inclusive_scan_u32(c0 + c1);
+          const uint32_t o0 = sum - (c0 + c1), o1 = sum - c1;
+          s_off[2 * tid] = o0;
+          s_off[2 * tid + 1] = o1;
+          if (tid == kWave - 1) s_off[kMaxWindows] = sum;
+          s_cnt[2 * tid] = 0;
+          s_cnt[2 * tid + 1] = 0;
+          s_base[2 * tid] = b0 - o0;  // (modulo 2^32)
+          s_base[2 * tid + 1] = b1 - o1;
         }
         __syncthreads();
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-          if (win[u] != 0xffffffffu) {
-            const uint32_t pos = s_off[win[u]] + rank[u];
-            BinPair<F> o;
-            o.rel = rel[u];
-            o.val = val[u];
-            s_sorted[pos] = o;
-            s_window[pos] = static_cast<uint8_t>(win[u]);
+          if (col[u] != 0xffffffffu) {
+            const uint32_t w = col[u] >> shift;
+            const uint32_t pos = s_off[w] + rank[u];
+            s_val[pos] = val[u];
+            s_rel[pos] = (col[u] & ((1u << shift) - 1u)) | (w << kWindowIdShift);
           }
         }
         __syncthreads();
         const uint32_t round_total = s_off[kMaxWindows];
-        for (uint32_t i = tid; i < round_total; i += kBinThreads) {
-          const uint32_t w = s_window[i];
-          const BinPair<F> o = s_sorted[i];
-          const uint32_t slot = s_base[w] + (i - s_off[w]);
-          if (slot < cap) {
-            if (HETER) pairs[static_cast<uint64_t>(w * kSubRuns + sub) * cap + slot] = o;
-            else run_columns[static_cast<uint64_t>(w * kSubRuns + sub) * cap + slot] = o.rel;
-          } else if (HETER) atomic_add(y + ((w << shift) | o.rel), o.val);
-          else add_synapse_count(y + ((w << shift) | o.rel), 1u);  // (the consumer turns counts into sums)
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const uint32_t i = tid + u * kBinThreads;
+          if (i < round_total) {
+            const uint32_t key = s_rel[i], w = key >> kWindowIdShift, rel = key & ((1u << kWindowIdShift) - 1u);
+            const uint32_t slot = s_base[w] + i;
+            if (slot < cap) {
+              const uint64_t at = static_cast<uint64_t>(w * kSubRuns + sub) * cap + slot;
+              if (HETER) {
+                BinPair<F> o;
+                o.rel = rel, o.val = s_val[i];
+                pairs[at] = o;
+              } else {
+                run_columns[at] = rel;
+              }
+            } else if (HETER) {
+              atomic_add(y + ((w << shift) | rel), s_val[i]);
+            } else {
+              add_synapse_count(y + ((w << shift) | rel), 1u);  // (the consumer turns counts into sums)
+            }
+          }
         }
-        __syncthreads();
-        if (tid < kMaxWindows) s_cnt[tid] = 0;
-        __syncthreads();
 #pragma unroll
         for (int u = 0; u < U; ++u) col[u] = ncol[u], val[u] = nval[u];
       }
@@ -1421,7 +1480,8 @@ size_t bin_event_scatter_min_bytes(uint32_t n_col) {
 template <typename F, typename I>
 bool bin_event_scatter(hipStream_t stream, const F *data, bool heter, const I *indices, const I *indptr,
                        F *y, uint32_t n_row, uint32_t n_col, uint32_t *active_count, const uint2 *active_list,
-                       uint32_t list_cap, void *scratch, size_t scratch_bytes, const uint32_t *active_colbase) {
+                       uint32_t list_cap, void *scratch, size_t scratch_bytes, const uint32_t *active_colbase,
+                       uint32_t entries) {
   const uint32_t shift = event_window_shift(n_col);
   const uint32_t n_win = div_up(n_col, 1u << shift);
   if (scratch_bytes < bin_event_scatter_min_bytes<F>(n_col)) return false;
@@ -1452,10 +1512,10 @@ bool bin_event_scatter(hipStream_t stream, const F *data, bool heter, const I *i
   const uint32_t producers = 2u * num_cu;
   if (heter)
     hipLaunchKernelGGL((bin_active_rows_kernel<F, true, I>), dim3(producers), dim3(kBinThreads), 0, stream, data, indices,
-                       indptr, n_row, active_count, active_list, list_cap, active_colbase, y, shift, cap, pairs, fill);
+                       indptr, n_row, active_count, active_list, list_cap, active_colbase, entries, y, shift, cap, pairs, fill);
   else
     hipLaunchKernelGGL((bin_active_rows_kernel<F, false, I>), dim3(producers), dim3(kBinThreads), 0, stream, data, indices,
-                       indptr, n_row, active_count, active_list, list_cap, active_colbase, y, shift, cap, pairs, fill);
+                       indptr, n_row, active_count, active_list, list_cap, active_colbase, entries, y, shift, cap, pairs, fill);
   hipLaunchKernelGGL(add_kernel, dim3(n_win * slices * parts), dim3(kBinThreads), lds, stream, y, n_col, shift,
                      lds_shift, parts, cap, pairs, fill, active_count, data, indices, active_list, active_colbase);
   return true;
@@ -1623,16 +1683,16 @@ template size_t bin_event_scatter_min_bytes<float>(uint32_t);
 template size_t bin_event_scatter_min_bytes<double>(uint32_t);
 template bool bin_event_scatter<float, uint32_t>(hipStream_t, const float *, bool, const uint32_t *, const uint32_t *, float *,
                                                  uint32_t, uint32_t, uint32_t *, const uint2 *, uint32_t, void *, size_t,
-                                                 const uint32_t *);
+                                                 const uint32_t *, uint32_t);
 template bool bin_event_scatter<double, uint32_t>(hipStream_t, const double *, bool, const uint32_t *, const uint32_t *,
                                                   double *, uint32_t, uint32_t, uint32_t *, const uint2 *, uint32_t, void *,
-                                                  size_t, const uint32_t *);
+                                                  size_t, const uint32_t *, uint32_t);
 template bool bin_event_scatter<float, uint64_t>(hipStream_t, const float *, bool, const uint64_t *, const uint64_t *, float *,
                                                  uint32_t, uint32_t, uint32_t *, const uint2 *, uint32_t, void *, size_t,
-                                                 const uint32_t *);
+                                                 const uint32_t *, uint32_t);
 template bool bin_event_scatter<double, uint64_t>(hipStream_t, const double *, bool, const uint64_t *, const uint64_t *,
                                                   double *, uint32_t, uint32_t, uint32_t *, const uint2 *, uint32_t, void *,
-                                                  size_t, const uint32_t *);
+                                                  size_t, const uint32_t *, uint32_t);
 template bool flat_window_scatter<float>(const char *, hipStream_t, const float *, bool, const uint32_t *, const uint32_t *,
                                          const float *, float *, uint32_t, uint32_t);
 template bool flat_window_scatter<double>(const char *, hipStream_t, const double *, bool, const uint32_t *,

@@ -506,6 +506,41 @@ def test_event_scatter_sorted_by_output_window(cuda, oracle_mod, dtype):
       assert np.array_equal(got, want)  # a homogeneous weight is added once per synapse: the reference's bits
 
 
+@pytest.mark.parametrize("listed", [1, 1023, 1025, 4096, 4097])
+@pytest.mark.parametrize("columns", ["sorted", "descending", "random", "one"])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_event_scatter_shares_the_listed_rows_nonzeros(cuda, listed, columns, dtype):
+  # up to 4,096 listed rows are shared out by their nonzeros, longer lists by rows; a producer's share may begin and end
+  # within a row (one row holds half of all nonzeros), a wave's columns come in runs of any length of one window.
+  # Weights are small whole numbers: every order of the additions gives the same sums.
+  rng = np.random.default_rng(listed)
+  n_row, n_col = 2 * listed + 8192, 60_001
+  lengths = np.zeros(n_row, dtype=np.int64)
+  on = rng.permutation(n_row)[:listed]
+  lengths[on] = np.maximum(1, rng.lognormal(np.log(140_000 / listed), 1.0, listed).astype(np.int64))
+  lengths[on[listed // 2]] = 140_000
+  lengths[rng.permutation(n_row)[:listed]] += 3  # (also rows without an event)
+  indptr = np.concatenate([[0], np.cumsum(lengths)]).astype(np.uint32)
+  rows = np.repeat(np.arange(n_row), lengths)
+  indices = rng.integers(0, 300 if columns == "one" else n_col, rows.shape[0])
+  if columns == "one":
+    indices[:] = np.where(rows % 2, 7, n_col - 1)
+  elif columns != "random":
+    order = np.lexsort((indices if columns == "sorted" else -indices, rows))
+    indices = indices[order]
+  data = rng.integers(-8, 9, rows.shape[0]).astype(dtype)
+  ev = np.zeros(n_row, dtype=bool)
+  ev[on] = True
+  for kind in (ev, ev.astype(dtype)):
+    got = bpl.event_csr_matvec(data, indices.astype(np.uint32), indptr, kind, shape=(n_row, n_col), transpose=True).cpu().numpy()
+    want = np.zeros(n_col)
+    np.add.at(want, indices[ev[rows]], data[ev[rows]])
+    assert np.array_equal(got, want)
+    got = bpl.event_csr_matvec(np.array([2.0], dtype=dtype), indices.astype(np.uint32), indptr, kind, shape=(n_row, n_col),
+                               transpose=True).cpu().numpy()
+    assert np.array_equal(got, 2.0 * np.bincount(indices[ev[rows]], minlength=n_col))
+
+
 def test_scatter_through_the_active_row_list(cuda, oracle_mod):
   # more than 32,768 rows: the active rows are first gathered into one list that the row groups
   # share; both input kinds, activity concentrated in one corner of the matrix, twice in a row
