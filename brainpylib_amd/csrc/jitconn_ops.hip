@@ -440,8 +440,8 @@ __global__ __launch_bounds__(kColBinThreads, sizeof(T1) == 4 ? 8 : 4) void jitco
   }
   __syncthreads();
   const uint64_t region = static_cast<uint64_t>(p) * n_win * cap;  // first place of this workgroup's bins
-  T1 *const packed_val = static_cast<T1 *>(pairs);
-  uint16_t *const packed_rel = reinterpret_cast<uint16_t *>(packed_val + n_pairs);
+  unsigned char *const region_val = static_cast<unsigned char *>(pairs) + region * (packed ? sizeof(T1) : sizeof(BinPair<T1>));
+  unsigned char *const region_rel = static_cast<unsigned char *>(pairs) + n_pairs * sizeof(T1) + region * 2u;  // (packed)
   uint32_t *st = s_state + wave * kWords;
   const uint32_t n_list = n_list_dev ? *n_list_dev : n_list_host;
 
@@ -460,7 +460,7 @@ __global__ __launch_bounds__(kColBinThreads, sizeof(T1) == 4 ? 8 : 4) void jitco
         return;
       }
     }
-    walk_stream<T1, W, W == kNormal, kShort>(st, lane, seed + col, pre, n_out, skips, wa, wb, [&](uint32_t idx, T1 w, bool valid, bool) {
+    walk_stream<T1, W, true, kShort>(st, lane, seed + col, pre, n_out, skips, wa, wb, [&](uint32_t idx, T1 w, bool valid, bool partial) {
       const uint32_t b = idx >> shift;
       // The positions rise from lane to lane and the lanes that hold a synapse are the first ones of the
       // wave, so the lanes of a batch that meet in one window are neighbours (sixteen of them with
@@ -469,34 +469,37 @@ __global__ __launch_bounds__(kColBinThreads, sizeof(T1) == 4 ? 8 : 4) void jitco
       // has a counter of its own), so the first lane of every run of equal windows reserves the places
       // of the whole run and the others fetch its answer (12 cycles with the shuffle): 3 to 6 % of the
       // walk, whose larger cost is the scattered stores of the pairs.  Lanes 0 and 32 begin runs of their
-      // own, which keeps the masks at 32 bits.
-      const uint32_t n_valid = static_cast<uint32_t>(__popcll(__ballot(valid)));
-      const uint64_t heads = __ballot(b != wave_shift_up1(b)) | 0x100000001ull;
+      // own, which keeps the masks at 32 bits, and so does the first lane without a synapse: run lengths then need no bound.
+      const uint64_t valids = partial ? __builtin_amdgcn_ballot_w64(valid) : ~0ull;
+      const uint64_t heads = __builtin_amdgcn_ballot_w64(b != wave_shift_up1(b)) | 0x100000001ull | (valids + 1ull);
       const uint32_t half = lane < 32 ? static_cast<uint32_t>(heads) : static_cast<uint32_t>(heads >> 32);
-      const uint32_t up = 31u - (static_cast<uint32_t>(lane) & 31u);  // lanes above this one in its half
-      const uint32_t rank = static_cast<uint32_t>(__builtin_clz(half << up));  // lanes from the run's first to this one
-      // the next run begins `run` lanes above this one (a run ends with its half at the latest)
-      const uint32_t above = ((half >> 1) >> (31u - up)) | (0x80000000u >> (31u - up));
-      uint32_t run = static_cast<uint32_t>(__builtin_ctz(above)) + 1u;
-      if (run > n_valid - static_cast<uint32_t>(lane)) run = n_valid - static_cast<uint32_t>(lane);
+      const uint32_t in_half = static_cast<uint32_t>(lane) & 31u;
+      const uint32_t rank = static_cast<uint32_t>(__builtin_clz(half << (31u - in_half)));  // lanes from the run's first to this one
       uint32_t first_slot = 0;
-      if (valid && rank == 0u) first_slot = atomicAdd(&s_cnt[b], run);
-      const uint32_t slot = static_cast<uint32_t>(__shfl(static_cast<int>(first_slot), lane - static_cast<int>(rank))) + rank;
+      if (__builtin_amdgcn_inverse_ballot_w64(heads & valids)) {
+        // the next run begins `run` lanes above this one (a run ends with its half at the latest)
+        const uint32_t above = (half >> in_half) & ~1u;
+        const uint32_t run = above != 0u ? static_cast<uint32_t>(__builtin_ctz(above)) : 32u - in_half;
+        first_slot = atomicAdd(&s_cnt[b], run);
+      }
+      const uint32_t slot = static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(static_cast<int>(4u * (static_cast<uint32_t>(lane) - rank)),
+                                                                              static_cast<int>(first_slot))) + rank;
       if (valid) {
         T1 add;
         if (IN == kInDense) add = (W == kHomo) ? val : static_cast<T1>(w * val);
         else add = w;  // homo: w == 1
         if (slot < cap) {
-          const uint64_t at = region + static_cast<uint64_t>(b) * cap + slot;
+          // (within the workgroup's region, whose bytes are counted in 32 bits; a window's number has seven, `cap` at most 24)
+          const uint32_t at = static_cast<uint32_t>(__umul24(b, cap)) + slot;
           const uint32_t rel = idx & ((1u << shift) - 1u);
           if (packed) {
-            packed_val[at] = add;
-            packed_rel[at] = static_cast<uint16_t>(rel);
+            *reinterpret_cast<T1 *>(region_val + at * static_cast<uint32_t>(sizeof(T1))) = add;
+            *reinterpret_cast<uint16_t *>(region_rel + at * 2u) = static_cast<uint16_t>(rel);
           } else {
             BinPair<T1> e;
             e.rel = rel;
             e.val = add;
-            static_cast<BinPair<T1> *>(pairs)[at] = e;
+            *reinterpret_cast<BinPair<T1> *>(region_val + at * static_cast<uint32_t>(sizeof(BinPair<T1>))) = e;
           }
         } else {
           atomic_add(&out[idx], add);
@@ -522,11 +525,15 @@ __global__ __launch_bounds__(kColBinThreads, sizeof(T1) == 4 ? 8 : 4) void jitco
         col = list_col != nullptr ? list_col[k] : first + k;
       }
       const uint32_t left = mine - j * kFuseBatch;
-      mt_seed_batch(st, lane, seed + col, ring + static_cast<size_t>(slot) * kFuseBatch * kMtN,
-                    left < kFuseBatch ? left : kFuseBatch);
+      uint32_t *const to = ring + static_cast<size_t>(slot) * kFuseBatch * kMtN;
+      if (left >= kFuseBatch) mt_seed_batch<kSeedGuarded>(st, lane, seed + col, to, left);
+      else mt_seed_batch<kSeedSoon>(st, lane, seed + col, to, left);
       __hip_atomic_store(&s_ready[slot], j + 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
     };
     if (wave == 0 && batches != 0) seed_batch(0);
+    // (One batch: the others wait at the barrier, where they take no issue slots from the wave that seeds.  More: the wave that
+    // takes the first entry seeds batch 1 beside it; 1,000,000 streams of 18 synapses, both walks, 1,908 us, behind the barrier 1,950.)
+    if (batches <= 1u) __syncthreads();
     for (;;) {
       // (every lane adds one: the counter advances by 64 per task, any lane's old value / 64 is the task)
       const uint32_t t = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(
@@ -549,9 +556,9 @@ __global__ __launch_bounds__(kColBinThreads, sizeof(T1) == 4 ? 8 : 4) void jitco
       for (uint32_t spin = 0; spin < kFuseSpin; ++spin) {
         flag = __hip_atomic_load(&s_ready[slot], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
         if ((flag & ~kFuseNotSeeded) >= j + 1u) break;
-        flag = kFuseNotSeeded;
-        __builtin_amdgcn_s_sleep(2);
+        __builtin_amdgcn_s_sleep(8);
       }
+      if ((flag & ~kFuseNotSeeded) < j + 1u) flag = kFuseNotSeeded;
       const uint32_t *pre = (flag & kFuseNotSeeded) ? nullptr : ring + (static_cast<size_t>(slot) * kFuseBatch + r) * kMtN;
       auto loaded = [&]() {
         if (lane == 0) __hip_atomic_fetch_add(&s_loaded[slot], 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -583,8 +590,8 @@ __global__ __launch_bounds__(kSeedThreads) void mt_seed_streams_kernel(uint32_t 
   const uint32_t mine = base + static_cast<uint32_t>(lane);  // lane l seeds stream base + l
   uint32_t x = seed + first + mine;
   if (ids != nullptr) x = seed + (mine < count ? ids[mine] : 0u);
-  mt_seed_batch(s_tile[wave], lane, x, states + static_cast<size_t>(base) * kMtN,
-                count - base < static_cast<uint32_t>(kWave) ? count - base : static_cast<uint32_t>(kWave));
+  mt_seed_batch<kSeedGuarded>(s_tile[wave], lane, x, states + static_cast<size_t>(base) * kMtN,
+                              count - base < static_cast<uint32_t>(kWave) ? count - base : static_cast<uint32_t>(kWave));
 }
 
 }  // namespace
@@ -851,6 +858,10 @@ void launch_colwalk(hipStream_t stream, const VT *in, T1 *out, uint32_t n_out, u
     const size_t val_bytes = (IN == kInEvent) ? round_up(static_cast<size_t>(n_in) * sizeof(T1)) : 0;
     uint32_t *list_count = (IN == kInEvent) ? stream_counters(stream) : nullptr;
     if (cap_d < 4.0e9 && pair_bytes <= (static_cast<size_t>(32) << 30) && (IN == kInDense || list_count != nullptr)) {
+      // (a producer's region is addressed with 32 bits of bytes, a bin's places with 24: more than scratch memory holds, but
+      // for a handful of producers)
+      const double addressable = 4294967040.0 / (static_cast<double>(n_win) * sizeof(BinPair<T1>));
+      cap_d = std::fmin(cap_d, std::floor(std::fmin(addressable, 16777212.0) / 4.0) * 4.0);
       const uint32_t cap = static_cast<uint32_t>(cap_d);
       unsigned char *ws = static_cast<unsigned char *>(
         stream_workspace(stream, pair_bytes + count_bytes + state_bytes + list_bytes + val_bytes));

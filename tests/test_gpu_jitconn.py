@@ -510,6 +510,27 @@ def test_column_walk_through_bins_events_and_overflow(cuda, oracle_mod):
     assert np.array_equal(got, want)
 
 
+@pytest.mark.parametrize("w_kind,a,b", [("homo", 0.0, 0.0), ("uniform", 0.25, 1.75), ("normal", 0.1, 1.0)])
+@pytest.mark.parametrize("active", [1, 16, 512 * 16, 512 * 17 + 1, 512 * 63, 512 * 64, 512 * 64 + 1])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_column_walk_last_batch_of_streams(cuda, oracle_mod, w_kind, a, b, active, dtype):
+  # a workgroup seeds 64 streams at a time, and a batch of fewer stores no state beyond its own: 1, 16, 17 and 63 to a
+  # workgroup, one whole batch, one more.  Rows of about 400 over ten windows, each ending within a batch of synapses.
+  n_out, n_in = 40_000, 40_000
+  lp = oracle_mod.log_p_of(0.01)
+  rng = np.random.default_rng(active)
+  ev = np.zeros(n_in, dtype=bool)
+  ev[rng.permutation(n_in)[:active]] = True
+  kw = dict(w_kind=w_kind, w_a=a, w_b=b, log_p=lp, seed=41, n_row=n_out, n_col=n_in, col_walk=True, dense=False)
+  for x in ([ev] if dtype == np.float32 else [ev.astype(np.float64)]):
+    got = kernel_call(x, **kw)
+    want, mag = oracle_mod.jitconn_matvec(x, return_abs=True, **kw)
+    if w_kind == "homo":
+      assert np.array_equal(got, want)
+    else:
+      assert_close_reordered(got, want, mag, dtype, what="column walk, last batch %s" % w_kind)
+
+
 @pytest.mark.parametrize("seed", [1, 2, 3])
 def test_random_shapes_walks_weights_and_inputs_against_oracle(cuda, oracle_mod, seed):
   # shapes up to two million inputs / outputs, both walks, all weight kinds, bool / float events and
