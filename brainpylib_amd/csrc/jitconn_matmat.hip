@@ -24,16 +24,35 @@ namespace {
 
 constexpr int kTile = 32;
 
+constexpr int kPrepareThreads = kTile * 8;
+
 // XT[r / pass_rows][c][r % pass_rows] = X[r][c] for r < m: the transposed operand in slices of pass_rows rows of
 // X (a multiple of 32), every slice contiguous, its rows pass_rows entries long; rows m .. m_pad - 1 are zero.
 // (In one array of rows of m_pad entries the pieces that a pass reads lie m_pad entries apart and share a
 // fraction of the L2's sets.)
+// The first seed_groups workgroups do not transpose: one wave of each seeds the generators of 64 of the `count` columns,
+// which it does in 8.6 us, beside the transposition (128 x 10,000: the launch takes 12.5 us, without the seeding 6.1).
 template <typename T>
-__global__ __launch_bounds__(kTile * 8) void transpose_pad_kernel(const T *__restrict__ X, T *__restrict__ XT,
-                                                                  uint32_t m, uint32_t k, uint32_t m_pad,
-                                                                  uint32_t pass_rows) {
-  __shared__ T tile[kTile][kTile + 1];
-  const uint32_t c0 = blockIdx.x * kTile, r0 = blockIdx.y * kTile;
+__global__ __launch_bounds__(kPrepareThreads) void matmat_prepare_kernel(const T *__restrict__ X, T *__restrict__ XT,
+                                                                         uint32_t m, uint32_t k, uint32_t m_pad,
+                                                                         uint32_t pass_rows, uint32_t col_tiles,
+                                                                         uint32_t seed, uint32_t count,
+                                                                         uint32_t seed_groups,
+                                                                         uint32_t *__restrict__ states) {
+  constexpr size_t kTileBytes = sizeof(T) * kTile * (kTile + 1), kSeedBytes = sizeof(uint32_t) * kMtSeedTileWords;
+  __shared__ __attribute__((aligned(16))) unsigned char s_mem[kTileBytes > kSeedBytes ? kTileBytes : kSeedBytes];
+  if (blockIdx.x < seed_groups) {
+    const uint32_t base = blockIdx.x * kWave;
+    const int lane = lane_id();
+    if (threadIdx.x < kWave)
+      mt_seed_batch<kSeedSoon>(reinterpret_cast<uint32_t *>(s_mem), lane, seed + base + static_cast<uint32_t>(lane),
+                               states + static_cast<size_t>(base) * kMtN,
+                               count - base < static_cast<uint32_t>(kWave) ? count - base : static_cast<uint32_t>(kWave));
+    return;
+  }
+  T(*tile)[kTile + 1] = reinterpret_cast<T(*)[kTile + 1]>(s_mem);
+  const uint32_t at = blockIdx.x - seed_groups;
+  const uint32_t c0 = at % col_tiles * kTile, r0 = at / col_tiles * kTile;
   const uint32_t tx = threadIdx.x % kTile, ty = threadIdx.x / kTile;  // 32 x 8
   for (uint32_t i = ty; i < kTile; i += 8) {
     const uint32_t r = r0 + i, c = c0 + tx;
@@ -86,7 +105,7 @@ __global__ __launch_bounds__(256) void jitconn_matmat_kernel(const T1 *__restric
   const char *xt_base = reinterpret_cast<const char *>(XT + static_cast<size_t>(pass) * k * (MT * kWave));
   const uint32_t lane_bytes = static_cast<uint32_t>(lane) * static_cast<uint32_t>(sizeof(T1));
 
-  // columns first .. first + count - 1 of M, their generators seeded ahead: states[c] for column first + c
+  // columns first .. first + count - 1 of M; states[c]: the generator of column first + c, if they are seeded ahead
   for (uint32_t c = blockIdx.x * kWaves + wave; c < count; c += gridDim.x * kWaves) {
     const uint32_t j = first + c;
     T1 acc[MT];
@@ -140,7 +159,7 @@ __global__ __launch_bounds__(256) void jitconn_matmat_kernel(const T1 *__restric
         take(static_cast<uint32_t>(__popcll(__ballot(valid0)) + __popcll(__ballot(valid1))));
       });
     } else {
-      walk_stream<T1, W>(st, lane, seed + j, pre, k, skips, wa, wb, [&](uint32_t idx, T1 w, bool valid, bool) {
+      walk_stream<T1, W, true>(st, lane, seed + j, pre, k, skips, wa, wb, [&](uint32_t idx, T1 w, bool valid, bool) {
         __builtin_amdgcn_wave_barrier();
         if (valid) put(static_cast<uint32_t>(lane), idx, w);
         __builtin_amdgcn_wave_barrier();
@@ -189,22 +208,35 @@ void matmat_entry(const char *target, hipStream_t stream, void **buffers, const 
   }
   // scratch memory: [XT][the generator states of a chunk of columns, seeded ahead on the vector unit]
   const size_t xt_bytes = (static_cast<size_t>(k) * m_pad * sizeof(T1) + 255) / 256 * 256;
-  // (from 32,768 columns on: with fewer a wave walks one or two columns and seeds them itself while others
-  // compute: 10,000 columns 234 us, seeded ahead 259; 1,000,000 columns of 20 synapses 5.6 ms, seeded ahead 3.3)
-  const bool ahead = n >= 32768;
+  // Seeded ahead where a CU has more columns than one workgroup's: its one scalar unit seeds a generator in 1.3 us (and
+  // no wave in less than 5), all columns together on the vector units take 8.6 us.  Float32, in place / ahead:
+  // 1,000 inputs 1,024 columns 16.3 / 18.4 us, 1,500 21.1 / 19.3, 3,000 26.5 / 20.8; 20,000 inputs of 4 rows, 20,000 columns
+  // of 100 synapses 132.7 / 49.4; 10,000 columns of 1,000 synapses 209 / 204, with normal weights 241 / 233.
   const uint32_t chunk = n < kSeedChunk ? n : kSeedChunk;
-  const size_t state_bytes = ahead ? static_cast<size_t>(chunk) * kMtN * sizeof(uint32_t) : 0;
-  unsigned char *ws = static_cast<unsigned char *>(stream_workspace(stream, xt_bytes + state_bytes));
+  const size_t state_bytes = static_cast<size_t>(chunk) * kMtN * sizeof(uint32_t);
+  bool ahead = n > 4u * static_cast<uint32_t>(device_info().num_cu);
+  // From 32,768 columns on (in place a million columns of 20 synapses take 5.6 ms, ahead 3.3) the states are required;
+  // with fewer a call that finds no room for them, a captured one above all, goes on without.
+  const bool optional = ahead && n < 32768;
+  unsigned char *ws =
+      static_cast<unsigned char *>(stream_workspace(stream, xt_bytes + (ahead ? state_bytes : 0), optional));
+  if (ws == nullptr && optional) {
+    bpl_clear_error();
+    ahead = false;
+    ws = static_cast<unsigned char *>(stream_workspace(stream, xt_bytes));
+  }
   if (ws == nullptr) return;
   T1 *XT = reinterpret_cast<T1 *>(ws);
   uint32_t *states = reinterpret_cast<uint32_t *>(ws + xt_bytes);
-  hipLaunchKernelGGL(transpose_pad_kernel<T1>, dim3(div_up(k, kTile), div_up(m_pad, kTile)), dim3(kTile * 8), 0,
-                     stream, X, XT, m, k, m_pad, pass_rows);
+  const uint32_t col_tiles = div_up(k, kTile), seed_groups = ahead ? div_up(chunk, kWave) : 0;
+  hipLaunchKernelGGL(matmat_prepare_kernel<T1>, dim3(seed_groups + col_tiles * div_up(m_pad, kTile)),
+                     dim3(kPrepareThreads), 0, stream, X, XT, m, k, m_pad, pass_rows, col_tiles, d.seed, chunk,
+                     seed_groups, states);
   const T1 wa = static_cast<T1>(d.w_a), wb = static_cast<T1>(d.w_b);
   const uint32_t tiles = pass_rows / kWave, passes = m_pad / pass_rows;
   for (uint32_t first = 0; first < n; first += chunk) {
     const uint32_t count = n - first < chunk ? n - first : chunk;
-    if (ahead) jitconn_seed_streams(stream, d.seed, first, count, states);
+    if (ahead && first != 0) jitconn_seed_streams(stream, d.seed, first, count, states);
     const unsigned grid_x = div_up(count, 4);
     const uint32_t *pre = ahead ? states : nullptr;
     for (uint32_t pass = 0; pass < passes; ++pass) {

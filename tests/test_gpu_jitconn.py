@@ -368,6 +368,18 @@ def test_matmat_with_generators_seeded_ahead(cuda, oracle_mod, n):
     assert got.shape == (m, n) and np.array_equal(got, want)
 
 
+@pytest.mark.parametrize("m,k,columns", [(3, 31, 0), (64, 33, 1), (65, 500, 63), (130, 64, 64), (9, 900, 65)])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_matmat_from_one_workgroup_for_every_cu_on(cuda, oracle_mod, m, k, columns, dtype):
+  # with more than four columns for every CU their generators are seeded beside the transposition of X, 64 to a wave
+  # (up to there by the waves that walk them); tiles of 32 inputs and 64 rows of X, the last ones partly filled
+  n = 4 * torch.cuda.get_device_properties(0).multi_processor_count + columns
+  X = np.random.default_rng(k).standard_normal((m, k)).astype(dtype)
+  want = oracle_mod.jitconn_matmat(X, w_kind="uniform", w_a=-0.5, w_b=1.5, log_p=oracle_mod.log_p_of(0.2), seed=3, n=n)
+  got = bpl.matmat_prob_conn_uniform_weight(X, w_low=-0.5, w_high=1.5, conn_prob=0.2, shape=(k, n), seed=3).cpu().numpy()
+  assert got.shape == (m, n) and np.array_equal(got, want)  # the same operations in the same order
+
+
 def test_config_jitconn_matmat_full_size(cuda, oracle_mod):
   # 10,000 x 10,000 implicit matrix, conn_prob 0.1, N(0, 0.01^2) from seed 7, times B[10000, 128]:
   # out = (B^T @ M)^T in the reference's orientation (X = B^T, m = 128).

@@ -190,6 +190,34 @@ def test_normal_row_walk_is_captured_on_a_cold_stream(cuda, n_in, capfd):
     torch.testing.assert_close(out, want, rtol=3e-7, atol=1e-6)
 
 
+def test_matmat_is_captured_where_there_is_no_room_for_generator_states(cuda, capfd):
+  # the stream's scratch memory holds the transposed operand (64 rows of 4,000 inputs) and not the states of 3,000
+  # columns: the waves of a captured call seed their own generators, with the same result
+  hip = ctypes.CDLL("libamdhip64.so")
+  handle = ctypes.c_void_p()
+  assert hip.hipStreamCreate(ctypes.byref(handle)) == 0
+  s, g = torch.cuda.ExternalStream(handle.value), torch.cuda.CUDAGraph()
+  X = torch.from_numpy(np.random.default_rng(5).standard_normal((64, 4000)).astype(np.float32)).to(cuda)
+  call = lambda n: bpl.matmat_prob_conn_uniform_weight(X, w_low=-0.5, w_high=1.5, conn_prob=0.01, shape=(4000, n), seed=5)
+  want = call(3000)
+  torch.cuda.synchronize()
+  with torch.cuda.stream(s):
+    call(100)
+  s.synchronize()
+  before = _query(s.cuda_stream)
+  assert before[0] and before[2] < 3000 * 624 * 4
+  capfd.readouterr()
+  with torch.cuda.graph(g, stream=s):
+    out = call(3000)
+  assert "brainpylib_amd" not in capfd.readouterr().err
+  assert _query(s.cuda_stream) == before, "nothing was allocated"
+  for _ in range(3):
+    out.zero_()
+    g.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(out, want)
+
+
 def test_row_walk_is_captured_where_the_stream_has_rings_but_no_counters(cuda, capfd):
   # more than four batches of streams for each of 512 workgroups, and no counter to take them from: they are shared out evenly, and the
   # call, which succeeds, prints nothing
