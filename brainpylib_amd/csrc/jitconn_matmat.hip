@@ -30,6 +30,7 @@ constexpr int kPrepareThreads = kTile * 8;
 // X (a multiple of 32), every slice contiguous, its rows pass_rows entries long; rows m .. m_pad - 1 are zero.
 // (In one array of rows of m_pad entries the pieces that a pass reads lie m_pad entries apart and share a
 // fraction of the L2's sets.)
+// Float64: 64 rows at a time, the low words of the 64 and then the high words, for the walk reads XT word by word.
 // The first seed_groups workgroups do not transpose: one wave of each seeds the generators of 64 of the `count` columns,
 // which it does in 8.6 us, beside the transposition (128 x 10,000: the launch takes 12.5 us, without the seeding 6.1).
 template <typename T>
@@ -61,8 +62,15 @@ __global__ __launch_bounds__(kPrepareThreads) void matmat_prepare_kernel(const T
   __syncthreads();
   for (uint32_t i = ty; i < kTile; i += 8) {
     const uint32_t c = c0 + i, r = r0 + tx;
-    if (c < k && r < m_pad)
-      XT[(static_cast<size_t>(r / pass_rows) * k + c) * pass_rows + r % pass_rows] = tile[tx][i];
+    if (c < k && r < m_pad) {
+      constexpr uint32_t kWords = sizeof(T) / 4;
+      uint32_t *to = reinterpret_cast<uint32_t *>(XT + (static_cast<size_t>(r / pass_rows) * k + c) * pass_rows) +
+                     r % pass_rows / kWave * (kWave * kWords) + r % kWave;
+      uint32_t w[kWords];
+      __builtin_memcpy(w, &tile[tx][i], sizeof(T));
+#pragma unroll
+      for (uint32_t part = 0; part < kWords; ++part) to[part * kWave] = w[part];
+    }
   }
 }
 
@@ -89,22 +97,35 @@ __global__ __launch_bounds__(256) void jitconn_matmat_kernel(const T1 *__restric
                                                              uint32_t first, uint32_t count,
                                                              const uint32_t *__restrict__ states, uint32_t pass) {
   constexpr int kWaves = 4;
-  constexpr int kWords = StreamLds<T1, W>::words;
-  __shared__ __attribute__((aligned(8))) uint32_t s_state[kWaves * kWords];
+  constexpr int kStreamWords = StreamLds<T1, W>::words;
+  __shared__ __attribute__((aligned(8))) uint32_t s_state[kWaves * kStreamWords];
   constexpr int kSlots = W == kNormal ? 2 * kWave : kWave;  // normal weights come two to a lane
   __shared__ __attribute__((aligned(16))) Synapse<T1> s_syn[kWaves * kSlots];
   const int lane = lane_id();
   const uint32_t wave = threadIdx.x / kWave;
-  uint32_t *st = s_state + wave * kWords;
+  uint32_t *st = s_state + wave * kStreamWords;
   Synapse<T1> *syn = s_syn + wave * kSlots;
   const uint32_t row_base = pass * (MT * kWave);  // first row of Y of this pass
-  // byte offsets into the pass's slice of XT fit 32 bits (checked by the host): one add per synapse instead of a
-  // 64-bit product
+  // The walk is bound by these reads, 512 bytes per synapse and pass of 128 float32 rows, at 27 of the 33 TB/s that 64 bytes
+  // per clock and CU come to, with the vector issue (two thirds of its rate) beside them.  A load takes the wave-uniform byte offset
+  // of a row of the slice (32 bits, checked by the host), an immediate one, and four times the lane, which the buffer's
+  // descriptor adds (stride 4, thread number enabled): no address arithmetic per synapse, one instruction of 8.6 less: 10,000 x
+  // 10,000 of 1,000 synapses x 128 203 -> 200 us, 1,000 x 200,000 of 20 396 -> 390.  Loads of 4 bytes a lane reach that
+  // rate; of 8 bytes 17.6 TB/s, as they did the float64 rows before these were stored as two words apart (5,000 x 10,000 of
+  // 250 x 100: 166 -> 124 us; with 16 bytes a lane 124 too, but there 64 rows are half a wave) and float32 rows of 128 as pairs (300 us).
+  constexpr uint32_t kWords = sizeof(T1) / 4;
   constexpr uint32_t row_bytes = MT * kWave * static_cast<uint32_t>(sizeof(T1));
-  // (a wave-uniform base and a 32-bit offset per lane: one address add per synapse and the base in scalar registers)
-  const char *xt_base = reinterpret_cast<const char *>(XT + static_cast<size_t>(pass) * k * (MT * kWave));
-  const uint32_t lane_bytes = static_cast<uint32_t>(lane) * static_cast<uint32_t>(sizeof(T1));
-
+  const __amdgpu_buffer_rsrc_t slice = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<T1 *>(XT + static_cast<size_t>(pass) * k * (MT * kWave)), 4, static_cast<int>(k * row_bytes), 0x00807000);
+  auto load = [&](uint32_t off, uint32_t t) {  // tile t of the row at byte `off`: the lane's entry
+    uint32_t w[kWords];
+#pragma unroll
+    for (uint32_t i = 0; i < kWords; ++i)
+      w[i] = __builtin_amdgcn_raw_buffer_load_b32(slice, static_cast<int>(off + (t * kWords + i) * kWave * 4), 0, 0);
+    T1 x;
+    __builtin_memcpy(&x, w, sizeof(T1));
+    return x;
+  };
   // columns first .. first + count - 1 of M; states[c]: the generator of column first + c, if they are seeded ahead
   for (uint32_t c = blockIdx.x * kWaves + wave; c < count; c += gridDim.x * kWaves) {
     const uint32_t j = first + c;
@@ -115,7 +136,7 @@ __global__ __launch_bounds__(256) void jitconn_matmat_kernel(const T1 *__restric
     // Every valid lane leaves its synapses (the byte offset of their rows of XT, their weights) in the
     // wave's LDS slots, in lane order (which is stream order); every lane then reads the slots
     // one after the other (one address per read: a broadcast), so a synapse costs one LDS read,
-    // one address add, MT loads and MT multiply-adds, with U synapses' loads in flight.
+    // its loads and MT multiply-adds, with U synapses' loads in flight.
     auto take = [&](uint32_t count) {
       constexpr int U = 8;
       uint32_t i = 0;
@@ -126,9 +147,8 @@ __global__ __launch_bounds__(256) void jitconn_matmat_kernel(const T1 *__restric
         for (int u = 0; u < U; ++u) {
           const Synapse<T1> e = syn[i + u];
           ws[u] = e.w;
-          const T1 *row = reinterpret_cast<const T1 *>(xt_base + (e.off + lane_bytes));
 #pragma unroll
-          for (int t = 0; t < MT; ++t) x[u][t] = row[t * kWave];
+          for (int t = 0; t < MT; ++t) x[u][t] = load(e.off, t);
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -138,9 +158,8 @@ __global__ __launch_bounds__(256) void jitconn_matmat_kernel(const T1 *__restric
       }
       for (; i < count; ++i) {
         const Synapse<T1> e = syn[i];
-        const T1 *row = reinterpret_cast<const T1 *>(xt_base + (e.off + lane_bytes));
 #pragma unroll
-        for (int t = 0; t < MT; ++t) acc[t] = add_rn(acc[t], mul_rn(e.w, row[t * kWave]));
+        for (int t = 0; t < MT; ++t) acc[t] = add_rn(acc[t], mul_rn(e.w, load(e.off, t)));
       }
     };
     auto put = [&](uint32_t slot, uint32_t idx, T1 w) {
