@@ -23,6 +23,7 @@
 
 #include "bins.h"
 #include "common.h"
+#include "jitconn_lane.h"
 #include "jitconn_stream.h"
 #include "targets.h"
 
@@ -280,6 +281,50 @@ __global__ __launch_bounds__(1024, (FORM == 2 || (W == kNormal && sizeof(T1) == 
       __syncthreads();
       if (threadIdx.x == 0 && atomicAdd(&next[1], 1u) == gridDim.x - 1u) next[0] = 0u, next[1] = 0u;
     }
+  }
+}
+
+// ---- row walk of short streams ------------------------------------------------------------------------
+// A lane per output (jitconn_lane.h): workgroups of one wave, 64 outputs each, the events probed where they lie.  The rare
+// stream that is longer than its lane can draw is walked again by the whole wave, which seeds it itself.
+template <typename T1, typename VT, int IN, int W>
+__global__ __launch_bounds__(kWave, 8) void jitconn_rows_by_lane_kernel(const VT *__restrict__ in, T1 *__restrict__ out,
+                                                                        uint32_t n_out, uint32_t n_in, uint32_t seed,
+                                                                        SkipParams skips, T1 wa, T1 wb, uint32_t words) {
+  __shared__ __attribute__((aligned(8))) uint32_t st[StreamLds<T1, W, true>::words];
+  const int lane = lane_id();
+  const uint32_t o = blockIdx.x * kWave + static_cast<uint32_t>(lane);
+  double acc = 0.0;
+  uint32_t cnt = 0;
+  // what a synapse meets is looked at when the next one is drawn
+  VT late = VT();
+  T1 late_w = T1(0);
+  bool late_valid = false;
+  auto use = [&](bool valid, VT v, T1 w) {
+    if constexpr (IN == kInEvent) {
+      const bool on = is_event(v) && valid;
+      if (W == kHomo) cnt += on ? 1u : 0u;
+      else acc += on ? static_cast<double>(w) : 0.0;
+    } else {
+      const T1 x = static_cast<T1>(v);
+      if (valid) acc += static_cast<double>(W == kHomo ? x : static_cast<T1>(w * x));
+    }
+  };
+  auto result = [&]() { return (IN == kInEvent && W == kHomo) ? static_cast<T1>(cnt) : static_cast<T1>(acc); };
+  uint64_t longer = walk_lane_streams<T1, W>(seed + o, o < n_out, n_in, skips, wa, wb, words, [&](uint32_t idx, T1 w, bool valid) {
+    use(late_valid, late, late_w);
+    late = in[idx], late_w = w, late_valid = valid;
+  });
+  use(late_valid, late, late_w);
+  if (o < n_out && !__builtin_amdgcn_inverse_ballot_w64(longer)) out[o] = result();
+  for (; longer != 0; longer &= longer - 1ull) {
+    const uint32_t row = blockIdx.x * kWave + static_cast<uint32_t>(__builtin_ctzll(longer));
+    acc = 0.0, cnt = 0;
+    walk_stream<T1, W, true, true>(st, lane, seed + row, nullptr, n_in, skips, wa, wb,
+                                   [&](uint32_t idx, T1 w, bool valid, bool) { use(valid, in[idx], w); });
+    if (IN == kInEvent && W == kHomo) cnt = wave_inclusive_scan_u32(cnt);
+    else acc = wave_sum(acc);
+    if (lane == ((IN == kInEvent && W == kHomo) ? kWave - 1 : 0)) out[row] = result();
   }
 }
 
@@ -753,10 +798,35 @@ uint32_t rowwalk_exact_bytes(uint32_t n_out) {
   return fused ? rowwalk_coarse_bytes<T1, W>() : rowwalk_bytes_for_two<T1, W, true>();
 }
 
+// Whether a lane walks a stream (jitconn_lane.h) rather than a wave: where its time, in us, is the smaller one by this fit of
+// both, and no more than one stream in 10^5 is expected to need more words than a lane can draw (4.5 standard deviations
+// of the synapses of a row).  A synapse takes a wave 0.27 us or, with weights, up to 2.1 while it waits for its own
+// instructions, longer from one wave to a SIMD on; a wave to a stream is bound by the seeding: on the CU's scalar unit (1.3 us
+// a stream) or, from kSeedAheadMin on, by the states' way through memory.  Either side at the line: 2,000 rows of 30 17.7 / 17.5
+// us, of 44 17.9 / 21; 40,000 of 70 44 / 30; 70,000 of 100 67 / 53, of 130 67 / 68; uniform weights 2,000 of 20 15.9 / 15.3, of 30
+// 15.9 / 19.3; normal ones 20,000 of 20 35 / 32, of 30 35 / 39; in double 1,000 of 3 19.6 / 18.5, 20,000 of 10 48 / 33, of 20 49 / 51.
+template <typename T1, int W>
+bool streams_by_lane(uint32_t streams, uint32_t n, double log_p, const SkipParams &sp) {
+  const double mean = -std::expm1(log_p) * static_cast<double>(n);
+  constexpr double words = W == kHomo ? 2.0 : W == kUniform ? 2.0 + WeightWords<T1>::value : sizeof(T1) == 4 ? 3.27 : 4.55;
+  if (!sp.narrow || n > 0xf0000000u || words * (mean + 4.5 * std::sqrt(mean)) > kLaneWords - 2.0) return false;
+  constexpr double step = W == kHomo ? 0.27 : W == kUniform ? (sizeof(T1) == 4 ? 0.35 : 0.45) : sizeof(T1) == 4 ? 1.0 : 2.1;
+  const double steps = mean + 0.7 * std::fmax(0.0, mean - kLaneFirst / words);
+  const double by_lane = 8.0 + step * steps * std::fmax(1.0, 0.8 + streams / 120e3);
+  const double by_wave = streams < kSeedAheadMin ? 7.0 + streams / 195.0 : std::fmax(31.0, 6.0 + streams * 0.74e-3);
+  return by_lane < by_wave;
+}
+
 template <typename T1, typename VT, int IN, int W>
 void launch_rowwalk(hipStream_t stream, const VT *in, T1 *out, uint32_t n_out, uint32_t n_in, uint32_t seed,
                     double log_p, T1 wa, T1 wb) {
   if (n_out == 0) return;
+  const SkipParams sp = make_skip_params(log_p);
+  if (streams_by_lane<T1, W>(n_out, n_in, log_p, sp)) {
+    hipLaunchKernelGGL((jitconn_rows_by_lane_kernel<T1, VT, IN, W>), dim3(div_up(n_out, kWave)), dim3(kWave), 0, stream, in,
+                       out, n_out, n_in, seed, sp, wa, wb, kLaneWords);
+    return;
+  }
   constexpr bool kEvents = IN == kInEvent;
   const size_t words = (static_cast<size_t>(n_in) + 31) / 32;
   // A longer event bitmap (rowwalk_exact_bytes): two levels, the exact bitmap packed into global memory and a

@@ -368,6 +368,44 @@ def test_matmat_with_generators_seeded_ahead(cuda, oracle_mod, n):
     assert got.shape == (m, n) and np.array_equal(got, want)
 
 
+@pytest.mark.parametrize("w_kind,a,b", [("homo", 0.0, 0.0), ("uniform", 0.25, 1.75), ("normal", 0.5, 2.0)])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n_out,n_in,p", [(5001, 900, 0.001), (10_000, 4000, 0.0025), (70_063, 3, 1.0), (70_063, 40, 0.5), (140_000, 1500, 0.04)])
+def test_row_walk_of_short_streams(cuda, oracle_mod, w_kind, a, b, dtype, n_out, n_in, p):
+  # a lane to a stream: outputs that are not a multiple of 64, streams without a synapse, every index connected, streams that go on
+  # behind word 227 of the generator (1,500 x 0.04: 120 words with homogeneous weights, 273 with normal ones in double)
+  rng = np.random.default_rng(n_out)
+  ev, vec = rng.random(n_in) < 0.3, rng.uniform(0.5, 2.0, n_in).astype(dtype)
+  oracle_mod.set_threads(min(16, len(os.sched_getaffinity(0))))
+  kw = dict(w_kind=w_kind, w_a=a, w_b=b, log_p=oracle_mod.log_p_of(p), seed=21, n_row=n_out, n_col=n_in, out_dtype=dtype)
+  for inp, dense in ((ev, False), (vec, True)):
+    want, mag = oracle_mod.jitconn_matvec(inp, dense=dense, return_abs=True, **kw)
+    got = kernel_call(inp, col_walk=False, dense=dense, **kw)
+    if w_kind == "homo" and not dense: assert np.array_equal(got, want)
+    assert_close_reordered(got, want, mag, dtype, what="row walk of short streams")
+  oracle_mod.set_threads(1)
+
+
+@pytest.mark.parametrize("w_kind,mean,most", [("homo", 167.0, 226), ("uniform", 104.0, 150)])
+def test_row_walk_of_streams_that_outlast_their_lane(cuda, oracle_mod, w_kind, mean, most):
+  # among streams of so many synapses in the mean a few need more words than a lane can draw (454): those are walked
+  # again by their wave
+  n_out, n_in = 300_000, 600_000
+  ones = np.ones(n_in, bool)
+  oracle_mod.set_threads(min(16, len(os.sched_getaffinity(0))))
+  kw = dict(log_p=oracle_mod.log_p_of(mean / n_in), seed=400_012, n_row=n_out, n_col=n_in, w_kind=w_kind, w_a=1.0, w_b=1.0,
+            out_dtype=np.float32)
+  counts = oracle_mod.jitconn_matvec(ones, dense=False, **kw)  # (every weight is 1)
+  assert counts.max() > most, "no stream is long enough"
+  assert np.array_equal(kernel_call(ones, col_walk=False, dense=False, **kw), counts)
+  kw.update(w_b=2.0)
+  vec = np.random.default_rng(7).uniform(0.5, 2.0, n_in).astype(np.float32)
+  want, mag = oracle_mod.jitconn_matvec(vec, dense=True, return_abs=True, **kw)
+  oracle_mod.set_threads(1)
+  assert_close_reordered(kernel_call(vec, col_walk=False, dense=True, **kw), want, mag, np.float32,
+                         what="streams that outlast their lane")
+
+
 @pytest.mark.parametrize("m,k,columns", [(3, 31, 0), (64, 33, 1), (65, 500, 63), (130, 64, 64), (9, 900, 65)])
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 def test_matmat_from_one_workgroup_for_every_cu_on(cuda, oracle_mod, m, k, columns, dtype):
