@@ -58,13 +58,12 @@ struct LaneGenerator {
 
 // Walks stream std::mt19937{stream_seed} of each lane over [0, n): calls f(index, weight, valid) with the whole wave converged,
 // one synapse of every lane that has one (`valid`; the others get index 0) per call, in the order of each stream.  Returns the lanes
-// whose stream needs more than `words` words (at most kLaneWords); what they gave is a part of their streams.
+// whose stream needs more than `words` words (at most kLaneWords): they gave what lies in front of their position `pos`.
 // The skips fit: sp.narrow and n <= 0xf0000000, so that a position never leads around 2^32.
 template <typename T1, int W, typename F>
 __device__ __forceinline__ uint64_t walk_lane_streams(uint32_t stream_seed, bool alive, uint32_t n, const SkipParams &sp,
-                                                      T1 wa, T1 wb, uint32_t words, F &&f) {
+                                                      T1 wa, T1 wb, uint32_t words, uint32_t &pos, F &&f) {
   LaneGenerator gen(stream_seed);
-  uint32_t pos;
   {
     const uint32_t lo = gen.raw<false>(), hi = gen.word<false>();
     pos = skip_from_words<true, false>(lo, hi, sp, __builtin_amdgcn_ballot_w64(alive));

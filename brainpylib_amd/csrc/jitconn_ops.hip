@@ -311,7 +311,8 @@ __global__ __launch_bounds__(kWave, 8) void jitconn_rows_by_lane_kernel(const VT
     }
   };
   auto result = [&]() { return (IN == kInEvent && W == kHomo) ? static_cast<T1>(cnt) : static_cast<T1>(acc); };
-  uint64_t longer = walk_lane_streams<T1, W>(seed + o, o < n_out, n_in, skips, wa, wb, words, [&](uint32_t idx, T1 w, bool valid) {
+  uint32_t pos;
+  uint64_t longer = walk_lane_streams<T1, W>(seed + o, o < n_out, n_in, skips, wa, wb, words, pos, [&](uint32_t idx, T1 w, bool valid) {
     use(late_valid, late, late_w);
     late = in[idx], late_w = w, late_valid = valid;
   });
@@ -617,6 +618,89 @@ __global__ __launch_bounds__(kColBinThreads, sizeof(T1) == 4 ? 8 : 4) void jitco
   if (threadIdx.x < n_win) counts[static_cast<size_t>(threadIdx.x) * gridDim.x + p] = s_cnt[threadIdx.x];
 }
 
+// ---- column walk of short streams ---------------------------------------------------------------------
+// The same with a lane to a column (jitconn_lane.h): batches of 64 entries, one to a workgroup before any has a second.
+// The synapses that 64 columns have at one time lie anywhere, so every lane reserves a place for itself, or, where there is
+// one window, the wave for all.  The rare stream that is longer than its lane can draw is finished by the whole wave.
+template <typename T1, typename VT, int IN, int W>
+__global__ __launch_bounds__(kColBinThreads, sizeof(T1) == 4 ? 8 : 4) void jitconn_columns_by_lane_kernel(
+    const VT *__restrict__ in, T1 *__restrict__ out, uint32_t n_out, uint32_t seed, SkipParams skips, T1 wa, T1 wb,
+    uint32_t first, uint32_t n_list_host, const uint32_t *__restrict__ n_list_dev,
+    const uint32_t *__restrict__ list_col, const T1 *__restrict__ list_val, uint32_t n_win, uint32_t shift, uint32_t cap,
+    void *__restrict__ pairs, uint64_t n_pairs, uint32_t packed, uint32_t *__restrict__ counts, uint32_t words) {
+  constexpr uint32_t kWaves = kColBinThreads / kWave;
+  constexpr int kStateWords = StreamLds<T1, W, true>::words;
+  __shared__ __attribute__((aligned(8))) uint32_t s_state[kWaves * kStateWords];
+  __shared__ uint32_t s_cnt[kBinMaxWindows];
+  const int lane = lane_id();
+  const uint32_t wave = threadIdx.x / kWave, p = blockIdx.x;
+  if (threadIdx.x < n_win) s_cnt[threadIdx.x] = counts[static_cast<size_t>(threadIdx.x) * gridDim.x + p];
+  __syncthreads();
+  const uint64_t region = static_cast<uint64_t>(p) * n_win * cap;  // first place of this workgroup's bins
+  unsigned char *const region_val = static_cast<unsigned char *>(pairs) + region * (packed ? sizeof(T1) : sizeof(BinPair<T1>));
+  unsigned char *const region_rel = static_cast<unsigned char *>(pairs) + n_pairs * sizeof(T1) + region * 2u;  // (packed)
+  uint32_t *const st = s_state + wave * kStateWords;
+  const uint32_t n_list = n_list_dev ? *n_list_dev : n_list_host;
+  auto append = [&](uint32_t idx, T1 add, bool valid) {  // (the whole wave)
+    const uint32_t b = idx >> shift;
+    uint32_t slot = cap;
+    if (cap != 0) {
+      if (n_win == 1) {
+        const uint64_t valids = __builtin_amdgcn_ballot_w64(valid);
+        uint32_t base = 0;
+        if (lane == 0) base = atomicAdd(&s_cnt[0], static_cast<uint32_t>(__popcll(valids)));
+        slot = lanes_below(valids, static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(base))));
+      } else if (valid) {
+        slot = atomicAdd(&s_cnt[b], 1u);
+      }
+    }
+    if (!valid) return;
+    if (slot < cap) {
+      const uint32_t at = static_cast<uint32_t>(__umul24(b, cap)) + slot;
+      const uint32_t rel = idx & ((1u << shift) - 1u);
+      if (packed) {
+        *reinterpret_cast<T1 *>(region_val + at * static_cast<uint32_t>(sizeof(T1))) = add;
+        *reinterpret_cast<uint16_t *>(region_rel + at * 2u) = static_cast<uint16_t>(rel);
+      } else {
+        BinPair<T1> e;
+        e.rel = rel;
+        e.val = add;
+        *reinterpret_cast<BinPair<T1> *>(region_val + at * static_cast<uint32_t>(sizeof(BinPair<T1>))) = e;
+      }
+    } else {
+      atomic_add(&out[idx], add);
+    }
+  };
+  for (uint32_t batch = p + wave * gridDim.x; batch < (n_list + kWave - 1u) / kWave; batch += kWaves * gridDim.x) {
+    const uint32_t k = batch * kWave + static_cast<uint32_t>(lane);
+    bool on = k < n_list;
+    uint32_t col = 0;
+    T1 val = T1(0);
+    if (on) {
+      col = list_col != nullptr ? list_col[k] : first + k;
+      val = list_col != nullptr ? list_val[k] : static_cast<T1>(in[col]);
+      on = is_event(val);  // (a zero input adds nothing)
+    }
+    auto addend = [&](T1 w, T1 v) { return IN == kInDense ? (W == kHomo ? v : static_cast<T1>(w * v)) : w; };  // (homo: w == 1)
+    uint32_t pos;
+    uint64_t longer = walk_lane_streams<T1, W>(seed + col, on, n_out, skips, wa, wb, words, pos,
+                                               [&](uint32_t idx, T1 w, bool valid) { append(idx, addend(w, val), valid); });
+    for (; longer != 0; longer &= longer - 1ull) {
+      const int of = static_cast<int>(__builtin_ctzll(longer));
+      const uint32_t its_col = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(col), of));
+      const uint32_t from = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(pos), of));
+      const T1 its_val = list_col != nullptr ? list_val[batch * kWave + of] : static_cast<T1>(in[its_col]);
+      walk_stream<T1, W, true, true>(st, lane, seed + its_col, nullptr, n_out, skips, wa, wb, [&](uint32_t idx, T1 w, bool valid, bool) {
+        append(idx, addend(w, its_val), valid && idx >= from);
+      });
+    }
+  }
+  __syncthreads();
+  uint32_t win = threadIdx.x;
+  asm volatile("" : "+v"(win));  // (else the address from above is kept, in memory with normal weights)
+  if (win < n_win) counts[static_cast<size_t>(win) * gridDim.x + p] = s_cnt[win];
+}
+
 // ---- seeding ahead ------------------------------------------------------------------------------------
 constexpr int kSeedThreads = 128;
 
@@ -805,14 +889,23 @@ uint32_t rowwalk_exact_bytes(uint32_t n_out) {
 // a stream) or, from kSeedAheadMin on, by the states' way through memory.  Either side at the line: 2,000 rows of 30 17.7 / 17.5
 // us, of 44 17.9 / 21; 40,000 of 70 44 / 30; 70,000 of 100 67 / 53, of 130 67 / 68; uniform weights 2,000 of 20 15.9 / 15.3, of 30
 // 15.9 / 19.3; normal ones 20,000 of 20 35 / 32, of 30 35 / 39; in double 1,000 of 3 19.6 / 18.5, 20,000 of 10 48 / 33, of 20 49 / 51.
+//
+// Columns: a synapse's place in the bins and its store come on top.  All columns, 5,000 outputs: 30,000 columns of 20 73 / 34 us, of
+// 60 50 / 55; normal weights of 20 74 / 108, of 3 43 / 21; 130,000 of 60 173 / 69, normal ones 197 / 127.  Those of the events only:
+// their number is not known here, and a wave to each of a few takes 17 us (100 columns of 20 27 / 23 us, of 60 27 / 35; 13,000 of
+// 3 34 / 19, of 20 48 / 49; normal ones of 3 35 / 24, of 20 48 / 53).
+enum StreamUse { kGathers, kScatters, kScattersSome };
 template <typename T1, int W>
-bool streams_by_lane(uint32_t streams, uint32_t n, double log_p, const SkipParams &sp) {
+bool streams_by_lane(uint32_t streams, uint32_t n, double log_p, const SkipParams &sp, StreamUse use) {
   const double mean = -std::expm1(log_p) * static_cast<double>(n);
   constexpr double words = W == kHomo ? 2.0 : W == kUniform ? 2.0 + WeightWords<T1>::value : sizeof(T1) == 4 ? 3.27 : 4.55;
   if (!sp.narrow || n > 0xf0000000u || words * (mean + 4.5 * std::sqrt(mean)) > kLaneWords - 2.0) return false;
-  constexpr double step = W == kHomo ? 0.27 : W == kUniform ? (sizeof(T1) == 4 ? 0.35 : 0.45) : sizeof(T1) == 4 ? 1.0 : 2.1;
+  const double step = (W == kHomo ? 0.27 : W == kUniform ? (sizeof(T1) == 4 ? 0.35 : 0.45) : sizeof(T1) == 4 ? 1.0 : 2.1) +
+                      (use == kGathers ? 0.0 : 0.15);
   const double steps = mean + 0.7 * std::fmax(0.0, mean - kLaneFirst / words);
+  if (use == kScattersSome) return 8.0 + step * steps < 15.0;
   const double by_lane = 8.0 + step * steps * std::fmax(1.0, 0.8 + streams / 120e3);
+  if (use == kScatters) return by_lane < std::fmax(24.0, 6.0 + streams * 0.74e-3);
   const double by_wave = streams < kSeedAheadMin ? 7.0 + streams / 195.0 : std::fmax(31.0, 6.0 + streams * 0.74e-3);
   return by_lane < by_wave;
 }
@@ -822,7 +915,7 @@ void launch_rowwalk(hipStream_t stream, const VT *in, T1 *out, uint32_t n_out, u
                     double log_p, T1 wa, T1 wb) {
   if (n_out == 0) return;
   const SkipParams sp = make_skip_params(log_p);
-  if (streams_by_lane<T1, W>(n_out, n_in, log_p, sp)) {
+  if (streams_by_lane<T1, W>(n_out, n_in, log_p, sp, kGathers)) {
     hipLaunchKernelGGL((jitconn_rows_by_lane_kernel<T1, VT, IN, W>), dim3(div_up(n_out, kWave)), dim3(kWave), 0, stream, in,
                        out, n_out, n_in, seed, sp, wa, wb, kLaneWords);
     return;
@@ -885,7 +978,9 @@ void launch_colwalk(hipStream_t stream, const VT *in, T1 *out, uint32_t n_out, u
   const uint32_t n_win = div_up(n_out, 1u << shift);
   const double p_conn = -std::expm1(log_p);
   const double full = static_cast<double>(n_in) * static_cast<double>(n_out) * p_conn;
-  const bool bins = n_win <= kBinMaxWindows && full >= (IN == kInDense ? 1048576.0 : 1.0e7);
+  const SkipParams sp = make_skip_params(log_p);
+  const bool by_lane = (IN == kInDense || n_in >= 2048) && streams_by_lane<T1, W>(n_in, n_out, log_p, sp, IN == kInDense ? kScatters : kScattersSome);
+  const bool bins = n_win <= kBinMaxWindows && full >= (IN == kInEvent ? 1.0e7 : by_lane ? 131072.0 : 1048576.0);
   // Event input and fewer pairs: the same list of active columns and the same seeding on the vector unit, but
   // the walk adds its pairs to `out` with atomics.  (A wave that seeds its own stream spends 2 us of the CU's one
   // scalar unit on it: with 200,000 active columns of ten synapses each the walk without a list took 1.2 ms.)
@@ -898,7 +993,8 @@ void launch_colwalk(hipStream_t stream, const VT *in, T1 *out, uint32_t n_out, u
     const uint32_t n_win = bins ? div_up(n_out, 1u << bin_window_shift(n_out)) : 1u;  // (no bins: every pair overflows)
     const uint32_t shift = bins ? bin_window_shift(n_out) : 31u;
     uint32_t producers = 2u * static_cast<uint32_t>(device_info().num_cu);
-    if (producers > div_up(n_in, kColBinThreads / kWave)) producers = div_up(n_in, kColBinThreads / kWave);
+    const uint32_t least = by_lane ? kWave : kColBinThreads / kWave;  // columns that occupy a producer
+    if (producers > div_up(n_in, least)) producers = div_up(n_in, least);
     auto round_up = [](size_t v) { return (v + 255) / 256 * 256; };
     // Dense input: the bins are emptied (added to `out`) after every `group` chunks of kSeedChunk columns,
     // the largest number of chunks whose pairs fit kColBinBytesMax of scratch memory (every column of a
@@ -911,9 +1007,12 @@ void launch_colwalk(hipStream_t stream, const VT *in, T1 *out, uint32_t n_out, u
     size_t pair_bytes = 0;
     for (;;) {
       const double share = (group >= chunks) ? 1.0 : static_cast<double>(group) * kSeedChunk / static_cast<double>(n_in);
-      const double per_bin = full * share / (static_cast<double>(producers) * n_win);  // every column active
+      double per_bin = full * share / (static_cast<double>(producers) * n_win);  // every column active
+      // (by lane a producer has whole batches)
+      const double batch = full / n_in * kWave / n_win;
+      if (by_lane && IN == kInDense) per_bin = std::ceil(std::ceil(share * n_in / kWave) / producers) * batch;
       cap_d = 1.25 * per_bin + 6.0 * std::sqrt(per_bin) + 128.0;
-      if (IN == kInEvent) cap_d = cap_d / 8.0 < 512.0 ? 512.0 : cap_d / 8.0;
+      if (IN == kInEvent) cap_d = std::fmax(cap_d / 8.0, by_lane ? std::fmax(512.0, 2.0 * batch + 128.0) : 512.0);
       cap_d = std::floor(cap_d / 4.0) * 4.0;  // (packed bins begin at multiples of four places)
       pair_bytes = round_up(static_cast<size_t>(producers) * n_win * static_cast<size_t>(cap_d) * pair_size);
       if (IN == kInEvent || group == 1 || pair_bytes <= kColBinBytesMax) break;
@@ -923,7 +1022,7 @@ void launch_colwalk(hipStream_t stream, const VT *in, T1 *out, uint32_t n_out, u
     if (!bins) cap_d = 0.0, pair_bytes = 0, group = chunks;
     const size_t count_bytes = round_up(static_cast<size_t>(n_win) * producers * sizeof(uint32_t));
     // the workgroups' rings of generator states, seeded inside the walk
-    const size_t state_bytes = round_up(static_cast<size_t>(producers) * kFuseRingBytes);
+    const size_t state_bytes = by_lane ? 0 : round_up(static_cast<size_t>(producers) * kFuseRingBytes);
     const size_t list_bytes = (IN == kInEvent) ? round_up(static_cast<size_t>(n_in) * 4) : 0;
     const size_t val_bytes = (IN == kInEvent) ? round_up(static_cast<size_t>(n_in) * sizeof(T1)) : 0;
     uint32_t *list_count = (IN == kInEvent) ? stream_counters(stream) : nullptr;
@@ -943,28 +1042,44 @@ void launch_colwalk(hipStream_t stream, const VT *in, T1 *out, uint32_t n_out, u
         uint32_t *list_col = list_bytes ? reinterpret_cast<uint32_t *>(ws + pair_bytes + count_bytes + state_bytes) : nullptr;
         T1 *list_val = val_bytes ? reinterpret_cast<T1 *>(ws + pair_bytes + count_bytes + state_bytes + list_bytes) : nullptr;
         auto walk = jitconn_colwalk_bins_kernel<T1, VT, IN, W, true>;
+        auto walk_lanes = jitconn_columns_by_lane_kernel<T1, VT, IN, W>;
         out_cleared = true;
         if (IN == kInEvent) {
           // the active columns, then one walk that seeds their generators as it goes
           hipLaunchKernelGGL((collect_active_columns_kernel<T1, VT>), dim3(div_up(n_in, kCollectCols)), dim3(1024), 0, stream,
                              in, n_in, list_count, list_col, list_val, counts, n_win * producers, out, n_out);
-          hipLaunchKernelGGL(walk, dim3(producers), dim3(kColBinThreads), 0, stream, in, out, n_out, seed,
-                             make_skip_params(log_p), wa, wb,
-                             0u, 0u, static_cast<const uint32_t *>(list_count), static_cast<const uint32_t *>(list_col),
-                             static_cast<const T1 *>(list_val), states, 0u, n_win, shift, cap, pairs, n_pairs, packed ? 1u : 0u, counts);
+          if (by_lane) {
+            hipLaunchKernelGGL(walk_lanes, dim3(producers), dim3(kColBinThreads), 0, stream, in, out, n_out, seed, sp, wa,
+                               wb, 0u, 0u, static_cast<const uint32_t *>(list_count), static_cast<const uint32_t *>(list_col),
+                               static_cast<const T1 *>(list_val), n_win, shift, cap, pairs, n_pairs, packed ? 1u : 0u, counts,
+                               kLaneWords);
+          } else {
+            hipLaunchKernelGGL(walk, dim3(producers), dim3(kColBinThreads), 0, stream, in, out, n_out, seed, sp, wa, wb,
+                               0u, 0u, static_cast<const uint32_t *>(list_count), static_cast<const uint32_t *>(list_col),
+                               static_cast<const T1 *>(list_val), states, 0u, n_win, shift, cap, pairs, n_pairs, packed ? 1u : 0u, counts);
+          }
         } else {
-          // every column, a chunk at a time; the bins are emptied after every `group` chunks
+          // every column, a chunk at a time; the bins are emptied after every `group` chunks (by lane: after every launch)
           fill_zero(stream, out, n_out);
           fill_zero(stream, counts, n_win * producers);
           uint32_t in_bins = 0;
-          for (uint32_t first = 0; first < n_in; first += kSeedChunk) {
-            const uint32_t count = (n_in - first < kSeedChunk) ? n_in - first : kSeedChunk;
-            hipLaunchKernelGGL(walk, dim3(producers), dim3(kColBinThreads), 0, stream, in, out, n_out, seed,
-                               make_skip_params(log_p), wa,
-                               wb, first, count, static_cast<const uint32_t *>(nullptr),
-                               static_cast<const uint32_t *>(nullptr), static_cast<const T1 *>(nullptr), states, 0u,
-                               n_win, shift, cap, pairs, n_pairs, packed ? 1u : 0u, counts);
-            if (++in_bins == group && first + kSeedChunk < n_in) {
+          const uint64_t span = by_lane ? static_cast<uint64_t>(group) * kSeedChunk : kSeedChunk;
+          if (by_lane) group = 1;
+          for (uint64_t at = 0; at < n_in; at += span) {
+            const uint32_t first = static_cast<uint32_t>(at);
+            const uint32_t count = static_cast<uint32_t>(n_in - at < span ? n_in - at : span);
+            if (by_lane) {
+              hipLaunchKernelGGL(walk_lanes, dim3(producers), dim3(kColBinThreads), 0, stream, in, out, n_out, seed, sp, wa,
+                                 wb, first, count, static_cast<const uint32_t *>(nullptr),
+                                 static_cast<const uint32_t *>(nullptr), static_cast<const T1 *>(nullptr), n_win, shift, cap,
+                                 pairs, n_pairs, packed ? 1u : 0u, counts, kLaneWords);
+            } else {
+              hipLaunchKernelGGL(walk, dim3(producers), dim3(kColBinThreads), 0, stream, in, out, n_out, seed, sp, wa,
+                                 wb, first, count, static_cast<const uint32_t *>(nullptr),
+                                 static_cast<const uint32_t *>(nullptr), static_cast<const T1 *>(nullptr), states, 0u,
+                                 n_win, shift, cap, pairs, n_pairs, packed ? 1u : 0u, counts);
+            }
+            if (++in_bins == group && at + span < n_in) {
               if (!add_uniform_bins<T1>("jitconn column walk", stream, out, n_out, shift, producers, cap, pairs, packed, counts,
                                         static_cast<uint32_t *>(nullptr)))
                 return;  // (the error stands: part of the pairs is in `out` already)

@@ -386,6 +386,26 @@ def test_row_walk_of_short_streams(cuda, oracle_mod, w_kind, a, b, dtype, n_out,
   oracle_mod.set_threads(1)
 
 
+@pytest.mark.parametrize("w_kind,a,b", [("homo", 0.0, 0.0), ("uniform", 0.25, 1.75), ("normal", 0.5, 2.0)])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n_out,n_in,p", [(900, 5001, 0.001), (30_000, 33_000, 0.0003), (3, 70_063, 1.0), (40, 70_063, 0.5),
+                                          (17_000, 140_000, 0.0035), (2_200_000, 2100, 0.0001)])
+def test_column_walk_of_short_streams(cuda, oracle_mod, w_kind, a, b, dtype, n_out, n_in, p):
+  # a lane to a column: batches of 64 that do not come out even, one window and several, windows of more than 16 bits of
+  # positions, no bins at all (events with few pairs), several launches (140,000 columns), streams beyond word 227
+  rng = np.random.default_rng(n_out)
+  ev, vec = rng.random(n_in) < 0.1, rng.uniform(0.5, 2.0, n_in).astype(dtype) * (rng.random(n_in) < 0.9)
+  oracle_mod.set_threads(min(16, len(os.sched_getaffinity(0))))
+  kw = dict(w_kind=w_kind, w_a=a, w_b=b, log_p=oracle_mod.log_p_of(p), seed=21, n_row=n_out, n_col=n_in, out_dtype=dtype,
+            col_walk=True)
+  for inp, dense in ((ev, False), (vec.astype(dtype), True)):
+    want, mag = oracle_mod.jitconn_matvec(inp, dense=dense, return_abs=True, **kw)
+    got = kernel_call(inp, dense=dense, **kw)
+    if w_kind == "homo" and not dense: assert np.array_equal(got, want)
+    assert_close_reordered(got, want, mag, dtype, what="column walk of short streams")
+  oracle_mod.set_threads(1)
+
+
 @pytest.mark.parametrize("w_kind,mean,most", [("homo", 167.0, 226), ("uniform", 104.0, 150)])
 def test_row_walk_of_streams_that_outlast_their_lane(cuda, oracle_mod, w_kind, mean, most):
   # among streams of so many synapses in the mean a few need more words than a lane can draw (454): those are walked
@@ -401,9 +421,14 @@ def test_row_walk_of_streams_that_outlast_their_lane(cuda, oracle_mod, w_kind, m
   kw.update(w_b=2.0)
   vec = np.random.default_rng(7).uniform(0.5, 2.0, n_in).astype(np.float32)
   want, mag = oracle_mod.jitconn_matvec(vec, dense=True, return_abs=True, **kw)
-  oracle_mod.set_threads(1)
   assert_close_reordered(kernel_call(vec, col_walk=False, dense=True, **kw), want, mag, np.float32,
                          what="streams that outlast their lane")
+  # the same streams as columns (homogeneous ones of that length are walked by waves): their wave finishes them
+  kw.update(n_row=n_in, n_col=n_out, col_walk=True, w_b=1.0)
+  ones = np.ones(n_out, np.float32)
+  want = oracle_mod.jitconn_matvec(ones, dense=True, **kw)
+  oracle_mod.set_threads(1)
+  assert np.array_equal(kernel_call(ones, dense=True, **kw), want)
 
 
 @pytest.mark.parametrize("m,k,columns", [(3, 31, 0), (64, 33, 1), (65, 500, 63), (130, 64, 64), (9, 900, 65)])
