@@ -1472,9 +1472,17 @@ __global__ __launch_bounds__(1024, (MODE == kEvent && BITS == 1) ? 8 : 4) void c
       }
     }
     if (mean >= 384) { gpb = 1; hub_len = hub_length(mean, kWaveStep, wave_least); gather_rows_wave<F, VT, HETER, MODE, BITS, 8>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
+    // Few long rows leave most groups of eight lanes one row and the longest of them sets the time; many of them are better
+    // fed by sixteen lanes where hits have weights to wait for.  (8 / 32 lanes, even rows and log-normal ones, weights per nonzero, 10 %
+    // events: 3,000 rows of 300 12.7 / 9.2 and 26 / 16 us, 20,000 of 220 14.1 / 12.3 and 37.5 / 28.8, 40,000 of 200 20.5 / 16.6 and 54 /
+    // 42, 60,000 of 200 23.5 / 21.2 but at 1 % 17.4 / 19.1; one weight 3,000 of 300 10.3 / 9.3 and 17.2 / 12.3, 9,000 of 250 9.3 / 10.1;
+    // 8 / 16 lanes: 200,000 of 200 73 / 64 and 126 / 121, of 100 37 / 30 and 57 / 54, 70,000 of 100 at 1 % 12.5 / 13.2, one weight
+    // 400,000 of 100 41.7 / 44.7.  Wide bitmaps lose: 30,000 rows of 380, 500,000 columns, at 1 % 24.3 / 29.5.)
+    else if (MODE == kEvent && mean >= 192u && n_col <= 131072u && n_row < (HETER ? 40960u : 4096u)) { gpb = blockDim.x / 32; hub_len = hub_of_group(4 * 32); gather_rows<F, VT, HETER, MODE, BITS, 32, 4>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
+    else if (MODE == kEvent && HETER && mean >= 96u && n_col <= 131072u && n_row >= 131072u) { gpb = blockDim.x / 16; hub_len = hub_of_group(8 * 16); gather_rows<F, VT, HETER, MODE, BITS, 16, 8>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
+    else if (MODE == kEvent && mean >= 48u) { gpb = blockDim.x / 8; hub_len = hub_of_group(8 * 8); gather_rows<F, VT, HETER, MODE, BITS, 8, 8>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
     // (a dense vector is gathered from L2: for rows of 48 .. 191 nonzeros the pipelined 32-lane walk keeps more
     // of those gathers in flight than a wave per row does)
-    else if (MODE == kEvent && mean >= 48u) { gpb = blockDim.x / 8; hub_len = hub_of_group(8 * 8); gather_rows<F, VT, HETER, MODE, BITS, 8, 8>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
     else if (MODE == kDense && mean >= 192u) { gpb = 1; hub_len = hub_length(mean, 2 * kWave); gather_rows_wave<F, VT, HETER, MODE, BITS, 2>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
     else if (mean >= 48) { gpb = blockDim.x / 32; hub_len = hub_of_group(4 * 32); gather_rows<F, VT, HETER, MODE, BITS, 32, 4>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
     else if (MODE == kEvent && mean >= 24) { gpb = blockDim.x / 8; hub_len = hub_of_group(8 * 8); gather_rows<F, VT, HETER, MODE, BITS, 8, 8>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }

@@ -195,6 +195,27 @@ def test_ragged_rows_and_all_row_length_modes(cuda, oracle_mod):
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n_row,n_col,mean", [(4095, 5000, 200), (4097, 5000, 200), (300, 131_072, 383), (40_959, 3000, 192),
+                                              (40_961, 3000, 192), (131_072, 700, 96), (131_071, 700, 97)])
+def test_event_gather_lanes_for_few_and_for_many_rows(cuda, oracle_mod, n_row, n_col, mean, dtype):
+  # groups of 8, 16 or 32 lanes for a row by the number of rows: log-normal rows on either side of each line, empty
+  # ones and rows of a step and one more or less, weights per nonzero and one weight
+  rng = np.random.default_rng(n_row + mean)
+  counts = np.minimum(rng.lognormal(np.log(mean) - 0.32, 0.8, size=n_row).astype(np.int64), n_col // 2)
+  counts[:7] = (0, 1, 127, 128, 129, 255, 257)
+  counts[7:] += max(0, int(np.ceil((mean * n_row - counts.sum()) / (n_row - 7))))
+  indices, indptr = synth.counted_csr(counts, n_col, seed=n_row)
+  assert mean <= indices.shape[0] // n_row < 384
+  ev = rng.random(n_col) < 0.1
+  for data in (rng.standard_normal(indices.shape[0]).astype(dtype), np.array([0.7], dtype)):
+    want = oracle_mod.event_csr_matvec(data, indices, indptr, ev, shape=(n_row, n_col))
+    mag = oracle_mod.event_csr_matvec(np.abs(data), indices, indptr, ev, shape=(n_row, n_col))
+    got = bpl.event_csr_matvec(data, indices, indptr, ev, shape=(n_row, n_col)).cpu().numpy()
+    assert_close_reordered(got, want, mag, dtype, what="event gather, few and many rows")
+
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
 def test_gather_long_rows_that_begin_at_different_steps(cuda, oracle_mod, dtype):
   # rows of 384 nonzeros or more take a wave each, in steps of 512 (float64: the same walk), and begin at a full
   # step chosen by the row's number: rows of exactly 1, 2, 3, 4 and 9 full steps, with and without a partial
