@@ -633,7 +633,7 @@ __global__ __launch_bounds__(kColBinThreads, sizeof(T1) == 4 ? 8 : 4) void jitco
   __shared__ __attribute__((aligned(8))) uint32_t s_state[kWaves * kStateWords];
   __shared__ uint32_t s_cnt[kBinMaxWindows];
   const int lane = lane_id();
-  const uint32_t wave = threadIdx.x / kWave, p = blockIdx.x;
+  const uint32_t wave = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / kWave))), p = blockIdx.x;
   if (threadIdx.x < n_win) s_cnt[threadIdx.x] = counts[static_cast<size_t>(threadIdx.x) * gridDim.x + p];
   __syncthreads();
   const uint64_t region = static_cast<uint64_t>(p) * n_win * cap;  // first place of this workgroup's bins
