@@ -46,7 +46,7 @@ __global__ __launch_bounds__(kPrepareThreads) void matmat_prepare_kernel(const T
     const uint32_t base = blockIdx.x * kWave;
     const int lane = lane_id();
     if (threadIdx.x < kWave)
-      mt_seed_batch<kSeedSoon>(reinterpret_cast<uint32_t *>(s_mem), lane, seed + base + static_cast<uint32_t>(lane),
+      mt_seed_batch<true>(reinterpret_cast<uint32_t *>(s_mem), lane, seed + base + static_cast<uint32_t>(lane),
                                states + static_cast<size_t>(base) * kMtN,
                                count - base < static_cast<uint32_t>(kWave) ? count - base : static_cast<uint32_t>(kWave));
     return;

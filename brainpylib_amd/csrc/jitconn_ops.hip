@@ -572,8 +572,8 @@ __global__ __launch_bounds__(kColBinThreads, sizeof(T1) == 4 ? 8 : 4) void jitco
       }
       const uint32_t left = mine - j * kFuseBatch;
       uint32_t *const to = ring + static_cast<size_t>(slot) * kFuseBatch * kMtN;
-      if (left >= kFuseBatch) mt_seed_batch<kSeedGuarded>(st, lane, seed + col, to, left);
-      else mt_seed_batch<kSeedSoon>(st, lane, seed + col, to, left);
+      if (left >= kFuseBatch) mt_seed_batch(st, lane, seed + col, to, left);
+      else mt_seed_batch<true>(st, lane, seed + col, to, left);
       __hip_atomic_store(&s_ready[slot], j + 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
     };
     if (wave == 0 && batches != 0) seed_batch(0);
@@ -719,7 +719,7 @@ __global__ __launch_bounds__(kSeedThreads) void mt_seed_streams_kernel(uint32_t 
   const uint32_t mine = base + static_cast<uint32_t>(lane);  // lane l seeds stream base + l
   uint32_t x = seed + first + mine;
   if (ids != nullptr) x = seed + (mine < count ? ids[mine] : 0u);
-  mt_seed_batch<kSeedGuarded>(s_tile[wave], lane, x, states + static_cast<size_t>(base) * kMtN,
+  mt_seed_batch(s_tile[wave], lane, x, states + static_cast<size_t>(base) * kMtN,
                               count - base < static_cast<uint32_t>(kWave) ? count - base : static_cast<uint32_t>(kWave));
 }
 

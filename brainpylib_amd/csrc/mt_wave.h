@@ -75,14 +75,13 @@ __device__ __forceinline__ void mt_load(uint32_t *st, const uint32_t *__restrict
 // of 3.1 ms.)  `dst` is wave uniform: the stores take it as a buffer whose lane offset never changes.
 constexpr int kMtSeedPairStride = 160;  // words from a pair of words of the 64 streams to the next: neighbours in other banks
 constexpr int kMtSeedTileWords = 3 * kMtSeedPairStride + 2 * kWave;
-//
-// kSeedAll: all 64 streams are stored.  kSeedGuarded: the first n_streams, a branch around every store: 78 * 4 of them, 12.5 to
-// 15 us a batch for a wave alone.  kSeedSoon: the first n_streams, by a buffer that ends with the last one's state (the hardware
-// leaves out what lies behind it), and three rounds to a turn of the loop: 8.6 us (10.1 with one round; the recurrence alone takes
-// 5.3), for batches that are waited for.  (Where batch after batch is seeded beside waves that walk, throughput counts, and the
-// guarded form is the better one: column walk of 1,000,000 streams of 18 synapses with the row walk 1,907 us, with the other two 1,945.)
-enum : int { kSeedAll = 0, kSeedGuarded = 1, kSeedSoon = 2 };
-template <int FORM = kSeedAll>
+
+// The first n_streams are stored.  Otherwise than SOON: a branch around every store of a batch of fewer than 64: 78 * 4 of them,
+// 12.5 to 15 us a batch for a wave alone.  SOON: by a buffer that ends with the last one's state (the hardware leaves out what
+// lies behind it), and three rounds to a turn of the loop: 8.6 us (10.1 with one round; the recurrence alone takes 5.3), for
+// batches that are waited for.  (Where batch after batch is seeded beside waves that walk, throughput counts, and the branches
+// are the better form: column walk of 1,000,000 streams of 18 synapses with the row walk 1,907 us, without them 1,945.)
+template <bool SOON = false>
 __device__ __forceinline__ void mt_seed_batch(uint32_t *tile, int lane, uint32_t lane_seed, uint32_t *dst,
                                               uint32_t n_streams = kWave) {
   typedef uint32_t Pair __attribute__((ext_vector_type(2)));
@@ -91,20 +90,20 @@ __device__ __forceinline__ void mt_seed_batch(uint32_t *tile, int lane, uint32_t
   Pair *const put = reinterpret_cast<Pair *>(tile) + lane;
   const Pair *const get = reinterpret_cast<const Pair *>(tile) + (pair * (kMtSeedPairStride / 2) + sub);
   const __amdgpu_buffer_rsrc_t out = __builtin_amdgcn_make_buffer_rsrc(
-      dst, 0, static_cast<int>(FORM == kSeedSoon ? n_streams * (kMtN * 4u) : kWave * kMtN * 4u), 0x00027000);
+      dst, 0, static_cast<int>(SOON ? n_streams * (kMtN * 4u) : kWave * kMtN * 4u), 0x00027000);
   // (streams 16 q + sub; the 16 q are added on the scalar unit, but where they have to count in the lane's offset)
   constexpr uint32_t kRow16 = 16u * kMtN * 4u;
   const uint32_t lane_offset = (sub * kMtN + 2u * pair) * 4u;
   auto store = [&](uint32_t q, uint32_t w0, Pair v) {  // streams 16 q + sub: words w0 + 2 pair, + 1
-    if (FORM == kSeedGuarded && !(16u * q + sub < n_streams)) return;
-    __builtin_amdgcn_raw_buffer_store_b64(v, out, static_cast<int>(lane_offset + (FORM == kSeedSoon ? kRow16 * q : 0u)),
-                                          static_cast<int>((FORM == kSeedSoon ? 0u : kRow16 * q) + w0 * 4u), 0);
+    if (!SOON && !(16u * q + sub < n_streams)) return;
+    __builtin_amdgcn_raw_buffer_store_b64(v, out, static_cast<int>(lane_offset + (SOON ? kRow16 * q : 0u)),
+                                          static_cast<int>(SOON ? w0 * 4u : (16u * q * kMtN + w0) * 4u), 0);
   };
   // The words of a tile are read back from LDS at the end of a round and stored at the start of the next
   // one, behind its eight steps of the recurrence, so that the chain of multiplications does not wait for
   // the LDS (a wave's LDS operations complete in order: the next round's writes cannot overtake the reads).
   Pair v[4];
-#pragma unroll(FORM == kSeedSoon ? 3 : 1)
+#pragma unroll(SOON ? 3 : 1)
   for (uint32_t w0 = 0; w0 < kMtN; w0 += 8) {
 #pragma unroll
     for (uint32_t i = 0; i < 8; i += 2) {  // words w0 + i and w0 + i + 1 of stream `lane`
