@@ -107,9 +107,9 @@ __global__ __launch_bounds__(256) void jitconn_matmat_kernel(const T1 *__restric
   Synapse<T1> *syn = s_syn + wave * kSlots;
   const uint32_t row_base = pass * (MT * kWave);  // first row of Y of this pass
   // The walk is bound by these reads, 512 bytes per synapse and pass of 128 float32 rows, at 27 of the 33 TB/s that 64 bytes
-  // per clock and CU come to, with the vector issue (two thirds of its rate) beside them.  A load takes the wave-uniform byte offset
+  // per clock and CU come to, with the vector issue (0.6 of its rate) beside them.  A load takes the wave-uniform byte offset
   // of a row of the slice (32 bits, checked by the host), an immediate one, and four times the lane, which the buffer's
-  // descriptor adds (stride 4, thread number enabled): no address arithmetic per synapse, one instruction of 8.6 less: 10,000 x
+  // descriptor adds (stride 4, thread number enabled): no address arithmetic per synapse, one instruction less, 6.9 now: 10,000 x
   // 10,000 of 1,000 synapses x 128 203 -> 200 us, 1,000 x 200,000 of 20 396 -> 390.  Loads of 4 bytes a lane reach that
   // rate; of 8 bytes 17.6 TB/s, as they did the float64 rows before these were stored as two words apart (5,000 x 10,000 of
   // 250 x 100: 166 -> 124 us; with 16 bytes a lane 124 too, but there 64 rows are half a wave) and float32 rows of 128 as pairs (300 us).
