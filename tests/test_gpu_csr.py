@@ -527,6 +527,27 @@ def test_event_scatter_sorted_by_output_window(cuda, oracle_mod, dtype):
       assert np.array_equal(got, want)  # a homogeneous weight is added once per synapse: the reference's bits
 
 
+@pytest.mark.parametrize("rows", [3000, 4097])
+@pytest.mark.parametrize("per_cu", [2048, 3072, 5120])
+@pytest.mark.parametrize("more", [0, 1])
+def test_event_scatter_producers_on_either_side_of_one_round(cuda, rows, per_cu, more):
+  # one workgroup to a compute unit as long as a round holds its share, then two: pairs that fill the round of every
+  # compute unit to the last place, and one more.  Whole numbers: every order of the additions gives the same sums.
+  nnz = torch.cuda.get_device_properties(0).multi_processor_count * per_cu + more
+  rng = np.random.default_rng(nnz + rows)
+  n_col = 70_003
+  cut = np.sort(rng.choice(np.arange(1, nnz), rows - 1, replace=False))
+  indptr = np.concatenate([[0], cut, [nnz]]).astype(np.uint32)
+  indices = rng.integers(0, n_col, nnz).astype(np.uint32)
+  ev = np.ones(rows, dtype=bool)
+  for dtype in (np.float32, np.float64):
+    data = rng.integers(-8, 9, nnz).astype(dtype)
+    got = bpl.event_csr_matvec(data, indices, indptr, ev, shape=(rows, n_col), transpose=True).cpu().numpy()
+    assert np.array_equal(got, np.bincount(indices, weights=data, minlength=n_col))
+    got = bpl.event_csr_matvec(np.array([2.0], dtype), indices, indptr, ev, shape=(rows, n_col), transpose=True).cpu().numpy()
+    assert np.array_equal(got, 2.0 * np.bincount(indices, minlength=n_col))
+
+
 @pytest.mark.parametrize("listed", [1, 1023, 1025, 4096, 4097])
 @pytest.mark.parametrize("columns", ["sorted", "descending", "random", "one"])
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
