@@ -386,6 +386,44 @@ def test_row_walk_of_short_streams(cuda, oracle_mod, w_kind, a, b, dtype, n_out,
   oracle_mod.set_threads(1)
 
 
+@pytest.mark.parametrize("signed", [False, True])
+@pytest.mark.parametrize("n_out,mean", [(3000, 20.0), (130_000, 100.0), (300_000, 167.0)])
+def test_sums_of_short_streams_in_double(cuda, oracle_mod, n_out, mean, signed):
+  # A lane adds a whole row.  The vector is cut in two whose sums are exact in whatever order: 40 bits behind the point, and the
+  # 13 bits and fewer that are left.  The result may be half a unit of the last place off plus what is lost of the lost parts: at
+  # most 2^-53 of each, which are 2^-53 of a partial sum each, of which there are at most 250 (300,000 rows: some by wave, in
+  # 64 sums of a few addends and a tree of six additions, as many half units of the sum of the sizes)
+  n_in = 600_000 if mean > 150 else 20_000
+  rng = np.random.default_rng(n_out)
+  vec = rng.uniform(0.5, 2.0, n_in) * (rng.choice([-1.0, 1.0], n_in) if signed else 1.0)
+  high = np.round(vec * 2.0 ** 40) * 2.0 ** -40
+  oracle_mod.set_threads(min(16, len(os.sched_getaffinity(0))))
+  kw = dict(w_kind="homo", log_p=oracle_mod.log_p_of(mean / n_in), seed=400_012, n_row=n_out, n_col=n_in, dense=True)
+  (a, mag), b = oracle_mod.jitconn_matvec(high, return_abs=True, **kw), oracle_mod.jitconn_matvec(vec - high, **kw)
+  counts = oracle_mod.jitconn_matvec(np.ones(n_in), **kw)
+  oracle_mod.set_threads(1)
+  assert np.finfo(np.longdouble).nmant >= 63
+  want = a.astype(np.longdouble) + b.astype(np.longdouble)
+  off = np.abs(kernel_call(vec, col_walk=False, **kw).astype(np.longdouble) - want).astype(np.float64)
+  bound = 2.0 ** -53 * np.abs(want).astype(np.float64) * (1 + 2.0 ** -50) + 250 ** 2 * 2.0 ** -106 * mag
+  bound[counts > 226] = 10 * 2.0 ** -53 * mag[counts > 226]
+  assert np.all(off <= bound), (off / np.abs(want).astype(np.float64)).max()
+
+
+def test_sums_of_short_streams_with_infinities(cuda, oracle_mod):
+  # infinite addends give what a plain sum gives: an infinity, or NaN where both kinds meet
+  n_out, n_in = 5000, 900
+  vec = np.random.default_rng(3).uniform(0.5, 2.0, n_in)
+  vec[5], vec[400], vec[77] = np.inf, -np.inf, np.finfo(np.float64).max
+  kw = dict(w_kind="homo", log_p=oracle_mod.log_p_of(0.03), seed=3, n_row=n_out, n_col=n_in, dense=True)
+  want = oracle_mod.jitconn_matvec(vec, **kw)
+  assert np.isnan(want).any() and (want == np.inf).any() and (want == -np.inf).any() and (np.abs(want) < 1e3).any()
+  got = kernel_call(vec, col_walk=False, **kw)
+  finite = np.isfinite(want)
+  np.testing.assert_array_equal(got[~finite], want[~finite])
+  np.testing.assert_allclose(got[finite], want[finite], rtol=50 * 2.0 ** -53)  # (some 50 addends of one sign)
+
+
 @pytest.mark.parametrize("w_kind,a,b", [("homo", 0.0, 0.0), ("uniform", 0.25, 1.75), ("normal", 0.5, 2.0)])
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 @pytest.mark.parametrize("n_out,n_in,p", [(900, 5001, 0.001), (30_000, 33_000, 0.0003), (3, 70_063, 1.0), (40, 70_063, 0.5),
