@@ -199,3 +199,29 @@ def test_batching_transposed_with_every_event_set(cuda):
       t1.synchronize()
       times[b].append(t0.elapsed_time(t1) / b)
   assert min(times[batch]) < 2.0 * min(times[8]), times
+
+
+def test_batching_transposed_shares_out_long_rows_of_more_nonzeros_than_32_bits_count(cuda):
+  # 600 rows of a million nonzeros: eight entries of them are 4.8e9, seven 4.2e9 (below 2^32).  Two rows are active: they
+  # are shared out among the workgroups in either case (a workgroup to a row takes some 200 rounds one after the other).
+  n_row, n_col = 600, 1_000_000
+  indices = torch.arange(n_col, dtype=torch.int32, device=cuda).repeat(n_row)[None]
+  indptr = (torch.arange(n_row + 1, dtype=torch.int64, device=cuda) * n_col).to(torch.int32)[None]
+  one = torch.ones((1, 1), device=cuda)
+  times = {}
+  for batch in (7, 8):
+    events = torch.zeros((batch, n_row), dtype=torch.bool, device=cuda)
+    events[0, 0], events[batch - 1, n_row - 1] = True, True
+    call = lambda: bpl.event_csr_matvec_batching(one, indices, indptr, events, batch_size=batch, shape=(n_row, n_col), transpose=True)
+    got = call()
+    assert bool((got == events.any(1).float()[:, None]).all())
+    times[batch] = []
+    for _ in range(5):
+      t0, t1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+      t0.record()
+      call()
+      t1.record()
+      t1.synchronize()
+      times[batch].append(t0.elapsed_time(t1))
+  print(times)
+  assert min(times[8]) < 2.0 * min(times[7]), times
