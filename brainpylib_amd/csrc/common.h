@@ -138,7 +138,8 @@ bool flat_window_scatter(const char *target, hipStream_t stream, const F *data, 
 // through direct atomics, far more slowly), and bin_event_scatter_bytes() is the size to ask for.
 // Batched calls (several event vectors, one matrix) hand in one list over all batch entries, n_col
 // = batch * columns, and `active_colbase` = what to add to the columns of each listed row (its
-// batch entry * columns); n_row stays the matrix's row count (indptr has n_row + 1 entries).
+// batch entry * columns); n_row stays the matrix's row count (indptr has n_row + 1 entries), and `entries` is
+// how many entries the list is over (the listed rows hold at most that many times the matrix's nonzeros).
 constexpr size_t kBinEventFillBytes = 131072;
 // How many entries of a batch (one matrix of nnz nonzeros, entries' columns side by side) such a chain takes, and how many
 // pairs its runs are to hold.
@@ -162,7 +163,7 @@ template <typename F, typename I>
 bool bin_event_scatter(hipStream_t stream, const F *data, bool heter, const I *indices, const I *indptr,
                        F *y, uint32_t n_row, uint32_t n_col, uint32_t *active_count, const uint2 *active_list,
                        uint32_t list_cap, void *scratch, size_t scratch_bytes,
-                       const uint32_t *active_colbase = nullptr);
+                       const uint32_t *active_colbase = nullptr, uint32_t entries = 1);
 // csr_event_sum with 64-bit index arrays through the sorted event scatter (csr_ops.hip).  1: enqueued (a matrix of
 // 2^32 nonzeros or more leaves the zeroed result untouched); 0: nothing enqueued, take another path; -1: failed.
 template <typename F, bool HETER>

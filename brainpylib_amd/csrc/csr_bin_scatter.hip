@@ -717,8 +717,8 @@ template <typename F, bool HETER, typename I>
 __global__ __launch_bounds__(kBinThreads, 8) __attribute__((amdgpu_num_sgpr(80))) void bin_active_rows_kernel(
     const F *__restrict__ data, const I *__restrict__ indices, const I *__restrict__ indptr,
     uint32_t n_row, const uint32_t *__restrict__ active_count, const uint2 *__restrict__ active_list,
-    uint32_t list_cap, const uint32_t *__restrict__ active_colbase, F *__restrict__ y, uint32_t shift, uint32_t cap,
-    BinPair<F> *__restrict__ pairs, uint32_t *__restrict__ fill) {
+    uint32_t list_cap, const uint32_t *__restrict__ active_colbase, uint32_t entries, F *__restrict__ y, uint32_t shift,
+    uint32_t cap, BinPair<F> *__restrict__ pairs, uint32_t *__restrict__ fill) {
   __shared__ uint32_t s_ptr[kTileRows + 1];     // nonzeros of the tile's rows before row k
   __shared__ uint32_t s_start[kTileRows];       // first nonzero of row k in the matrix
   __shared__ uint32_t s_colbase[kTileRows];     // added to row k's columns (batched calls: batch entry * n_col)
@@ -727,7 +727,6 @@ __global__ __launch_bounds__(kBinThreads, 8) __attribute__((amdgpu_num_sgpr(80))
   __shared__ uint32_t s_off[kMaxWindows + 1];   // their offsets in the sorted round
   __shared__ uint32_t s_base[kMaxWindows];      // place in the window's run of the pair at position i of the round: s_base + i
   __shared__ uint32_t s_wave[kBinThreads / kWave];
-  __shared__ uint64_t s_wave_sum[kBinThreads / kWave];
   __shared__ uint32_t s_share[4];               // this producer's first and last row, the nonzeros it leaves out of them
   constexpr int U = (sizeof(F) == 4) ? 5 : 3;
   constexpr uint32_t kRound = U * kBinThreads;
@@ -737,30 +736,30 @@ __global__ __launch_bounds__(kBinThreads, 8) __attribute__((amdgpu_num_sgpr(80))
   const uint32_t total = active_count[0] < list_cap ? active_count[0] : list_cap;  // (never beyond the list)
   const uint32_t nnz = static_cast<uint32_t>(indptr[n_row]);  // (64-bit offsets: listed only below 2^32 nonzeros)
   // the listed rows' nonzeros: exact where every producer can look at the whole list, else from the mean row length
-  // (Summed in 64 bits: rows of several batch entries may hold more than 2^32 together, and a few long ones are still shared out.
-  // A thread has four rows at most, whose sum is scanned in its lower 24 bits and those above.)
+  // (counted in 32 bits: where the rows of several batch entries may hold more, 16 nonzeros at a time; entries are 8 at most then.
+  // Sums of 64 bits cost every call 0.4 us.)
   uint64_t work = static_cast<uint64_t>(total) * (nnz / n_row + 1u);
   const bool exact = total <= kExactRows;
+  const uint32_t unit = static_cast<uint64_t>(nnz) * entries <= 0xffffffffu ? 0u : 4u;
+  auto units = [&](uint32_t length) { return unit ? length / 16u + (length % 16u ? 1u : 0u) : length; };
   const uint32_t each = (total + kBinThreads - 1u) / kBinThreads;  // (of these, listed rows a thread)
-  uint64_t before_mine = 0;
+  uint32_t before_mine = 0;
   if (exact) {
-    static_assert(kExactRows <= 256u * kBinThreads, "lower halves: at most 64 * 2^24");
-    uint64_t mine = 0;
+    uint32_t mine = 0;
     for (uint32_t e = 0; e < each; ++e) {
       const uint32_t k = tid * each + e;
-      mine += k < total ? active_list[k].y : 0u;
+      mine += k < total ? units(active_list[k].y) : 0u;
     }
-    const uint32_t low = static_cast<uint32_t>(mine) & 0xffffffu, high = static_cast<uint32_t>(mine >> 24);
-    const uint64_t incl = (static_cast<uint64_t>(wave_inclusive_scan_u32(high)) << 24) + wave_inclusive_scan_u32(low);
-    if (lane == kWave - 1) s_wave_sum[wave] = incl;
+    const uint32_t incl = wave_inclusive_scan_u32(mine);
+    if (lane == kWave - 1) s_wave[wave] = incl;
     __syncthreads();
-    uint64_t all = 0;
+    uint32_t all = 0;
     for (uint32_t w = 0; w < kBinThreads / kWave; ++w) {
       if (w == wave) before_mine = all;
-      all += s_wave_sum[w];
+      all += s_wave[w];
     }
     before_mine += incl - mine;
-    work = all;
+    work = static_cast<uint64_t>(all) << unit;
   }
   // With little activity a few producers finish sooner than a chip full of them, and as long as one round holds their shares,
   // one to a CU sooner than more: 720,000 pairs of 1,365 rows over 126,766 columns 22.7 us with 352, 21.2 with 256; 990,000
@@ -780,11 +779,13 @@ __global__ __launch_bounds__(kBinThreads, 8) __attribute__((amdgpu_num_sgpr(80))
   // first `end` of row hi - 1: an equal share of the nonzeros, or, of a long list, of the rows.
   uint32_t lo, hi, skip = 0, end = 0xffffffffu;
   if (exact) {
-    const uint64_t a = p * work / producers, b = (p + 1u) * work / producers;  // (work is below 2^44)
+    const uint32_t all = static_cast<uint32_t>(work >> unit);
+    const uint32_t a = static_cast<uint32_t>(static_cast<uint64_t>(p) * all / producers);
+    const uint32_t b = static_cast<uint32_t>(static_cast<uint64_t>(p + 1u) * all / producers);
     for (uint32_t e = 0; e < each; ++e) {  // (listed rows are never empty: one row holds nonzero a, one nonzero b - 1)
-      const uint32_t k = tid * each + e, len = k < total ? active_list[k].y : 0u;
-      if (a - before_mine < len) s_share[0] = k, s_share[2] = static_cast<uint32_t>(a - before_mine);
-      if (b - 1u - before_mine < len) s_share[1] = k + 1u, s_share[3] = static_cast<uint32_t>(b - before_mine);
+      const uint32_t k = tid * each + e, len = k < total ? units(active_list[k].y) : 0u;
+      if (a - before_mine < len) s_share[0] = k, s_share[2] = (a - before_mine) << unit;
+      if (b - 1u - before_mine < len) s_share[1] = k + 1u, s_share[3] = b - before_mine < len ? (b - before_mine) << unit : 0xffffffffu;
       before_mine += len;
     }
     __syncthreads();
@@ -1483,7 +1484,8 @@ size_t bin_event_scatter_min_bytes(uint32_t n_col) {
 template <typename F, typename I>
 bool bin_event_scatter(hipStream_t stream, const F *data, bool heter, const I *indices, const I *indptr,
                        F *y, uint32_t n_row, uint32_t n_col, uint32_t *active_count, const uint2 *active_list,
-                       uint32_t list_cap, void *scratch, size_t scratch_bytes, const uint32_t *active_colbase) {
+                       uint32_t list_cap, void *scratch, size_t scratch_bytes, const uint32_t *active_colbase,
+                       uint32_t entries) {
   const uint32_t shift = event_window_shift(n_col);
   const uint32_t n_win = div_up(n_col, 1u << shift);
   if (scratch_bytes < bin_event_scatter_min_bytes<F>(n_col)) return false;
@@ -1514,10 +1516,10 @@ bool bin_event_scatter(hipStream_t stream, const F *data, bool heter, const I *i
   const uint32_t producers = 2u * num_cu;
   if (heter)
     hipLaunchKernelGGL((bin_active_rows_kernel<F, true, I>), dim3(producers), dim3(kBinThreads), 0, stream, data, indices,
-                       indptr, n_row, active_count, active_list, list_cap, active_colbase, y, shift, cap, pairs, fill);
+                       indptr, n_row, active_count, active_list, list_cap, active_colbase, entries, y, shift, cap, pairs, fill);
   else
     hipLaunchKernelGGL((bin_active_rows_kernel<F, false, I>), dim3(producers), dim3(kBinThreads), 0, stream, data, indices,
-                       indptr, n_row, active_count, active_list, list_cap, active_colbase, y, shift, cap, pairs, fill);
+                       indptr, n_row, active_count, active_list, list_cap, active_colbase, entries, y, shift, cap, pairs, fill);
   hipLaunchKernelGGL(add_kernel, dim3(n_win * slices * parts), dim3(kBinThreads), lds, stream, y, n_col, shift,
                      lds_shift, parts, cap, pairs, fill, active_count, data, indices, active_list, active_colbase);
   return true;
@@ -1685,16 +1687,16 @@ template size_t bin_event_scatter_min_bytes<float>(uint32_t);
 template size_t bin_event_scatter_min_bytes<double>(uint32_t);
 template bool bin_event_scatter<float, uint32_t>(hipStream_t, const float *, bool, const uint32_t *, const uint32_t *, float *,
                                                  uint32_t, uint32_t, uint32_t *, const uint2 *, uint32_t, void *, size_t,
-                                                 const uint32_t *);
+                                                 const uint32_t *, uint32_t);
 template bool bin_event_scatter<double, uint32_t>(hipStream_t, const double *, bool, const uint32_t *, const uint32_t *,
                                                   double *, uint32_t, uint32_t, uint32_t *, const uint2 *, uint32_t, void *,
-                                                  size_t, const uint32_t *);
+                                                  size_t, const uint32_t *, uint32_t);
 template bool bin_event_scatter<float, uint64_t>(hipStream_t, const float *, bool, const uint64_t *, const uint64_t *, float *,
                                                  uint32_t, uint32_t, uint32_t *, const uint2 *, uint32_t, void *, size_t,
-                                                 const uint32_t *);
+                                                 const uint32_t *, uint32_t);
 template bool bin_event_scatter<double, uint64_t>(hipStream_t, const double *, bool, const uint64_t *, const uint64_t *,
                                                   double *, uint32_t, uint32_t, uint32_t *, const uint2 *, uint32_t, void *,
-                                                  size_t, const uint32_t *);
+                                                  size_t, const uint32_t *, uint32_t);
 template bool flat_window_scatter<float>(const char *, hipStream_t, const float *, bool, const uint32_t *, const uint32_t *,
                                          const float *, float *, uint32_t, uint32_t);
 template bool flat_window_scatter<double>(const char *, hipStream_t, const double *, bool, const uint32_t *,

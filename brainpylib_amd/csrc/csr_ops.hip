@@ -2427,7 +2427,7 @@ void event_csr_batching_entry(const char *target, hipStream_t stream, void **buf
                              static_cast<uint32_t>(kBinEventFillBytes / sizeof(uint32_t)), o,
                              static_cast<uint64_t>(g) * d.n_col);
           if (!bin_event_scatter<F>(stream, values, HETER, indices, indptr, o, d.n_row, g * d.n_col, counters, list,
-                                    static_cast<uint32_t>(vrows), scratch, scratch_bytes, colbase)) {
+                                    static_cast<uint32_t>(vrows), scratch, scratch_bytes, colbase, g)) {
             set_error("%s: the sorted scatter could not be enqueued", target);
             return;
           }
