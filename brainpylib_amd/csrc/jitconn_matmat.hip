@@ -25,6 +25,7 @@ namespace {
 constexpr int kTile = 32;
 
 constexpr int kPrepareThreads = kTile * 8;
+constexpr uint32_t kPrepareGroups = 1u << 22;  // workgroups that transpose, at most
 
 // XT[r / pass_rows][c][r % pass_rows] = X[r][c] for r < m: the transposed operand in slices of pass_rows rows of
 // X (a multiple of 32), every slice contiguous, its rows pass_rows entries long; rows m .. m_pad - 1 are zero.
@@ -33,10 +34,11 @@ constexpr int kPrepareThreads = kTile * 8;
 // Float64: 64 rows at a time, the low words of the 64 and then the high words, for the walk reads XT word by word.
 // The first seed_groups workgroups do not transpose: one wave of each seeds the generators of 64 of the `count` columns,
 // which it does in 8.6 us, beside the transposition (128 x 10,000: the launch takes 12.5 us, without the seeding 6.1).
+// The others take the tiles in turn: a launch has fewer than 2^32 threads, an X of 2^34 entries as many tiles as 2^32 threads.
 template <typename T>
 __global__ __launch_bounds__(kPrepareThreads) void matmat_prepare_kernel(const T *__restrict__ X, T *__restrict__ XT,
                                                                          uint32_t m, uint32_t k, uint32_t m_pad,
-                                                                         uint32_t pass_rows, uint32_t col_tiles,
+                                                                         uint32_t pass_rows, uint32_t col_tiles, uint32_t tiles,
                                                                          uint32_t seed, uint32_t count,
                                                                          uint32_t seed_groups,
                                                                          uint32_t *__restrict__ states) {
@@ -52,25 +54,29 @@ __global__ __launch_bounds__(kPrepareThreads) void matmat_prepare_kernel(const T
     return;
   }
   T(*tile)[kTile + 1] = reinterpret_cast<T(*)[kTile + 1]>(s_mem);
-  const uint32_t at = blockIdx.x - seed_groups;
-  const uint32_t c0 = at % col_tiles * kTile, r0 = at / col_tiles * kTile;
   const uint32_t tx = threadIdx.x % kTile, ty = threadIdx.x / kTile;  // 32 x 8
-  for (uint32_t i = ty; i < kTile; i += 8) {
-    const uint32_t r = r0 + i, c = c0 + tx;
-    tile[i][tx] = (r < m && c < k) ? X[static_cast<size_t>(r) * k + c] : T(0);
-  }
-  __syncthreads();
-  for (uint32_t i = ty; i < kTile; i += 8) {
-    const uint32_t c = c0 + i, r = r0 + tx;
-    if (c < k && r < m_pad) {
-      constexpr uint32_t kWords = sizeof(T) / 4;
-      uint32_t *to = reinterpret_cast<uint32_t *>(XT + (static_cast<size_t>(r / pass_rows) * k + c) * pass_rows) +
-                     r % pass_rows / kWave * (kWave * kWords) + r % kWave;
-      uint32_t w[kWords];
-      __builtin_memcpy(w, &tile[tx][i], sizeof(T));
-#pragma unroll
-      for (uint32_t part = 0; part < kWords; ++part) to[part * kWave] = w[part];
+  for (uint32_t at = blockIdx.x - seed_groups;;) {
+    const uint32_t c0 = at % col_tiles * kTile, r0 = at / col_tiles * kTile;
+    for (uint32_t i = ty; i < kTile; i += 8) {
+      const uint32_t r = r0 + i, c = c0 + tx;
+      tile[i][tx] = (r < m && c < k) ? X[static_cast<size_t>(r) * k + c] : T(0);
     }
+    __syncthreads();
+    for (uint32_t i = ty; i < kTile; i += 8) {
+      const uint32_t c = c0 + i, r = r0 + tx;
+      if (c < k && r < m_pad) {
+        constexpr uint32_t kWords = sizeof(T) / 4;
+        uint32_t *to = reinterpret_cast<uint32_t *>(XT + (static_cast<size_t>(r / pass_rows) * k + c) * pass_rows) +
+                       r % pass_rows / kWave * (kWave * kWords) + r % kWave;
+        uint32_t w[kWords];
+        __builtin_memcpy(w, &tile[tx][i], sizeof(T));
+#pragma unroll
+        for (uint32_t part = 0; part < kWords; ++part) to[part * kWave] = w[part];
+      }
+    }
+    at += gridDim.x - seed_groups;
+    if (at >= tiles) break;
+    __syncthreads();  // the tile is read
   }
 }
 
@@ -248,8 +254,10 @@ void matmat_entry(const char *target, hipStream_t stream, void **buffers, const 
   T1 *XT = reinterpret_cast<T1 *>(ws);
   uint32_t *states = reinterpret_cast<uint32_t *>(ws + xt_bytes);
   const uint32_t col_tiles = div_up(k, kTile), seed_groups = ahead ? div_up(chunk, kWave) : 0;
-  hipLaunchKernelGGL(matmat_prepare_kernel<T1>, dim3(seed_groups + col_tiles * div_up(m_pad, kTile)),
-                     dim3(kPrepareThreads), 0, stream, X, XT, m, k, m_pad, pass_rows, col_tiles, d.seed, chunk,
+  // (an X that fits the device has fewer than 2^32 tiles)
+  const uint32_t all_tiles = static_cast<uint32_t>(static_cast<uint64_t>(col_tiles) * div_up(m_pad, kTile));
+  hipLaunchKernelGGL(matmat_prepare_kernel<T1>, dim3(seed_groups + (all_tiles < kPrepareGroups ? all_tiles : kPrepareGroups)),
+                     dim3(kPrepareThreads), 0, stream, X, XT, m, k, m_pad, pass_rows, col_tiles, all_tiles, d.seed, chunk,
                      seed_groups, states);
   const T1 wa = static_cast<T1>(d.w_a), wb = static_cast<T1>(d.w_b);
   const uint32_t tiles = pass_rows / kWave, passes = m_pad / pass_rows;

@@ -5,6 +5,7 @@ Generator contract: stream i is std::mt19937{seed + i}; output row i of a row-wa
 single stream.  Checked against (a) golden vectors produced by the reference's compiled CPU
 kernels one stream at a time, (b) the per-stream oracle, (c) exact integer probes that pin the
 generated index sets, (d) full-size properties."""
+import ctypes
 import json
 import os
 
@@ -467,6 +468,33 @@ def test_row_walk_of_streams_that_outlast_their_lane(cuda, oracle_mod, w_kind, m
   want = oracle_mod.jitconn_matvec(ones, dense=True, **kw)
   oracle_mod.set_threads(1)
   assert np.array_equal(kernel_call(ones, dense=True, **kw), want)
+
+
+def test_matmat_of_more_tiles_than_a_launch_has_threads_for(cuda, oracle_mod):
+  # X of 2,200 x 8,000,000 is transposed in 1.8e7 tiles of 32 x 32, 256 threads each: more than 2^32 (4e6 workgroups take them
+  # in turn).  70 GB and their transpose, which is the scratch memory of a stream of its own.
+  m, k, n, seed = 2_200, 8_000_000, 8, 5
+  if torch.cuda.mem_get_info()[0] < 170 << 30:
+    pytest.skip("150 GB of device memory are needed")
+  handle = ctypes.c_void_p()
+  hip = ctypes.CDLL("libamdhip64.so")
+  assert hip.hipStreamCreate(ctypes.byref(handle)) == 0
+  lp = oracle_mod.log_p_of(1e-5)
+  X = torch.empty((m, k), device=cuda)
+  for i in range(0, m, 50):
+    X[i:i + 50].uniform_(0.5, 2.0)
+  torch.cuda.synchronize()
+  with torch.cuda.stream(torch.cuda.ExternalStream(handle.value)):
+    got = bpl.matmat_prob_conn_uniform_weight(X, w_low=0.5, w_high=1.5, conn_prob=1e-5, shape=(k, n), seed=seed)
+  torch.cuda.synchronize()
+  for j in range(n):
+    idx, w = oracle_mod.jitconn_stream_weights(seed + j, "uniform", 0.5, 1.5, lp, k, dtype=np.float32)
+    assert idx.shape[0] > 20
+    want = X[:, torch.from_numpy(idx.astype(np.int64)).to(cuda)].double() @ torch.from_numpy(w.astype(np.float64)).to(cuda)
+    # (some 80 addends of one sign, added in float32 one after the other)
+    torch.testing.assert_close(got[:, j].double(), want, rtol=idx.shape[0] * 2.0 ** -23, atol=0.0)
+  del X, got, want
+  torch.cuda.empty_cache()
 
 
 @pytest.mark.parametrize("m,k,columns", [(3, 31, 0), (64, 33, 1), (65, 500, 63), (130, 64, 64), (9, 900, 65)])
