@@ -403,6 +403,7 @@ __global__ __launch_bounds__(kColThreads) void jitconn_colwalk_kernel(const VT *
 // first, so that one atomic reserves all their positions (atomics of many workgroups on the one
 // counter are served one after the other).
 constexpr uint32_t kCollectCols = 4096;
+constexpr double kColBinEventMin = 1.0e7;  // synapses of all columns from which a walk of event columns has bins (launch_colwalk)
 
 template <typename T1, typename VT>
 __global__ __launch_bounds__(1024) void collect_active_columns_kernel(const VT *__restrict__ in, uint32_t n_in,
@@ -895,31 +896,80 @@ uint32_t rowwalk_exact_bytes(uint32_t n_out) {
   return fused ? rowwalk_coarse_bytes<T1, W>() : rowwalk_bytes_for_two<T1, W, true>();
 }
 
-// Whether a lane walks a stream (jitconn_lane.h) rather than a wave: where its time, in us, is the smaller one by this fit of
-// both, and no more than one stream in 10^5 is expected to need more words than a lane can draw (4.5 standard deviations
-// of the synapses of a row).  A synapse takes a wave 0.27 us or, with weights, up to 2.1 while it waits for its own
-// instructions, longer from one wave to a SIMD on; a wave to a stream is bound by the seeding: on the CU's scalar unit (1.3 us
-// a stream) or, from kSeedAheadMin on, by the states' way through memory.  Either side at the line: 2,000 rows of 30 17.7 / 17.5
-// us, of 44 17.9 / 21; 40,000 of 70 44 / 30; 70,000 of 100 67 / 53, of 130 67 / 68; uniform weights 2,000 of 20 15.9 / 15.3, of 30
-// 15.9 / 19.3; normal ones 20,000 of 20 35 / 32, of 30 35 / 39; in double 1,000 of 3 19.6 / 18.5, 20,000 of 10 48 / 33, of 20 49 / 51.
+// Whether a lane walks a stream (jitconn_lane.h) rather than a wave: where its time, in us, is the smaller one by these fits of
+// both (every kernel with either walk over 1,000 to 1,000,000 streams of 3 to 165 synapses, 3,000 to 600,000 places), and no more
+// than one stream in 10^5 is expected to need more words than a lane can draw (4.5 standard deviations of the synapses of a row).
 //
-// Columns: a synapse's place in the bins and its store come on top.  All columns, 5,000 outputs: 30,000 columns of 20 73 / 34 us, of
-// 60 50 / 55; normal weights of 20 74 / 108, of 3 43 / 21; 130,000 of 60 173 / 69, normal ones 197 / 127.  Those of the events only:
-// their number is not known here, and a wave to each of a few takes 17 us (100 columns of 20 27 / 23 us, of 60 27 / 35; 13,000 of
-// 3 34 / 19, of 20 48 / 49; normal ones of 3 35 / 24, of 20 48 / 53).
+// By lane a wave takes what its longest stream takes, 2.4 standard deviations over the mean, from word 227 on more: a begin
+// and a share for each of its synapses, while they wait for their own instructions, longer from one wave to a SIMD on.  By wave the
+// seeding counts: on the CU's scalar unit, 11.3 us for 2,048 streams, or, from kSeedAheadMin on, for 64 streams a CU at a time.
+//
+// Rows, by wave / by lane at the line, floats: 4,000 of 55, 3,000 inputs 28.1 / 26.2 us, of 75 28.3 / 30.9; 10,000 of 25 22.0 / 17.9, of 55
+// 22.5 / 26.9; 20,000 of 55 29.9 / 27.0, of 75 31.8 / 33.0; 80,000 of 130 70 / 66, of 165 72 / 81; uniform weights 16,000 of 25 24.1 / 17.4,
+// of 55 24.3 / 28.5; normal ones 10,000 of 8 24.4 / 21.5, of 15 24.4 / 27.4, 80,000 of 40 72 / 62, of 55 73.5 / 80; in double 20,000 of 15
+// 45.7 / 42.1, of 25 48 / 58.  Events whose vector the L2s do not hold lose what the walk by wave gains from their bitmap
+// (500,000 rows of 167, 1,500,000 inputs of doubles 418 / 470).
+//
+// Columns of a dense vector: a synapse's place in the bins and its store come on top, and a walk by wave has bins from 1,048,576
+// synapses on.  5,000 outputs: 4,000 columns of 25 26.6 / 25.8 us, of 40 30.5 / 40.2; 10,000 of 100 96 / 69, of 130 36 / 83; 60,000 of 55 71 / 62,
+// of 100 78 / 87; doubles, whose 512 workgroups do not fit the device at once, 20,000 of 40 75 / 66, of 55 53 / 79; normal ones 8,000 of 3 36 / 26, of 15 39 / 50.
+//
+// Those of the events only: their number is not known here, and a wave to each of a few takes 20 us (5,000 outputs, 15 columns
+// of 15 21.2 / 20.1 us, of 25 21.4 / 23.5; normal ones of 3 19.3 / 17.4, of 8 19.0 / 20.8).
 enum StreamUse { kGathers, kScatters, kScattersSome };
 template <typename T1, int W>
-bool streams_by_lane(uint32_t streams, uint32_t n, double log_p, const SkipParams &sp, StreamUse use) {
-  const double mean = -std::expm1(log_p) * static_cast<double>(n);
-  constexpr double words = W == kHomo ? 2.0 : W == kUniform ? 2.0 + WeightWords<T1>::value : sizeof(T1) == 4 ? 3.27 : 4.55;
+bool streams_by_lane(uint32_t streams, uint32_t n, double log_p, const SkipParams &sp, StreamUse use, uint64_t event_bytes = 0) {
+  constexpr bool wide = sizeof(T1) == 8;
+  const double mean = -std::expm1(log_p) * static_cast<double>(n), count = streams;
+  constexpr double words = W == kHomo ? 2.0 : W == kUniform ? 2.0 + WeightWords<T1>::value : wide ? 4.55 : 3.27;
   if (!sp.narrow || n > 0xf0000000u || words * (mean + 4.5 * std::sqrt(mean)) > kLaneWords - 2.0) return false;
-  const double step = (W == kHomo ? 0.27 : W == kUniform ? (sizeof(T1) == 4 ? 0.35 : 0.45) : sizeof(T1) == 4 ? 1.0 : 2.1) +
-                      (use == kGathers ? 0.0 : 0.15);
-  const double steps = mean + 0.7 * std::fmax(0.0, mean - kLaneFirst / words);
-  if (use == kScattersSome) return 8.0 + step * steps < 15.0;
-  const double by_lane = 8.0 + step * steps * std::fmax(1.0, 0.8 + streams / 120e3);
-  if (use == kScatters) return by_lane < std::fmax(24.0, 6.0 + streams * 0.74e-3);
-  const double by_wave = streams < kSeedAheadMin ? 7.0 + streams / 195.0 : std::fmax(31.0, 6.0 + streams * 0.74e-3);
+  const double longest = mean + 2.4 * std::sqrt(mean), steps = longest + 0.5 * std::fmax(0.0, longest - kLaneFirst / words);
+  // the share of a wave's steps whose skips the upper word alone does not decide
+  const double undecided = sp.quick ? -std::expm1(-128.0 * 0x1p-33 * sp.quick_band) : 1.0;
+  auto of = [](double homo, double uniform, double uniform_wide, double normal, double normal_wide) {
+    return W == kHomo ? homo : W == kUniform ? (wide ? uniform_wide : uniform) : wide ? normal_wide : normal;
+  };
+  if (use == kGathers) {
+    if (event_bytes > (8u << 20)) return false;
+    const double turns = std::ceil(count / 65536.0);  // waves of 64 to a SIMD
+    const double step = of(wide ? 0.262 : 0.25, 0.33, 0.42, 0.73, 1.25) * (1.0 + undecided * of(0.4, 0.15, 0.1, 0.1, 0.05));
+    const double by_lane = of(8.0, 6.0, 6.0, 9.0, 10.5) + step * steps * (1.0 + of(0.32, 0.42, 0.42, 0.42, 0.6) * (turns - 1.0));
+    double by_wave = streams < kSeedAheadMin ? of(5.5, 4.0, 4.3, 4.7, 5.5) + 11.3 * std::ceil(count / 2048.0)
+                     : streams <= 16384u     ? of(21.6, 21.3, 23.3, 24.0, 29.0) + (streams > 12288u ? 1.5 : 0.0)
+                     : streams <= 32768u     ? of(29.6, 29.4, 33.0, 33.0, 45.0) + (streams > 24576u ? 1.5 : 0.0)
+                                             : of(10.0, 10.0, 11.0, 11.0, 24.0) + count * (W == kNormal && wide ? 0.91e-3 : 0.75e-3);
+    if (event_bytes != 0) {
+      by_wave += 1.9;  // (the bitmap; one in two levels)
+      if (n > 8u * kRowwalkCoarseMost) by_wave = streams <= 4096u ? 37.0 : streams < kSeedAheadMin ? 59.0 : by_wave + 5.0;
+    } else if (static_cast<uint64_t>(n) * sizeof(T1) > (2u << 20) && streams > 32768u) {
+      by_wave *= of(1.4, 1.25, 1.25, 1.25, 1.1);  // (a vector that the L2s hardly hold)
+    }
+    return by_lane < by_wave;
+  }
+  if (use == kScattersSome) {
+    // (without bins the synapses that lanes have at one time meet few outputs in any order, a wave's are neighbours: 200,000 columns of
+    // 16, 10 / 30 % events, 5,000 outputs 49 / 107, by lane 56 / 135, 20,000 outputs 43 / 90, by lane 35 / 74)
+    if (!wide && n <= 10000u && mean >= 11.0 && mean * count >= 2.0e6 && mean * count < kColBinEventMin) return false;
+    return steps * of(0.27, 0.31, 0.33, 0.8, 1.0) < 7.2;
+  }
+  const double synapses = mean * count, outs = 26e-6 * n, slower = 1.0 + 0.1 * undecided;
+  double by_lane;
+  if (synapses < 131072.0) {  // (no bins)
+    by_lane = of(16.0, 13.0, 14.5, 15.0, 16.5) + of(0.28, 0.34, 0.41, 0.82, 1.35) * slower * steps;
+  } else if (streams <= (wide ? 16384u : 32768u)) {
+    by_lane = of(21.0, 19.0, 20.0, 22.0, 22.0) + outs + of(0.42, 0.43, 0.56, 0.92, 1.55) * slower * steps;
+  } else {
+    const double step = of(wide ? 0.85 : 0.55, 0.62, 1.08, 1.17, 2.95) * slower;
+    by_lane = of(wide ? 26.0 : 22.5, 22.0, 26.0, 24.0, 36.0) + (wide && n > 16384u ? 7.0 : 0.0) + outs + 45e-6 * count + step * std::fmax(1.0, count / 220e3) * steps;
+  }
+  double by_wave;
+  if (synapses < 1048576.0) {
+    const double begin = streams <= 4096u ? of(20.0, 18.5, 18.5, 18.5, 19.5) : wide ? 33.0 : of(22.0, 20.5, 20.5, 20.5, 20.5);
+    const double each = n <= 16384u ? (wide ? 0.05e-3 : 0.06e-3) : wide ? 0.035e-3 : 0.04e-3;  // (fewer outputs: more atomics to one)
+    by_wave = std::fmax(begin + each * synapses, 12.0 + 0.79e-3 * count + 0.025e-3 * synapses);
+  } else {
+    by_wave = 0.75 * outs + (streams <= 32768u ? (wide ? 42.0 : 29.0) + 0.35e-3 * count + 0.06 * mean : (wide ? 16.0 : 10.0) + 0.9e-3 * count + mean * (streams <= 98304u ? 0.14 : 4e-6 * count));
+  }
   return by_lane < by_wave;
 }
 
@@ -928,7 +978,7 @@ void launch_rowwalk(hipStream_t stream, const VT *in, T1 *out, uint32_t n_out, u
                     double log_p, T1 wa, T1 wb) {
   if (n_out == 0) return;
   const SkipParams sp = make_skip_params(log_p);
-  if (streams_by_lane<T1, W>(n_out, n_in, log_p, sp, kGathers)) {
+  if (streams_by_lane<T1, W>(n_out, n_in, log_p, sp, kGathers, IN == kInEvent ? n_in * sizeof(VT) : 0)) {
     hipLaunchKernelGGL((jitconn_rows_by_lane_kernel<T1, VT, IN, W>), dim3(div_up(n_out, kWave)), dim3(kWave), 0, stream, in,
                        out, n_out, n_in, seed, sp, wa, wb, kLaneWords);
     return;
@@ -993,7 +1043,7 @@ void launch_colwalk(hipStream_t stream, const VT *in, T1 *out, uint32_t n_out, u
   const double full = static_cast<double>(n_in) * static_cast<double>(n_out) * p_conn;
   const SkipParams sp = make_skip_params(log_p);
   const bool by_lane = (IN == kInDense || n_in >= 2048) && streams_by_lane<T1, W>(n_in, n_out, log_p, sp, IN == kInDense ? kScatters : kScattersSome);
-  const bool bins = n_win <= kBinMaxWindows && full >= (IN == kInEvent ? 1.0e7 : by_lane ? 131072.0 : 1048576.0);
+  const bool bins = n_win <= kBinMaxWindows && full >= (IN == kInEvent ? kColBinEventMin : by_lane ? 131072.0 : 1048576.0);
   // Event input and fewer pairs: the same list of active columns and the same seeding on the vector unit, but
   // the walk adds its pairs to `out` with atomics.  (A wave that seeds its own stream spends 2 us of the CU's one
   // scalar unit on it: with 200,000 active columns of ten synapses each the walk without a list took 1.2 ms.)
@@ -1288,6 +1338,24 @@ extern "C" int bpl_selfcheck_jitconn_rowwalk(bpl_stream_t stream, const uint8_t 
   hipLaunchKernelGGL(kernel, dim3(groups), dim3(1024), lds, s, events, out, n_out, n_in, seed, make_skip_params(log_p),
                      0.0f, 0.0f, counters ? counters + kWalkCounters : nullptr, static_cast<uint32_t *>(rings));
   return check_launch(name) ? 0 : 1;
+}
+
+extern "C" int bpl_selfcheck_jitconn_by_lane(uint32_t weights, uint32_t value_bytes, uint32_t streams, uint32_t n, double log_p,
+                                             uint32_t use, uint32_t event_bytes) {
+  if (weights > 2u || (value_bytes != 4u && value_bytes != 8u) || use > 2u) {
+    set_error("bpl_selfcheck_jitconn_by_lane: no such weights, values or use");
+    return -1;
+  }
+  auto ask = [&](auto value, auto kind) {
+    return streams_by_lane<decltype(value), decltype(kind)::value>(streams, n, log_p, make_skip_params(log_p), static_cast<StreamUse>(use),
+                                                                 static_cast<uint64_t>(event_bytes) * n);
+  };
+  auto of = [&](auto value) {
+    return weights == 0u ? ask(value, std::integral_constant<int, kHomo>())
+                         : weights == 1u ? ask(value, std::integral_constant<int, kUniform>())
+                                         : ask(value, std::integral_constant<int, kNormal>());
+  };
+  return value_bytes == 4u ? of(0.0f) : of(0.0);
 }
 
 #define BPL_DEFINE(name, ...)                                                                      \

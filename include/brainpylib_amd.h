@@ -240,6 +240,14 @@ int bpl_selfcheck_jitconn_trust(bpl_stream_t stream, uint32_t seed, uint64_t n_d
 int bpl_selfcheck_jitconn_rowwalk(bpl_stream_t stream, const uint8_t *events, float *out, uint32_t n_out, uint32_t n_in,
                                   uint32_t seed, double log_p, uint32_t polls, uint32_t groups, int counter);
 
+/* Which of the two walks the jitconn matvec operators choose (no counterpart in the reference): 1 if a lane walks a
+ * stream, 0 if a wave does, -1 with an error for what there is not.  `weights` 0 homogeneous, 1 uniform, 2 normal;
+ * `value_bytes` 4 or 8; `streams` generators over `n` places each; `use` 0 for a stream per output, 1 for a stream per
+ * element of a dense vector, 2 for one per event (of at least 2,048 inputs); `event_bytes` the size of an event where
+ * the outputs read events, else 0.  No device is touched. */
+int bpl_selfcheck_jitconn_by_lane(uint32_t weights, uint32_t value_bytes, uint32_t streams, uint32_t n, double log_p,
+                                  uint32_t use, uint32_t event_bytes);
+
 /* ------------------------------------------------------------------------------------------
  * event_csr_matvec  (lib/gpu_event_csr_matvec.cu:222-260; launchers :148-217)
  *   buffers = [data, indices, indptr, events, out]

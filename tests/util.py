@@ -103,3 +103,19 @@ def batched_csr(shape, mean, batch, seed, dtype=np.float32):
     indptr.append(ip)
     data.append(rng.standard_normal(ix.shape[0]).astype(dtype))
   return np.stack(data), np.stack(indices), np.stack(indptr)
+
+
+def jitconn_by_lane(weights, value_bytes, streams, n, conn_prob, use=0, event_bytes=0):
+  """Whether a lane walks a stream of a jitconn matvec (weights 0 homogeneous, 1 uniform, 2 normal or their names; use 0: a
+  stream per output, 1: per element of a dense vector, 2: per event; event_bytes: size of an event that outputs read)."""
+  import ctypes
+
+  import numpy as np
+
+  from brainpylib_amd import _lib
+  check = _lib.lib().bpl_selfcheck_jitconn_by_lane
+  check.argtypes = [ctypes.c_uint32] * 4 + [ctypes.c_double] + [ctypes.c_uint32] * 2
+  weights = {"homo": 0, "uniform": 1, "normal": 2}.get(weights, weights)
+  got = check(weights, value_bytes, streams, n, float(np.log1p(-conn_prob)), use, event_bytes)
+  assert got in (0, 1), _lib.last_error()
+  return got == 1
