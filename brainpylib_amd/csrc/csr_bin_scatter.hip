@@ -942,7 +942,14 @@ __global__ __launch_bounds__(kBinThreads, 8) __attribute__((amdgpu_num_sgpr(80))
             const uint32_t slot = s_base[w] + i;
             if (slot < cap) {
               const uint64_t at = static_cast<uint64_t>(w * kSubRuns + sub) * cap + slot;
-              if (HETER) {
+              if constexpr (HETER && sizeof(F) == 8) {
+                // (one store of 16 bytes, those between the two among them: of 12 it is two stores, and lines that memory has to
+                // complete; with the loads that the adding kernel makes of them, 1.2e7 pairs, 100,000 columns, whole call 132.5 -> 109.5 us)
+                typedef uint32_t Whole __attribute__((ext_vector_type(4)));
+                const F v = s_val[i];
+                Whole o = {rel, 0u, static_cast<uint32_t>(__double2loint(v)), static_cast<uint32_t>(__double2hiint(v))};
+                *reinterpret_cast<Whole *>(pairs + at) = o;
+              } else if constexpr (HETER) {
                 BinPair<F> o;
                 o.rel = rel, o.val = s_val[i];
                 pairs[at] = o;
@@ -1261,7 +1268,10 @@ __global__ __launch_bounds__(kBinThreads) void add_window_runs_kernel(F *__restr
   // that the compiler can wait for one step's loads while the next one's are on their way.  Which run a step lies in is
   // found once for the wave, on the scalar unit: looked up pair by pair it took 20 vector instructions each (98 windows of
   // 51,000 pairs: 10.6 us, now 9.0; one weight, 98 workgroups, the whole call 47 -> 36).
-  using Item = typename std::conditional<heter, BinPair<F>, uint32_t>::type;  // (one weight: a run holds columns only)
+  constexpr bool whole = heter && sizeof(F) == 8;
+  typedef uint32_t Whole __attribute__((ext_vector_type(4)));  // (a pair of doubles in one load)
+  using Item = typename std::conditional<whole, Whole, typename std::conditional<heter, BinPair<F>, uint32_t>::type>::type;  // (one
+                                                                                           // weight: a run holds columns only)
   const Item *runs = reinterpret_cast<const Item *>(pairs) + static_cast<uint64_t>(b) * kSubRuns * cap;
   struct Step {
     Item e[U];
@@ -1312,9 +1322,13 @@ __global__ __launch_bounds__(kBinThreads) void add_window_runs_kernel(F *__restr
     __syncthreads();
     walk([&](const Step &st) {
 #pragma unroll
-      for (uint32_t u = 0; u < U; ++u)
-        if (u * kWave + lane < st.left && st.e[u].rel - r0 < width)
-          atomicAdd(&window[st.e[u].rel - r0], static_cast<double>(st.e[u].val));  // (wraps below r0)
+      for (uint32_t u = 0; u < U; ++u) {
+        uint32_t rel;
+        double val;
+        if constexpr (whole) rel = st.e[u].x, val = __hiloint2double(static_cast<int>(st.e[u].w), static_cast<int>(st.e[u].z));
+        else rel = st.e[u].rel, val = static_cast<double>(st.e[u].val);
+        if (u * kWave + lane < st.left && rel - r0 < width) atomicAdd(&window[rel - r0], val);  // (wraps below r0)
+      }
     });
     __syncthreads();
     for (uint32_t i = tid; i < width; i += kBinThreads) {
