@@ -708,7 +708,9 @@ constexpr uint32_t kExactRows = 4 * kBinThreads;
 // 7 the rows' nonzeros, 4 the copy-out, the rest ranks, scan, reservation and sort between the three barriers of a round.
 // The nonzeros of a row mostly come in the order of their columns: runs of a wave's lanes meet in one window.  Their first
 // lane takes the ranks of the run; lane by lane their atomics on one counter took turns (4.8e6 pairs of rows of
-// 400 over five windows 33 -> 20 us).
+// 400 over five windows 33 -> 20 us).  Where a row has few nonzeros to a window that only costs: by runs from three on (whole calls,
+// lane by lane / by runs: 3e6 pairs of rows of 200, 500,000 columns in 123 windows, 31.3 / 32.9 us; rows of 300 on average, log-normal, in
+// 92 windows, where the longer ones hold most, 25.6 / 24.2; 5e6 of 1,600 in 98 38.4 / 34.2).
 //
 // (At most 80 scalar registers: measured on this device, a 1,024-thread workgroup whose waves hold
 // 81..96 of them is alone on its CU, as it would be with more than 64 vector registers; the
@@ -717,8 +719,8 @@ template <typename F, bool HETER, typename I>
 __global__ __launch_bounds__(kBinThreads, 8) __attribute__((amdgpu_num_sgpr(80))) void bin_active_rows_kernel(
     const F *__restrict__ data, const I *__restrict__ indices, const I *__restrict__ indptr,
     uint32_t n_row, const uint32_t *__restrict__ active_count, const uint2 *__restrict__ active_list,
-    uint32_t list_cap, const uint32_t *__restrict__ active_colbase, uint32_t entries, F *__restrict__ y, uint32_t shift,
-    uint32_t cap, BinPair<F> *__restrict__ pairs, uint32_t *__restrict__ fill) {
+    uint32_t list_cap, const uint32_t *__restrict__ active_colbase, uint32_t entries, uint32_t row_cols, F *__restrict__ y,
+    uint32_t shift, uint32_t cap, BinPair<F> *__restrict__ pairs, uint32_t *__restrict__ fill) {
   __shared__ uint32_t s_ptr[kTileRows + 1];     // nonzeros of the tile's rows before row k
   __shared__ uint32_t s_start[kTileRows];       // first nonzero of row k in the matrix
   __shared__ uint32_t s_colbase[kTileRows];     // added to row k's columns (batched calls: batch entry * n_col)
@@ -810,6 +812,8 @@ __global__ __launch_bounds__(kBinThreads, 8) __attribute__((amdgpu_num_sgpr(80))
   lo = uniform(lo), hi = uniform(hi), skip = uniform(skip), end = uniform(end);
   if (tid < kMaxWindows) s_cnt[tid] = 0;
   const F w_homo = HETER ? F(0) : data[0];
+  // the nonzeros that a row has to a window
+  const bool by_runs = static_cast<uint64_t>(nnz / n_row) << shift >= 3ull * row_cols;
   // homogeneous weight: a run holds the pairs' columns only, `cap` of them
   uint32_t *run_columns = reinterpret_cast<uint32_t *>(pairs);
 
@@ -893,18 +897,23 @@ __global__ __launch_bounds__(kBinThreads, 8) __attribute__((amdgpu_num_sgpr(80))
         for (int u = 0; u < U; ++u) ncol[u] = 0xffffffffu, nval[u] = F(0);
         if (base + step < seg_end) fetch(base + step, ncol, nval);
         uint32_t rank[U];
+        if (by_runs) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-          const uint32_t w = col[u] != 0xffffffffu ? col[u] >> shift : kMaxWindows;
-          const uint32_t prev = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(
-              static_cast<int>(~w), static_cast<int>(w), 0x138 /* wave_shr:1 */, 0xf, 0xf, false));
-          const uint64_t heads = __builtin_amdgcn_ballot_w64(w != prev);
-          const uint32_t off = static_cast<uint32_t>(__builtin_clzll(heads << (kWave - 1u - lane)));  // (lane 0 is a head)
-          const uint64_t behind = (heads >> lane) >> 1;
-          uint32_t taken = 0;
-          if (off == 0u && w != kMaxWindows)
-            taken = atomicAdd(&s_cnt[w], behind ? static_cast<uint32_t>(__builtin_ctzll(behind)) + 1u : kWave - lane);
-          rank[u] = static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(static_cast<int>(4u * (lane - off)), static_cast<int>(taken))) + off;
+          for (int u = 0; u < U; ++u) {
+            const uint32_t w = col[u] != 0xffffffffu ? col[u] >> shift : kMaxWindows;
+            const uint32_t prev = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(
+                static_cast<int>(~w), static_cast<int>(w), 0x138 /* wave_shr:1 */, 0xf, 0xf, false));
+            const uint64_t heads = __builtin_amdgcn_ballot_w64(w != prev);
+            const uint32_t off = static_cast<uint32_t>(__builtin_clzll(heads << (kWave - 1u - lane)));  // (lane 0 is a head)
+            const uint64_t behind = (heads >> lane) >> 1;
+            uint32_t taken = 0;
+            if (off == 0u && w != kMaxWindows)
+              taken = atomicAdd(&s_cnt[w], behind ? static_cast<uint32_t>(__builtin_ctzll(behind)) + 1u : kWave - lane);
+            rank[u] = static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(static_cast<int>(4u * (lane - off)), static_cast<int>(taken))) + off;
+          }
+        } else {
+#pragma unroll
+          for (int u = 0; u < U; ++u) rank[u] = col[u] != 0xffffffffu ? atomicAdd(&s_cnt[col[u] >> shift], 1u) : 0u;
         }
         __syncthreads();
         if (tid < kWave) {  // two windows per lane: offsets within the round, room in the windows' runs
@@ -1541,10 +1550,10 @@ bool bin_event_scatter(hipStream_t stream, const F *data, bool heter, const I *i
   const uint32_t producers = 2u * num_cu;
   if (heter)
     hipLaunchKernelGGL((bin_active_rows_kernel<F, true, I>), dim3(producers), dim3(kBinThreads), 0, stream, data, indices,
-                       indptr, n_row, active_count, active_list, list_cap, active_colbase, entries, y, shift, cap, pairs, fill);
+                       indptr, n_row, active_count, active_list, list_cap, active_colbase, entries, n_col / entries, y, shift, cap, pairs, fill);
   else
     hipLaunchKernelGGL((bin_active_rows_kernel<F, false, I>), dim3(producers), dim3(kBinThreads), 0, stream, data, indices,
-                       indptr, n_row, active_count, active_list, list_cap, active_colbase, entries, y, shift, cap, pairs, fill);
+                       indptr, n_row, active_count, active_list, list_cap, active_colbase, entries, n_col / entries, y, shift, cap, pairs, fill);
   hipLaunchKernelGGL(add_kernel, dim3(n_win * slices * parts), dim3(kBinThreads), lds, stream, y, n_col, shift,
                      lds_shift, parts, cap, pairs, fill, active_count, data, indices, active_list, active_colbase);
   return true;

@@ -214,7 +214,6 @@ def test_event_gather_lanes_for_few_and_for_many_rows(cuda, oracle_mod, n_row, n
     assert_close_reordered(got, want, mag, dtype, what="event gather, few and many rows")
 
 
-
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 def test_gather_long_rows_that_begin_at_different_steps(cuda, oracle_mod, dtype):
   # rows of 384 nonzeros or more take a wave each, in steps of 512 (float64: the same walk), and begin at a full
@@ -581,6 +580,30 @@ def test_event_scatter_shares_the_listed_rows_nonzeros(cuda, listed, columns, dt
     got = bpl.event_csr_matvec(np.array([2.0], dtype=dtype), indices.astype(np.uint32), indptr, kind, shape=(n_row, n_col),
                                transpose=True).cpu().numpy()
     assert np.array_equal(got, 2.0 * np.bincount(indices[ev[rows]], minlength=n_col))
+
+
+@pytest.mark.parametrize("columns", ["sorted", "descending", "random", "two"])
+@pytest.mark.parametrize("mean", [292, 293, 294, 700])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_event_scatter_ranks_of_a_round(cuda, columns, mean, dtype):
+  # 50,001 columns are 98 windows of 512: from 293 nonzeros a row on (three to a window) a wave's pairs take their ranks by runs of
+  # lanes, below lane by lane.  Small whole weights: every order of the additions gives the same sums.
+  n_row, n_col = 605, 50_001
+  rng = np.random.default_rng(mean)
+  indptr = (np.arange(n_row + 1) * mean).astype(np.uint32)
+  indices = rng.integers(0, n_col, (n_row, mean))
+  if columns == "two":
+    indices = np.where(indices % 2, 511, n_col - 1)
+  elif columns != "random":
+    indices = np.sort(indices, axis=1)[:, ::1 if columns == "sorted" else -1]
+  indices = indices.reshape(-1).astype(np.uint32)
+  data = rng.integers(-8, 9, indices.shape[0]).astype(dtype)
+  ev = rng.random(n_row) < 0.9
+  on = np.repeat(ev, mean)
+  got = bpl.event_csr_matvec(data, indices, indptr, ev, shape=(n_row, n_col), transpose=True).cpu().numpy()
+  assert np.array_equal(got, np.bincount(indices[on], weights=data[on], minlength=n_col))
+  got = bpl.event_csr_matvec(np.array([2.0], dtype), indices, indptr, ev, shape=(n_row, n_col), transpose=True).cpu().numpy()
+  assert np.array_equal(got, 2.0 * np.bincount(indices[on], minlength=n_col))
 
 
 def test_scatter_through_the_active_row_list(cuda, oracle_mod):
