@@ -194,14 +194,19 @@ def test_ragged_rows_and_all_row_length_modes(cuda, oracle_mod):
     assert_close_reordered(got, want, mag, what="event scatter mean %d" % mean)
 
 
+@pytest.mark.parametrize("even", [False, True])
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 @pytest.mark.parametrize("n_row,n_col,mean", [(4095, 5000, 200), (4097, 5000, 200), (300, 131_072, 383), (40_959, 3000, 192),
-                                              (40_961, 3000, 192), (131_072, 700, 96), (131_071, 700, 97)])
-def test_event_gather_lanes_for_few_and_for_many_rows(cuda, oracle_mod, n_row, n_col, mean, dtype):
-  # groups of 8, 16 or 32 lanes for a row by the number of rows: log-normal rows on either side of each line, empty
-  # ones and rows of a step and one more or less, weights per nonzero and one weight
+                                              (40_961, 3000, 192), (131_072, 700, 96), (131_071, 700, 97), (24_576, 3000, 192),
+                                              (24_577, 3000, 192), (32_768, 3000, 192), (32_769, 3000, 192)])
+def test_event_gather_lanes_for_few_and_for_many_rows(cuda, oracle_mod, n_row, n_col, mean, even, dtype):
+  # groups of 8, 16 or 32 lanes for a row by the number of rows and, from 24,577 to 32,768 of them, by whether 64 of them look even:
+  # log-normal and even rows on either side of each line, empty ones and rows of a step and one more or less, weights per nonzero and
+  # one weight
   rng = np.random.default_rng(n_row + mean)
   counts = np.minimum(rng.lognormal(np.log(mean) - 0.32, 0.8, size=n_row).astype(np.int64), n_col // 2)
+  if even:
+    counts[:] = rng.integers(mean - 30, mean + 31, n_row)
   counts[:7] = (0, 1, 127, 128, 129, 255, 257)
   counts[7:] += max(0, int(np.ceil((mean * n_row - counts.sum()) / (n_row - 7))))
   indices, indptr = synth.counted_csr(counts, n_col, seed=n_row)
