@@ -1483,10 +1483,9 @@ __global__ __launch_bounds__(1024, (MODE == kEvent && BITS == 1) ? 8 : 4) void c
     // events: 3,000 rows of 300 12.7 / 9.2 and 26 / 16 us, 20,000 of 220 14.1 / 12.3 and 37.5 / 28.8, 40,000 of 200 20.5 / 16.6 and 54 /
     // 42, 60,000 of 200 23.5 / 21.2 but at 1 % 17.4 / 19.1; one weight 3,000 of 300 10.3 / 9.3 and 17.2 / 12.3, 9,000 of 250 9.3 / 10.1;
     // 8 / 16 lanes: 200,000 of 200 73 / 64 and 126 / 121, of 100 37 / 30 and 57 / 54, 70,000 of 100 at 1 % 12.5 / 13.2, one weight
-    // 400,000 of 100 41.7 / 44.7.  Wide bitmaps lose: 30,000 rows of 380, 500,000 columns, at 1 % 24.3 / 29.5.  Even rows that nearly fill
-    // the groups of eight lanes once leave none idle (the look at them takes 0.5 us): 30,000 of 250 at 1 / 10 % 14.3 / 15.7 and 16.8 / 17.4, 23,000 of 300 15.7 /
-    // 13.0 and 17.1 / 15.5, log-normal ones of 300
-    // 30,000 44 / 35 and 51 / 42.  At 0.5 % events 16 lanes lose where the mean is 112 to 160: 200,000 of 145 33.5 / 35.9, at 2 % 40.0 / 39.4.)
+    // 400,000 of 100 41.7 / 44.7, at 0.5 % events 200,000 of 145 33.5 / 35.9.  Wide bitmaps lose: 30,000 rows of 380, 500,000 columns, at 1 %
+    // 24.3 / 29.5.  Even rows that nearly fill the groups of eight lanes once leave none idle: 30,000 of 250 at 1 / 10 % 13.8 / 15.7 and
+    // 16.3 / 17.4, but log-normal ones of 300 44 / 35 and 51 / 42; the look at them takes 0.5 us.)
     else if (MODE == kEvent && mean >= 192u && n_col <= 131072u && n_row < (HETER ? 40960u : 4096u) &&
              !(HETER && n_row > 24576u && n_row <= 32768u && rows_look_even(indptr, n_row, mean))) { gpb = blockDim.x / 32; hub_len = hub_of_group(4 * 32); gather_rows<F, VT, HETER, MODE, BITS, 32, 4>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }
     else if (MODE == kEvent && HETER && mean >= 96u && n_col <= 131072u && n_row >= 131072u) { gpb = blockDim.x / 16; hub_len = hub_of_group(8 * 16); gather_rows<F, VT, HETER, MODE, BITS, 16, 8>(data, indices, indptr, x, y, n_row, s_bits, coarse_g, hub_len); }

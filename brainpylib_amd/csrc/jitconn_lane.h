@@ -58,11 +58,11 @@ struct LaneGenerator {
 
 // Walks stream std::mt19937{stream_seed} of each lane over [0, n): calls f(index, weight, valid) with the whole wave converged,
 // one synapse of every lane that has one (`valid`; the others get index 0) per call, in the order of each stream.  Returns the lanes
-// whose stream needs more than `words` words (at most kLaneWords): they gave what lies in front of their position `pos`.
+// whose stream needs more than kLaneWords words: they gave what lies in front of their position `pos`.
 // The skips fit: sp.narrow and n <= 0xf0000000, so that a position never leads around 2^32.
 template <typename T1, int W, typename F>
 __device__ __forceinline__ uint64_t walk_lane_streams(uint32_t stream_seed, bool alive, uint32_t n, const SkipParams &sp,
-                                                      T1 wa, T1 wb, uint32_t words, uint32_t &pos, F &&f) {
+                                                      T1 wa, T1 wb, uint32_t &pos, F &&f) {
   LaneGenerator gen(stream_seed);
   {
     const uint32_t lo = gen.raw<false>(), hi = gen.word<false>();
@@ -125,8 +125,8 @@ __device__ __forceinline__ uint64_t walk_lane_streams(uint32_t stream_seed, bool
       }
     }
   };
-  walk(std::false_type(), words < kLaneFirst ? words : kLaneFirst);
-  walk(std::true_type(), words);
+  walk(std::false_type(), kLaneFirst);
+  walk(std::true_type(), kLaneWords);
   return left;
 }
 

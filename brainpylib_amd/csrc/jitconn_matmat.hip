@@ -49,8 +49,8 @@ __global__ __launch_bounds__(kPrepareThreads) void matmat_prepare_kernel(const T
     const int lane = lane_id();
     if (threadIdx.x < kWave)
       mt_seed_batch<true>(reinterpret_cast<uint32_t *>(s_mem), lane, seed + base + static_cast<uint32_t>(lane),
-                               states + static_cast<size_t>(base) * kMtN,
-                               count - base < static_cast<uint32_t>(kWave) ? count - base : static_cast<uint32_t>(kWave));
+                          states + static_cast<size_t>(base) * kMtN,
+                          count - base < static_cast<uint32_t>(kWave) ? count - base : static_cast<uint32_t>(kWave));
     return;
   }
   T(*tile)[kTile + 1] = reinterpret_cast<T(*)[kTile + 1]>(s_mem);

@@ -290,7 +290,7 @@ __global__ __launch_bounds__(1024, (FORM == 2 || (W == kNormal && sizeof(T1) == 
 template <typename T1, typename VT, int IN, int W>
 __global__ __launch_bounds__(kWave, 8) void jitconn_rows_by_lane_kernel(const VT *__restrict__ in, T1 *__restrict__ out,
                                                                         uint32_t n_out, uint32_t n_in, uint32_t seed,
-                                                                        SkipParams skips, T1 wa, T1 wb, uint32_t words) {
+                                                                        SkipParams skips, T1 wa, T1 wb) {
   __shared__ __attribute__((aligned(8))) uint32_t st[StreamLds<T1, W, true>::words];
   const int lane = lane_id();
   const uint32_t o = blockIdx.x * kWave + static_cast<uint32_t>(lane);
@@ -325,7 +325,7 @@ __global__ __launch_bounds__(kWave, 8) void jitconn_rows_by_lane_kernel(const VT
   };
   auto result = [&]() { return (IN == kInEvent && W == kHomo) ? static_cast<T1>(cnt) : static_cast<T1>(total()); };
   uint32_t pos;
-  uint64_t longer = walk_lane_streams<T1, W>(seed + o, o < n_out, n_in, skips, wa, wb, words, pos, [&](uint32_t idx, T1 w, bool valid) {
+  uint64_t longer = walk_lane_streams<T1, W>(seed + o, o < n_out, n_in, skips, wa, wb, pos, [&](uint32_t idx, T1 w, bool valid) {
     use(late_valid, late, late_w);
     late = in[idx], late_w = w, late_valid = valid;
   });
@@ -457,8 +457,7 @@ __global__ __launch_bounds__(1024) void collect_active_columns_kernel(const VT *
 // [0, n_list) of a list: column list_col[k] with value list_val[k] (event input: the active
 // columns), or, without a list, column first + k with value in[first + k] (dense input).  Waves
 // take entries round robin over the whole grid, so every wave walks the same number of streams.
-// Not FUSED: the generators of the first n_seeded entries were seeded ahead on the vector unit (`states`);
-// a wave seeding its own generator does it on the CU's one scalar unit, about 2 us each, and a
+// A wave seeding its own generator does it on the CU's one scalar unit, about 2 us each, and a
 // CU's waves queue up for it.  A pair for output window b (2^shift outputs) of workgroup p goes to
 // place (p * n_win + b) * cap + position of the bins; the positions continue from `counts` (zero before
 // the first launch of a call), so that a call may be split into several launches; a pair that finds
@@ -470,18 +469,18 @@ constexpr int kColBinThreads = 1024;  // 16 waves share one set of bins: 4 times
 constexpr size_t kColBinBytesMax = static_cast<size_t>(3) << 30;  // bins of the dense column walk (scratch memory)
 
 //
-// FUSED: the generators are seeded inside this kernel instead, as in the row walk: workgroup p takes the
+// So the generators are seeded inside this kernel on the vector unit, as in the row walk: workgroup p takes the
 // entries p, p + G, p + 2 G, ... (G workgroups), 64 of them are a batch, its waves take (batch, entry) tasks
 // from a counter in LDS, and the wave that takes the first entry of batch j first seeds batch j + 1 on the
 // vector unit (lane per stream) into slot (j + 1) % 3 of the workgroup's ring of seeded states in device
 // memory (`states`, kFuseRingBytes per workgroup), which the other waves read back from the L2.  Only the
-// first batch of a workgroup is waited for; n_seeded is not used.
-template <typename T1, typename VT, int IN, int W, bool FUSED>
+// first batch of a workgroup is waited for.
+template <typename T1, typename VT, int IN, int W>
 __global__ __launch_bounds__(kColBinThreads, sizeof(T1) == 4 ? 8 : 4) void jitconn_colwalk_bins_kernel(
     const VT *__restrict__ in, T1 *__restrict__ out, uint32_t n_out, uint32_t seed, SkipParams skips, T1 wa, T1 wb,
     uint32_t first, uint32_t n_list_host, const uint32_t *__restrict__ n_list_dev,
     const uint32_t *__restrict__ list_col, const T1 *__restrict__ list_val, uint32_t *states,
-    uint32_t n_seeded, uint32_t n_win, uint32_t shift, uint32_t cap, void *__restrict__ pairs, uint64_t n_pairs,
+    uint32_t n_win, uint32_t shift, uint32_t cap, void *__restrict__ pairs, uint64_t n_pairs,
     uint32_t packed, uint32_t *__restrict__ counts) {
   constexpr int kWaves = kColBinThreads / kWave;
   constexpr bool kShort = W == kNormal;  // (sixteen waves' states and queues within 64 KB of static LDS)
@@ -568,67 +567,62 @@ __global__ __launch_bounds__(kColBinThreads, sizeof(T1) == 4 ? 8 : 4) void jitco
     }, loaded);
   };
 
-  if constexpr (!FUSED) {
-    for (uint32_t k = wave * gridDim.x + p; k < n_list; k += gridDim.x * kWaves)
-      walk_entry(k, (k < n_seeded) ? states + static_cast<size_t>(k) * kMtN : nullptr, NoLoadHook());
-  } else {
-    // this workgroup's entries: p + i * G for i < mine
-    const uint32_t mine = n_list > p ? (n_list - p + gridDim.x - 1u) / gridDim.x : 0u;
-    const uint32_t batches = (mine + kFuseBatch - 1u) / kFuseBatch;
-    uint32_t *ring = states + static_cast<size_t>(p) * kFuseSlots * kFuseBatch * kMtN;
-    auto seed_batch = [&](uint32_t j) {
-      const uint32_t slot = j % kFuseSlots;
-      const uint32_t i = j * kFuseBatch + static_cast<uint32_t>(lane);
-      uint32_t col = 0;
-      if (i < mine) {
-        const uint32_t k = p + i * gridDim.x;
-        col = list_col != nullptr ? list_col[k] : first + k;
-      }
-      const uint32_t left = mine - j * kFuseBatch;
-      uint32_t *const to = ring + static_cast<size_t>(slot) * kFuseBatch * kMtN;
-      // (a short last batch: the quick form, for it is soon waited for; not the second of two with normal weights, whose walk of the
-      // first lasts longer than the seeding: 65,000 columns of 20 116.2 -> 113.0 us)
-      if (left >= kFuseBatch || (W == kNormal && j != 0u && batches == 2u)) mt_seed_batch(st, lane, seed + col, to, left);
-      else mt_seed_batch<true>(st, lane, seed + col, to, left);
-      __hip_atomic_store(&s_ready[slot], j + 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
-    };
-    if (wave == 0 && batches != 0) seed_batch(0);
-    // (One batch: the others wait at the barrier, where they take no issue slots from the wave that seeds.  More: the wave that
-    // takes the first entry seeds batch 1 beside it; 1,000,000 streams of 18 synapses, both walks, 1,908 us, behind the barrier 1,950.)
-    if (batches <= 1u) __syncthreads();
-    for (;;) {
-      // (every lane adds one: the counter advances by 64 per task, any lane's old value / 64 is the task)
-      const uint32_t t = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(
-                             static_cast<int>(atomicAdd(&s_task, 1u)))) / kWave;
-      const uint32_t j = t / kFuseBatch, r = t % kFuseBatch;
-      if (j >= batches) break;
-      if (r == 0 && j + 1 < batches) {
-        // slot (j + 1) % 3 last held batch j - 2: (j + 1) / 3 batches have used it, 64 loads each
-        const uint32_t slot = (j + 1u) % kFuseSlots, need = ((j + 1u) / kFuseSlots) * kFuseBatch;
-        bool free_ = false;
-        for (uint32_t spin = 0; spin < kFuseSpin && !free_; ++spin) {
-          free_ = __hip_atomic_load(&s_loaded[slot], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) >= need;
-          if (!free_) __builtin_amdgcn_s_sleep(2);
-        }
-        if (free_) seed_batch(j + 1u);
-        else __hip_atomic_store(&s_ready[slot], kFuseNotSeeded | (j + 2u), __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
-      }
-      const uint32_t slot = j % kFuseSlots;
-      uint32_t flag = 0;
-      for (uint32_t spin = 0; spin < kFuseSpin; ++spin) {
-        flag = __hip_atomic_load(&s_ready[slot], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
-        if ((flag & ~kFuseNotSeeded) >= j + 1u) break;
-        __builtin_amdgcn_s_sleep(8);
-      }
-      if ((flag & ~kFuseNotSeeded) < j + 1u) flag = kFuseNotSeeded;
-      const uint32_t *pre = (flag & kFuseNotSeeded) ? nullptr : ring + (static_cast<size_t>(slot) * kFuseBatch + r) * kMtN;
-      auto loaded = [&]() {
-        if (lane == 0) __hip_atomic_fetch_add(&s_loaded[slot], 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
-      };
-      const uint32_t i = j * kFuseBatch + r;
-      if (i < mine) walk_entry(p + i * gridDim.x, pre, loaded);
-      else loaded();
+  // this workgroup's entries: p + i * G for i < mine
+  const uint32_t mine = n_list > p ? (n_list - p + gridDim.x - 1u) / gridDim.x : 0u;
+  const uint32_t batches = (mine + kFuseBatch - 1u) / kFuseBatch;
+  uint32_t *ring = states + static_cast<size_t>(p) * kFuseSlots * kFuseBatch * kMtN;
+  auto seed_batch = [&](uint32_t j) {
+    const uint32_t slot = j % kFuseSlots;
+    const uint32_t i = j * kFuseBatch + static_cast<uint32_t>(lane);
+    uint32_t col = 0;
+    if (i < mine) {
+      const uint32_t k = p + i * gridDim.x;
+      col = list_col != nullptr ? list_col[k] : first + k;
     }
+    const uint32_t left = mine - j * kFuseBatch;
+    uint32_t *const to = ring + static_cast<size_t>(slot) * kFuseBatch * kMtN;
+    // (a short last batch: the quick form, for it is soon waited for; not the second of two with normal weights, whose walk of the
+    // first lasts longer than the seeding: 65,000 columns of 20 116.2 -> 113.0 us)
+    if (left >= kFuseBatch || (W == kNormal && j != 0u && batches == 2u)) mt_seed_batch(st, lane, seed + col, to, left);
+    else mt_seed_batch<true>(st, lane, seed + col, to, left);
+    __hip_atomic_store(&s_ready[slot], j + 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+  };
+  if (wave == 0 && batches != 0) seed_batch(0);
+  // (One batch: the others wait at the barrier, where they take no issue slots from the wave that seeds.  More: the wave that
+  // takes the first entry seeds batch 1 beside it; 1,000,000 streams of 18 synapses, both walks, 1,908 us, behind the barrier 1,950.)
+  if (batches <= 1u) __syncthreads();
+  for (;;) {
+    // (every lane adds one: the counter advances by 64 per task, any lane's old value / 64 is the task)
+    const uint32_t t = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(
+                           static_cast<int>(atomicAdd(&s_task, 1u)))) / kWave;
+    const uint32_t j = t / kFuseBatch, r = t % kFuseBatch;
+    if (j >= batches) break;
+    if (r == 0 && j + 1 < batches) {
+      // slot (j + 1) % 3 last held batch j - 2: (j + 1) / 3 batches have used it, 64 loads each
+      const uint32_t slot = (j + 1u) % kFuseSlots, need = ((j + 1u) / kFuseSlots) * kFuseBatch;
+      bool free_ = false;
+      for (uint32_t spin = 0; spin < kFuseSpin && !free_; ++spin) {
+        free_ = __hip_atomic_load(&s_loaded[slot], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) >= need;
+        if (!free_) __builtin_amdgcn_s_sleep(2);
+      }
+      if (free_) seed_batch(j + 1u);
+      else __hip_atomic_store(&s_ready[slot], kFuseNotSeeded | (j + 2u), __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    const uint32_t slot = j % kFuseSlots;
+    uint32_t flag = 0;
+    for (uint32_t spin = 0; spin < kFuseSpin; ++spin) {
+      flag = __hip_atomic_load(&s_ready[slot], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
+      if ((flag & ~kFuseNotSeeded) >= j + 1u) break;
+      __builtin_amdgcn_s_sleep(8);
+    }
+    if ((flag & ~kFuseNotSeeded) < j + 1u) flag = kFuseNotSeeded;
+    const uint32_t *pre = (flag & kFuseNotSeeded) ? nullptr : ring + (static_cast<size_t>(slot) * kFuseBatch + r) * kMtN;
+    auto loaded = [&]() {
+      if (lane == 0) __hip_atomic_fetch_add(&s_loaded[slot], 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+    };
+    const uint32_t i = j * kFuseBatch + r;
+    if (i < mine) walk_entry(p + i * gridDim.x, pre, loaded);
+    else loaded();
   }
   __syncthreads();
   if (threadIdx.x < n_win) counts[static_cast<size_t>(threadIdx.x) * gridDim.x + p] = s_cnt[threadIdx.x];
@@ -643,7 +637,7 @@ __global__ __launch_bounds__(kColBinThreads, sizeof(T1) == 4 ? 8 : 4) void jitco
     const VT *__restrict__ in, T1 *__restrict__ out, uint32_t n_out, uint32_t seed, SkipParams skips, T1 wa, T1 wb,
     uint32_t first, uint32_t n_list_host, const uint32_t *__restrict__ n_list_dev,
     const uint32_t *__restrict__ list_col, const T1 *__restrict__ list_val, uint32_t n_win, uint32_t shift, uint32_t cap,
-    void *__restrict__ pairs, uint64_t n_pairs, uint32_t packed, uint32_t *__restrict__ counts, uint32_t words) {
+    void *__restrict__ pairs, uint64_t n_pairs, uint32_t *__restrict__ counts) {
   constexpr uint32_t kWaves = kColBinThreads / kWave;
   constexpr int kStateWords = StreamLds<T1, W, true>::words;
   __shared__ __attribute__((aligned(8))) uint32_t s_state[kWaves * kStateWords];
@@ -653,8 +647,8 @@ __global__ __launch_bounds__(kColBinThreads, sizeof(T1) == 4 ? 8 : 4) void jitco
   if (threadIdx.x < n_win) s_cnt[threadIdx.x] = counts[static_cast<size_t>(threadIdx.x) * gridDim.x + p];
   __syncthreads();
   const uint64_t region = static_cast<uint64_t>(p) * n_win * cap;  // first place of this workgroup's bins
-  unsigned char *const region_val = static_cast<unsigned char *>(pairs) + region * (packed ? sizeof(T1) : sizeof(BinPair<T1>));
-  unsigned char *const region_rel = static_cast<unsigned char *>(pairs) + n_pairs * sizeof(T1) + region * 2u;  // (packed)
+  unsigned char *const region_val = static_cast<unsigned char *>(pairs) + region * sizeof(T1);
+  unsigned char *const region_rel = static_cast<unsigned char *>(pairs) + n_pairs * sizeof(T1) + region * 2u;
   uint32_t *const st = s_state + wave * kStateWords;
   const uint32_t n_list = n_list_dev ? *n_list_dev : n_list_host;
   auto append = [&](uint32_t idx, T1 add, bool valid) {  // (the whole wave)
@@ -674,15 +668,8 @@ __global__ __launch_bounds__(kColBinThreads, sizeof(T1) == 4 ? 8 : 4) void jitco
     if (slot < cap) {
       const uint32_t at = static_cast<uint32_t>(__umul24(b, cap)) + slot;
       const uint32_t rel = idx & ((1u << shift) - 1u);
-      if (packed) {
-        *reinterpret_cast<T1 *>(region_val + at * static_cast<uint32_t>(sizeof(T1))) = add;
-        *reinterpret_cast<uint16_t *>(region_rel + at * 2u) = static_cast<uint16_t>(rel);
-      } else {
-        BinPair<T1> e;
-        e.rel = rel;
-        e.val = add;
-        *reinterpret_cast<BinPair<T1> *>(region_val + at * static_cast<uint32_t>(sizeof(BinPair<T1>))) = e;
-      }
+      *reinterpret_cast<T1 *>(region_val + at * static_cast<uint32_t>(sizeof(T1))) = add;
+      *reinterpret_cast<uint16_t *>(region_rel + at * 2u) = static_cast<uint16_t>(rel);
     } else {
       atomic_add(&out[idx], add);
     }
@@ -699,7 +686,7 @@ __global__ __launch_bounds__(kColBinThreads, sizeof(T1) == 4 ? 8 : 4) void jitco
     }
     auto addend = [&](T1 w, T1 v) { return IN == kInDense ? (W == kHomo ? v : static_cast<T1>(w * v)) : w; };  // (homo: w == 1)
     uint32_t pos;
-    uint64_t longer = walk_lane_streams<T1, W>(seed + col, on, n_out, skips, wa, wb, words, pos,
+    uint64_t longer = walk_lane_streams<T1, W>(seed + col, on, n_out, skips, wa, wb, pos,
                                                [&](uint32_t idx, T1 w, bool valid) { append(idx, addend(w, val), valid); });
     for (; longer != 0; longer &= longer - 1ull) {
       const int of = static_cast<int>(__builtin_ctzll(longer));
@@ -736,7 +723,7 @@ __global__ __launch_bounds__(kSeedThreads) void mt_seed_streams_kernel(uint32_t 
   uint32_t x = seed + first + mine;
   if (ids != nullptr) x = seed + (mine < count ? ids[mine] : 0u);
   mt_seed_batch(s_tile[wave], lane, x, states + static_cast<size_t>(base) * kMtN,
-                              count - base < static_cast<uint32_t>(kWave) ? count - base : static_cast<uint32_t>(kWave));
+                count - base < static_cast<uint32_t>(kWave) ? count - base : static_cast<uint32_t>(kWave));
 }
 
 }  // namespace
@@ -982,7 +969,7 @@ void launch_rowwalk(hipStream_t stream, const VT *in, T1 *out, uint32_t n_out, u
   const SkipParams sp = make_skip_params(log_p);
   if (streams_by_lane<T1, W>(n_out, n_in, log_p, sp, kGathers, IN == kInEvent ? n_in * sizeof(VT) : 0)) {
     hipLaunchKernelGGL((jitconn_rows_by_lane_kernel<T1, VT, IN, W>), dim3(div_up(n_out, kWave)), dim3(kWave), 0, stream, in,
-                       out, n_out, n_in, seed, sp, wa, wb, kLaneWords);
+                       out, n_out, n_in, seed, sp, wa, wb);
     return;
   }
   constexpr bool kEvents = IN == kInEvent;
@@ -1044,7 +1031,8 @@ void launch_colwalk(hipStream_t stream, const VT *in, T1 *out, uint32_t n_out, u
   const double p_conn = -std::expm1(log_p);
   const double full = static_cast<double>(n_in) * static_cast<double>(n_out) * p_conn;
   const SkipParams sp = make_skip_params(log_p);
-  const bool by_lane = (IN == kInDense || n_in >= 2048) && streams_by_lane<T1, W>(n_in, n_out, log_p, sp, IN == kInDense ? kScatters : kScattersSome);
+  // (streams that a lane can draw reach windows of 2^16 outputs at most, which streams_by_lane() has seen to: positions of 16 bits)
+  const bool by_lane = (IN == kInDense || n_in >= 2048) && shift <= 16u && streams_by_lane<T1, W>(n_in, n_out, log_p, sp, IN == kInDense ? kScatters : kScattersSome);
   const bool bins = n_win <= kBinMaxWindows && full >= (IN == kInEvent ? kColBinEventMin : by_lane ? 131072.0 : 1048576.0);
   // Event input and fewer pairs: the same list of active columns and the same seeding on the vector unit, but
   // the walk adds its pairs to `out` with atomics.  (A wave that seeds its own stream spends 2 us of the CU's one
@@ -1106,7 +1094,7 @@ void launch_colwalk(hipStream_t stream, const VT *in, T1 *out, uint32_t n_out, u
         uint32_t *states = reinterpret_cast<uint32_t *>(ws + pair_bytes + count_bytes);
         uint32_t *list_col = list_bytes ? reinterpret_cast<uint32_t *>(ws + pair_bytes + count_bytes + state_bytes) : nullptr;
         T1 *list_val = val_bytes ? reinterpret_cast<T1 *>(ws + pair_bytes + count_bytes + state_bytes + list_bytes) : nullptr;
-        auto walk = jitconn_colwalk_bins_kernel<T1, VT, IN, W, true>;
+        auto walk = jitconn_colwalk_bins_kernel<T1, VT, IN, W>;
         auto walk_lanes = jitconn_columns_by_lane_kernel<T1, VT, IN, W>;
         out_cleared = true;
         if (IN == kInEvent) {
@@ -1116,12 +1104,11 @@ void launch_colwalk(hipStream_t stream, const VT *in, T1 *out, uint32_t n_out, u
           if (by_lane) {
             hipLaunchKernelGGL(walk_lanes, dim3(producers), dim3(kColBinThreads), 0, stream, in, out, n_out, seed, sp, wa,
                                wb, 0u, 0u, static_cast<const uint32_t *>(list_count), static_cast<const uint32_t *>(list_col),
-                               static_cast<const T1 *>(list_val), n_win, shift, cap, pairs, n_pairs, packed ? 1u : 0u, counts,
-                               kLaneWords);
+                               static_cast<const T1 *>(list_val), n_win, shift, cap, pairs, n_pairs, counts);
           } else {
             hipLaunchKernelGGL(walk, dim3(producers), dim3(kColBinThreads), 0, stream, in, out, n_out, seed, sp, wa, wb,
                                0u, 0u, static_cast<const uint32_t *>(list_count), static_cast<const uint32_t *>(list_col),
-                               static_cast<const T1 *>(list_val), states, 0u, n_win, shift, cap, pairs, n_pairs, packed ? 1u : 0u, counts);
+                               static_cast<const T1 *>(list_val), states, n_win, shift, cap, pairs, n_pairs, packed ? 1u : 0u, counts);
           }
         } else {
           // every column, a chunk at a time; the bins are emptied after every `group` chunks (by lane: after every launch)
@@ -1137,11 +1124,11 @@ void launch_colwalk(hipStream_t stream, const VT *in, T1 *out, uint32_t n_out, u
               hipLaunchKernelGGL(walk_lanes, dim3(producers), dim3(kColBinThreads), 0, stream, in, out, n_out, seed, sp, wa,
                                  wb, first, count, static_cast<const uint32_t *>(nullptr),
                                  static_cast<const uint32_t *>(nullptr), static_cast<const T1 *>(nullptr), n_win, shift, cap,
-                                 pairs, n_pairs, packed ? 1u : 0u, counts, kLaneWords);
+                                 pairs, n_pairs, counts);
             } else {
               hipLaunchKernelGGL(walk, dim3(producers), dim3(kColBinThreads), 0, stream, in, out, n_out, seed, sp, wa,
                                  wb, first, count, static_cast<const uint32_t *>(nullptr),
-                                 static_cast<const uint32_t *>(nullptr), static_cast<const T1 *>(nullptr), states, 0u,
+                                 static_cast<const uint32_t *>(nullptr), static_cast<const T1 *>(nullptr), states,
                                  n_win, shift, cap, pairs, n_pairs, packed ? 1u : 0u, counts);
             }
             if (++in_bins == group && at + span < n_in) {

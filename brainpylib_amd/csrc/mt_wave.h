@@ -103,7 +103,7 @@ __device__ __forceinline__ void mt_seed_batch(uint32_t *tile, int lane, uint32_t
   // one, behind its eight steps of the recurrence, so that the chain of multiplications does not wait for
   // the LDS (a wave's LDS operations complete in order: the next round's writes cannot overtake the reads).
   Pair v[4];
-#pragma unroll(SOON ? 3 : 1)
+#pragma unroll (SOON ? 3 : 1)
   for (uint32_t w0 = 0; w0 < kMtN; w0 += 8) {
 #pragma unroll
     for (uint32_t i = 0; i < 8; i += 2) {  // words w0 + i and w0 + i + 1 of stream `lane`

@@ -27,6 +27,7 @@ TWO_PER_CU = [
   (r"jitconn_rowwalk_kernel<\w+, bpl::PackedBits, 0, \d, 2, (true|false)>", "jitconn row walk with the two-level bitmap"),
   (r"jitconn_rowwalk_kernel<float, [\w: ]+, \d, 2, \d, (true|false)>", "jitconn row walk, float normal weights"),
   (r"jitconn_colwalk_bins_kernel<float,", "jitconn column walk into bins, float"),
+  (r"jitconn_columns_by_lane_kernel<float,", "jitconn column walk, a lane to a column, float"),
 ]
 
 
