@@ -206,7 +206,7 @@ def test_event_gather_lanes_for_few_and_for_many_rows(cuda, oracle_mod, n_row, n
   rng = np.random.default_rng(n_row + mean)
   counts = np.minimum(rng.lognormal(np.log(mean) - 0.32, 0.8, size=n_row).astype(np.int64), n_col // 2)
   if even:
-    counts[:] = rng.integers(mean, mean + 31, n_row)
+    counts[:] = rng.integers(mean, min(mean + 30, 383) + 1, n_row)
   counts[:7] = (0, 1, 127, 128, 129, 255, 257)
   counts[7:] += max(0, int(np.ceil((mean * n_row - counts.sum()) / (n_row - 7))))
   indices, indptr = synth.counted_csr(counts, n_col, seed=n_row)

@@ -16,7 +16,7 @@ import torch
 import brainpylib_amd as bpl
 from brainpylib_amd import _lib
 import benchdata as synth
-from util import JIT_SHAPES, assert_close, assert_close_reordered
+from util import JIT_SHAPES, assert_close, assert_close_reordered, jitconn_by_lane
 
 pytestmark = pytest.mark.gpu
 GOLD = os.path.join(os.path.dirname(__file__), "golden")
@@ -373,8 +373,8 @@ def test_matmat_with_generators_seeded_ahead(cuda, oracle_mod, n):
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 @pytest.mark.parametrize("n_out,n_in,p", [(5001, 900, 0.001), (10_000, 4000, 0.0025), (70_063, 3, 1.0), (70_063, 40, 0.5), (140_000, 1500, 0.04)])
 def test_row_walk_of_short_streams(cuda, oracle_mod, w_kind, a, b, dtype, n_out, n_in, p):
-  # a lane to a stream: outputs that are not a multiple of 64, streams without a synapse, every index connected, streams that go on
-  # behind word 227 of the generator (1,500 x 0.04: 120 words with homogeneous weights, 273 with normal ones in double)
+  # a lane to a stream: outputs that are not a multiple of 64, streams without a synapse, every index connected (what is longer, with
+  # normal weights 140,000 rows of 60 and some others, goes by wave: test_row_walk_of_normal_weights_that_go_on_behind_the_first_words)
   rng = np.random.default_rng(n_out)
   ev, vec = rng.random(n_in) < 0.3, rng.uniform(0.5, 2.0, n_in).astype(dtype)
   oracle_mod.set_threads(min(16, len(os.sched_getaffinity(0))))
@@ -430,8 +430,8 @@ def test_sums_of_short_streams_with_infinities(cuda, oracle_mod):
 @pytest.mark.parametrize("n_out,n_in,p", [(900, 5001, 0.001), (30_000, 33_000, 0.0003), (3, 70_063, 1.0), (40, 70_063, 0.5),
                                           (17_000, 140_000, 0.0035), (2_200_000, 2100, 0.0001)])
 def test_column_walk_of_short_streams(cuda, oracle_mod, w_kind, a, b, dtype, n_out, n_in, p):
-  # a lane to a column: batches of 64 that do not come out even, one window and several, windows of more than 16 bits of
-  # positions, no bins at all (events with few pairs), several launches (140,000 columns), streams beyond word 227
+  # a lane to a column: batches of 64 that do not come out even, one window and several, no bins at all (events with few pairs);
+  # 2,100 columns of 220 are walked by waves, into windows of 15 bits
   rng = np.random.default_rng(n_out)
   ev, vec = rng.random(n_in) < 0.1, rng.uniform(0.5, 2.0, n_in).astype(dtype) * (rng.random(n_in) < 0.9)
   oracle_mod.set_threads(min(16, len(os.sched_getaffinity(0))))
@@ -468,6 +468,74 @@ def test_row_walk_of_streams_that_outlast_their_lane(cuda, oracle_mod, w_kind, m
   want = oracle_mod.jitconn_matvec(ones, dense=True, **kw)
   oracle_mod.set_threads(1)
   assert np.array_equal(kernel_call(ones, dense=True, **kw), want)
+
+
+@pytest.mark.parametrize("n_out,mean,dtype,most", [(1_000_000, 92.0, np.float32, 139), (1_000_000, 38.0, np.float64, 60)])
+def test_row_walk_of_normal_weights_that_go_on_behind_the_first_words(cuda, oracle_mod, n_out, mean, dtype, most):
+  # A synapse takes 3.27 words, in double 4.55: the streams go on behind word 227, where words are made of new words, and of those of
+  # 92 a few need more than the 454 that a lane can draw (139 synapses and more): their wave walks them.
+  n_in, p = 3000, mean / 3000
+  assert jitconn_by_lane("normal", np.dtype(dtype).itemsize, n_out, n_in, p, event_bytes=1)
+  assert jitconn_by_lane("normal", np.dtype(dtype).itemsize, n_out, n_in, p)
+  rng = np.random.default_rng(n_out)
+  oracle_mod.set_threads(min(16, len(os.sched_getaffinity(0))))
+  kw = dict(w_kind="normal", log_p=oracle_mod.log_p_of(p), seed=77, n_row=n_out, n_col=n_in, out_dtype=dtype)
+  counts = oracle_mod.jitconn_matvec(np.ones(n_in, bool), dense=False, w_a=1.0, w_b=0.0, **kw)  # (every weight is 1)
+  assert counts.max() >= most, counts.max()
+  for inp, dense in ((rng.random(n_in) < 0.5, False), (rng.uniform(0.5, 2.0, n_in).astype(dtype), True)):
+    want, mag = oracle_mod.jitconn_matvec(inp, dense=dense, return_abs=True, w_a=0.5, w_b=2.0, **kw)
+    got = kernel_call(inp, col_walk=False, dense=dense, w_a=0.5, w_b=2.0, **kw)
+    assert_close_reordered(got, want, mag, dtype, what="normal weights by lane")
+  oracle_mod.set_threads(1)
+
+
+@pytest.mark.parametrize("mean,dtype", [(80.0, np.float32), (30.0, np.float64)])
+def test_column_walk_of_normal_weights_that_go_on_behind_the_first_words(cuda, oracle_mod, mean, dtype):
+  n_in, n_out, p = 300_000, 20_000, mean / 20_000
+  assert jitconn_by_lane("normal", np.dtype(dtype).itemsize, n_in, n_out, p, use=1)
+  vec = np.random.default_rng(5).uniform(0.5, 2.0, n_in).astype(dtype)
+  oracle_mod.set_threads(min(16, len(os.sched_getaffinity(0))))
+  kw = dict(w_kind="normal", w_a=0.5, w_b=2.0, log_p=oracle_mod.log_p_of(p), seed=7, n_row=n_out, n_col=n_in, col_walk=True, dense=True)
+  want, mag = oracle_mod.jitconn_matvec(vec, return_abs=True, **kw)
+  oracle_mod.set_threads(1)
+  assert_close_reordered(kernel_call(vec, **kw), want, mag, dtype, what="columns with normal weights by lane")
+
+
+def test_column_walk_by_lane_in_several_launches(cuda, oracle_mod):
+  # 4.8e8 synapses are more than the bins hold (3 GiB at 6 bytes and a quarter to spare): the columns are walked in two launches by
+  # lane, with the bins emptied in between.  Whole numbers: every order of the additions gives the same sums.
+  n_in, n_out, p = 8_000_000, 5000, 60.0 / 5000
+  assert jitconn_by_lane("homo", 4, n_in, n_out, p, use=1) and n_in * 60.0 * 1.25 * 6 > 3 << 30
+  rng = np.random.default_rng(8)
+  vec = np.zeros(n_in, np.float32)
+  on = rng.choice(n_in, 40_000, replace=False)
+  vec[on] = rng.integers(1, 4, on.shape[0])
+  kw = dict(log_p=oracle_mod.log_p_of(p), n_row=n_out)
+  got = kernel_call(vec, w_kind="homo", seed=3, n_col=n_in, col_walk=True, dense=True, **kw)
+  want = np.zeros(n_out)
+  for c in on:
+    idx, _ = oracle_mod.jitconn_stream_weights(3 + int(c), "homo", 0.0, 0.0, kw["log_p"], n_out, dtype=np.float32)
+    want[idx] += vec[c]
+  assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("w_kind,mean", [("homo", 15.0), ("uniform", 12.0), ("normal", 11.0)])
+@pytest.mark.parametrize("rate", [0.004, 0.1, 0.6])
+def test_column_walk_of_events_by_lane_into_bins(cuda, oracle_mod, w_kind, mean, rate):
+  # a million columns have more than 1e7 synapses: bins, sized for an eighth of the columns (0.6: what finds them full goes to the
+  # output directly).  Normal weights of that length go by wave.
+  n_in, n_out, p = 1_000_000, 6007, mean / 6007
+  assert jitconn_by_lane(w_kind, 4, n_in, n_out, p, use=2) == (w_kind != "normal") and n_in * mean > 1e7
+  ev = np.random.default_rng(int(mean)).random(n_in) < rate
+  oracle_mod.set_threads(min(16, len(os.sched_getaffinity(0))))
+  kw = dict(w_kind=w_kind, w_a=0.25, w_b=1.75, log_p=oracle_mod.log_p_of(p), seed=7, n_row=n_out, n_col=n_in, col_walk=True, dense=False)
+  want, mag = oracle_mod.jitconn_matvec(ev, return_abs=True, **kw)
+  oracle_mod.set_threads(1)
+  got = kernel_call(ev, **kw)
+  if w_kind == "homo":
+    assert np.array_equal(got, want)
+  else:
+    assert_close_reordered(got, want, mag, np.float32, what="event columns by lane into bins")
 
 
 def test_matmat_of_more_tiles_than_a_launch_has_threads_for(cuda, oracle_mod):
@@ -814,10 +882,12 @@ def test_normal_weights_on_both_sides_of_the_bitmaps_and_skip_paths(cuda, oracle
                          what="normal weights, events")
 
 
+@pytest.mark.parametrize("mean", [70.0, 240.0])
 @pytest.mark.parametrize("w_kind,dtype,last", [("homo", np.float32, 268_288), ("uniform", np.float32, 235_520),
                                                ("uniform", np.float64, 219_136), ("normal", np.float32, 151_552),
                                                ("normal", np.float64, 90_112)])
-def test_row_walk_on_both_sides_of_the_exact_bitmaps(cuda, oracle_mod, w_kind, dtype, last):
+def test_row_walk_on_both_sides_of_the_exact_bitmaps(cuda, oracle_mod, w_kind, dtype, last, mean):
+  # (rows of 240 synapses are walked by waves, most of those of 70 by lanes, which have no bitmaps)
   # (outputs, inputs): exact bitmaps of up to 311,296 inputs where one workgroup a CU has all rows; two workgroups of
   # fewer waves; two turns of one; two 16-wave workgroups, up to `last` inputs (16,384 outputs: one)
   place = {"homo": 311_296, "uniform": 311_296, "normal": 151_552 if dtype == np.float32 else 153_600}[w_kind]
@@ -825,8 +895,9 @@ def test_row_walk_on_both_sides_of_the_exact_bitmaps(cuda, oracle_mod, w_kind, d
   for n_out, n_in in ((301, 311_296), (301, 311_297), (4_101, place), (4_101, place + 1), (6_000, place), (8_191, place),
                       (16_384, 311_296), (16_385, last), (16_385, last + 1)):
     ev = rng.random(n_in) < 0.2
-    kw = dict(w_kind=w_kind, w_a=0.5, w_b=2.0, log_p=oracle_mod.log_p_of(70.0 / n_in), seed=9, n_row=n_out, n_col=n_in)
+    kw = dict(w_kind=w_kind, w_a=0.5, w_b=2.0, log_p=oracle_mod.log_p_of(mean / n_in), seed=9, n_row=n_out, n_col=n_in)
     print("case", n_out, n_in, flush=True)
+    assert mean < 240 or not jitconn_by_lane(w_kind, np.dtype(dtype).itemsize, n_out, n_in, mean / n_in, event_bytes=1)
     want, mag = oracle_mod.jitconn_matvec(ev, dense=False, return_abs=True, out_dtype=dtype, **kw)
     got = kernel_call(ev, col_walk=False, dense=False, out_dtype=dtype, **kw)
     if w_kind == "homo":
@@ -886,15 +957,18 @@ def test_waves_that_do_not_wait_for_their_generators_write_their_rows_all_the_sa
     np.testing.assert_array_equal(out.cpu().numpy(), want)
 
 
-@pytest.mark.parametrize("n_out,per_row", [(33_001, 30), (60_000, 100), (81_921, 250), (135_000, 20)])
+@pytest.mark.parametrize("n_out,per_row", [(33_001, 30), (60_000, 100), (81_921, 250), (135_000, 20), (33_001, 240), (60_000, 240),
+                                           (135_000, 240)])
 def test_row_walk_whose_batches_are_shared_out_or_taken(cuda, oracle_mod, n_out, per_row):
   # two batches for some workgroups, seeded side by side and one after the other; taken from the counter from two and a
-  # half and from four batches a workgroup on
+  # half (rows of 200 synapses and more) and from four batches a workgroup on.  Rows of 240 and 250 are walked by waves, the shorter
+  # ones by lanes, but for 60,000 uniform ones of 100.
   n_in = 3000
   ev = np.random.default_rng(n_out).random(n_in) < 0.1
   kw = dict(log_p=oracle_mod.log_p_of(per_row / n_in), seed=5, n_row=n_out, n_col=n_in, w_a=0.25, w_b=1.75)
   print("case", n_out, per_row, flush=True)
   for w_kind in ("homo", "uniform"):
+    assert per_row < 240 or not jitconn_by_lane(w_kind, 4, n_out, n_in, per_row / n_in, event_bytes=1)
     want, mag = oracle_mod.jitconn_matvec(ev, w_kind=w_kind, dense=False, per_stream_seed=True, return_abs=True, **kw)
     for _ in range(3):
       got = kernel_call(ev, w_kind=w_kind, col_walk=False, dense=False, **kw)

@@ -10,6 +10,7 @@ import torch
 import brainpylib_amd as bpl
 from brainpylib_amd import _lib, sparse_ops
 import benchdata as synth
+from util import jitconn_by_lane
 
 pytestmark = pytest.mark.gpu
 
@@ -218,9 +219,10 @@ def test_matmat_is_captured_where_there_is_no_room_for_generator_states(cuda, ca
     assert torch.equal(out, want)
 
 
-def test_row_walk_is_captured_where_the_stream_has_rings_but_no_counters(cuda, capfd):
+@pytest.mark.parametrize("conn_prob", [0.005, 0.012])
+def test_row_walk_is_captured_where_the_stream_has_rings_but_no_counters(cuda, capfd, conn_prob):
   # more than four batches of streams for each of 512 workgroups, and no counter to take them from: they are shared out evenly, and the
-  # call, which succeeds, prints nothing
+  # call, which succeeds, prints nothing.  (Rows of 240 synapses; those of 100 are walked by lanes, which need neither.)
   rng = np.random.default_rng(3)
   handle = ctypes.c_void_p()  # (a stream of its own: torch's come from a pool and may have counters from elsewhere)
   assert ctypes.CDLL("libamdhip64.so").hipStreamCreate(ctypes.byref(handle)) == 0
@@ -233,7 +235,8 @@ def test_row_walk_is_captured_where_the_stream_has_rings_but_no_counters(cuda, c
   before = _query(s.cuda_stream)
   n_in = 20_000
   ev = torch.zeros(n_in, dtype=torch.bool, device=cuda)
-  kw = dict(weight=1.0, conn_prob=0.005, shape=(140_001, n_in), seed=5, outdim_parallel=True)
+  kw = dict(weight=1.0, conn_prob=conn_prob, shape=(140_001, n_in), seed=5, outdim_parallel=True)
+  assert jitconn_by_lane("homo", 4, 140_001, n_in, conn_prob, event_bytes=1) == (conn_prob < 0.01)
   bpl.event_matvec_prob_conn_homo_weight(ev, **kw)
   torch.cuda.synchronize()
   capfd.readouterr()
